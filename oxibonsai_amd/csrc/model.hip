@@ -71,6 +71,7 @@ struct Model {
     uint32_t pf_cap = 0;
     float *pf_hidden = nullptr, *pf_qkv = nullptr, *pf_attn = nullptr, *pf_gu = nullptr;
     std::vector<void*> pf_allocs;
+    DevBuf pf_part;     // the prefill attention's sums of runs of keys
     GemmWorkspace gws;  // GEMM scratch of the captured large-batch decode step: sized at creation, never moved
     DevBuf gpack;       // quantised activation vectors of the captured GEMV-based step (batches of two to eight): likewise
     DevBuf gpack_o;     // the O projection's quantised input where the attention kernel writes it itself; starts as zeros (= zero vectors) and
@@ -126,6 +127,7 @@ static void free_model(Model& m) {
     for (void* p : m.pf_allocs) (void)hipFree(p);
     m.pf_allocs.clear();
     m.pf_cap = 0;
+    m.pf_part.release();
     m.gws.release();
     m.gpack.release();
     m.gpack_o.release();
@@ -561,7 +563,9 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
         ap.hd = d.hd;
         ap.max_seq = d.max_seq;
         ap.scale = 1.0f / sqrtf((float)d.hd);
-        OXB_TRY_HIP(oxb_launch_attn_prefill(ap, st), "kernel launch failed: attn_prefill");
+        OXB_TRY(m.pf_part.ensure(oxb_attn_prefill_part_bytes(ap, g_rt.n_cus)));
+        ap.part = (float*)m.pf_part.ptr;
+        OXB_TRY_HIP(oxb_launch_attn_prefill(ap, g_rt.n_cus, st), "kernel launch failed: attn_prefill");
         OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f));
         // SwiGLU in the epilogue of the gate || up product: the activation [M][inter] is all that is written
         OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps));

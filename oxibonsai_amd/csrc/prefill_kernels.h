@@ -22,6 +22,13 @@ struct OxbPrefillAttnParams {
     uint32_t M, pos_start;            // query t sits at position pos_start + t and sees keys 0 .. pos_start + t
     uint32_t nq, nkv, hd, max_seq;
     float scale;                      // 1 / sqrt(hd)
+    float* part;                      // oxb_attn_prefill_part_bytes(...) of scratch where that is not 0: sums of the runs of keys
+    uint32_t blocks_per_split;        // key blocks of a run (filled by the launcher)
 };
 
-hipError_t oxb_launch_attn_prefill(const OxbPrefillAttnParams& p, hipStream_t st);
+// How the launcher cuts the work: q heads per workgroup, query tiles per wave, workgroups, runs of keys.
+struct OxbPrefillAttnPlan { uint32_t hpw, qt, wgs, n_splits, blocks_per_split; };
+#define OXB_PF_ATTN_MAX_SPLITS 32u
+
+size_t oxb_attn_prefill_part_bytes(const OxbPrefillAttnParams& p, uint32_t n_cus);
+hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipStream_t st);

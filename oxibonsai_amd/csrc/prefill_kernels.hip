@@ -20,78 +20,176 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // ---------------------------------------------------------------------------
 // Causal attention of M query tokens (positions pos_start .. pos_start + M - 1) over keys 0 .. own position
 // of one sequence, GQA, online softmax (semantics: block/functions.rs:78-127 -> layers/attention_fused.rs:329-400
-// applied per token).  One wave = 16 queries of one q head.
+// applied per token).  One wave = QT tiles of 16 queries of one q head.
 //
 // Both products run on v_mfma_f32_16x16x32_f16 in transposed form, so the score tile comes out with the
 // query in the lane (column) and needs no transposition before the second product:
 //   S^T[key][q]  = sum_d K[key][d] Q[q][d]      A = K rows (16 bytes per lane),
-//                                               B = Q * scale, split into fp16 hi + lo (two MFMAs: the
+//                                               B = Q * scale * log2 e, split into fp16 hi + lo (two MFMAs: the
 //                                               scores keep fp32-level accuracy)
-//   O^T[d][q]   += sum_key V[key][d] P[q][key]  B = the lane's own 8 probabilities of a 32-key block,
-//                                               A = V gathered for exactly those 8 keys
-// Lane (q = lane % 16, g = lane / 16) holds keys {4g..4g+3} and {16+4g..16+4g+3} of each 32-key block.
+//   O^T[d][q]   += sum_key V[key][d] P[q][key]  B = the lane's own 8 probabilities of 32 keys,
+//                                               A = V gathered for exactly those 8 keys (two transposing LDS reads)
+// Lane (q = lane % 16, g = lane / 16) holds keys {4g..4g+3} and {16+4g..16+4g+3} of every 32 keys.  The sum of the
+// probabilities is one more MFMA, against an operand of ones: it adds the same rounded values the numerator adds.
 //
 // The four waves of a workgroup walk the same keys and values: they take `hpw` q heads of ONE kv head (4, 2 or 1,
-// whatever divides the group) times 4 / hpw consecutive query tiles.  Each 32-key block of K and V is fetched once
-// per workgroup into LDS, double-buffered: while block i is being used, block i+1 waits in registers and is
-// written to the other buffer before the barrier that ends the block.  Waves of an earlier query tile see the
-// last block(s) fully masked.
-// ---------------------------------------------------------------------------
+// whatever divides the group) times 4 / hpw consecutive runs of QT query tiles.  Each block of KB keys (K and V) is
+// fetched once per workgroup into LDS, double-buffered: fp16 rows go there directly (global_load_lds), quantised rows
+// wait in registers and are widened on their way.  Rows are stored without padding, their 16-byte pieces permuted by an
+// XOR with the row number, which keeps both kinds of read free of bank conflicts.
+//
+// What bounds it: the SIMDs' issue slots.  With 16 queries per wave and 32-key blocks the kernel issued about 200 vector
+// instructions around 24 MFMAs per block (94 us per layer for 2048 tokens of the 8B shape, 201 us for 301 tokens behind
+// 6000 INT8 positions).  Two query tiles per wave halve the LDS reads per MFMA; a running maximum that is replaced only
+// when a score exceeds it by more than 8 (powers of two: the result does not depend on when) takes the rescaling of the
+// accumulators out of nearly every block; the visibility tests run only in blocks that some query of the wave sees in part:
+// 77 us and 76 us per layer for the two.
+//
 // Options as in the decode attention: quantised cache rows (template KVM; the codes are widened to exact fp16
 // numbers on their way into LDS, V already multiplied by its row scale there, the K row scale multiplies the
 // score) and a sliding window with attention sinks (key visible to the query at qpos iff key < sinks or
 // qpos - key < window - sinks; blocks no query of the workgroup can see are skipped).
-template <int HD, int KVM, bool OPT>  // OPT: a window and / or a paged cache may be in use (else neither costs anything)
-__global__ __launch_bounds__(256) void attn_prefill_kernel(OxbPrefillAttnParams p, uint32_t hpw) {
+//
+// Few queries behind a long cache leave most of the chip idle when a workgroup walks all keys: then blockIdx.y splits the
+// walk into runs of p.blocks_per_split blocks, each run leaves its un-normalised sums in p.part, and
+// attn_prefill_merge_kernel adds them in order.
+// ---------------------------------------------------------------------------
+// Keys per block: 64, or 32 where the LDS (4 x KB x 2 HD bytes) or the registers that hold a block of codes leave no room.
+constexpr int pf_block_keys(int hd, bool quantised) { return hd == 256 || (hd == 128 && quantised) ? 32 : 64; }
+
+template <int HD, int KVM, bool OPT, int QT>  // OPT: a window and / or a paged cache may be in use (else neither costs anything)
+__global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(OxbPrefillAttnParams p, uint32_t hpw) {
     constexpr bool QC = KVM != OXB_KV_F16;
-    constexpr int KS = HD / 32, NS = HD / 16;
-    constexpr int STR = HD + 8;                      // LDS row stride in fp16 (16 bytes of padding: conflict-free rows)
-    constexpr int PPR = QC ? HD / 16 : HD / 8;       // 16-byte pieces per cache row
-    constexpr int PIECES = 32 * PPR;                 // pieces of a 32-key block
-    constexpr int PP = (PIECES + 255) / 256;         // pieces per thread
-    __shared__ __attribute__((aligned(16))) _Float16 ks[2][32 * STR];
-    __shared__ __attribute__((aligned(16))) _Float16 vs[2][32 * STR];
-    __shared__ __attribute__((aligned(16))) float kscale[2][32];                // K row scales of the block (quantised cache)
+    constexpr int KS = HD / 32, NS = HD / 16, KB = pf_block_keys(HD, QC);
+    constexpr int RPW = KB / 4;                                      // rows of a block that a wave fetches
+    constexpr int PPR = HD / 8;                                      // 16-byte pieces of an LDS row
+    constexpr int RB = PPR >= 16 ? 1 : 16 / PPR, PM = (PPR < 16 ? PPR : 16) - 1;  // rows per 256 bytes; mask of the permutation
+    constexpr int NI = QC ? (RPW * HD / 16 + 63) / 64 : RPW * PPR / 64;  // 16-byte pieces per lane and block, of K and of V
+    constexpr float LAZY = 8.0f;
+    __shared__ __attribute__((aligned(16))) _Float16 ks0[KB * HD], ks1[KB * HD], vs0[KB * HD], vs1[KB * HD];
+    __shared__ __attribute__((aligned(16))) float kscale0[KB], kscale1[KB];  // K row scales of the block (quantised cache)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, qi = lane & 15u, g = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t n_qt = (p.M + 15u) / 16u, hq = p.nq / hpw, tpw = 4u / hpw, n_tg = (n_qt + tpw - 1) / tpw;
-    const uint32_t tg = n_tg - 1 - blockIdx.x / hq;                       // long (late) query tiles first
+    const uint32_t tpw = 4u / hpw, n_qt = (p.M + 15u) / 16u, per_wg = tpw * QT, n_tg = (n_qt + per_wg - 1) / per_wg, hq = p.nq / hpw;
+    // Late query tiles walk more keys than early ones.  Workgroups are handed out in order, one to a CU, then a second
+    // one to each: the first half of the tiles goes from the latest down, the second half from the earliest up, so that the
+    // longest walk shares its CU with the shortest.
+    const uint32_t tb = blockIdx.x / hq, tg = 2 * tb < n_tg ? n_tg - 1 - tb : tb - (n_tg + 1) / 2;
     const uint32_t head = (blockIdx.x % hq) * hpw + wave % hpw;
-    const uint32_t qt_own = tg * tpw + wave / hpw;
-    const bool active = qt_own < n_qt;                                    // a tile past the end: the wave only helps with the loads
-    const uint32_t qt = active ? qt_own : n_qt - 1;
     const uint32_t kvh = head / (p.nq / p.nkv);                           // the same for the four waves
-    const uint32_t t_q = min(qt * 16 + qi, p.M - 1);                      // rows past M repeat the last one and are not stored
-    const uint32_t qpos = p.pos_start + t_q;
-    const uint32_t kv_len = p.pos_start + min((tg * tpw + tpw - 1) * 16 + 15, p.M - 1) + 1;  // keys the workgroup's last query sees
-    typedef typename std::conditional<QC, uint8_t, _Float16>::type cache_t;
-    const cache_t* K = reinterpret_cast<const cache_t*>(p.k_cache);
-    const cache_t* V = reinterpret_cast<const cache_t*>(p.v_cache);
-    const float* Ksc = p.k_scale;
-    const float* Vsc = p.v_scale;
+    const uint32_t t_first = (tg * per_wg + (wave / hpw) * QT) * 16;      // first query of this wave
+    const uint32_t kv_len = p.pos_start + min((tg + 1) * per_wg * 16, p.M);  // keys the workgroup's last query sees
+    const uint32_t last = kv_len - 1;
+    uint32_t t_q[QT], qpos[QT];
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+        t_q[t] = min(t_first + t * 16 + qi, p.M - 1);                     // rows past M repeat the last one and are not stored
+        qpos[t] = p.pos_start + t_q[t];
+    }
+    const uint32_t q_lo = p.pos_start + min(t_first, p.M - 1), q_hi = p.pos_start + min(t_first + QT * 16 - 1, p.M - 1);
     const bool paged = OPT && p.kv.page_table != nullptr;
     const uint32_t window = OPT ? p.window : 0u;
     const size_t row0 = paged ? 0 : kv_row(p.kv, p.seq, p.layer, kvh, 0);
-    auto row_of = [&](uint32_t key) -> size_t { return paged ? kv_row(p.kv, p.seq, p.layer, kvh, key) : row0 + key; };
-    // sliding window: this query sees [0, sinks) and (qpos - budget, qpos]; the workgroup's earliest query sits at
-    // q_first, so no query of it sees a key in [sinks, q_first + 1 - budget): whole 32-key blocks in there are skipped
+    // sliding window: a query sees [0, sinks) and (qpos - budget, qpos]; the workgroup's earliest query sits at
+    // q_first, so no query of it sees a key in [sinks, q_first + 1 - budget): whole blocks in there are left out of the walk
     const uint32_t budget = window > p.sinks ? window - p.sinks : 0u;
-    const uint32_t q_first = p.pos_start + tg * tpw * 16;
-    const uint32_t skip_from = window ? (p.sinks + 31u) & ~31u : 0u;
-    const uint32_t skip_to = window && q_first + 1 > budget ? (q_first + 1 - budget) & ~31u : 0u;
-    auto next_block = [&](uint32_t key0) {  // the block after key0 that some query may see
-        key0 += 32;
-        return key0 >= skip_from && key0 < skip_to ? skip_to : key0;
-    };
+    const uint32_t q_first = p.pos_start + tg * per_wg * 16;
+    const uint32_t sink_blocks = window ? (p.sinks + KB - 1) / KB : 0u;
+    const uint32_t seen_from = window && q_first + 1 > budget ? (q_first + 1 - budget) / KB : 0u;
+    const uint32_t gap = seen_from > sink_blocks ? seen_from - sink_blocks : 0u;  // blocks left out behind the sinks
+    auto key_of = [&](uint32_t i) -> uint32_t { return (gap && i >= sink_blocks ? i + gap : i) * KB; };
+    const uint32_t n_blk = (last / KB + 1) - min(gap, last / KB + 1);
+    const uint32_t i0 = min(blockIdx.y * p.blocks_per_split, n_blk), i1 = blockIdx.y + 1 == gridDim.y ? n_blk : min(i0 + p.blocks_per_split, n_blk);
 
-    // Q of this lane's query: per-head RMSNorm, RoPE on the pairs (d, d + hd/2), times 1/sqrt(hd)
+    // ---- fetching: wave w takes rows w * RPW .. of a block; they lie in one page, so the base is uniform.  Rows past the
+    // last key repeat it (their scores are masked, their probabilities 0).
+    const uint8_t* const Kc = reinterpret_cast<const uint8_t*>(p.k_cache);
+    const uint8_t* const Vc = reinterpret_cast<const uint8_t*>(p.v_cache);
+    constexpr uint32_t ROWB = HD * (QC ? 1 : 2), SPR = ROWB / 16;  // bytes and 16-byte pieces of a cache row
+    // (worked out again for every block from an opaque copy of the lane: kept, they would cost the registers of a wave)
+    auto piece_of = [&](uint32_t l, int i, uint32_t& row, uint32_t& off) {
+        const uint32_t id = i * 64 + l;
+        row = id / SPR;
+        off = QC ? (id % SPR) * 16u : ((id % SPR) ^ (((wave * RPW + row) / RB) & PM)) * 16u;
+    };
+    const bool f_on = RPW * HD / 16 >= 64 || !QC || lane < RPW * HD / 16;  // (hd 32, quantised: half a wave holds all pieces)
+    auto group = [&](uint32_t key0, uint32_t& lim) -> size_t {
+        const uint32_t g0 = min(key0 + wave * RPW, last & ~(uint32_t)(RPW - 1));
+        lim = min((uint32_t)RPW - 1, last - g0);
+        return paged ? kv_row(p.kv, p.seq, p.layer, kvh, g0) : row0 + g0;
+    };
+    v4i kreg[QC ? NI : 1], vreg[QC ? NI : 1];
+    float vsreg[QC ? NI : 1], ksreg = 0.f;
+    auto request = [&](uint32_t key0, _Float16* kd, _Float16* vd) {
+        uint32_t lim;
+        const size_t row = group(key0, lim);
+        const uint8_t *kb = Kc + row * ROWB, *vb = Vc + row * ROWB;
+        uint32_t l = lane;
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            uint32_t f_row, f_off;
+            piece_of(l, i, f_row, f_off);
+            const uint32_t off = min(f_row, lim) * ROWB + f_off;
+            if constexpr (QC) {
+                if (f_on) {
+                    kreg[i] = *reinterpret_cast<const v4i*>(kb + off);
+                    vreg[i] = *reinterpret_cast<const v4i*>(vb + off);
+                    vsreg[i] = p.v_scale[row + min(f_row, lim)];
+                }
+            } else {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kb + off),
+                                                 (__attribute__((address_space(3))) void*)(kd + (wave * RPW * PPR + i * 64) * 8), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vb + off),
+                                                 (__attribute__((address_space(3))) void*)(vd + (wave * RPW * PPR + i * 64) * 8), 16, 0, 0);
+            }
+        }
+        if constexpr (QC) ksreg = p.k_scale[row + min(lane & (RPW - 1), lim)];
+    };
+    auto deliver = [&](_Float16* kd, _Float16* vd, float* scd) {
+        if constexpr (QC) {
+            uint32_t l = lane;
+            asm volatile("" : "+v"(l));
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                if (!f_on) continue;
+                uint32_t f_row, f_off;
+                piece_of(l, i, f_row, f_off);
+                uint32_t kw[8], vw[8];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    kv_dec4<KVM>((uint32_t)kreg[i][e], kw[2 * e], kw[2 * e + 1]);
+                    kv_dec4<KVM>((uint32_t)vreg[i][e], vw[2 * e], vw[2 * e + 1]);
+                }
+                // V leaves for LDS as code * scale in fp16 (the probabilities it meets are fp16 as well)
+                const _Float16 sc = (_Float16)vsreg[i];
+                const kvh2_t sc2 = {sc, sc};
+#pragma unroll
+                for (int e = 0; e < 8; e++) vw[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvh2_t, vw[e]) * sc2);
+                const uint32_t row = wave * RPW + f_row, x = (row / RB) & PM, c = f_off / 8u;  // the piece becomes LDS pieces c, c + 1
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const uint32_t at = (row * PPR + ((c + e) ^ x)) * 8;
+                    *reinterpret_cast<v4i*>(kd + at) = (v4i){(int)kw[4 * e], (int)kw[4 * e + 1], (int)kw[4 * e + 2], (int)kw[4 * e + 3]};
+                    *reinterpret_cast<v4i*>(vd + at) = (v4i){(int)vw[4 * e], (int)vw[4 * e + 1], (int)vw[4 * e + 2], (int)vw[4 * e + 3]};
+                }
+            }
+            if (lane < RPW) scd[wave * RPW + lane] = ksreg;
+        }
+        // the barrier that ends a block: every wave has read it, and the next one is complete in LDS
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    if (i0 < i1) request(key_of(i0), ks0, vs0);
+
+    // Q of this lane's queries: per-head RMSNorm, RoPE on the pairs (d, d + hd/2), times log2(e)/sqrt(hd)
     // (fused_qk_norm_rope, gpu_backend/cuda_attn_kernels.rs:160-226), then split into fp16 hi + lo.  The lane holds
     // elements 32 s + 8 g + e; for hd >= 64 both elements of a pair are its own (steps s and s + KS / 2), for hd = 32
     // the partner sits in lane g ^ 2.
-    v8h qh[KS], ql[KS];
-    {
+    v8h qh[QT][KS], ql[QT][KS];
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
         constexpr int half = HD / 2;
-        const float* qr = p.qkv + (size_t)t_q * p.qkv_stride + (size_t)head * HD + 8 * g;
+        const float* qr = p.qkv + (size_t)t_q[t] * p.qkv_stride + (size_t)head * HD + 8 * g;
         float x[KS][8], ss = 0.f;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
@@ -109,8 +207,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(OxbPrefillAttnParams 
         for (int s = 0; s < KS; s++)
 #pragma unroll
             for (int e = 0; e < 8; e++) x[s][e] = p.q_norm[32 * s + 8 * g + e] * x[s][e] * inv;
-        const float* cs = p.cos_t + (size_t)qpos * half;
-        const float* sn = p.sin_t + (size_t)qpos * half;
+        const float* cs = p.cos_t + (size_t)qpos[t] * half;
+        const float* sn = p.sin_t + (size_t)qpos[t] * half;
         float r[KS][8];
         if constexpr (KS >= 2) {
 #pragma unroll
@@ -131,185 +229,281 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(OxbPrefillAttnParams 
                 r[0][e] = g < 2 ? mine * c - other * sv : other * sv + mine * c;
             }
         }
+        const float mul = p.scale * 1.44269504088896340736f;
 #pragma unroll
         for (int s = 0; s < KS; s++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float v = r[s][e] * p.scale;
+                const float v = r[s][e] * mul;
                 const _Float16 hi = (_Float16)v;
-                qh[s][e] = hi;
-                ql[s][e] = (_Float16)(v - (float)hi);
+                qh[t][s][e] = hi;
+                ql[t][s][e] = (_Float16)(v - (float)hi);
             }
     }
-    v4f O[NS];
+    // reading: offset (in halves) of the K operand of step 0 in key tile 0 and of the V tile of dimensions 0..15 in keys
+    // 0..15.  Step s and dimension tile sl are an XOR with a constant away (32 s, 16 sl), the other key tiles whole multiples
+    // of 16 rows, where the permutation is the same.
+    const uint32_t k_at = (qi * PPR + (g ^ ((qi / RB) & PM))) * 8;
+    const uint32_t v_row = 4 * g + (qi >> 2), v_at = (v_row * PPR + (((qi >> 1) & 1u) ^ ((v_row / RB) & PM))) * 8 + (qi & 1u) * 4;
+    v8h ones;
 #pragma unroll
-    for (int i = 0; i < NS; i++) O[i] = (v4f){0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
+    for (int e = 0; e < 8; e++) ones[e] = (_Float16)1.0f;
 
-    // this thread's pieces of a block: piece id = i * 256 + tid -> row id / PPR, 16-byte column id % PPR;
-    // rows past the last key repeat it (their scores are masked, their probabilities 0)
-    v4i kreg[PP], vreg[PP];
-    float vsreg[PP], ksreg = 0.f;  // quantised cache: the V row scale of each piece, one K row scale (threads 0..31)
-    auto fetch = [&](uint32_t key0) {
+    v4f O[QT][NS], lsum[QT];
+    float m_ref[QT];
 #pragma unroll
-        for (int i = 0; i < PP; i++) {
-            const uint32_t id = i * 256 + tid;
-            if (PIECES % 256 == 0 || id < (uint32_t)PIECES) {
-                const uint32_t col = id % PPR;
-                const size_t row = row_of(min(key0 + id / PPR, kv_len - 1));
-                kreg[i] = *reinterpret_cast<const v4i*>(reinterpret_cast<const uint8_t*>(K + row * HD) + col * 16);
-                vreg[i] = *reinterpret_cast<const v4i*>(reinterpret_cast<const uint8_t*>(V + row * HD) + col * 16);
-                if constexpr (QC) vsreg[i] = Vsc[row];
-            }
-        }
-        if constexpr (QC)
-            if (tid < 32) ksreg = Ksc[row_of(min(key0 + tid, kv_len - 1))];
-    };
-    auto stash = [&](int buf) {
+    for (int t = 0; t < QT; t++) {
 #pragma unroll
-        for (int i = 0; i < PP; i++) {
-            const uint32_t id = i * 256 + tid;
-            if (PIECES % 256 == 0 || id < (uint32_t)PIECES) {
-                if constexpr (QC) {
-                    uint32_t kd[8], vd[8];
-                    kv_dec4<KVM>((uint32_t)kreg[i].x, kd[0], kd[1]);
-                    kv_dec4<KVM>((uint32_t)kreg[i].y, kd[2], kd[3]);
-                    kv_dec4<KVM>((uint32_t)kreg[i].z, kd[4], kd[5]);
-                    kv_dec4<KVM>((uint32_t)kreg[i].w, kd[6], kd[7]);
-                    kv_dec4<KVM>((uint32_t)vreg[i].x, vd[0], vd[1]);
-                    kv_dec4<KVM>((uint32_t)vreg[i].y, vd[2], vd[3]);
-                    kv_dec4<KVM>((uint32_t)vreg[i].z, vd[4], vd[5]);
-                    kv_dec4<KVM>((uint32_t)vreg[i].w, vd[6], vd[7]);
-                    // V leaves for LDS as code * scale in fp16 (the probabilities it meets are fp16 as well)
-                    const _Float16 sc = (_Float16)vsreg[i];
-                    const kvh2_t sc2 = {sc, sc};
+        for (int i = 0; i < NS; i++) O[t][i] = (v4f){0.f, 0.f, 0.f, 0.f};
+        lsum[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+        m_ref[t] = -INFINITY;
+    }
+    auto block = [&](const _Float16* kb, const _Float16* vb, const float* ksc, uint32_t blk_key0) {
+        uint32_t ka = k_at, va = v_at;
+        asm volatile("" : "+v"(ka), "+v"(va));  // (the XORs below stay in the loop: their results would cost 12 registers)
+        constexpr int NH = KB / 32, NV = QC && QT == 2 && NS >= 4 ? NS / 4 : NS / 2;  // (V operands read ahead: rows waiting in registers leave room for fewer)
+        // (where rows wait in registers there is no room to hold the requests' order: the compiler's own has no spills)
+        constexpr bool FENCE = !QC || QT == 1;
+        v8h K[2][KS];
+        auto read_k = [&](int hb) {
 #pragma unroll
-                    for (int e = 0; e < 8; e++) vd[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvh2_t, vd[e]) * sc2);
-                    _Float16* kd_ = &ks[buf][(id / PPR) * STR + (id % PPR) * 16];
-                    _Float16* vd_ = &vs[buf][(id / PPR) * STR + (id % PPR) * 16];
-                    *reinterpret_cast<v4i*>(kd_) = (v4i){(int)kd[0], (int)kd[1], (int)kd[2], (int)kd[3]};
-                    *reinterpret_cast<v4i*>(kd_ + 8) = (v4i){(int)kd[4], (int)kd[5], (int)kd[6], (int)kd[7]};
-                    *reinterpret_cast<v4i*>(vd_) = (v4i){(int)vd[0], (int)vd[1], (int)vd[2], (int)vd[3]};
-                    *reinterpret_cast<v4i*>(vd_ + 8) = (v4i){(int)vd[4], (int)vd[5], (int)vd[6], (int)vd[7]};
-                } else {
-                    *reinterpret_cast<v4i*>(&ks[buf][(id / PPR) * STR + (id % PPR) * 8]) = kreg[i];
-                    *reinterpret_cast<v4i*>(&vs[buf][(id / PPR) * STR + (id % PPR) * 8]) = vreg[i];
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++) K[kt][s] = *reinterpret_cast<const v8h*>(kb + (ka ^ (32u * s)) + (2 * hb + kt) * 16 * HD);
+        };
+        auto read_v = [&](int hb, int sl) -> v8h {
+            const _Float16* tile = vb + (va ^ (16u * sl)) + hb * 32 * HD;
+            const v4h_t t0 = lds_read_tr16(tile), t1 = lds_read_tr16(tile + 16 * HD);
+            return (v8h){t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
+        };
+        read_k(0);
+#pragma unroll
+        for (int hb = 0; hb < NH; hb++) {  // 32 keys at a time
+            const uint32_t key0 = blk_key0 + hb * 32;
+            if (hb && key0 > q_hi) continue;  // (wave-uniform) above the diagonal of every query of the wave
+            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);  // all K operands have been requested: their latency is paid once
+            v4f S[QT][2];
+#pragma unroll
+            for (int t = 0; t < QT; t++) S[t][0] = S[t][1] = (v4f){0.f, 0.f, 0.f, 0.f};
+            // four independent chains of products at a time
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int hl = 0; hl < 2; hl++)
+#pragma unroll
+                    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                        for (int t = 0; t < QT; t++)
+                            S[t][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(K[kt][s], hl ? ql[t][s] : qh[t][s], S[t][kt], 0, 0, 0);
+            // the next half's K and the first V operands travel while the probabilities are worked out
+            if (hb + 1 < NH) read_k(hb + 1);
+            v8h V[NV];
+#pragma unroll
+            for (int sl = 0; sl < NV; sl++) V[sl] = read_v(hb, sl);
+            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (QC) {
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++) {
+                    const float4 a = *reinterpret_cast<const float4*>(ksc + 16 * (2 * hb + kt) + 4 * g);
+#pragma unroll
+                    for (int t = 0; t < QT; t++) S[t][kt][0] *= a.x, S[t][kt][1] *= a.y, S[t][kt][2] *= a.z, S[t][kt][3] *= a.w;
                 }
             }
+            // (wave-uniform) every query of the wave sees all of these keys, or the tests run
+            const bool all = key0 + 31 <= q_lo && (!window || key0 + 32 <= p.sinks || q_hi - key0 < budget);
+            if (!all) {
+#pragma unroll
+                for (int t = 0; t < QT; t++)
+#pragma unroll
+                    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const uint32_t key = key0 + 16 * kt + 4 * g + v;
+                            const bool vis = key <= qpos[t] && (!window || key < p.sinks || qpos[t] - key < budget);
+                            S[t][kt][v] = vis ? S[t][kt][v] : -INFINITY;
+                        }
+            }
+            float mx[QT];
+            bool grow = false;
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                const float m0 = max_raw(max_raw(S[t][0][0], S[t][0][1]), max_raw(S[t][0][2], S[t][0][3]));
+                const float m1 = max_raw(max_raw(S[t][1][0], S[t][1][1]), max_raw(S[t][1][2], S[t][1][3]));
+                mx[t] = max_rows4_raw(max_raw(m0, m1));
+                grow |= mx[t] > m_ref[t] + LAZY;
+            }
+            if (__builtin_amdgcn_ballot_w64(grow)) {
+#pragma unroll
+                for (int t = 0; t < QT; t++) {
+                    // a whole number: the factors are powers of two and leave every bit of the sums as it is
+                    const float m_new = mx[t] > m_ref[t] ? ceilf(mx[t]) : m_ref[t];
+                    const float alpha = m_ref[t] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
+                    m_ref[t] = m_new;
+#pragma unroll
+                    for (int sl = 0; sl < NS; sl++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) O[t][sl][v] *= alpha;
+#pragma unroll
+                    for (int v = 0; v < 4; v++) lsum[t][v] *= alpha;
+                }
+            }
+            v8h P[QT];
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                // (a query that has seen nothing yet keeps its empty state: every probability 0)
+                const float m = m_ref[t] == -INFINITY ? 0.f : m_ref[t];
+#pragma unroll
+                for (int e = 0; e < 8; e++) P[t][e] = (_Float16)__builtin_amdgcn_exp2f(S[t][e >> 2][e & 3] - m);
+            }
+            v8h V2[NS - NV];
+#pragma unroll
+            for (int sl = NV; sl < NS; sl++) V2[sl - NV] = read_v(hb, sl);
+            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int sl = 0; sl < NS; sl++)
+#pragma unroll
+                for (int t = 0; t < QT; t++)
+                    O[t][sl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl < NV ? V[sl < NV ? sl : 0] : V2[sl < NV ? 0 : sl - NV], P[t], O[t][sl], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < QT; t++) lsum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, P[t], lsum[t], 0, 0, 0);
         }
-        if constexpr (QC)
-            if (tid < 32) kscale[buf][tid] = ksreg;
     };
-    fetch(0);
-    stash(0);
-    if (next_block(0) < kv_len) fetch(next_block(0));
-    __syncthreads();
-
-    int buf = 0;
-    for (uint32_t key0 = 0; key0 < kv_len;) {
-        const uint32_t key1 = next_block(key0), key2 = next_block(key1);
-        const _Float16* kb = ks[buf];
-        const _Float16* vb = vs[buf];
-        v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < KS; s++) {
-            const v8h k0 = *reinterpret_cast<const v8h*>(kb + qi * STR + 32 * s + 8 * g);
-            const v8h k1 = *reinterpret_cast<const v8h*>(kb + (16 + qi) * STR + 32 * s + 8 * g);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qh[s], s0, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, ql[s], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qh[s], s1, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, ql[s], s1, 0, 0, 0);
+    if (i0 < i1) {
+        deliver(ks0, vs0, kscale0);
+        for (uint32_t i = i0;;) {
+            if (i + 1 < i1) request(key_of(i + 1), ks1, vs1);
+            block(ks0, vs0, kscale0, key_of(i));
+            if (++i == i1) break;
+            deliver(ks1, vs1, kscale1);
+            if (i + 1 < i1) request(key_of(i + 1), ks0, vs0);
+            block(ks1, vs1, kscale1, key_of(i));
+            if (++i == i1) break;
+            deliver(ks0, vs0, kscale0);
         }
-        if constexpr (QC) {
-            const float4 a = *reinterpret_cast<const float4*>(&kscale[buf][4 * g]), b = *reinterpret_cast<const float4*>(&kscale[buf][16 + 4 * g]);
-            s0[0] *= a.x, s0[1] *= a.y, s0[2] *= a.z, s0[3] *= a.w;
-            s1[0] *= b.x, s1[1] *= b.y, s1[2] *= b.z, s1[3] *= b.w;
-        }
-        float sv[8];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const uint32_t ka = key0 + 4 * g + v, kb_ = ka + 16;
-            const bool va = ka <= qpos && (!window || ka < p.sinks || qpos - ka < budget);
-            const bool vb_ = kb_ <= qpos && (!window || kb_ < p.sinks || qpos - kb_ < budget);
-            sv[v] = va ? s0[v] : -INFINITY;
-            sv[4 + v] = vb_ ? s1[v] : -INFINITY;
-            mx = fmaxf(mx, fmaxf(sv[v], sv[4 + v]));
-        }
-        mx = max_rows4(mx);
-        // without a window key 0 is visible to every query, so the maximum is finite from the first block on; with
-        // one, a query may see nothing yet: it keeps its empty state (all probabilities 0)
-        const float m_new = fmaxf(m_run, mx);
-        const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = __expf(m_run - m_ref);  // 0 for the first block
-        float sum = 0.f;
-        v8h pb;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const float pe = __expf(sv[e] - m_ref);
-            sum += pe;
-            pb[e] = (_Float16)pe;
-        }
-        sum = sum_rows4(sum);
-        l_run = l_run * alpha + sum;
-        m_run = m_new;
-#pragma unroll
-        for (int sl = 0; sl < NS; sl++) {
-            // a[e] = V[4 g + e][16 sl + qi], a[4 + e] = V[16 + 4 g + e][16 sl + qi]: two transposing reads
-            const _Float16* tile = vb + (4 * g + (qi >> 2)) * STR + 16 * sl + 4 * (qi & 3u);
-            const v4h_t t0 = lds_read_tr16(tile), t1 = lds_read_tr16(tile + 16 * STR);
-            const v8h a = {t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
-#pragma unroll
-            for (int v = 0; v < 4; v++) O[sl][v] *= alpha;
-            O[sl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb, O[sl], 0, 0, 0);
-        }
-        // the next block goes into the other buffer (last read one block ago, before the previous barrier);
-        // the block after it is requested now
-        if (key1 < kv_len) {
-            stash(buf ^ 1);
-            if (key2 < kv_len) fetch(key2);
-        }
-        __syncthreads();
-        buf ^= 1;
-        key0 = key1;
     }
-    if (active && qt * 16 + qi < p.M) {
-        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
-        float* o = p.out + ((size_t)(qt * 16 + qi) * p.nq + head) * HD + 4 * g;
 #pragma unroll
-        for (int sl = 0; sl < NS; sl++)
-            *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[sl][0] * inv, O[sl][1] * inv, O[sl][2] * inv, O[sl][3] * inv);
+    for (int t = 0; t < QT; t++) {
+        const uint32_t tok = t_first + t * 16 + qi;
+        if (tok >= p.M) continue;
+        const float l = lsum[t][0];
+        if (gridDim.y == 1) {
+            const float inv = l > 0.f ? 1.0f / l : 0.f;
+            float* o = p.out + ((size_t)tok * p.nq + head) * HD + 4 * g;
+#pragma unroll
+            for (int sl = 0; sl < NS; sl++)
+                *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[t][sl][0] * inv, O[t][sl][1] * inv, O[t][sl][2] * inv, O[t][sl][3] * inv);
+        } else {
+            const size_t at = ((size_t)blockIdx.y * p.M + tok) * p.nq + head;
+            if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_ref[t], l);
+            if (!(l == 0.f)) {  // (an empty run is left out of the merge)
+                float* o = p.part + (size_t)gridDim.y * p.M * p.nq * 2 + at * HD + 4 * g;
+#pragma unroll
+                for (int sl = 0; sl < NS; sl++)
+                    *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[t][sl][0], O[t][sl][1], O[t][sl][2], O[t][sl][3]);
+            }
+        }
     }
 }
 
-hipError_t oxb_launch_attn_prefill(const OxbPrefillAttnParams& p, hipStream_t st) {
+// out[t][head] = the runs' sums brought to a common exponent, added in order, over the total of their probabilities.
+// A thread owns four dimensions.
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint32_t n_splits, uint32_t rows,
+                                                                  uint32_t hd4, float* __restrict__ out) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, row = i / hd4, c = i % hd4;
+    if (row >= rows) return;
+    const float2* ml = reinterpret_cast<const float2*>(part);
+    const float4* po = reinterpret_cast<const float4*>(part + (size_t)n_splits * rows * 2);
+    float m = -INFINITY;
+    for (uint32_t s = 0; s < n_splits; s++) {
+        const float2 v = ml[(size_t)s * rows + row];
+        m = v.y == 0.f ? m : fmaxf(m, v.x);
+    }
+    float l = 0.f;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t s = 0; s < n_splits; s++) {
+        const float2 v = ml[(size_t)s * rows + row];
+        if (v.y == 0.f) continue;
+        const float w = __builtin_amdgcn_exp2f(v.x - m);
+        const float4 o = po[((size_t)s * rows + row) * hd4 + c];
+        l = fmaf(v.y, w, l);
+        a.x = fmaf(o.x, w, a.x), a.y = fmaf(o.y, w, a.y), a.z = fmaf(o.z, w, a.z), a.w = fmaf(o.w, w, a.w);
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    reinterpret_cast<float4*>(out)[(size_t)row * hd4 + c] = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+}
+
+// Query tiles per wave and runs of keys.  Two tiles per wave where there are enough queries for both (from 49 on);
+// keys are split where a walk by one workgroup per tile would leave the chip idle: the cost of a plan is (rounds of
+// workgroups, two to a CU) x blocks of the longest run, 64 keys counting 1 us, and a split adds the merge: 6 us and the
+// partial sums' way to memory and back at 3 TB/s.
+static OxbPrefillAttnPlan plan_attn(const OxbPrefillAttnParams& p, uint32_t n_cus) {
+    const uint32_t G = p.nq / p.nkv, hpw = G % 4u == 0 ? 4u : (G % 2u == 0 ? 2u : 1u), KB = (uint32_t)pf_block_keys((int)p.hd, p.kv_mode != OXB_KV_F16);
+    const uint32_t qt = p.M > 48 && p.hd != 256 ? 2u : 1u, per_wg = (4u / hpw) * qt;
+    const uint32_t n_tg = ((p.M + 15u) / 16u + per_wg - 1) / per_wg, wgs = n_tg * (p.nq / hpw);
+    uint32_t keys = p.pos_start + p.M;
+    if (p.window) {  // sinks, window and the workgroup's own queries
+        const uint64_t seen = (uint64_t)p.sinks + p.window + per_wg * 16 + 2 * KB;
+        if (seen < keys) keys = (uint32_t)seen;
+    }
+    const uint32_t n_blk = (keys + KB - 1) / KB + (p.window ? 1 : 0);
+    OxbPrefillAttnPlan best = {hpw, qt, wgs, 1, n_blk};
+    float best_cost = 1e30f;
+    for (uint32_t s = 1; s <= OXB_PF_ATTN_MAX_SPLITS && s <= n_blk; s++) {
+        const uint32_t bps = (n_blk + s - 1) / s, used = (n_blk + bps - 1) / bps;
+        if (used != s) continue;
+        const uint32_t rounds = (uint32_t)(((uint64_t)wgs * s + 2 * n_cus - 1) / (2 * n_cus));
+        const float cost = (float)rounds * (float)(bps * KB) / 64.0f + (s > 1 ? 6.0f + 2.0f * (float)s * p.M * p.nq * p.hd * 4.0f / 3e6f : 0.f);
+        if (cost < best_cost) best_cost = cost, best.n_splits = s, best.blocks_per_split = bps;
+    }
+    return best;
+}
+
+size_t oxb_attn_prefill_part_bytes(const OxbPrefillAttnParams& p, uint32_t n_cus) {
+    const OxbPrefillAttnPlan pl = plan_attn(p, n_cus);
+    return pl.n_splits > 1 ? (size_t)pl.n_splits * p.M * p.nq * (p.hd + 2) * sizeof(float) : 0;
+}
+
+hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipStream_t st) {
     if (p.M == 0 || p.nq == 0 || p.nkv == 0 || p.nq % p.nkv || !p.qkv || !p.q_norm || !p.cos_t || !p.sin_t || p.pos_start + p.M > p.max_seq || p.kv_mode > OXB_KV_FP8_E4M3 ||
         (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale)) || (p.kv.page_table && (p.kv.page_shift < 4 || p.kv.page_shift > 7)))
         return hipErrorInvalidValue;
-    const uint32_t G = p.nq / p.nkv, hpw = G % 4u == 0 ? 4u : (G % 2u == 0 ? 2u : 1u), tpw = 4u / hpw;
-    const uint32_t n_qt = (p.M + 15u) / 16u, grid = ((n_qt + tpw - 1) / tpw) * (p.nq / hpw);
+    const OxbPrefillAttnPlan pl = plan_attn(p, n_cus);
+    if (pl.n_splits > 1 && !p.part) return hipErrorInvalidValue;
+    p.blocks_per_split = pl.blocks_per_split;
+    const dim3 grid(pl.wgs, pl.n_splits);
     const bool opt = p.window != 0 || p.kv.page_table != nullptr;
-    switch (p.hd) {
-#define OXB_PF_LAUNCH(HD_, KVM_)                                                                                     \
-    if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true>), dim3(grid), dim3(256), 0, st, p, hpw);        \
-    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false>), dim3(grid), dim3(256), 0, st, p, hpw);
-#define OXB_PF_CASE(HD_)                                           \
-    case HD_:                                                      \
-        if (p.kv_mode == OXB_KV_I8) {                              \
-            OXB_PF_LAUNCH(HD_, OXB_KV_I8)                          \
-        } else if (p.kv_mode == OXB_KV_FP8_E4M3) {                 \
-            OXB_PF_LAUNCH(HD_, OXB_KV_FP8_E4M3)                    \
-        } else {                                                   \
-            OXB_PF_LAUNCH(HD_, OXB_KV_F16)                         \
-        }                                                          \
+#define OXB_PF_LAUNCH(HD_, KVM_, QT_)                                                                                     \
+    if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, QT_>), grid, dim3(256), 0, st, p, pl.hpw);          \
+    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, QT_>), grid, dim3(256), 0, st, p, pl.hpw);
+#define OXB_PF_KVM(HD_, QT_)                                       \
+    if (p.kv_mode == OXB_KV_I8) {                                  \
+        OXB_PF_LAUNCH(HD_, OXB_KV_I8, QT_)                         \
+    } else if (p.kv_mode == OXB_KV_FP8_E4M3) {                     \
+        OXB_PF_LAUNCH(HD_, OXB_KV_FP8_E4M3, QT_)                   \
+    } else {                                                       \
+        OXB_PF_LAUNCH(HD_, OXB_KV_F16, QT_)                        \
+    }
+#define OXB_PF_CASE(HD_)               \
+    case HD_:                          \
+        if (pl.qt == 2) {              \
+            OXB_PF_KVM(HD_, 2)         \
+        } else {                       \
+            OXB_PF_KVM(HD_, 1)         \
+        }                              \
         break;
+    switch (p.hd) {
         OXB_PF_CASE(32)
         OXB_PF_CASE(64)
         OXB_PF_CASE(128)
-        OXB_PF_CASE(256)
-#undef OXB_PF_LAUNCH
-#undef OXB_PF_CASE
+        case 256: OXB_PF_KVM(256, 1) break;
         default: return hipErrorInvalidValue;
     }
+#undef OXB_PF_LAUNCH
+#undef OXB_PF_KVM
+#undef OXB_PF_CASE
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || pl.n_splits == 1) return e;
+    const uint32_t rows = p.M * p.nq, hd4 = p.hd / 4;
+    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((uint32_t)(((uint64_t)rows * hd4 + 255) / 256)), dim3(256), 0, st, p.part, pl.n_splits, rows, hd4, p.out);
     return hipGetLastError();
 }
