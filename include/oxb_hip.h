@@ -298,6 +298,13 @@ int  oxb_hip_sample_logits(const float* logits, uint32_t vocab, uint32_t batch, 
 int  oxb_hip_prefill_tokens(uint64_t model, uint64_t embedding, uint32_t seq, const uint32_t* ids, uint32_t n_tokens,
                             uint32_t pos_start, float* logits_or_null, uint32_t* token_out_or_null);
 
+/* ---- pinned host memory for results (no counterpart in the reference): a host output buffer that lies in such a block is
+ * written by the device itself, without a copy through the library's staging.  Any host output parameter above may point
+ * into one; freed blocks are kept for reuse up to 128 MiB, and at most 512 MiB are handed out at a time
+ * (OXB_HIP_OUT_OF_MEMORY beyond: use ordinary memory).  Safe from any thread. */
+int  oxb_hip_host_alloc(void** p, size_t n_bytes);
+int  oxb_hip_host_free(void* p);
+
 /* ---- host-only helpers (no GPU needed): the upload-time repack, exposed so it can be checked on any machine.
  * reformat_q1_aos_to_soa / reformat_tq2_blocks_to_soa (KG/cuda_graph/cudagraph_reformat_*_group.rs). */
 int  oxb_hip_repack_sizes(int fmt, uint32_t n_rows, uint32_t k, size_t* codes_bytes, size_t* scales_bytes);

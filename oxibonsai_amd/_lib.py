@@ -33,12 +33,12 @@ _SIGNATURES = {
     "oxb_hip_free_weight": ([C.c_uint64], C.c_int),
     "oxb_hip_weight_info": ([C.c_uint64, C.POINTER(C.c_int), u32p, u32p, szp], C.c_int),
     "oxb_hip_dequant": ([C.c_uint64, f32p, C.c_size_t], C.c_int),
-    "oxb_hip_gemv": ([C.c_uint64, f32p, f32p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
+    "oxb_hip_gemv": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_gemv_dev": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_profile_gemv": ([u64p, C.c_uint32, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32,
                               C.c_uint32, f32p], C.c_int),
     "oxb_hip_profile_gemv_floor": ([u64p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, f32p], C.c_int),
-    "oxb_hip_gemm": ([C.c_uint64, f32p, f32p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
+    "oxb_hip_gemm": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_gemm_dev": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_gemm_dev_static": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_profile_gemm": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32,
@@ -53,7 +53,7 @@ _SIGNATURES = {
     "oxb_hip_model_create": ([C.c_void_p, u64p], C.c_int),
     "oxb_hip_model_reset": ([C.c_uint64], C.c_int),
     "oxb_hip_model_destroy": ([C.c_uint64], C.c_int),
-    "oxb_hip_decode": ([C.c_uint64, f32p, u32p, f32p, u32p], C.c_int),
+    "oxb_hip_decode": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "oxb_hip_decode_hidden": ([C.c_uint64, f32p, u32p, f32p], C.c_int),
     "oxb_hip_model_set_lm_head": ([C.c_uint64, C.c_uint64, C.c_uint64, C.c_uint32], C.c_int),
     "oxb_hip_model_set_rope_rows": ([C.c_uint64, C.c_uint32, C.c_uint32, f32p, f32p], C.c_int),
@@ -82,6 +82,8 @@ _SIGNATURES = {
     "oxb_hip_sum_in_order": ([f32p, C.c_uint32, f32p], C.c_int),
     "oxb_hip_set_gemv_packed_min_batch": ([C.c_uint32], C.c_int),
     "oxb_hip_prefill_tokens": ([C.c_uint64, C.c_uint64, C.c_uint32, u32p, C.c_uint32, C.c_uint32, f32p, u32p], C.c_int),
+    "oxb_hip_host_alloc": ([C.POINTER(C.c_void_p), C.c_size_t], C.c_int),
+    "oxb_hip_host_free": ([C.c_void_p], C.c_int),
     "oxb_hip_repack_sizes": ([C.c_int, C.c_uint32, C.c_uint32, szp, szp], C.c_int),
     "oxb_hip_repack": ([C.c_int, u8p, C.c_size_t, C.c_uint32, C.c_uint32, u8p, C.c_size_t, u8p, C.c_size_t], C.c_int),
     "oxb_hip_unpack": ([C.c_int, u8p, C.c_size_t, u8p, C.c_size_t, C.c_uint32, C.c_uint32, u8p, C.c_size_t], C.c_int),

@@ -1,0 +1,255 @@
+// host_io.hip — host buffers to the device and back.
+//
+// A caller's buffers are ordinary pageable memory.  hipMemcpyAsync on such memory goes through the runtime's own staging
+// or pins the pages for the transfer: 14 / 22 us for 4 KB in / out, 110 us for 256 KB, 18 GB/s out of the device for
+// large results.  Here every transfer goes through pinned memory that the library keeps - a host copy runs at 80 GB/s out
+// of the caches, faster than the 56 GB/s of the bus - and is made by a small kernel in the caller's stream, so no copy
+// engine has to be synchronised with it.  The last transfer of a call raises a flag in pinned memory that the host polls:
+// three dependent launches and a poll take 12.6 us where the same three and hipStreamSynchronize take 18.
+#include <hip/hip_runtime.h>
+
+#include <chrono>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "../../include/oxb_hip.h"
+#include "host_io.h"
+#include "runtime_internal.h"
+
+// 64 workgroups move a large buffer at the rate of the bus; with more of them the fences in front of the flag cost
+// more than they gain (1.2 MB out: 34 us with 64 workgroups, 50 with 256).
+#define OXB_IO_GRID 64u
+
+// Pieces of 16 bytes (4, where a buffer lies otherwise), then what is left byte by byte.  With `flag`: the workgroup that finishes last stores seq there once every
+// workgroup's part is visible to the host; *arrived is 0 before and after.
+template <typename T>
+__global__ __launch_bounds__(256) void io_copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t bytes,
+                                                       uint32_t* arrived, uint32_t* flag, uint32_t seq) {
+    const size_t n = bytes / sizeof(T), step = (size_t)gridDim.x * 256;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step)
+        reinterpret_cast<T*>(dst)[i] = reinterpret_cast<const T*>(src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < bytes % sizeof(T)) dst[n * sizeof(T) + threadIdx.x] = src[n * sizeof(T) + threadIdx.x];
+    if (!flag) return;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (before == gridDim.x - 1) {
+            *arrived = 0;
+            __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
+namespace oxb {
+namespace {
+
+constexpr size_t kChunk = (size_t)1 << 20;      // host copy of one piece while the bus moves the one before
+constexpr size_t kStaging = (size_t)32 << 20;   // per direction; larger buffers take turns in it
+constexpr size_t kPoolOut = (size_t)512 << 20;  // result memory handed out at a time
+constexpr size_t kPoolFree = (size_t)128 << 20; // ... and kept for reuse
+constexpr uint32_t kSyncEvery = 256;            // calls after which the stream is synchronised all the same (the runtime retires its commands there)
+
+struct Io {
+    uint8_t *in = nullptr, *out = nullptr;
+    size_t in_cap = 0, out_cap = 0, in_used = 0, out_used = 0;
+    uint32_t *flag = nullptr, *arrived = nullptr, seq = 0, seq_begin = 0, calls = 0;
+    bool open = false;  // something may still be reading or writing the staging buffers
+    struct Late { void* dst; size_t at, bytes; uint32_t seq; };
+    std::vector<Late> late;  // results that wait in staging for the device
+} io;
+
+int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two up to kStaging; nothing is in flight
+    if (want > kStaging) want = kStaging;
+    if (*cap >= want) return OXB_HIP_OK;
+    size_t n = (size_t)256 << 10;
+    while (n < want) n *= 2;
+    if (*p) (void)hipHostFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    if (hipHostMalloc((void**)p, n, hipHostMallocCoherent) != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+        return fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: pinned staging of %zu bytes", n);
+    }
+    *cap = n;
+    return OXB_HIP_OK;
+}
+
+int ensure_flag() {
+    if (io.flag) return OXB_HIP_OK;
+    if (hipHostMalloc((void**)&io.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&io.arrived, 4) != hipSuccess ||
+        hipMemset(io.arrived, 0, 4) != hipSuccess) {
+        (void)hipGetLastError();
+        if (io.flag) (void)hipHostFree(io.flag);
+        io.flag = nullptr;
+        return fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: completion flag");
+    }
+    *io.flag = io.seq;
+    return OXB_HIP_OK;
+}
+
+int copy(const void* src, void* dst, size_t bytes, uint32_t* flag, uint32_t seq) {
+    const size_t wgs = (bytes / 16 + 255) / 256;
+    const uint32_t grid = wgs < 1 ? 1u : wgs < OXB_IO_GRID ? (uint32_t)wgs : OXB_IO_GRID;
+    const uintptr_t at = (uintptr_t)src | (uintptr_t)dst;
+    if (at & 3) return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: a buffer of %zu bytes is not aligned to 4", bytes);
+    if (at & 15) hipLaunchKernelGGL(io_copy_kernel<uint32_t>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, io.arrived, flag, seq);
+    else hipLaunchKernelGGL(io_copy_kernel<uint4>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, io.arrived, flag, seq);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? OXB_HIP_OK : hip_fail(e, "kernel launch failed: io_copy");
+}
+
+int sync_all(const char* what) {
+    const hipError_t e = hipStreamSynchronize(g_rt.stream);
+    return e == hipSuccess ? OXB_HIP_OK : fail(OXB_HIP_SYNC_FAILED, "device synchronization failed: %s: %s", what, hipGetErrorString(e));
+}
+
+// Polls for a few milliseconds; a longer wait (or a stream in error, which never raises the flag) is the runtime's.
+int wait_for(uint32_t seq, const char* what) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t n = 1; (int32_t)(__atomic_load_n(io.flag, __ATOMIC_ACQUIRE) - seq) < 0; n++) {
+        __builtin_ia32_pause();
+        if ((n & 1023u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(4)) return sync_all(what);
+    }
+    return OXB_HIP_OK;
+}
+
+struct Pool {
+    std::mutex mu;
+    std::map<const uint8_t*, size_t> out;              // handed out: start -> size
+    std::multimap<size_t, uint8_t*> free_blocks;       // kept: size -> start
+    size_t out_bytes = 0, free_bytes = 0;
+} pool;
+
+bool is_pinned(const void* p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(pool.mu);
+    auto it = pool.out.upper_bound((const uint8_t*)p);
+    if (it == pool.out.begin()) return false;
+    --it;
+    return (const uint8_t*)p + bytes <= it->first + it->second;
+}
+
+}  // namespace
+
+int io_begin() {
+    int rc = ensure_flag();
+    if (rc) return rc;
+    if (io.open) {  // the call before ended in an error: whatever it left may still use the staging buffers
+        (void)hipDeviceSynchronize();
+        (void)hipMemset(io.arrived, 0, 4);
+    }
+    io.open = true;
+    io.in_used = io.out_used = 0;
+    io.seq_begin = io.seq;
+    io.late.clear();
+    return OXB_HIP_OK;
+}
+
+int io_upload(void* d_dst, const void* src, size_t bytes) {
+    const uint8_t* s = (const uint8_t*)src;
+    uint8_t* d = (uint8_t*)d_dst;
+    if (((uintptr_t)s & 15) == 0 && is_pinned(s, bytes)) return copy(s, d, bytes, nullptr, 0);
+    int rc;
+    if (io.in_used == 0 && (rc = staging(&io.in, &io.in_cap, bytes))) return rc;
+    while (bytes) {
+        const size_t n = bytes < kChunk ? bytes : kChunk;
+        if (io.in_used + n > io.in_cap) {  // every piece has been used once: wait for the device to be done with them
+            if ((rc = sync_all("input upload"))) return rc;
+            io.in_used = 0;
+            if ((rc = staging(&io.in, &io.in_cap, bytes))) return rc;
+        }
+        memcpy(io.in + io.in_used, s, n);
+        if ((rc = copy(io.in + io.in_used, d, n, nullptr, 0))) return rc;
+        io.in_used += (n + 255) & ~(size_t)255;
+        s += n, d += n, bytes -= n;
+    }
+    return OXB_HIP_OK;
+}
+
+int io_download(void* dst, const void* d_src, size_t bytes) {
+    if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, io.flag, ++io.seq);
+    int rc;
+    if (io.out_used == 0 && (rc = staging(&io.out, &io.out_cap, bytes))) return rc;
+    uint8_t* d = (uint8_t*)dst;
+    const uint8_t* s = (const uint8_t*)d_src;
+    while (bytes) {
+        const size_t n = bytes < kChunk ? bytes : kChunk;
+        if (io.out_used + n > io.out_cap) {  // staging is full of results: hand them over first
+            if ((rc = sync_all("output download"))) return rc;
+            for (const Io::Late& l : io.late) memcpy(l.dst, io.out + l.at, l.bytes);
+            io.late.clear();
+            io.out_used = 0;
+            if ((rc = staging(&io.out, &io.out_cap, bytes))) return rc;
+        }
+        if ((rc = copy(s, io.out + io.out_used, n, io.flag, ++io.seq))) return rc;
+        io.late.push_back({d, io.out_used, n, io.seq});
+        io.out_used += (n + 255) & ~(size_t)255;
+        s += n, d += n, bytes -= n;
+    }
+    return OXB_HIP_OK;
+}
+
+int io_finish(const char* what) {
+    int rc;
+    if (io.seq == io.seq_begin && (rc = sync_all(what))) return rc;  // nothing came back
+    for (const Io::Late& l : io.late) {  // one piece is copied on the host while the next ones cross the bus
+        if ((rc = wait_for(l.seq, what))) return rc;
+        memcpy(l.dst, io.out + l.at, l.bytes);
+    }
+    io.late.clear();
+    if ((rc = wait_for(io.seq, what))) return rc;
+    if (++io.calls % kSyncEvery == 0 && (rc = sync_all(what))) return rc;
+    io.open = false;
+    return OXB_HIP_OK;
+}
+
+void* pinned_alloc(size_t bytes) {
+    const size_t unit = bytes < kChunk ? (size_t)64 << 10 : kChunk, n = (bytes + unit - 1) / unit * unit;
+    std::lock_guard<std::mutex> lk(pool.mu);
+    uint8_t* p = nullptr;
+    auto it = pool.free_blocks.find(n);
+    if (it != pool.free_blocks.end()) {
+        p = it->second;
+        pool.free_blocks.erase(it);
+        pool.free_bytes -= n;
+    } else if (!bytes || pool.out_bytes + n > kPoolOut || hipHostMalloc((void**)&p, n, hipHostMallocCoherent) != hipSuccess) {
+        if (bytes) (void)hipGetLastError();
+        return nullptr;
+    }
+    pool.out[p] = n;
+    pool.out_bytes += n;
+    return p;
+}
+
+bool pinned_free(void* p) {
+    std::lock_guard<std::mutex> lk(pool.mu);
+    auto it = pool.out.find((const uint8_t*)p);
+    if (it == pool.out.end()) return false;
+    const size_t n = it->second;
+    pool.out.erase(it);
+    pool.out_bytes -= n;
+    if (pool.free_bytes + n > kPoolFree) {
+        (void)hipHostFree(p);
+    } else {
+        pool.free_blocks.emplace(n, (uint8_t*)p);
+        pool.free_bytes += n;
+    }
+    return true;
+}
+
+void io_shutdown() {  // results that a caller still holds stay
+    if (io.in) (void)hipHostFree(io.in);
+    if (io.out) (void)hipHostFree(io.out);
+    if (io.flag) (void)hipHostFree(io.flag);
+    if (io.arrived) (void)hipFree(io.arrived);
+    io = Io();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    for (auto& b : pool.free_blocks) (void)hipHostFree(b.second);
+    pool.free_blocks.clear();
+    pool.free_bytes = 0;
+}
+
+}  // namespace oxb

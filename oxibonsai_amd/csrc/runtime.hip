@@ -19,6 +19,7 @@
 #include "../../include/oxb_hip_measure.h"
 #include "gemm_kernels.h"
 #include "gemv_kernels.h"
+#include "host_io.h"
 #include "layout.h"
 #include "repack.h"
 #include "runtime_internal.h"
@@ -404,6 +405,7 @@ void oxb_hip_shutdown(void) {
     g_rt.weights.clear();
     for (auto& kv : g_rt.vectors) (void)hipFree(kv.second.d);
     g_rt.vectors.clear();
+    io_shutdown();
     g_rt.ws_x.release();
     g_rt.ws_y.release();
     g_rt.ws_aux.release();
@@ -518,11 +520,11 @@ int oxb_hip_dequant(uint64_t id, float* out, size_t out_len) {
     if (!out || out_len < n) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: output holds %zu values, %zu needed", out_len, n);
     int rc = g_rt.ws_y.ensure(n * sizeof(float));
     if (rc) return rc;
+    if ((rc = io_begin())) return rc;
     hipError_t e = oxb_launch_dequant(w->L, w->d_codes, w->d_scales, (float*)g_rt.ws_y.ptr, g_rt.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch failed: dequant");
-    e = hipMemcpyAsync(out, g_rt.ws_y.ptr, n * sizeof(float), hipMemcpyDeviceToHost, g_rt.stream);
-    if (e != hipSuccess) return hip_fail(e, "dequant download");
-    return sync_stream("dequant");
+    if ((rc = io_download(out, g_rt.ws_y.ptr, n * sizeof(float)))) return rc;
+    return io_finish("dequant");
     OXB_API_END
 }
 
@@ -683,13 +685,11 @@ int oxb_hip_gemm(uint64_t id, const float* x, float* y, uint32_t m, uint32_t n_r
     const size_t xb = (size_t)m * k * sizeof(float), yb = (size_t)m * n_rows * sizeof(float);
     if ((rc = g_rt.ws_x.ensure(xb))) return rc;
     if ((rc = g_rt.ws_y.ensure(yb))) return rc;
-    hipError_t e = hipMemcpyAsync(g_rt.ws_x.ptr, x, xb, hipMemcpyHostToDevice, g_rt.stream);
-    if (e != hipSuccess) return hip_fail(e, "input upload");
+    if ((rc = io_begin()) || (rc = io_upload(g_rt.ws_x.ptr, x, xb))) return rc;
     rc = gemm_device(*w, (const float*)g_rt.ws_x.ptr, k, (float*)g_rt.ws_y.ptr, m, n_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_IDENT, nullptr, 0.f);
     if (rc) return rc;
-    e = hipMemcpyAsync(y, g_rt.ws_y.ptr, yb, hipMemcpyDeviceToHost, g_rt.stream);
-    if (e != hipSuccess) return hip_fail(e, "output download");
-    return sync_stream("gemm");
+    if ((rc = io_download(y, g_rt.ws_y.ptr, yb))) return rc;
+    return io_finish("gemm");
     OXB_API_END
 }
 
@@ -757,13 +757,11 @@ int oxb_hip_gemv(uint64_t id, const float* x, float* y, uint32_t n_rows, uint32_
     const size_t xb = (size_t)batch * k * sizeof(float), yb = (size_t)batch * n_rows * sizeof(float);
     if ((rc = g_rt.ws_x.ensure(xb))) return rc;
     if ((rc = g_rt.ws_y.ensure(yb))) return rc;
-    hipError_t e = hipMemcpyAsync(g_rt.ws_x.ptr, x, xb, hipMemcpyHostToDevice, g_rt.stream);
-    if (e != hipSuccess) return hip_fail(e, "input upload");
+    if ((rc = io_begin()) || (rc = io_upload(g_rt.ws_x.ptr, x, xb))) return rc;
     rc = gemv_device(*w, (const float*)g_rt.ws_x.ptr, (float*)g_rt.ws_y.ptr, batch, n_rows, OXB_GEMV_STORE, nullptr);
     if (rc) return rc;
-    e = hipMemcpyAsync(y, g_rt.ws_y.ptr, yb, hipMemcpyDeviceToHost, g_rt.stream);
-    if (e != hipSuccess) return hip_fail(e, "output download");
-    return sync_stream("gemv");
+    if ((rc = io_download(y, g_rt.ws_y.ptr, yb))) return rc;
+    return io_finish("gemv");
     OXB_API_END
 }
 
@@ -780,6 +778,26 @@ int oxb_hip_gemv_tq2_g128(const uint8_t* aos, size_t n_bytes, const float* x, si
     OXB_API_BEGIN
     std::lock_guard<std::recursive_mutex> lk(g_mu);
     return oneshot_gemv(OXB_FMT_TQ2, aos, n_bytes, x, x_len, y, y_len, n_rows, k);
+    OXB_API_END
+}
+
+int oxb_hip_host_alloc(void** p, size_t n_bytes) {
+    OXB_API_BEGIN
+    if (!p) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: null pointer");
+    *p = nullptr;
+    {
+        std::lock_guard<std::recursive_mutex> lk(g_mu);
+        int rc = ensure_init();
+        if (rc) return rc;
+    }
+    *p = pinned_alloc(n_bytes);
+    return *p ? OXB_HIP_OK : fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: %zu bytes of pinned result memory", n_bytes);
+    OXB_API_END
+}
+
+int oxb_hip_host_free(void* p) {
+    OXB_API_BEGIN
+    return pinned_free(p) ? OXB_HIP_OK : fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: not a block of oxb_hip_host_alloc");
     OXB_API_END
 }
 

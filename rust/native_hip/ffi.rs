@@ -182,6 +182,9 @@ extern "C" {
                                  tokens_out: *mut u32) -> c_int;
     pub fn oxb_hip_prefill_tokens(model: u64, embedding: u64, seq: u32, ids: *const u32, n_tokens: u32, pos_start: u32,
                                   logits_or_null: *mut f32, token_out_or_null: *mut u32) -> c_int;
+    // pinned host memory for results
+    pub fn oxb_hip_host_alloc(p: *mut *mut c_void, n_bytes: usize) -> c_int;
+    pub fn oxb_hip_host_free(p: *mut c_void) -> c_int;
     // host-only repack helpers
     pub fn oxb_hip_repack_sizes(fmt: c_int, n_rows: u32, k: u32, codes_bytes: *mut usize, scales_bytes: *mut usize) -> c_int;
     pub fn oxb_hip_repack(fmt: c_int, aos: *const u8, n_bytes: usize, n_rows: u32, k: u32, codes: *mut u8, codes_cap: usize,
