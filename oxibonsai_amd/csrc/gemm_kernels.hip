@@ -35,18 +35,35 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 // Activation packer, fused with the row-wise producer of the activations:
 //   OXB_PACK_IDENT   a[m][k] = x[m][k]
 //   OXB_PACK_RMSNORM a[m][k] = w[k] * x[m][k] / sqrt(mean_k x[m][k]^2 + eps)      (simd_float_ops.rs:204-215)
-// Two kernels: row_stats (one workgroup per token row) finds the row's multiplier - the producer's scalar
-// times the power of two that puts the row's largest |a| into [2^14, 2^15) - and the exponent that undoes the
-// power of two; xh_pack (one workgroup = 16 token rows x a share of the blocks) recomputes a from x and writes
-// fp16 in MFMA B-operand order.  The normalised activations never go to memory in fp32.  (SwiGLU is not a packer
-// operation: the gate || up GEMM applies it in its epilogue, simd_float_ops.rs:217-236.)  A few token rows (decode batches)
-// take both steps in one launch, xh_pack_rows, one workgroup per row.
+// Two steps: the row's multiplier - the producer's scalar times the power of two that puts the row's largest |a| into
+// [2^14, 2^15) - with the exponent that undoes the power of two; then the fp16 values in MFMA B-operand order.  The
+// normalised activations never go to memory in fp32.  (SwiGLU is not a packer operation: the gate || up GEMM applies it in
+// its epilogue, simd_float_ops.rs:217-236.)  Both steps take one launch: xh_pack_rows, one workgroup per row, for up to
+// OXB_PACK_ROWS_MAX rows, xh_pack_wide beyond.  Rows too long for either to hold in registers take row_stats (one workgroup
+// per token row) and xh_pack (one workgroup = 16 token rows x a share of the blocks), which read x twice.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     const v2h h = {(_Float16)a, (_Float16)b};
     return __builtin_bit_cast(uint32_t, h);
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
+
+// Multiplier and exponent of one token row from its sum of squares, its largest |a| before the producer's scalar and
+// whether it holds something non-finite.
+template <int OP>
+__device__ __forceinline__ void row_scale(float ss, float mx, int bad, uint32_t k, float eps, float* mul_out, int32_t* xsh_out) {
+    float scalar = 1.0f;
+    if (OP == OXB_PACK_RMSNORM) {
+        scalar = 1.0f / sqrtf(ss / (float)k + eps);
+        mx *= scalar;
+        bad |= !(fabsf(scalar) <= 3.402823466e38f) | !(fabsf(mx) <= 3.402823466e38f);
+    }
+    int E = 0;
+    if (mx > 0.0f) (void)frexpf(mx, &E);  // mx = f * 2^E, f in [0.5, 1)
+    const int shift = mx > 0.0f ? 15 - E : 0;
+    *mul_out = bad ? 0.0f : ldexpf(scalar, shift);
+    *xsh_out = bad ? INT32_MIN : -shift;
+}
 
 // Multiplier and exponent of one token row from the threads' partial results (sum of squares of x, largest |a|,
 // non-finite seen); all 256 threads of the workgroup call it, thread 0 gets the result.
@@ -85,22 +102,9 @@ __device__ __forceinline__ void row_finish(float ss, float mx, int bad, uint32_t
     bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
     if ((tid & 63u) == 0) red_s[tid >> 6] = ss, red_m[tid >> 6] = mx, red_b[tid >> 6] = bad;
     __syncthreads();
-    if (tid == 0) {
-        ss = red_s[0] + red_s[1] + red_s[2] + red_s[3];
-        mx = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
-        bad = red_b[0] | red_b[1] | red_b[2] | red_b[3];
-        float scalar = 1.0f;
-        if (OP == OXB_PACK_RMSNORM) {
-            scalar = 1.0f / sqrtf(ss / (float)k + eps);
-            mx *= scalar;
-            bad |= !(fabsf(scalar) <= 3.402823466e38f) | !(fabsf(mx) <= 3.402823466e38f);
-        }
-        int E = 0;
-        if (mx > 0.0f) (void)frexpf(mx, &E);  // mx = f * 2^E, f in [0.5, 1)
-        const int shift = mx > 0.0f ? 15 - E : 0;
-        *mul_out = bad ? 0.0f : ldexpf(scalar, shift);
-        *xsh_out = bad ? INT32_MIN : -shift;
-    }
+    if (tid == 0)
+        row_scale<OP>(red_s[0] + red_s[1] + red_s[2] + red_s[3], fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3])),
+                      red_b[0] | red_b[1] | red_b[2] | red_b[3], k, eps, mul_out, xsh_out);
 }
 
 template <int OP>
@@ -210,6 +214,92 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(const float* __restri
         const float4 p = a[it], q = b[it];
         xh[(size_t)id * M_pad + m] = make_uint4(pack_h2(p.x * mul, q.x * mul), pack_h2(p.y * mul, q.y * mul),
                                                 pack_h2(p.z * mul, q.z * mul), pack_h2(p.w * mul, q.w * mul));
+    }
+}
+
+// Both steps in one launch for many token rows: the eight waves of a workgroup own RPW rows (8, 4 or 2), 8 / RPW waves a
+// row.  A wave requests its whole share of the row at once (4 NI values per lane) and keeps it in registers, so x is read
+// once; the fp16 values then change from row order to chunk order through LDS, SEG pieces per lane at a time, and leave in
+// runs of RPW x 16 bytes (RPW rows side by side in a chunk).  row_stats_kernel + xh_pack_kernel read x twice in two
+// launches.  What bounds it is the way into and out of a CU (64 bytes a clock each) and, for few rows, the chain of one
+// memory round trip, two barriers and the stores.  A layer's four packs, 8B shape, two launches each before: 2048 rows
+// 93 -> 56 us, 301 rows 41 -> 26 us.
+template <int FMT, int OP, int RPW, int NI>
+__global__ __launch_bounds__(512) void xh_pack_wide_kernel(const float* __restrict__ x, const float* __restrict__ w, uint32_t ldx, uint32_t k,
+                                                            float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
+                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh) {
+    constexpr int WPR = 8 / RPW, SEG = NI <= 16 ? NI : NI == 48 ? 16 : 12;
+    static_assert(NI % SEG == 0, "whole segments");
+    constexpr uint32_t VALS = SEG * 256 * WPR, STR = VALS + 16;  // values of a row in a segment; LDS row stride (32 bytes of padding spread the rows over the banks)
+    constexpr int WG = OP == OXB_PACK_RMSNORM && NI > 16 ? 4 : SEG;  // norm weights requested at a time (registers)
+    __shared__ __attribute__((aligned(16))) _Float16 rows[RPW * STR];
+    __shared__ float red_s[8], red_m[8];
+    __shared__ int red_b[8];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, m0 = blockIdx.x * RPW;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), wr = wave / WPR, part = wave % WPR, m = m0 + wr;
+    const bool live = m < M;
+    const float* xr = x + (size_t)(live ? m : 0) * ldx;
+    auto at_of = [&](int i) -> uint32_t { return ((i * WPR + part) * 64 + lane) * 4; };
+    float4 a[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) a[i] = live && at_of(i) < k ? *reinterpret_cast<const float4*>(xr + at_of(i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float ss = 0.f, mx = 0.f;
+    int bad = 0;
+#pragma unroll
+    for (int i0 = 0; i0 < NI; i0 += WG) {
+        float4 g[OP == OXB_PACK_RMSNORM ? WG : 1];
+        if (OP == OXB_PACK_RMSNORM) {
+#pragma unroll
+            for (int i = 0; i < WG; i++) g[i] = at_of(i0 + i) < k ? *reinterpret_cast<const float4*>(w + at_of(i0 + i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int i = 0; i < WG; i++) {
+            float4& v = a[i0 + i];
+            if (OP == OXB_PACK_RMSNORM) {
+                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+                const float4 q = g[OP == OXB_PACK_RMSNORM ? i : 0];
+                v = make_float4(q.x * v.x, q.y * v.y, q.z * v.z, q.w * v.w);
+            }
+            bad |= !(fabsf(v.x) <= 3.402823466e38f) | !(fabsf(v.y) <= 3.402823466e38f) | !(fabsf(v.z) <= 3.402823466e38f) |
+                   !(fabsf(v.w) <= 3.402823466e38f);
+            mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+        }
+    }
+    ss = wave_sum_f32(ss);
+    mx = wave_max_f32(mx);
+    bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
+    if constexpr (WPR > 1) {  // the row's waves, added in wave order
+        if (lane == 0) red_s[wave] = ss, red_m[wave] = mx, red_b[wave] = bad;
+        __syncthreads();
+        ss = red_s[wr * WPR], mx = red_m[wr * WPR], bad = red_b[wr * WPR];
+#pragma unroll
+        for (int i = 1; i < WPR; i++) ss += red_s[wr * WPR + i], mx = fmaxf(mx, red_m[wr * WPR + i]), bad |= red_b[wr * WPR + i];
+    }
+    float mul;
+    int32_t e;
+    row_scale<OP>(ss, mx, bad, k, eps, &mul, &e);
+    if (!live) mul = 0.f;
+    else if (part == 0 && lane == 0) xsh[m] = e;
+#pragma unroll
+    for (int i0 = 0; i0 < NI; i0 += SEG) {
+        if (i0) __syncthreads();  // the segment before has been read
+#pragma unroll
+        for (int i = 0; i < SEG; i++) {
+            const float4 v = a[i0 + i];
+            *reinterpret_cast<uint2*>(&rows[wr * STR + at_of(i)]) = make_uint2(pack_h2(v.x * mul, v.y * mul), pack_h2(v.z * mul, v.w * mul));
+        }
+        __syncthreads();
+        const uint32_t blk0 = (uint32_t)(i0 / SEG) * (VALS / 128), blks = min(nblk_pad - min(nblk_pad, blk0), VALS / 128);  // blocks of this segment
+        for (uint32_t id = tid; id < blks * 16 * RPW; id += 512) {  // (chunk, row), rows first
+            const uint32_t row = id % RPW, c = id / RPW;
+            uint32_t o0, o1;
+            item_offsets<FMT>(c >> 4, c & 15u, &o0, &o1);
+            const uint2 p = *reinterpret_cast<const uint2*>(&rows[row * STR + o0]), q = *reinterpret_cast<const uint2*>(&rows[row * STR + o1]);
+            // values 0..3 of the first piece side by side with those of the second
+            xh[(size_t)(blk0 * 16 + c) * M_pad + m0 + row] =
+                make_uint4(__builtin_amdgcn_perm(q.x, p.x, 0x05040100u), __builtin_amdgcn_perm(q.x, p.x, 0x07060302u),
+                           __builtin_amdgcn_perm(q.y, p.y, 0x05040100u), __builtin_amdgcn_perm(q.y, p.y, 0x07060302u));
+        }
     }
 }
 
@@ -816,6 +906,23 @@ static void launch_pack_op(int fmt, const float* d_x, const float* d_w, uint32_t
         OXB_ROWS_CASE(1) OXB_ROWS_CASE(2) OXB_ROWS_CASE(4) OXB_ROWS_CASE(6) OXB_ROWS_CASE(8)
 #undef OXB_ROWS_CASE
     }
+    // Four rows per workgroup, two where four would leave half the CUs idle; eight for long rows where each CU has a
+    // workgroup all the same (2048 rows of 12288: 25 us against 28 with four and 36 with two; of 4096: 11, 10 and 12).
+    const uint32_t rpw = OP == OXB_PACK_IDENT && k > 8192 && M_pad >= 2048 ? 8 : M_pad >= 512 ? 4 : 2, per_lane = (nblk_pad * 4 * rpw + 63) / 64;  // pieces of four values per lane
+#define OXB_WIDE_CASE(RPW, NI)                                                                                                     \
+    if (rpw == RPW && per_lane <= NI) {                                                                                            \
+        if (fmt == OXB_FMT_Q1)                                                                                                     \
+            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_Q1, OP, RPW, NI>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                 \
+        else                                                                                                                       \
+            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_TQ2, OP, RPW, NI>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                 \
+        return;                                                                                                                    \
+    }
+    OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16) OXB_WIDE_CASE(4, 24) OXB_WIDE_CASE(2, 4) OXB_WIDE_CASE(2, 8) OXB_WIDE_CASE(2, 12)
+    if constexpr (OP == OXB_PACK_IDENT) { OXB_WIDE_CASE(8, 48) }
+    // (rows of more than 12288 values take two launches)
+#undef OXB_WIDE_CASE
     hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh);
     const dim3 grid(M_pad / 16, nblk_pad < 16 ? nblk_pad : 16);
     if (fmt == OXB_FMT_Q1)
