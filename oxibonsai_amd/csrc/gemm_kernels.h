@@ -8,7 +8,7 @@
 // STORE: y = W a;  RESIDUAL: y = residual + W a;  SWIGLU: W = gate || up (n_rows = 2 * inter, a multiple of 32),
 // y[m][i] = silu(gate_i . a) * (up_i . a) for i < inter, ldy >= inter.
 enum { OXB_GEMM_STORE = 0, OXB_GEMM_RESIDUAL = 2, OXB_GEMM_SWIGLU = 3 };
-#define OXB_GEMM_NARROW_MAX_M 32  // up to this many token rows the narrow kernel (K split over waves) is used
+#define OXB_GEMM_NARROW_MAX_M 32  // up to this many token rows the narrow kernel (K split over waves) is always used
 
 struct OxbGemmParams {
     const uint32_t* codes;   // resident codes section
@@ -27,6 +27,7 @@ struct OxbGemmParams {
     float* part;             // [ksplit][M][ldy] partial sums, needed when oxb_gemm_ksplit(...) > 1
     uint32_t codes_bytes, scales_bytes, xh_bytes;  // buffer extents (loads beyond them read 0)
     int mode;
+    bool no_split;           // keep K in one piece (a caller without room for partial sums)
 };
 
 // Bytes of the packed activation buffer for M token rows of length k.
@@ -40,5 +41,5 @@ enum { OXB_PACK_IDENT = 0, OXB_PACK_RMSNORM = 1 };
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
                               uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st);
 // Number of K slices the launcher will use for this shape (1: no workspace needed).
-uint32_t oxb_gemm_ksplit(const OxbGemmParams& p, uint32_t n_cus);
+uint32_t oxb_gemm_ksplit(int fmt, const OxbGemmParams& p, uint32_t n_cus);
 hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st);

@@ -704,11 +704,14 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 }
 
 // ---------------------------------------------------------------------------
-// GEMM for a few token rows (M <= 32: decode batches).  The wide kernel above would spend its time on barriers
+// GEMM for up to 128 token rows (decode batches, short prompts).  The wide kernel above would spend its time on barriers
 // and on MFMAs over padding; here the weights stream once at GEMV-like rates.  A workgroup = 8 waves owns RT row
 // tiles; the waves split K (contiguous runs of superblocks), each expands its weights and multiplies them with
 // B operands read straight from the packed activations (they stay in L2, no LDS stage, no barrier in the loop),
-// prefetched one block ahead; the eight partial sums meet in LDS and are added in wave order.
+// requested D - 1 steps ahead; the eight partial sums meet in LDS and are added in wave order.  What bounds it is the
+// activations' way into the CU: every workgroup takes in all of them, 16 CT rows of K at 64 bytes a clock.
+// Beyond 32 rows against the wide kernel with its 64-token tiles (kernel alone): 4096 x 4096 at 64 / 128 rows 14.9 -> 8.7 /
+// 15.5 -> 13.5 us, 6144 x 4096 at 77 15.8 -> 9.7, 4096 x 2048 (TQ2) at 64 / 128 10.5 -> 5.6 / 11.0 -> 8.2.
 // ---------------------------------------------------------------------------
 #define OXB_GEMM_NARROW_THREADS 512
 
@@ -716,8 +719,9 @@ template <int FMT, int RT, int CT>
 __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(const OxbGemmParams p) {
     // The partial sums meet in LDS in passes of PT row tiles (all of them up to four; pairs beyond, so that the
     // array stays within 64 KB): in SWIGLU mode a pass holds gate tiles and the up tiles of the same rows.
-    constexpr int PT = RT <= 4 ? RT : 2, NPASS = RT / PT;
+    constexpr int PT = RT * CT <= 8 || RT == 1 ? RT : 2, NPASS = RT / PT;
     static_assert(RT % PT == 0, "row tiles per pass");
+    constexpr int D = CT <= 2 && RT <= 4 ? 8 : 4;  // steps of B operands in registers (16 D CT registers)
     __shared__ float red[8][PT * CT * 4][64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, g = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -742,27 +746,28 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     if (sb0 < sb1) {
         const uint32_t blk_stride = 16u * p.M_pad * 16u;  // bytes of xh per block
         const uint32_t blk_end = sb1 * 4u;
-        // B operand of step s, token tile ct of a block: chunk 4g + s, token 16 ct + r
-        v8h B[2][4][CT];
-        auto load_b = [&](uint32_t blk, v8h (&dst)[4][CT]) {
+        // B operands of step s, token tile ct of a block: chunk 4g + s, token 16 ct + r.  A ring of D steps, D - 1 ahead.
+        v8h B[D][CT];
+        // One lane offset; step and block go into the wave-uniform part, the token tile into the instruction's constant.
+        const uint32_t b_off = (4u * g * p.M_pad + r) * 16u;
+        auto load_b = [&](uint32_t blk, int s, v8h (&dst)[CT]) {
+            const uint32_t at = blk < blk_end ? b_off : 0x7FFFF000u;  // (past the slice: out of range, a constant may still be added)
 #pragma unroll
-            for (int s = 0; s < 4; s++)
-#pragma unroll
-                for (int ct = 0; ct < CT; ct++) {
-                    const uint32_t off = ((4u * g + s) * p.M_pad + ct * 16u + r) * 16u;
-                    dst[s][ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, blk < blk_end ? off : OXB_OOB, blk * blk_stride));
-                }
+            for (int ct = 0; ct < CT; ct++) dst[ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, at + ct * 256u, blk * blk_stride + s * p.M_pad * 16u));
         };
         // RING: the next superblock's weights wait in a second register set; with more than four row tiles there
         // is no room for one, and a half is requested again in place once its second block has been prepared.
-        constexpr bool RING = RT <= 4;
+        constexpr bool RING = RT * CT <= 12 && RT <= 4;
         HalfRegs<FMT> H[RT][2], Hn[RING ? RT : 1][2];
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             load_half<FMT>(H[rt][0], rc, rs, tile_of(rt), valid(rt), p.n_sb, sb0, 0, lane);
             load_half<FMT>(H[rt][1], rc, rs, tile_of(rt), valid(rt), p.n_sb, sb0, 1, lane);
         }
-        load_b(sb0 * 4u, B[0]);
+        // (two blocks in registers: the next block's steps are requested together; else step by step)
+        constexpr bool BLOCKS = D == 8;
+#pragma unroll
+        for (int j = 0; j < (BLOCKS ? 4 : D - 1); j++) load_b(sb0 * 4u + (j >> 2), j & 3, B[j]);
         for (uint32_t sb = sb0; sb < sb1; sb++) {
             // next superblock's weights (all zero past the slice: never used)
             if (RING) {
@@ -774,7 +779,10 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
             }
 #pragma unroll
             for (int bi = 0; bi < 4; bi++) {
-                load_b(sb * 4u + bi + 1, B[(bi + 1) & 1]);
+                if (BLOCKS) {
+#pragma unroll
+                    for (int s = 0; s < 4; s++) load_b(sb * 4u + bi + 1, s, B[(4 * (bi + 1) + s) % D]);
+                }
                 BlockDec bd[RT];
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][bi >> 1], bi & 1);
@@ -784,13 +792,15 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
                 }
 #pragma unroll
                 for (int s = 0; s < 4; s++) {
+                    const int j = 4 * bi + s, jn = j + D - 1;
+                    if (!BLOCKS) load_b(sb * 4u + (jn >> 2), jn & 3, B[jn % D]);
                     v8h A[RT];
                     decode_step<FMT, RT>(bd, s, A);
 #pragma unroll
                     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
                         for (int rt = 0; rt < RT; rt++)  // row tiles past the range hold zero weights
-                            acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rt], B[bi & 1][s][ct], acc[rt][ct], 0, 0, 0);
+                            acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rt], B[j % D][ct], acc[rt][ct], 0, 0, 0);
                 }
             }
             if (RING) {
@@ -953,51 +963,89 @@ static hipError_t launch_gemm_case(const OxbGemmParams& p, uint32_t grid, hipStr
     return hipGetLastError();
 }
 
-struct GemmPlan { uint32_t rt, tpw, ksplit, sb_per_split, ct; };
+// What the launcher runs: the narrow kernel with rt row tiles per workgroup, or the wide one with rt row tiles per wave, tpw
+// per workgroup, 16 ct tokens per tile and K in ksplit slices of sb_per_split superblocks.
+struct GemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };
 
-// Row tiles per workgroup and K slices: minimise (rounds of workgroups over the CUs) x (time of one workgroup),
-// where a workgroup costs, per superblock of its K slice, its row tiles per wave plus about one more for staging,
-// barriers and operand latency, plus a fixed part for its start and epilogue.  Splitting K adds a pass over the
-// output per slice (the partial sums are written, then added in slice order).  Ties go to the larger tile.
-static GemmPlan plan_gemm(const OxbGemmParams& p, uint32_t n_cus) {
-    constexpr uint32_t BM = 128;
-    const uint32_t n_mt = (p.M + BM - 1) / BM;
-    static const uint32_t rts[] = {5, 4, 3, 2, 1};
-    GemmPlan best = {1, 4, 1, p.n_sb, 8};
-    if (p.mode == OXB_GEMM_SWIGLU) best = {2, 8, 1, p.n_sb, 8};
-    uint64_t best_cost = ~0ull;
-    const bool sw = p.mode == OXB_GEMM_SWIGLU;  // even tile counts per wave, no K split (the epilogue is not linear)
-    const bool can_split = (p.ldy & 3u) == 0 && !sw;
-    for (uint32_t ks = 1; ks <= (can_split ? 8u : 1u) && ks <= p.n_sb; ks++) {
-        const uint32_t spk = (p.n_sb + ks - 1) / ks;
-        if (ks > 1 && (p.n_sb + spk - 1) / spk != ks) continue;  // same slices as a smaller count
-        for (uint32_t rt : rts) {
-            // SWIGLU: a wave takes gate and up tiles in pairs.  One pair per wave (164 registers: two workgroups per
-            // CU, whose starts and epilogues overlap) measured faster than two pairs (308 registers, one workgroup per
-            // CU) on both quoted gate || up shapes at 2048 tokens: 24576 x 4096 357 against 368 us, 12288 x 2048 109
-            // against 121 us.
-            if (sw && rt != 2) continue;  // (three tiles per wave are considered below)
-            for (uint32_t tpw = 4 * rt; tpw > (sw ? 4 * rt - 1 : 4 * rt - 4); tpw--) {
-                const uint32_t groups = (p.n_tiles + tpw - 1) / tpw;
-                const uint64_t wgs = (uint64_t)groups * n_mt * ks;
-                uint64_t cost = ((wgs + n_cus - 1) / n_cus) * ((uint64_t)spk * (rt + 1) + 2 * rt + 2);
-                if (ks > 1) cost += (uint64_t)ks * 2 + 4;  // the reduction pass
-                if (cost < best_cost) best_cost = cost, best = {rt, tpw, ks, spk, 8};
-            }
+// Time of a wide plan in us, from 19 000 measured (shape, tokens, plan) triples - both formats, 1280 .. 24576 rows, K 1280 ..
+// 12288, 33 .. 2048 tokens - whose best plan it names within 2 % on average (the rule before it, 128-token tiles by rounds
+// of workgroups: 12 %).  Per 128-weight block a workgroup alone on its CU needs `lone`, a latency; workgroups that share
+// one need `busy` each, a rate.  More tokens per tile amortise the expansion of the weights, more row tiles the reading of
+// the token tile out of LDS; small tiles make more workgroups and less padding.
+static float wide_cost(bool tq2, const OxbGemmParams& p, const GemmPlan& g, uint32_t n_cus) {
+    // [format][ct = 4, 5, 8][rt - 1]; rt = 5 goes with ct = 8 only
+    static const float lone_us[2][3][5] = {{{0.34f, 0.50f, 0.68f, 0.82f}, {0.40f, 0.59f, 0.81f, 0.96f}, {0.66f, 0.86f, 1.18f, 1.42f, 1.69f}},
+                                           {{0.39f, 0.59f, 0.85f, 1.05f}, {0.45f, 0.70f, 0.96f, 1.19f}, {0.69f, 0.99f, 1.30f, 1.60f, 1.83f}}};
+    static const float busy_us[2][3][5] = {{{0.25f, 0.41f, 0.58f, 0.77f}, {0.31f, 0.51f, 0.70f, 0.92f}, {0.54f, 0.83f, 1.09f, 1.42f, 1.69f}},
+                                           {{0.28f, 0.49f, 0.68f, 0.94f}, {0.34f, 0.60f, 0.84f, 1.06f}, {0.57f, 0.85f, 1.17f, 1.60f, 1.83f}}};
+    static const float long_k_us[3][5] = {{0.14f, 0.05f, 0.03f, 0.02f}, {0.14f, 0.05f, 0.03f, 0.02f}, {0.03f, 0.03f}};  // on top of lone, K > 4608: the token panel leaves L2
+    static const uint32_t resident[3][5] = {{5, 4, 3, 2}, {4, 3, 3, 2}, {2, 2, 2, 1, 1}};  // workgroups per CU (registers, LDS)
+    const uint32_t ci = g.ct == 4 ? 0 : g.ct == 5 ? 1 : 2, ri = g.rt - 1, R = resident[ci][ri];
+    const uint32_t n_mt = (p.M + 16 * g.ct - 1) / (16 * g.ct), n_ng = (p.n_tiles + g.tpw - 1) / g.tpw;
+    const uint32_t q = (n_ng * n_mt * g.ksplit + n_cus - 1) / n_cus;  // workgroups on the CU that gets most
+    const float lone = lone_us[tq2][ci][ri] + (p.n_sb > 9 ? long_k_us[ci][ri] : 0.f), busy = busy_us[tq2][ci][ri];
+    auto round = [&](uint32_t w) { const float b = w * busy; return w == 0 ? 0.f : b > lone ? b : lone; };
+    const float us = 4.4f + 4.f * g.sb_per_split * ((float)(q / R) * round(R) + round(q % R)) + 0.158f * q * g.rt * g.ct;
+    // a K split writes its partial sums and adds them in a launch of its own
+    return g.ksplit > 1 ? 1.04f * (us + 2.2f + 0.73e-6f * g.ksplit * p.M * (float)p.n_rows) : us;
+}
+
+// The same for the narrow kernel (416 triples, rms 8 %): every workgroup takes in the whole packed activations, so its
+// time goes with K and the token tiles, little with its row tiles.
+static float narrow_cost(bool tq2, const OxbGemmParams& p, uint32_t rt, uint32_t n_cus) {
+    const uint32_t ct = (p.M + 15) / 16, R = (rt == 1 && ct <= 4) || (rt == 2 && ct == 3 && !tq2) ? 2 : 1;
+    const uint32_t wgs = p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + rt / 2 - 1) / (rt / 2) : (p.n_tiles + rt - 1) / rt, q = (wgs + n_cus - 1) / n_cus;
+    const float n_sb = (float)p.n_sb, busy = 0.119f * n_sb * ct + 0.063f * n_sb * rt * (tq2 ? 2.14f : 1.f), lone = 0.443f + busy;
+    auto round = [&](uint32_t w) { const float b = w * busy; return w == 0 ? 0.f : b > lone ? b : lone; };
+    return 1.34f + (float)(q / R) * round(R) + round(q % R) + 0.197f * q * rt * ct;
+}
+
+// The narrow kernel up to OXB_GEMM_NARROW_MAX_M token rows (the wide one would spend its time on barriers and padding),
+// the cheaper of the two up to 128, the wide one beyond.
+static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
+    const bool tq2 = fmt == OXB_FMT_TQ2, sw = p.mode == OXB_GEMM_SWIGLU;
+    GemmPlan best = {true, sw ? 2u : 1u, 0, 0, 1, p.n_sb};
+    if (p.M <= OXB_GEMM_NARROW_MAX_M) {
+        // Row tiles per workgroup (1, 2, 4 or - Q1 - 6): the count that minimises (rounds of workgroups over the CUs) x (row tiles + 2 - a
+        // workgroup's time grows with its tiles on top of a fixed part: its start, the K-split sum and the epilogue).  What
+        // counts is the last round: 384 workgroups of one tile leave half the CUs with two and the launch as long as those
+        // (QKV 6144 x 4096, 8 rows: 5.5 us against 4.7 us as 192 workgroups of two tiles; 32 rows: 8.2 against 6.1).  A tie
+        // goes to the larger workgroups (every workgroup reads all of the packed activations); 8B-shape decode with this rule
+        // against "as many tiles as leave a workgroup per CU": +2 % at 8 and at 32 sequences.  Six tiles (three gate and three up
+        // tiles in SWIGLU mode) make gate || up 24576 x 4096 one workgroup per CU: at four, the 384 workgroups - one resident per
+        // CU at their register count - ran in two rounds (32 rows: 17.4 -> 13.0 us per launch, the LM head 78 -> 74 us).
+        uint64_t best_cost = ~0ull;
+        static const uint32_t choices[4] = {1, 2, 4, 6};
+        for (uint32_t ci = sw ? 1 : 0; ci < (tq2 ? 3u : 4u); ci++) {  // (six tiles: Q1 only - the ternary decoder's registers do not fit)
+            const uint32_t r = choices[ci];
+            const uint32_t wgs = sw ? (p.n_tiles / 2 + r / 2 - 1) / (r / 2) : (p.n_tiles + r - 1) / r;
+            const uint64_t cost = (uint64_t)((wgs + n_cus - 1) / n_cus) * (r + 2);
+            if (cost <= best_cost) best_cost = cost, best.rt = r;
+        }
+        return best;
+    }
+    float best_us = 1e30f;
+    if (p.M <= 128) {
+        const uint32_t ct = (p.M + 15) / 16;
+        for (uint32_t rt = sw ? 2 : 1; rt <= (ct <= 4 ? 4u : ct <= 7 ? 2u : 1u); rt *= 2) {
+            const float us = narrow_cost(tq2, p, rt, n_cus);
+            if (us < best_us) best_us = us, best.rt = rt;
         }
     }
-    // Small matrices leave the 128-token tile short of workgroups (one or two row tiles per wave and still fewer
-    // workgroups than CUs): there a 64-token tile with one row tile per wave doubles their number.  Measured at 512
-    // tokens: 4096 x 4096 26.2 -> 23.0 us, 6144 x 4096 37.0 -> 33.2, 5120 x 2560 (TQ2) 26.6 -> 24.6, 4096 x 2048 17.5 ->
-    // 15.8, 2048 x 2048 14.9 -> 11.4; with more workgroups to begin with the wider tile wins.
-    if (!sw && best.ksplit == 1 && best.rt <= 2) {
-        const uint64_t wgs = (uint64_t)((p.n_tiles + best.tpw - 1) / best.tpw) * n_mt;
-        if (best.rt == 1 || wgs < n_cus) best = {1, 4, 1, p.n_sb, 4};
+    static const uint32_t cts[3] = {8, 5, 4}, splits[5] = {1, 2, 3, 4, 6};
+    const bool can_split = (p.ldy & 3u) == 0 && !sw && !p.no_split;  // (the SwiGLU epilogue is not linear)
+    for (uint32_t ks : splits) {
+        if (ks > (can_split ? p.n_sb : 1u)) break;
+        const uint32_t spk = (p.n_sb + ks - 1) / ks;
+        if ((p.n_sb + spk - 1) / spk != ks) continue;  // same slices as a smaller count
+        for (uint32_t ct : cts)
+            for (uint32_t rt = 1; rt <= (ct == 8 ? 5u : 4u); rt++) {
+                if (sw && rt != 2 && rt != 3) continue;  // a gate and an up tile per wave, or three tiles of either kind
+                const GemmPlan g = {false, rt, 4 * rt, ct, ks, spk};
+                const float us = wide_cost(tq2, p, g, n_cus);
+                if (us < best_us) best_us = us, best = g;
+            }
     }
-    // gate || up with three tiles per wave (two gate waves, two up waves; still two workgroups per CU): fewer LDS reads
-    // per MFMA than with two.  Measured at 2048 tokens (plain stores): 24576 x 4096 310 against 343 us, 19456 x 2560
-    // (TQ2) 181 against 193, 12288 x 2048 (TQ2) 92 against 101; taken where its workgroups still cover the CUs.
-    if (sw && (uint64_t)((p.n_tiles / 2 + 5) / 6) * n_mt >= n_cus) best = {3, 12, 1, p.n_sb, 8};
     return best;
 }
 
@@ -1008,77 +1056,54 @@ static hipError_t launch_narrow_case(const OxbGemmParams& p, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Row tiles per workgroup (1, 2, 4 or - Q1 - 6): the count that minimises (rounds of workgroups over the CUs) x (row tiles + 2 - a
-// workgroup's time grows with its tiles on top of a fixed part: its start, the K-split sum and the epilogue).  What
-// counts is the last round: 384 workgroups of one tile leave half the CUs with two and the launch as long as those
-// (QKV 6144 x 4096, 8 rows: 5.5 us against 4.7 us as 192 workgroups of two tiles; 32 rows: 8.2 against 6.1).  A tie
-// goes to the larger workgroups (every workgroup reads all of the packed activations); 8B-shape decode with this rule
-// against "as many tiles as leave a workgroup per CU": +2 % at 8 and at 32 sequences.  Six tiles (three gate and three up
-// tiles in SWIGLU mode) make gate || up 24576 x 4096 one workgroup per CU: at four, the 384 workgroups - one resident per
-// CU at their register count - ran in two rounds (32 rows: 17.4 -> 13.0 us per launch, the LM head 78 -> 74 us).
-static hipError_t launch_gemm_narrow(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st) {
+static hipError_t launch_gemm_narrow(int fmt, OxbGemmParams p, uint32_t rt, hipStream_t st) {
     p.ksplit = 1;
     p.sb_per_split = p.n_sb;
-    const bool sw = p.mode == OXB_GEMM_SWIGLU;
-    if (sw && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // gate and up halves of whole row tiles
     const uint32_t ct = p.M_pad / 16;
-    uint32_t rt = sw ? 2 : 1;
-    uint64_t best_cost = ~0ull;
-    static const uint32_t choices[4] = {1, 2, 4, 6};
-    for (uint32_t ci = sw ? 1 : 0; ci < (fmt == OXB_FMT_Q1 ? 4u : 3u); ci++) {  // (six tiles: Q1 only - the ternary decoder's registers do not fit)
-        const uint32_t r = choices[ci];
-        const uint32_t wgs = sw ? (p.n_tiles / 2 + r / 2 - 1) / (r / 2) : (p.n_tiles + r - 1) / r;
-        const uint64_t cost = (uint64_t)((wgs + n_cus - 1) / n_cus) * (r + 2);
-        if (cost <= best_cost) best_cost = cost, rt = r;
-    }
 #define OXB_NARROW_CASE(F, R, C) \
     if (fmt == F && rt == R && ct == C) return launch_narrow_case<F, R, C>(p, st);
-    OXB_NARROW_CASE(OXB_FMT_Q1, 1, 1) OXB_NARROW_CASE(OXB_FMT_Q1, 2, 1) OXB_NARROW_CASE(OXB_FMT_Q1, 4, 1)
-    OXB_NARROW_CASE(OXB_FMT_Q1, 1, 2) OXB_NARROW_CASE(OXB_FMT_Q1, 2, 2) OXB_NARROW_CASE(OXB_FMT_Q1, 4, 2)
-    OXB_NARROW_CASE(OXB_FMT_Q1, 6, 1) OXB_NARROW_CASE(OXB_FMT_Q1, 6, 2)
-    OXB_NARROW_CASE(OXB_FMT_TQ2, 1, 1) OXB_NARROW_CASE(OXB_FMT_TQ2, 2, 1) OXB_NARROW_CASE(OXB_FMT_TQ2, 4, 1)
-    OXB_NARROW_CASE(OXB_FMT_TQ2, 1, 2) OXB_NARROW_CASE(OXB_FMT_TQ2, 2, 2) OXB_NARROW_CASE(OXB_FMT_TQ2, 4, 2)
+#define OXB_NARROW_CASES(R, C) OXB_NARROW_CASE(OXB_FMT_Q1, R, C) OXB_NARROW_CASE(OXB_FMT_TQ2, R, C)
+    OXB_NARROW_CASES(1, 1) OXB_NARROW_CASES(2, 1) OXB_NARROW_CASES(4, 1) OXB_NARROW_CASE(OXB_FMT_Q1, 6, 1)
+    OXB_NARROW_CASES(1, 2) OXB_NARROW_CASES(2, 2) OXB_NARROW_CASES(4, 2) OXB_NARROW_CASE(OXB_FMT_Q1, 6, 2)
+    OXB_NARROW_CASES(1, 3) OXB_NARROW_CASES(2, 3) OXB_NARROW_CASES(4, 3)
+    OXB_NARROW_CASES(1, 4) OXB_NARROW_CASES(2, 4) OXB_NARROW_CASES(4, 4)
+    OXB_NARROW_CASES(1, 5) OXB_NARROW_CASES(2, 5)
+    OXB_NARROW_CASES(1, 6) OXB_NARROW_CASES(2, 6)
+    OXB_NARROW_CASES(1, 7) OXB_NARROW_CASES(2, 7)
+    OXB_NARROW_CASES(1, 8)
+#undef OXB_NARROW_CASES
 #undef OXB_NARROW_CASE
     return hipErrorInvalidValue;
 }
 
 
-uint32_t oxb_gemm_ksplit(const OxbGemmParams& p, uint32_t n_cus) {
-    if (p.M == 0 || p.n_rows == 0 || p.n_sb == 0 || p.M <= OXB_GEMM_NARROW_MAX_M) return 1;
-    return plan_gemm(p, n_cus).ksplit;
+uint32_t oxb_gemm_ksplit(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
+    if (p.M == 0 || p.n_rows == 0 || p.n_sb == 0) return 1;
+    return plan_gemm(fmt, p, n_cus).ksplit;
 }
 
 hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st) {
     if (p.M == 0 || p.n_rows == 0) return hipSuccess;
     if (p.n_sb == 0 || (uint64_t)p.n_tiles * p.n_sb * 2048ull >= 0xFFFFFFF0ull) return hipErrorInvalidValue;
-    p.M_pad = (p.M + 15u) / 16u * 16u;
-    if (p.M <= OXB_GEMM_NARROW_MAX_M) return launch_gemm_narrow(fmt, p, n_cus, st);
     if (p.mode == OXB_GEMM_SWIGLU && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // whole gate and up row tiles
-    const GemmPlan plan = plan_gemm(p, n_cus);
-    const uint32_t BM = 16 * plan.ct;  // tokens per workgroup tile
-    p.n_mt = (p.M + BM - 1) / BM;
-    const uint32_t best_rt = plan.rt, best_tpw = plan.tpw;
+    p.M_pad = (p.M + 15u) / 16u * 16u;
+    const GemmPlan plan = plan_gemm(fmt, p, n_cus);
+    if (plan.narrow) return launch_gemm_narrow(fmt, p, plan.rt, st);
+    p.n_mt = (p.M + 16 * plan.ct - 1) / (16 * plan.ct);
     p.ksplit = plan.ksplit;
     p.sb_per_split = plan.sb_per_split;
     if (p.ksplit > 1 && !p.part) return hipErrorInvalidValue;
-    p.tpw = best_tpw;
+    p.tpw = plan.tpw;
     p.n_ng = (p.n_tiles + p.tpw - 1) / p.tpw;
     const uint32_t grid = p.n_ng * p.n_mt * p.ksplit;
     hipError_t err = hipErrorInvalidValue;
-#define OXB_GEMM_CASE(F, R) \
-    if (fmt == F && best_rt == R && plan.ct == 8) err = launch_gemm_case<F, R, 8>(p, grid, st);
-    OXB_GEMM_CASE(OXB_FMT_Q1, 1)
-    OXB_GEMM_CASE(OXB_FMT_Q1, 2)
-    OXB_GEMM_CASE(OXB_FMT_Q1, 3)
-    OXB_GEMM_CASE(OXB_FMT_Q1, 4)
-    OXB_GEMM_CASE(OXB_FMT_Q1, 5)
-    OXB_GEMM_CASE(OXB_FMT_TQ2, 1)
-    OXB_GEMM_CASE(OXB_FMT_TQ2, 2)
-    OXB_GEMM_CASE(OXB_FMT_TQ2, 3)
-    OXB_GEMM_CASE(OXB_FMT_TQ2, 4)
-    OXB_GEMM_CASE(OXB_FMT_TQ2, 5)
+#define OXB_GEMM_CASE(R, C)                                                                        \
+    if (plan.rt == R && plan.ct == C)                                                              \
+        err = fmt == OXB_FMT_Q1 ? launch_gemm_case<OXB_FMT_Q1, R, C>(p, grid, st) : launch_gemm_case<OXB_FMT_TQ2, R, C>(p, grid, st);
+    OXB_GEMM_CASE(1, 8) OXB_GEMM_CASE(2, 8) OXB_GEMM_CASE(3, 8) OXB_GEMM_CASE(4, 8) OXB_GEMM_CASE(5, 8)
+    OXB_GEMM_CASE(1, 5) OXB_GEMM_CASE(2, 5) OXB_GEMM_CASE(3, 5) OXB_GEMM_CASE(4, 5)
+    OXB_GEMM_CASE(1, 4) OXB_GEMM_CASE(2, 4) OXB_GEMM_CASE(3, 4) OXB_GEMM_CASE(4, 4)
 #undef OXB_GEMM_CASE
-    if (plan.ct == 4 && best_rt == 1) err = fmt == OXB_FMT_Q1 ? launch_gemm_case<OXB_FMT_Q1, 1, 4>(p, grid, st) : launch_gemm_case<OXB_FMT_TQ2, 1, 4>(p, grid, st);
     if (err != hipSuccess || p.ksplit == 1) return err;
     const size_t plane = (size_t)p.M * p.ldy, n4 = plane / 4;
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, st, p.part, p.ksplit, plane,

@@ -284,8 +284,8 @@ static int size_gemm_workspaces(Model& m) {
         gp.n_sb = w->L.n_sb;
         gp.M = d.batch;
         gp.ldy = sh.n;
-        const size_t b = (size_t)oxb_gemm_ksplit(gp, g_rt.n_cus) * d.batch * sh.n * sizeof(float);
-        if (oxb_gemm_ksplit(gp, g_rt.n_cus) > 1 && b > part_bytes) part_bytes = b;
+        const size_t b = (size_t)oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus) * d.batch * sh.n * sizeof(float);
+        if (oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus) > 1 && b > part_bytes) part_bytes = b;
     }
     int rc;
     if ((rc = m.gws.xh.ensure(oxb_xh_bytes(kx, d.batch))) || (rc = m.gws.xsh.ensure(((size_t)d.batch + 16) * 4)) ||

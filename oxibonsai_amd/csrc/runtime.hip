@@ -309,7 +309,8 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
     p.scales_bytes = (uint32_t)w.L.scales_bytes;
     p.xh_bytes = (uint32_t)oxb_xh_bytes(k, m);
     p.mode = mode;
-    const uint32_t ksplit = oxb_gemm_ksplit(p, g_rt.n_cus);
+    p.no_split = ws->no_split;
+    const uint32_t ksplit = oxb_gemm_ksplit((int)w.L.fmt, p, g_rt.n_cus);
     if (ksplit > 1) {
         if ((rc = ws->part.ensure((size_t)ksplit * m * ldy * sizeof(float)))) return rc;
         p.part = (float*)ws->part.ptr;
@@ -652,16 +653,21 @@ int oxb_hip_gemm_dev_static(uint64_t id, const float* d_x, float* d_y, uint32_t 
     OxbGemmParams gp;
     memset(&gp, 0, sizeof gp);
     gp.n_rows = n_rows, gp.n_tiles = w->L.n_tiles, gp.n_sb = w->L.n_sb, gp.M = m, gp.ldy = n_rows;
-    const uint32_t ksplit = oxb_gemm_ksplit(gp, g_rt.n_cus);
+    const uint32_t ksplit = oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus);
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t need[4] = {up(oxb_xh_bytes(k, m)), up(((size_t)m + 16) * sizeof(int32_t)), up(((size_t)m + 16) * sizeof(float)),
-                            ksplit > 1 ? up((size_t)ksplit * m * n_rows * sizeof(float)) : 0};
-    const size_t total = need[0] + need[1] + need[2] + need[3];
+    size_t need[4] = {up(oxb_xh_bytes(k, m)), up(((size_t)m + 16) * sizeof(int32_t)), up(((size_t)m + 16) * sizeof(float)),
+                      ksplit > 1 ? up((size_t)ksplit * m * n_rows * sizeof(float)) : 0};
+    size_t total = need[0] + need[1] + need[2] + need[3];
+    GemmWorkspace ws;
+    if (total > OXB_STATIC_SCRATCH_BYTES && need[3]) {  // a K split is only a faster way: do without its partial sums
+        ws.no_split = true;
+        total -= need[3];
+        need[3] = 0;
+    }
     if (total > OXB_STATIC_SCRATCH_BYTES)
         return fail(OXB_HIP_INVALID_ARGUMENT,
                     "invalid argument: a GEMM of %u rows x %u x %u needs %zu bytes of scratch, the allocation-free entry point holds %u",
                     m, n_rows, k, total, OXB_STATIC_SCRATCH_BYTES);
-    GemmWorkspace ws;
     DevBuf* bufs[4] = {&ws.xh, &ws.xsh, &ws.rowmul, &ws.part};
     size_t off = 0;
     for (int i = 0; i < 4; i++) {

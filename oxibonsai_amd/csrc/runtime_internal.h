@@ -25,6 +25,7 @@ struct DevBuf {  // grow-only device scratch
 // own that never move.
 struct GemmWorkspace {
     DevBuf xh, xsh, rowmul, part;
+    bool no_split = false;  // no room for partial sums: K stays in one piece
     void release() { xh.release(); xsh.release(); rowmul.release(); part.release(); }
 };
 
