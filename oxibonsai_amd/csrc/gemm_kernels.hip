@@ -19,6 +19,7 @@
 // One workgroup = 4 waves stacked along the weight rows; they share one token tile of X that is staged per
 // 128-weight block through double-buffered LDS.  Wave w owns up to RT row tiles (16 rows each) and CT token
 // tiles (16 tokens each): RT*CT accumulator tiles, RT decoded A operands reused over CT B operands.
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -336,15 +337,15 @@ __device__ __forceinline__ void load_half(HalfRegs<FMT>& H, __amdgpu_buffer_rsrc
     const uint32_t unit = tile * n_sb + sb;  // wave-uniform
     ok = ok && sb < n_sb;
     if (FMT == OXB_FMT_Q1) {
-        const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rc, (int)(ok ? lane * 16u + half * 8u : OXB_OOB), (int)(unit * 1024u), 0);
+        const v2u v = __builtin_amdgcn_raw_buffer_load_b64(rc, (int)(ok ? lane * 16u : OXB_OOB), (int)(unit * 1024u + half * 8u), 0);
         H.c[0] = v.x, H.c[1] = v.y;
     } else {
-        const v4i v = buf_load_b128(rc, ok ? lane * 16u + half * 1024u : OXB_OOB, unit * 2048u);
+        const v4i v = buf_load_b128(rc, ok ? lane * 16u : OXB_OOB, unit * 2048u + half * 1024u);
         H.c[0] = (uint32_t)v.x, H.c[1] = (uint32_t)v.y, H.c[FMT == OXB_FMT_Q1 ? 0 : 2] = (uint32_t)v.z,
         H.c[FMT == OXB_FMT_Q1 ? 1 : 3] = (uint32_t)v.w;
     }
     // scales of blocks 2 * half and 2 * half + 1 of this lane's row lie side by side
-    const uint32_t sv = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(ok ? r * 8u + half * 4u : OXB_OOB), (int)(unit * 128u), 0);
+    const uint32_t sv = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(ok ? r * 8u : OXB_OOB), (int)(unit * 128u + half * 4u), 0);
     H.d[0] = sv & 0xFFFFu;
     H.d[1] = sv >> 16;
 }
@@ -706,10 +707,13 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 // ---------------------------------------------------------------------------
 // GEMM for up to 128 token rows (decode batches, short prompts).  The wide kernel above would spend its time on barriers
 // and on MFMAs over padding; here the weights stream once at GEMV-like rates.  A workgroup = 8 waves owns RT row
-// tiles; the waves split K (contiguous runs of superblocks), each expands its weights and multiplies them with
-// B operands read straight from the packed activations (they stay in L2, no LDS stage, no barrier in the loop),
+// tiles; the waves split K (contiguous runs of half superblocks, 256 values), each expands its weights and multiplies them
+// with B operands read straight from the packed activations (they stay in L2, no LDS stage, no barrier in the loop),
 // requested D - 1 steps ahead; the eight partial sums meet in LDS and are added in wave order.  What bounds it is the
 // activations' way into the CU: every workgroup takes in all of them, 16 CT rows of K at 64 bytes a clock.
+// Runs of halves and no request past a run against runs of superblocks: 2048 x 6144 (TQ2) at 16 / 77 rows 5.3 -> 4.8 /
+// 10.8 -> 10.0 us, 4096 x 4096 at 77 9.3 -> 8.6, 6144 x 4096 at 16 4.8 -> 4.4; the LM head 151936 x 4096 at 16 rows with
+// the plan below 53 -> 40, 19456 x 2560 (TQ2) at 16 14.1 -> 8.4.
 // Beyond 32 rows against the wide kernel with its 64-token tiles (kernel alone): 4096 x 4096 at 64 / 128 rows 14.9 -> 8.7 /
 // 15.5 -> 13.5 us, 6144 x 4096 at 77 15.8 -> 9.7, 4096 x 2048 (TQ2) at 64 / 128 10.5 -> 5.6 / 11.0 -> 8.2.
 // ---------------------------------------------------------------------------
@@ -729,11 +733,14 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     // RT even): RT/2 consecutive gate tiles and the up tiles of the same rows, so the epilogue holds both factors.
     const bool sw = p.mode == OXB_GEMM_SWIGLU;
     constexpr uint32_t HP = RT > 1 ? RT / 2 : 1;
-    const uint32_t t0 = sw ? blockIdx.x * HP : blockIdx.x * RT;
+    const uint32_t ng = blockIdx.x, ks = blockIdx.y;  // row group, K slice
+    const uint32_t t0 = sw ? ng * HP : ng * RT;
     const uint32_t t_lim = sw ? p.n_tiles / 2 : p.n_tiles;
     auto tile_of = [&](int rt) -> uint32_t { return sw ? ((uint32_t)rt < HP ? t0 + rt : p.n_tiles / 2 + t0 + rt - HP) : t0 + rt; };
     auto valid = [&](int rt) -> bool { return sw ? t0 + ((uint32_t)rt % HP) < t_lim : t0 + rt < t_lim; };
-    const uint32_t per = (p.n_sb + 7u) / 8u, sb0 = wave * per, sb1 = min(sb0 + per, p.n_sb);
+    // the wave's run of half superblocks (two blocks each) of the slice: with 2048 values of K every wave has one
+    const uint32_t s0 = ks * p.sb_per_split * 2u, s1 = min(s0 + p.sb_per_split * 2u, p.n_sb * 2u);
+    const uint32_t per = (s1 - s0 + 7u) / 8u, h0 = s0 + wave * per, h1 = min(h0 + per, s1);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
 
@@ -743,9 +750,9 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) acc[rt][ct] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-    if (sb0 < sb1) {
+    if (h0 < h1) {
         const uint32_t blk_stride = 16u * p.M_pad * 16u;  // bytes of xh per block
-        const uint32_t blk_end = sb1 * 4u;
+        const uint32_t blk_end = h1 * 2u;
         // B operands of step s, token tile ct of a block: chunk 4g + s, token 16 ct + r.  A ring of D steps, D - 1 ahead.
         v8h B[D][CT];
         // One lane offset; step and block go into the wave-uniform part, the token tile into the instruction's constant.
@@ -755,47 +762,54 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) dst[ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, at + ct * 256u, blk * blk_stride + s * p.M_pad * 16u));
         };
-        // RING: the next superblock's weights wait in a second register set; with more than four row tiles there
-        // is no room for one, and a half is requested again in place once its second block has been prepared.
-        constexpr bool RING = RT * CT <= 12 && RT <= 4;
-        HalfRegs<FMT> H[RT][2], Hn[RING ? RT : 1][2];
+        // Two halves of weights in registers: a half is requested again, for the one after next, as soon as both its blocks
+        // have been prepared (with many row tiles only once the second one has: there is no room for two prepared blocks).
+        constexpr bool EARLY = RT <= 4 && RT * CT <= 12;
+        HalfRegs<FMT> H[RT][2];
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
-            load_half<FMT>(H[rt][0], rc, rs, tile_of(rt), valid(rt), p.n_sb, sb0, 0, lane);
-            load_half<FMT>(H[rt][1], rc, rs, tile_of(rt), valid(rt), p.n_sb, sb0, 1, lane);
-        }
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int hh = 0; hh < 2; hh++) load_half<FMT>(H[rt][hh], rc, rs, tile_of(rt), valid(rt) && h0 + hh < h1, p.n_sb, (h0 + hh) >> 1, (int)((h0 + hh) & 1u), lane);
         // (two blocks in registers: the next block's steps are requested together; else step by step)
         constexpr bool BLOCKS = D == 8;
 #pragma unroll
-        for (int j = 0; j < (BLOCKS ? 4 : D - 1); j++) load_b(sb0 * 4u + (j >> 2), j & 3, B[j]);
-        for (uint32_t sb = sb0; sb < sb1; sb++) {
-            // next superblock's weights (all zero past the slice: never used)
-            if (RING) {
+        for (int j = 0; j < (BLOCKS ? 4 : D - 1); j++) load_b(h0 * 2u + (j >> 2), j & 3, B[j]);
+        // The two blocks of half superblock h, weights in set hh.  Where the registers allow the last half its own copy (PEEL),
+        // nothing is requested past the run: a load that is out of range still takes its turn on the way into the CU, which is
+        // what the kernel waits for (with K = 6144 a wave has three halves: 2048 x 6144, TQ2, 16 rows 5.3 -> 4.8 us).
+        constexpr bool PEEL = CT <= 6 && (RT * CT <= 8 || (FMT == OXB_FMT_Q1 && (RT * CT <= 10 || CT <= 3)));
+        auto half = [&](auto hh_c, auto refill_c, auto last_c, uint32_t h) {
+            constexpr int hh = hh_c;
+            constexpr bool REFILL = refill_c, LAST = last_c;
+            BlockDec bd[EARLY ? 2 : 1][RT];
+            auto refill = [&]() {
 #pragma unroll
-                for (int rt = 0; rt < RT; rt++) {
-                    load_half<FMT>(Hn[RING ? rt : 0][0], rc, rs, tile_of(rt), valid(rt) && sb + 1 < sb1, p.n_sb, sb + 1, 0, lane);
-                    load_half<FMT>(Hn[RING ? rt : 0][1], rc, rs, tile_of(rt), valid(rt) && sb + 1 < sb1, p.n_sb, sb + 1, 1, lane);
-                }
+                for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][hh], rc, rs, tile_of(rt), valid(rt) && h + 2 < h1, p.n_sb, (h + 2) >> 1, (int)(h & 1u), lane);
+            };
+            if (EARLY) {
+#pragma unroll
+                for (int bi = 0; bi < 2; bi++)
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) bd[EARLY ? bi : 0][rt] = prepare_block<FMT>(H[rt][hh], bi);
+                if (REFILL) refill();
             }
 #pragma unroll
-            for (int bi = 0; bi < 4; bi++) {
-                if (BLOCKS) {
+            for (int bi = 0; bi < 2; bi++) {
+                if (BLOCKS && !(LAST && bi)) {
 #pragma unroll
-                    for (int s = 0; s < 4; s++) load_b(sb * 4u + bi + 1, s, B[(4 * (bi + 1) + s) % D]);
+                    for (int s = 0; s < 4; s++) load_b(h * 2u + bi + 1, s, B[(4 * (bi + 1) + s) % D]);
                 }
-                BlockDec bd[RT];
+                if (!EARLY) {
 #pragma unroll
-                for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][bi >> 1], bi & 1);
-                if (!RING && (bi & 1) && sb + 1 < sb1) {  // (wave-uniform) both blocks of the half are in bd now
-#pragma unroll
-                    for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][bi >> 1], rc, rs, tile_of(rt), valid(rt), p.n_sb, sb + 1, bi >> 1, lane);
+                    for (int rt = 0; rt < RT; rt++) bd[0][rt] = prepare_block<FMT>(H[rt][hh], bi);
+                    if (REFILL && bi) refill();
                 }
 #pragma unroll
                 for (int s = 0; s < 4; s++) {
                     const int j = 4 * bi + s, jn = j + D - 1;
-                    if (!BLOCKS) load_b(sb * 4u + (jn >> 2), jn & 3, B[jn % D]);
+                    if (!BLOCKS && !(LAST && jn >= 8)) load_b(h * 2u + (jn >> 2), jn & 3, B[jn % D]);
                     v8h A[RT];
-                    decode_step<FMT, RT>(bd, s, A);
+                    decode_step<FMT, RT>(bd[EARLY ? bi : 0], s, A);
 #pragma unroll
                     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
@@ -803,11 +817,21 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
                             acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rt], B[j % D][ct], acc[rt][ct], 0, 0, 0);
                 }
             }
-            if (RING) {
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++) H[rt][0] = Hn[RING ? rt : 0][0], H[rt][1] = Hn[RING ? rt : 0][1];
-            }
+        };
+        constexpr std::integral_constant<int, 0> set0{};
+        constexpr std::integral_constant<int, 1> set1{};
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        uint32_t h = h0;
+        for (; h + 2 < (PEEL ? h1 : h1 + 1); h += 2) {
+            half(set0, yes, no, h);
+            half(set1, yes, no, h + 1);
         }
+        if (PEEL && h + 1 < h1) {
+            half(set0, no, no, h);
+            half(set1, no, yes, h + 1);
+        } else if (h < h1)
+            half(set0, no, yes, h);
     }
     // row tile behind slot q of pass ps: all tiles in order with a single pass; with pairs, SWIGLU mode takes a gate
     // tile and the up tile of the same rows, the plain modes two neighbours
@@ -852,8 +876,9 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
             for (int v = 0; v < 4; v++) o[v] = silu_mul(o[v], u[v]);
         }
-        float* yr = p.y + (size_t)m * p.ldy;
-        const float* rr = p.mode == OXB_GEMM_RESIDUAL ? p.residual + (size_t)m * p.ldy : nullptr;
+        // (with K split over workgroups, slice ks writes its partial sums to plane ks of the workspace)
+        float* yr = p.ksplit > 1 ? p.part + ((size_t)ks * p.M + m) * p.ldy : p.y + (size_t)m * p.ldy;
+        const float* rr = p.mode == OXB_GEMM_RESIDUAL && p.ksplit == 1 ? p.residual + (size_t)m * p.ldy : nullptr;
         const uint32_t n = (t0 + rt) * 16 + 4 * g, n_lim = sw ? p.n_rows / 2 : p.n_rows;
         if (vec_ok && n + 3 < n_lim) {
             if (rr) {
@@ -990,47 +1015,39 @@ static float wide_cost(bool tq2, const OxbGemmParams& p, const GemmPlan& g, uint
     return g.ksplit > 1 ? 1.04f * (us + 2.2f + 0.73e-6f * g.ksplit * p.M * (float)p.n_rows) : us;
 }
 
-// The same for the narrow kernel (416 triples, rms 8 %): every workgroup takes in the whole packed activations, so its
-// time goes with K and the token tiles, little with its row tiles.
-static float narrow_cost(bool tq2, const OxbGemmParams& p, uint32_t rt, uint32_t n_cus) {
-    const uint32_t ct = (p.M + 15) / 16, R = (rt == 1 && ct <= 4) || (rt == 2 && ct == 3 && !tq2) ? 2 : 1;
-    const uint32_t wgs = p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + rt / 2 - 1) / (rt / 2) : (p.n_tiles + rt - 1) / rt, q = (wgs + n_cus - 1) / n_cus;
-    const float n_sb = (float)p.n_sb, busy = 0.119f * n_sb * ct + 0.063f * n_sb * rt * (tq2 ? 2.14f : 1.f), lone = 0.443f + busy;
-    auto round = [&](uint32_t w) { const float b = w * busy; return w == 0 ? 0.f : b > lone ? b : lone; };
-    return 1.34f + (float)(q / R) * round(R) + round(q % R) + 0.197f * q * rt * ct;
+// Time of a narrow plan in us, from 1900 measured (shape, tokens, plan) triples - both formats, 1280 .. 151936 rows, K 1280 ..
+// 12288, 8 .. 128 tokens; rms 4 %; the plan it names is within 1 % of the best on average.  A workgroup's eight waves have a
+// latency (a round trip per half superblock, longer with more row tiles in flight); workgroups that share a CU queue for what
+// each takes in: all of the packed activations and its weights.  What counts is the fullest CU: 384 workgroups of one tile
+// leave half the CUs with two (QKV 6144 x 4096, 32 rows: 8.2 us against 5.9 as 192 workgroups of two tiles), six tiles make
+// gate || up 24576 x 4096 one workgroup per CU (11.8 us; as 384 of four: 16.6), while the LM head's 9496 tiles run best in
+// fours at 16 rows, two workgroups resident (39.6 us against 53 in sixes).
+static float narrow_cost(bool tq2, const OxbGemmParams& p, uint32_t rt, uint32_t ksplit, uint32_t n_cus) {
+    static const uint8_t resident[2][2][2] = {{{4, 2}, {2, 1}}, {{3, 2}, {2, 1}}};  // [format][rt = 1, 2][ct = 1, 2]: workgroups per CU (registers); else one
+    const uint32_t ct = (p.M + 15) / 16, R = rt > 2 || ct > 2 ? 1 : resident[tq2][rt - 1][ct - 1], spk = (p.n_sb + ksplit - 1) / ksplit;
+    const uint32_t wgs = (p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + rt / 2 - 1) / (rt / 2) : (p.n_tiles + rt - 1) / rt) * ksplit;
+    const uint32_t q = (wgs + n_cus - 1) / n_cus;  // workgroups on the CU that gets most
+    const float w_rt = rt * (tq2 ? 1.48f : 1.f), busy = spk * (0.096f * ct + 0.035f * w_rt + 0.012f * rt * ct) + 0.119f * rt * ct;
+    const float lat = 0.18f + (float)((2 * spk + 7) / 8) * 0.192f * w_rt;
+    return 1.91f + (float)(q / R) * (lat + R * busy) + (q % R ? lat + (q % R) * busy : 0.f);
 }
 
 // The narrow kernel up to OXB_GEMM_NARROW_MAX_M token rows (the wide one would spend its time on barriers and padding),
 // the cheaper of the two up to 128, the wide one beyond.
 static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
     const bool tq2 = fmt == OXB_FMT_TQ2, sw = p.mode == OXB_GEMM_SWIGLU;
-    GemmPlan best = {true, sw ? 2u : 1u, 0, 0, 1, p.n_sb};
-    if (p.M <= OXB_GEMM_NARROW_MAX_M) {
-        // Row tiles per workgroup (1, 2, 4 or - Q1 - 6): the count that minimises (rounds of workgroups over the CUs) x (row tiles + 2 - a
-        // workgroup's time grows with its tiles on top of a fixed part: its start, the K-split sum and the epilogue).  What
-        // counts is the last round: 384 workgroups of one tile leave half the CUs with two and the launch as long as those
-        // (QKV 6144 x 4096, 8 rows: 5.5 us against 4.7 us as 192 workgroups of two tiles; 32 rows: 8.2 against 6.1).  A tie
-        // goes to the larger workgroups (every workgroup reads all of the packed activations); 8B-shape decode with this rule
-        // against "as many tiles as leave a workgroup per CU": +2 % at 8 and at 32 sequences.  Six tiles (three gate and three up
-        // tiles in SWIGLU mode) make gate || up 24576 x 4096 one workgroup per CU: at four, the 384 workgroups - one resident per
-        // CU at their register count - ran in two rounds (32 rows: 17.4 -> 13.0 us per launch, the LM head 78 -> 74 us).
-        uint64_t best_cost = ~0ull;
-        static const uint32_t choices[4] = {1, 2, 4, 6};
-        for (uint32_t ci = sw ? 1 : 0; ci < (tq2 ? 3u : 4u); ci++) {  // (six tiles: Q1 only - the ternary decoder's registers do not fit)
-            const uint32_t r = choices[ci];
-            const uint32_t wgs = sw ? (p.n_tiles / 2 + r / 2 - 1) / (r / 2) : (p.n_tiles + r - 1) / r;
-            const uint64_t cost = (uint64_t)((wgs + n_cus - 1) / n_cus) * (r + 2);
-            if (cost <= best_cost) best_cost = cost, best.rt = r;
-        }
-        return best;
-    }
+    GemmPlan best = {true, 0, 0, 0, 1, p.n_sb};
     float best_us = 1e30f;
     if (p.M <= 128) {
-        const uint32_t ct = (p.M + 15) / 16;
-        for (uint32_t rt = sw ? 2 : 1; rt <= (ct <= 4 ? 4u : ct <= 7 ? 2u : 1u); rt *= 2) {
-            const float us = narrow_cost(tq2, p, rt, n_cus);
+        // row tiles per workgroup: as many as the registers hold next to the token tiles (six: Q1 only), two or more with SWIGLU
+        static const uint32_t choices[4] = {1, 2, 4, 6};
+        const uint32_t ct = (p.M + 15) / 16, most = ct <= 2 && !tq2 ? 6 : ct <= 4 ? 4 : ct <= 7 ? 2 : 1;
+        for (uint32_t rt : choices) {
+            if (rt > most || (sw && rt == 1)) continue;
+            const float us = narrow_cost(tq2, p, rt, 1, n_cus);
             if (us < best_us) best_us = us, best.rt = rt;
         }
+        if (p.M <= OXB_GEMM_NARROW_MAX_M) return best;
     }
     static const uint32_t cts[3] = {8, 5, 4}, splits[5] = {1, 2, 3, 4, 6};
     const bool can_split = (p.ldy & 3u) == 0 && !sw && !p.no_split;  // (the SwiGLU epilogue is not linear)
@@ -1051,14 +1068,12 @@ static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
 
 template <int FMT, int RT, int CT>
 static hipError_t launch_narrow_case(const OxbGemmParams& p, hipStream_t st) {
-    const uint32_t grid = p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + RT / 2 - 1) / (RT > 1 ? RT / 2 : 1) : (p.n_tiles + RT - 1) / RT;
-    hipLaunchKernelGGL((gemm_narrow_kernel<FMT, RT, CT>), dim3(grid), dim3(OXB_GEMM_NARROW_THREADS), 0, st, p);
+    hipLaunchKernelGGL((gemm_narrow_kernel<FMT, RT, CT>), dim3(p.n_ng, p.ksplit), dim3(OXB_GEMM_NARROW_THREADS), 0, st, p);
     return hipGetLastError();
 }
 
 static hipError_t launch_gemm_narrow(int fmt, OxbGemmParams p, uint32_t rt, hipStream_t st) {
-    p.ksplit = 1;
-    p.sb_per_split = p.n_sb;
+    p.n_ng = p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + rt / 2 - 1) / (rt > 1 ? rt / 2 : 1) : (p.n_tiles + rt - 1) / rt;
     const uint32_t ct = p.M_pad / 16;
 #define OXB_NARROW_CASE(F, R, C) \
     if (fmt == F && rt == R && ct == C) return launch_narrow_case<F, R, C>(p, st);
@@ -1088,11 +1103,11 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     if (p.mode == OXB_GEMM_SWIGLU && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // whole gate and up row tiles
     p.M_pad = (p.M + 15u) / 16u * 16u;
     const GemmPlan plan = plan_gemm(fmt, p, n_cus);
-    if (plan.narrow) return launch_gemm_narrow(fmt, p, plan.rt, st);
-    p.n_mt = (p.M + 16 * plan.ct - 1) / (16 * plan.ct);
     p.ksplit = plan.ksplit;
     p.sb_per_split = plan.sb_per_split;
     if (p.ksplit > 1 && !p.part) return hipErrorInvalidValue;
+    if (plan.narrow) return launch_gemm_narrow(fmt, p, plan.rt, st);
+    p.n_mt = (p.M + 16 * plan.ct - 1) / (16 * plan.ct);
     p.tpw = plan.tpw;
     p.n_ng = (p.n_tiles + p.tpw - 1) / p.tpw;
     const uint32_t grid = p.n_ng * p.n_mt * p.ksplit;
