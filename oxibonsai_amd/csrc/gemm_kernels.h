@@ -28,6 +28,7 @@ struct OxbGemmParams {
     uint32_t codes_bytes, scales_bytes, xh_bytes;  // buffer extents (loads beyond them read 0)
     int mode;
     bool no_split;           // keep K in one piece (a caller without room for partial sums)
+    bool sum_later;          // mode RESIDUAL: with K in slices leave the sums in `part`, the next pack of y adds them (OxbPackSum)
 };
 
 // Bytes of the packed activation buffer for M token rows of length k.
@@ -38,8 +39,12 @@ size_t oxb_xh_bytes(uint32_t k, uint32_t M);
 //   IDENT: a = x;  RMSNORM: a = w * x / rms(x) (w = d_w[k]).
 // d_rowmul: M floats of scratch (the multiplier applied to every row).
 enum { OXB_PACK_IDENT = 0, OXB_PACK_RMSNORM = 1 };
+// With `sum` (RMSNORM, ldx = k, a shape that oxb_pack_can_sum takes) x lacks the K slices' sums of the product it is the
+// result of: x += planes 0 .. n - 1, in that order, then as above; x is written back.
+struct OxbPackSum { const float* part; uint32_t n; size_t plane; };
+bool oxb_pack_can_sum(uint32_t k, uint32_t M);
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
-                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st);
+                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr);
 // Number of K slices the launcher will use for this shape (1: no workspace needed).
 uint32_t oxb_gemm_ksplit(int fmt, const OxbGemmParams& p, uint32_t n_cus);
 hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st);

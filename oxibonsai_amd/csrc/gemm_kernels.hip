@@ -149,6 +149,8 @@ __device__ __forceinline__ void item_offsets(uint32_t blk, uint32_t c, uint32_t*
     *o1 = *o0 + (FMT == OXB_FMT_Q1 ? 16 : 8);
 }
 
+__device__ __forceinline__ float4 add4(const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+
 // Both steps in one launch for a few token rows (decode batches): one workgroup per token row, one pass over the row.
 // A thread requests all of its items - the pieces it will pack, NI of them for rows of up to 2048 NI values - before
 // it uses any, keeps them in registers while the workgroup finds the row's multiplier, and packs them from there;
@@ -156,10 +158,12 @@ __device__ __forceinline__ void item_offsets(uint32_t blk, uint32_t c, uint32_t*
 // as its chain of memory round trips: this way it is one for the row and one for the store.  (The sum of squares adds
 // the row's values in another order than row_stats does: the multiplier may differ from the two-kernel route's in the
 // last bit, within what fp16 activations already cost.)
-template <int FMT, int OP, int NI>
-__global__ __launch_bounds__(256) void xh_pack_rows_kernel(const float* __restrict__ x, const float* __restrict__ w, uint32_t ldx,
+// SUM: x is a product's residual whose partial sums still lie in sum.n planes; they are added here, in slice order, and
+// x is written back (a launch of its own for that costs as much as the slices save).
+template <int FMT, int OP, int NI, bool SUM>
+__global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float* __restrict__ w, uint32_t ldx,
                                                             uint32_t k, float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh) {
+                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh, const OxbPackSum sum) {
     __shared__ float red_s[4], red_m[4];
     __shared__ int red_b[4];
     __shared__ float mul_s;
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(const float* __restri
         for (uint32_t id = tid; id < n_items; id += 256) xh[(size_t)id * M_pad + m] = make_uint4(0, 0, 0, 0);
         return;
     }
-    const float* xr = x + (size_t)m * ldx;
+    float* xr = x + (size_t)m * ldx;
     float4 a[NI], b[NI], wa[NI], wb[NI];
 #pragma unroll
     for (int it = 0; it < NI; it++) {
@@ -181,6 +185,44 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(const float* __restri
         if (OP == OXB_PACK_RMSNORM) {
             wa[it] = ok ? *reinterpret_cast<const float4*>(w + o0) : make_float4(0.f, 0.f, 0.f, 0.f);
             wb[it] = ok ? *reinterpret_cast<const float4*>(w + o1) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    if (SUM) {
+        const float* pr = sum.part + (size_t)m * ldx;
+        float4 ta[NI], tb[NI];
+        for (uint32_t s0 = 0; s0 < sum.n; s0 += 4) {  // four planes requested together
+            float4 pa[4][NI], pb[4][NI];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+#pragma unroll
+                for (int it = 0; it < NI; it++) {
+                    const uint32_t id = it * 256 + tid;
+                    uint32_t o0, o1;
+                    item_offsets<FMT>(id >> 4, id & 15u, &o0, &o1);
+                    const bool ok = s0 + j < sum.n && id < n_items && (id >> 4) * 128 < k;
+                    const float* q = pr + (s0 + j) * sum.plane;
+                    pa[j][it] = ok ? *reinterpret_cast<const float4*>(q + o0) : make_float4(0.f, 0.f, 0.f, 0.f);
+                    pb[j][it] = ok ? *reinterpret_cast<const float4*>(q + o1) : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+#pragma unroll
+                for (int it = 0; it < NI; it++) {
+                    ta[it] = s0 + j == 0 ? pa[j][it] : add4(ta[it], pa[j][it]);
+                    tb[it] = s0 + j == 0 ? pb[j][it] : add4(tb[it], pb[j][it]);
+                }
+        }
+#pragma unroll
+        for (int it = 0; it < NI; it++) {
+            const uint32_t id = it * 256 + tid;
+            uint32_t o0, o1;
+            item_offsets<FMT>(id >> 4, id & 15u, &o0, &o1);
+            a[it] = add4(ta[it], a[it]);
+            b[it] = add4(tb[it], b[it]);
+            if (id < n_items && (id >> 4) * 128 < k) {
+                *reinterpret_cast<float4*>(xr + o0) = a[it];
+                *reinterpret_cast<float4*>(xr + o1) = b[it];
+            }
         }
     }
     float ss = 0.f, mx = 0.f;
@@ -225,10 +267,11 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(const float* __restri
 // launches.  What bounds it is the way into and out of a CU (64 bytes a clock each) and, for few rows, the chain of one
 // memory round trip, two barriers and the stores.  A layer's four packs, 8B shape, two launches each before: 2048 rows
 // 93 -> 56 us, 301 rows 41 -> 26 us.
-template <int FMT, int OP, int RPW, int NI>
-__global__ __launch_bounds__(512) void xh_pack_wide_kernel(const float* __restrict__ x, const float* __restrict__ w, uint32_t ldx, uint32_t k,
+// (SUM as in xh_pack_rows_kernel.)
+template <int FMT, int OP, int RPW, int NI, bool SUM>
+__global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float* __restrict__ w, uint32_t ldx, uint32_t k,
                                                             float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh) {
+                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh, const OxbPackSum sum) {
     constexpr int WPR = 8 / RPW, SEG = NI <= 16 ? NI : NI == 48 ? 16 : 12;
     static_assert(NI % SEG == 0, "whole segments");
     constexpr uint32_t VALS = SEG * 256 * WPR, STR = VALS + 16;  // values of a row in a segment; LDS row stride (32 bytes of padding spread the rows over the banks)
@@ -239,11 +282,27 @@ __global__ __launch_bounds__(512) void xh_pack_wide_kernel(const float* __restri
     const uint32_t tid = threadIdx.x, lane = tid & 63u, m0 = blockIdx.x * RPW;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), wr = wave / WPR, part = wave % WPR, m = m0 + wr;
     const bool live = m < M;
-    const float* xr = x + (size_t)(live ? m : 0) * ldx;
+    float* xr = x + (size_t)(live ? m : 0) * ldx;
     auto at_of = [&](int i) -> uint32_t { return ((i * WPR + part) * 64 + lane) * 4; };
     float4 a[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) a[i] = live && at_of(i) < k ? *reinterpret_cast<const float4*>(xr + at_of(i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (SUM && live) {
+        const float* pr = sum.part + (size_t)m * ldx;
+        float4 t[NI];
+        for (uint32_t s = 0; s < sum.n; s++) {
+            float4 q[NI];
+#pragma unroll
+            for (int i = 0; i < NI; i++) q[i] = at_of(i) < k ? *reinterpret_cast<const float4*>(pr + s * sum.plane + at_of(i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < NI; i++) t[i] = s == 0 ? q[i] : add4(t[i], q[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            a[i] = add4(t[i], a[i]);
+            if (at_of(i) < k) *reinterpret_cast<float4*>(xr + at_of(i)) = a[i];
+        }
+    }
     float ss = 0.f, mx = 0.f;
     int bad = 0;
 #pragma unroll
@@ -895,7 +954,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     }
 }
 
-// y = (residual +) the K slices' partial sums, added in slice order (deterministic).
+// y = (residual +) the K slices' partial sums, added in slice order (deterministic): where no pack of the result follows.
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, uint32_t ksplit, size_t plane,
                                                                   const float* __restrict__ residual, float* __restrict__ y,
                                                                   size_t n4) {
@@ -923,22 +982,23 @@ size_t oxb_xh_bytes(uint32_t k, uint32_t M) {
 
 #define OXB_PACK_ROWS_MAX 64  // up to this many token rows (of at most 16384 values) the one-launch packer is used
 
-template <int OP>
-static void launch_pack_op(int fmt, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, uint32_t M, uint32_t M_pad,
-                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st) {
+template <int OP, bool SUM>
+static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, uint32_t k, uint32_t M, uint32_t M_pad,
+                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, const OxbPackSum& sum, hipStream_t st) {
     const uint32_t per_thread = (nblk_pad * 16 + 255) / 256;  // items of a row per thread of the one-launch packer
     if (M <= OXB_PACK_ROWS_MAX && per_thread <= 8) {
 #define OXB_ROWS_CASE(NI)                                                                                                      \
     if (per_thread <= NI) {                                                                                                    \
         if (fmt == OXB_FMT_Q1)                                                                                                 \
-            hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_Q1, OP, NI>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                        \
+            hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_Q1, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
+                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         else                                                                                                                   \
-            hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_TQ2, OP, NI>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                        \
+            hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_TQ2, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
+                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         return;                                                                                                                \
     }
-        OXB_ROWS_CASE(1) OXB_ROWS_CASE(2) OXB_ROWS_CASE(4) OXB_ROWS_CASE(6) OXB_ROWS_CASE(8)
+        OXB_ROWS_CASE(1) OXB_ROWS_CASE(2) OXB_ROWS_CASE(4)
+        if constexpr (!SUM) { OXB_ROWS_CASE(6) OXB_ROWS_CASE(8) }
 #undef OXB_ROWS_CASE
     }
     // Four rows per workgroup, two where four would leave half the CUs idle; eight for long rows where each CU has a
@@ -947,36 +1007,47 @@ static void launch_pack_op(int fmt, const float* d_x, const float* d_w, uint32_t
 #define OXB_WIDE_CASE(RPW, NI)                                                                                                     \
     if (rpw == RPW && per_lane <= NI) {                                                                                            \
         if (fmt == OXB_FMT_Q1)                                                                                                     \
-            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_Q1, OP, RPW, NI>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                 \
+            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_Q1, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                            \
         else                                                                                                                       \
-            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_TQ2, OP, RPW, NI>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh));                                 \
+            hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_TQ2, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                            \
         return;                                                                                                                    \
     }
     OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16) OXB_WIDE_CASE(4, 24) OXB_WIDE_CASE(2, 4) OXB_WIDE_CASE(2, 8) OXB_WIDE_CASE(2, 12)
     if constexpr (OP == OXB_PACK_IDENT) { OXB_WIDE_CASE(8, 48) }
     // (rows of more than 12288 values take two launches)
 #undef OXB_WIDE_CASE
-    hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh);
-    const dim3 grid(M_pad / 16, nblk_pad < 16 ? nblk_pad : 16);
-    if (fmt == OXB_FMT_Q1)
-        hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_Q1, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
-                           reinterpret_cast<uint4*>(d_xh));
-    else
-        hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_TQ2, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
-                           reinterpret_cast<uint4*>(d_xh));
+    if constexpr (!SUM) {
+        hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh);
+        const dim3 grid(M_pad / 16, nblk_pad < 16 ? nblk_pad : 16);
+        if (fmt == OXB_FMT_Q1)
+            hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_Q1, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
+                               reinterpret_cast<uint4*>(d_xh));
+        else
+            hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_TQ2, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
+                               reinterpret_cast<uint4*>(d_xh));
+    }
 }
 
+bool oxb_pack_can_sum(uint32_t k, uint32_t M) { return k <= (M <= OXB_PACK_ROWS_MAX ? 8192u : 12288u) && (k % OXB_QK) == 0; }
+
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
-                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st) {
+                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum) {
     if (M == 0 || k == 0 || (k % OXB_QK) != 0 || (ldx & 3u) != 0) return hipErrorInvalidValue;
     if (op == OXB_PACK_RMSNORM && !d_w) return hipErrorInvalidValue;
     const uint32_t nblk_pad = ((k + 511u) / 512u) * 4u, M_pad = (M + 15u) / 16u * 16u;
     if (oxb_xh_bytes(k, M) >= 0xFFFFFFF0ull) return hipErrorInvalidValue;
+    float* x = const_cast<float*>(d_x);  // (written with `sum` only)
+    if (sum && sum->n > 1) {
+        if (op != OXB_PACK_RMSNORM || !oxb_pack_can_sum(k, M) || ldx != k) return hipErrorInvalidValue;
+        launch_pack_op<OXB_PACK_RMSNORM, true>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, *sum, st);
+        return hipGetLastError();
+    }
+    const OxbPackSum none = {nullptr, 0, 0};
     switch (op) {
-        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT>(fmt, d_x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, st); break;
-        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM>(fmt, d_x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, st); break;
+        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, none, st); break;
+        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, none, st); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1011,8 +1082,8 @@ static float wide_cost(bool tq2, const OxbGemmParams& p, const GemmPlan& g, uint
     const float lone = lone_us[tq2][ci][ri] + (p.n_sb > 9 ? long_k_us[ci][ri] : 0.f), busy = busy_us[tq2][ci][ri];
     auto round = [&](uint32_t w) { const float b = w * busy; return w == 0 ? 0.f : b > lone ? b : lone; };
     const float us = 4.4f + 4.f * g.sb_per_split * ((float)(q / R) * round(R) + round(q % R)) + 0.158f * q * g.rt * g.ct;
-    // a K split writes its partial sums and adds them in a launch of its own
-    return g.ksplit > 1 ? 1.04f * (us + 2.2f + 0.73e-6f * g.ksplit * p.M * (float)p.n_rows) : us;
+    // a K split writes its partial sums and adds them in a launch of its own, or leaves them to the next pack
+    return g.ksplit > 1 ? 1.04f * (us + (p.sum_later ? 0.6f : 2.2f) + 0.73e-6f * g.ksplit * p.M * (float)p.n_rows) : us;
 }
 
 // Time of a narrow plan in us, from 1900 measured (shape, tokens, plan) triples - both formats, 1280 .. 151936 rows, K 1280 ..
@@ -1044,8 +1115,14 @@ static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
         const uint32_t ct = (p.M + 15) / 16, most = ct <= 2 && !tq2 ? 6 : ct <= 4 ? 4 : ct <= 7 ? 2 : 1;
         for (uint32_t rt : choices) {
             if (rt > most || (sw && rt == 1)) continue;
-            const float us = narrow_cost(tq2, p, rt, 1, n_cus);
-            if (us < best_us) best_us = us, best.rt = rt;
+            // K in slices where the next pack adds them anyway: with few row tiles they fill the chip, and a workgroup takes in
+            // its slice of the activations only (4096 x 12288, 32 rows: 9.6 us whole, 7.7 in four slices of 64 workgroups)
+            for (uint32_t ks = 1; ks <= (p.sum_later ? 4u : 1u); ks++) {
+                const uint32_t spk = (p.n_sb + ks - 1) / ks;
+                if ((p.n_sb + spk - 1) / spk != ks || (ks > 1 && (p.n_tiles + rt - 1) / rt * ks > 2 * n_cus)) continue;
+                const float us = narrow_cost(tq2, p, rt, ks, n_cus) + (ks > 1 ? 0.3f + 0.3f * ks : 0.f);
+                if (us < best_us) best_us = us, best.rt = rt, best.ksplit = ks, best.sb_per_split = spk;
+            }
         }
         if (p.M <= OXB_GEMM_NARROW_MAX_M) return best;
     }
@@ -1119,7 +1196,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     OXB_GEMM_CASE(1, 5) OXB_GEMM_CASE(2, 5) OXB_GEMM_CASE(3, 5) OXB_GEMM_CASE(4, 5)
     OXB_GEMM_CASE(1, 4) OXB_GEMM_CASE(2, 4) OXB_GEMM_CASE(3, 4) OXB_GEMM_CASE(4, 4)
 #undef OXB_GEMM_CASE
-    if (err != hipSuccess || p.ksplit == 1) return err;
+    if (err != hipSuccess || p.ksplit == 1 || p.sum_later) return err;
     const size_t plane = (size_t)p.M * p.ldy, n4 = plane / 4;
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, st, p.part, p.ksplit, plane,
                        p.mode == OXB_GEMM_RESIDUAL ? p.residual : nullptr, p.y, n4);

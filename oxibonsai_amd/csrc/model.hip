@@ -271,9 +271,9 @@ static int size_gemm_workspaces(Model& m) {
     uint32_t kx = d.h > d.inter ? d.h : d.inter;
     if (qd > kx) kx = qd;
     size_t part_bytes = 0;
-    const struct { uint64_t id; uint32_t n, k; } shapes[] = {{m.layers[0].qkv, qkv_rows, d.h}, {m.layers[0].o, d.h, qd},
-                                                             {m.layers[0].gate_up, 2 * d.inter, d.h},
-                                                             {m.layers[0].down, d.h, d.inter}, {d.lm_head, d.vocab, d.h}};
+    const struct { uint64_t id; uint32_t n, k; int mode; } shapes[] = {{m.layers[0].qkv, qkv_rows, d.h, OXB_GEMM_STORE}, {m.layers[0].o, d.h, qd, OXB_GEMM_RESIDUAL},
+                                                                       {m.layers[0].gate_up, 2 * d.inter, d.h, OXB_GEMM_SWIGLU},
+                                                                       {m.layers[0].down, d.h, d.inter, OXB_GEMM_RESIDUAL}, {d.lm_head, d.vocab, d.h, OXB_GEMM_STORE}};
     for (const auto& sh : shapes) {
         const Weight* w = find_weight(sh.id);
         if (!w) continue;  // a model without an LM head
@@ -284,6 +284,8 @@ static int size_gemm_workspaces(Model& m) {
         gp.n_sb = w->L.n_sb;
         gp.M = d.batch;
         gp.ldy = sh.n;
+        gp.mode = sh.mode;
+        gp.sum_later = sh.mode == OXB_GEMM_RESIDUAL && oxb_pack_can_sum(sh.n, d.batch);
         const size_t b = (size_t)oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus) * d.batch * sh.n * sizeof(float);
         if (oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus) > 1 && b > part_bytes) part_bytes = b;
     }
@@ -393,6 +395,7 @@ static int encode_decode_step_gemm(Model& m) {
     hipStream_t st = g_rt.stream;
     const uint32_t qd = d.nq * d.hd, kd = d.nkv * d.hd, qkv_rows = qd + 2 * kd, B = d.batch;
     int rc = OXB_HIP_OK;
+    OxbPackSum sum = {nullptr, 0, 0};  // partial sums that the next pack adds to m.hidden
     for (uint32_t L = 0; L < d.n_layers; L++) {
         const oxb_layer_ids& ly = m.layers[L];
         const float* attn_norm = vec_ptr(ly.attn_norm, d.h, "attn_norm", &rc);
@@ -404,17 +407,17 @@ static int encode_decode_step_gemm(Model& m) {
         const Weight* wgu = mat_ptr(ly.gate_up, d.fmt, 2 * d.inter, d.h, "gate_up", &rc);
         const Weight* wdn = mat_ptr(ly.down, d.fmt, d.h, d.inter, "down", &rc);
         if (rc) return rc;
-        OXB_TRY(gemm_device(*wqkv, m.hidden, d.h, m.qkv, B, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, &m.gws));
+        OXB_TRY(gemm_device(*wqkv, m.hidden, d.h, m.qkv, B, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, &m.gws, &sum));
         OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm));
-        OXB_TRY(gemm_device(*wo, m.attn_out, qd, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws));
+        OXB_TRY(gemm_device(*wo, m.attn_out, qd, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum));
         // SwiGLU in the epilogue of the gate || up product
-        OXB_TRY(gemm_device(*wgu, m.hidden, d.h, m.gu, B, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, &m.gws));
-        OXB_TRY(gemm_device(*wdn, m.gu, d.inter, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws));
+        OXB_TRY(gemm_device(*wgu, m.hidden, d.h, m.gu, B, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, &m.gws, &sum));
+        OXB_TRY(gemm_device(*wdn, m.gu, d.inter, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum));
     }
     const float* final_norm = vec_ptr(d.final_norm, d.h, "final_norm", &rc);
     const Weight* lm = mat_ptr(d.lm_head, d.fmt, d.vocab, d.h, "lm_head", &rc);
     if (rc) return rc;
-    OXB_TRY(gemm_device(*lm, m.hidden, d.h, m.logits, B, d.vocab, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, final_norm, d.eps, &m.gws));
+    OXB_TRY(gemm_device(*lm, m.hidden, d.h, m.logits, B, d.vocab, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, final_norm, d.eps, &m.gws, &sum));
     OXB_TRY_HIP(oxb_launch_argmax(m.logits, d.vocab, B, m.tokens, m.argmax_ws, st, m.h_tokens), "kernel launch failed: argmax");
     return OXB_HIP_OK;
 }
@@ -502,6 +505,7 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
     hipStream_t st = g_rt.stream;
     const uint32_t qd = d.nq * d.hd, kd = d.nkv * d.hd, qkv_rows = qd + 2 * kd;
     int rc = OXB_HIP_OK;
+    OxbPackSum sum = {nullptr, 0, 0};  // partial sums that the next pack adds to m.pf_hidden
     for (uint32_t L = 0; L < d.n_layers; L++) {
         const oxb_layer_ids& ly = m.layers[L];
         const float* attn_norm = vec_ptr(ly.attn_norm, d.h, "attn_norm", &rc);
@@ -513,7 +517,7 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
         const Weight* wgu = mat_ptr(ly.gate_up, d.fmt, 2 * d.inter, d.h, "gate_up", &rc);
         const Weight* wdn = mat_ptr(ly.down, d.fmt, d.h, d.inter, "down", &rc);
         if (rc) return rc;
-        OXB_TRY(gemm_device(*wqkv, m.pf_hidden, d.h, m.pf_qkv, M, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps));
+        OXB_TRY(gemm_device(*wqkv, m.pf_hidden, d.h, m.pf_qkv, M, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, nullptr, &sum));
         OxbQkParams qp;
         qp.qkv = m.pf_qkv;
         qp.qkv_stride = qkv_rows;
@@ -567,10 +571,12 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
         OXB_TRY(m.pf_part.ensure(oxb_attn_prefill_part_bytes(ap, g_rt.n_cus)));
         ap.part = (float*)m.pf_part.ptr;
         OXB_TRY_HIP(oxb_launch_attn_prefill(ap, g_rt.n_cus, st), "kernel launch failed: attn_prefill");
-        OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f));
+        OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr, &sum));
         // SwiGLU in the epilogue of the gate || up product: the activation [M][inter] is all that is written
-        OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps));
-        OXB_TRY(gemm_device(*wdn, m.pf_gu, d.inter, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f));
+        OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, nullptr, &sum));
+        // (no pack follows the last layer)
+        OXB_TRY(gemm_device(*wdn, m.pf_gu, d.inter, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr,
+                            L + 1 < d.n_layers ? &sum : nullptr));
     }
     if (!d.lm_head) return OXB_HIP_OK;  // the caller asked for the cache rows only
     // last token: final norm, LM head, greedy token (fp32-exact products, as in a decode step)

@@ -280,7 +280,7 @@ int gemv_device(const Weight& w, const float* d_x, float* d_y, uint32_t batch, u
 }
 
 int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uint32_t m, uint32_t ldy, int mode,
-                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws) {
+                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws, OxbPackSum* carry) {
     if (!ws) ws = &g_rt.gemm_ws;
     const uint32_t k = w.L.k;
     if ((uint64_t)m * k >= (1ull << 31))
@@ -290,8 +290,9 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
     if ((rc = ws->xsh.ensure(((size_t)m + 16) * sizeof(int32_t)))) return rc;
     if ((rc = ws->rowmul.ensure(((size_t)m + 16) * sizeof(float)))) return rc;
     hipError_t e = oxb_launch_xh_pack((int)w.L.fmt, pack_op, d_x, d_pack_w, ldx, k, eps, m, (float*)ws->rowmul.ptr,
-                                      (uint32_t*)ws->xh.ptr, (int32_t*)ws->xsh.ptr, g_rt.stream);
+                                      (uint32_t*)ws->xh.ptr, (int32_t*)ws->xsh.ptr, g_rt.stream, pack_op == OXB_PACK_RMSNORM ? carry : nullptr);
     if (e != hipSuccess) return hip_fail(e, "kernel launch failed: xh_pack");
+    if (carry) carry->n = 0;
     OxbGemmParams p;
     memset(&p, 0, sizeof p);
     p.codes = w.d_codes;
@@ -310,10 +311,12 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
     p.xh_bytes = (uint32_t)oxb_xh_bytes(k, m);
     p.mode = mode;
     p.no_split = ws->no_split;
+    p.sum_later = carry && mode == OXB_GEMM_RESIDUAL && ldy == w.L.n_rows && oxb_pack_can_sum(ldy, m);
     const uint32_t ksplit = oxb_gemm_ksplit((int)w.L.fmt, p, g_rt.n_cus);
     if (ksplit > 1) {
         if ((rc = ws->part.ensure((size_t)ksplit * m * ldy * sizeof(float)))) return rc;
         p.part = (float*)ws->part.ptr;
+        if (p.sum_later) *carry = {p.part, ksplit, (size_t)m * ldy};
     }
     e = oxb_launch_gemm((int)w.L.fmt, p, g_rt.n_cus, g_rt.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch failed: gemm");

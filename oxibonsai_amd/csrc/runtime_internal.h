@@ -8,6 +8,7 @@
 #include <string>
 #include <unordered_map>
 
+#include "gemm_kernels.h"
 #include "layout.h"
 
 namespace oxb {
@@ -89,8 +90,11 @@ uint32_t gemv_packed_min_batch(uint32_t k);
 // x (device, [m][ldx]) -> y (device, [m][ldy]) through the fp16 packer + MFMA GEMM.  pack_op (OXB_PACK_*) names the
 // row-wise producer fused into the packer: RMSNorm with weights d_pack_w and eps, or SwiGLU of x = [gate | up].
 // ws = nullptr uses (and may grow) the runtime's shared workspace.
+// With `carry` a residual product may leave its K slices' sums in the workspace (carry->n planes); the next product, which
+// packs the same rows through RMSNorm in the same workspace, is given the same carry and adds them.
 int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uint32_t m, uint32_t ldy, int mode,
-                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws = nullptr);
+                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws = nullptr,
+                OxbPackSum* carry = nullptr);
 void shutdown_models();
 
 // Every `int` entry point of the C ABI runs its body between these two, so that no C++ exception (a failed host
