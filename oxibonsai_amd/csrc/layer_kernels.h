@@ -32,19 +32,19 @@ struct OxbAttnParams {
     void *k_cache, *v_cache;             // cache rows of hd values each (fp16, or one-byte codes: kv_mode), placed by `kv`
     float *k_scale, *v_scale;            // quantised cache: one scale per row
     uint32_t kv_mode;                    // OXB_KV_* (kv_quant_device.h)
-    OxbKvLayout kv;                      // contiguous (row_stride a multiple of the chunk, >= max_seq) or paged (pages of 16..128 positions)
+    OxbKvLayout kv;                      // contiguous (row_stride a multiple of 128, >= max_seq) or paged (pages of 16..128 positions)
     uint32_t window, sinks;              // sliding window with attention sinks; window 0 = off
     float* part;                         // [batch][nq][n_splits][hd + OXB_ATTN_PART_PAD]: un-normalised output, maximum, sum
-    float* out_single;                   // optional, n_splits == 1 only: [batch][nq*hd] receives the finished output (no merge launch)
-    float* out_merged;                   // n_splits > 1: [batch][nq*hd], written by the last workgroup of each (sequence, kv head) to finish
+    float* out;                          // [batch][nq*hd], written by the last workgroup of each (sequence, kv head) to finish
     uint32_t* done;                      // n_splits > 1: [batch][nkv] arrival counters, zero before the launch; the kernel leaves them zero
     const uint32_t* pos;                 // [batch], device; seq_len = pos + 1
-    uint32_t nq, nkv, hd, max_seq, n_layers, layer, chunk, n_splits;
+    uint32_t nq, nkv, hd, max_seq, n_layers, layer, n_splits;
+    uint32_t wide;                       // eight waves (256 positions at a time) instead of four (128): one-byte rows and hd <= 128 only
     float scale;                         // 1 / sqrt(hd)
     // Optional: the workgroup that merges the slots of (sequence b, kv head) also leaves its 512 outputs quantised for
     // the O projection's packed GEMV (gemv_pack_device.h) as superblock `kv head` of vector b - instead of a pack launch
-    // between the two kernels.  Only where a kv head's q heads are exactly one superblock (nq / nkv * hd == 512) and the
-    // slots are merged in the kernel (n_splits > 1); pack_fmt = the O weight's format.
+    // between the two kernels.  Only where a kv head's q heads are exactly one superblock (nq / nkv * hd == 512);
+    // pack_fmt = the O weight's format.
     uint32_t* pack_out;                  // nullptr = off
     uint32_t pack_fmt, pack_n_sb, pack_nvg;
 };
@@ -55,7 +55,7 @@ hipError_t oxb_launch_kv_dequantize_rows(int kv_mode, const uint8_t* d_codes, co
 hipError_t oxb_launch_kv_quantize_rows(int kv_mode, const float* d_x, uint32_t n_rows, uint32_t n, uint8_t* d_codes, float* d_scales,
                                        hipStream_t st);
 hipError_t oxb_launch_qk_norm_rope_store(const OxbQkParams& p, uint32_t batch, hipStream_t st);
-#define OXB_ATTN_CHUNK_POSITIONS 128  // KV positions one attention workgroup covers at a time
+#define OXB_ATTN_CHUNK_POSITIONS 128  // KV positions a four-wave attention workgroup covers at a time
 #define OXB_ATTN_MAX_SPLITS 64        // slots the KV sequence is split over; slot s walks chunks s, s + n_splits, ...
 #define OXB_ATTN_PART_PAD 4           // floats after the hd outputs of a slot: maximum, sum, 2 unused (16-byte rows)
 // QK-norm, RoPE, KV store of the new position, split-KV attention (at most 16 q heads per kv head) into p.part and

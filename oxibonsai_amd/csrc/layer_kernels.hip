@@ -191,23 +191,21 @@ hipError_t oxb_launch_kv_quantize_rows(int kv_mode, const float* d_x, uint32_t n
     return hipGetLastError();
 }
 
-#define OXB_ATTN_CHUNK 128  // KV positions per chunk of the split-KV decode attention
-
 // ---------------------------------------------------------------------------
 // Decode attention, split over the KV sequence (flash-decode), on the matrix cores: softmax(q K^T / sqrt(hd)) V
 // with GQA (kv_head = q_head / (nq / nkv)) over positions 0..pos[b]
 // (batched_attn_scores_v2 / batched_softmax / batched_attn_weighted_sum, cuda_attn_kernels.rs:264-438;
 //  CPU: block/functions.rs:78-127 -> layers/attention_fused.rs:329-400), fused with what precedes it in the layer:
 // per-head QK-RMSNorm, RoPE and the FP16 store of the new position's K and V (fused_qk_norm_rope + fused_kv_store,
-// cuda_attn_kernels.rs:160-251).  Grid (n_splits, nkv, batch), 256 threads = 4 waves.  It writes, per q head and
+// cuda_attn_kernels.rs:160-251).  Grid (n_splits, nkv, batch), NW = 4 or 8 waves.  It writes, per q head and
 // slot, the un-normalised partial output, the running maximum and the running sum; the last workgroup of a
 // (sequence, kv head) to finish merges the slots (attn_last_arrival, attn_merge_heads).
 // A workgroup serves all q heads of one kv head (<= 16, the columns of the MFMA tiles) for one slot of the KV
-// sequence: slot s walks chunks s, s + n_splits, ... of 128 positions, wave w takes keys [32w, 32w + 32) of each.
+// sequence: slot s walks chunks s, s + n_splits, ... of 32 NW positions, wave w takes keys [32w, 32w + 32) of each.
 //   S^T[key][head] = sum_d K[key][d] Q[head][d]     A = K rows straight from the cache, B = Q * scale as fp16 hi + lo
 //   O^T[d][head]  += sum_key V[key][d] P[head][key]  A = V gathered from the wave's LDS copy of the block,
 //                                                    B = the lane's own probabilities as fp16 hi + lo
-// so scores and weighted sums keep fp32-level accuracy.  Every wave runs its own online softmax; the four results
+// so scores and weighted sums keep fp32-level accuracy.  Every wave runs its own online softmax; the results
 // meet in LDS.  The workgroup whose slot holds the new position computes K (norm + RoPE) and V of that position,
 // stores them to the cache and, after a barrier, reads them back like any other row.
 // ---------------------------------------------------------------------------
@@ -219,12 +217,25 @@ typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 //    (relative to a running largest scale `u`, so that the fp16 hi + lo pair of the product stays in range; the
 //    accumulator is kept in units of u and rescaled like the running maximum of the softmax).  A lane takes a
 //    contiguous quarter of a K row (hd / 4 bytes), so the Q operand follows that order.
+//    Eight waves widen the codes of one CU's walk twice as fast as four, but cost 1 us more to start, to meet and to
+//    merge; fp16 rows, which need no widening, are limited by the requests in flight either way: four waves, except for
+//    long walks of quantised rows (model.hip: attn_slots).  8B shape, us per launch with 4 / 8 waves: one FP8 sequence at
+//    32 000 28.2 / 22.4, at 8 000 13.5 / 14.0; 32 of INT8 at 2048 35.8 / 33.0, at 500 13.0 / 13.3; one of fp16 at 700
+//    8.7 / 10.8, at 20 000 21.0 / 22.5.
 //  * sliding window with attention sinks (is_in_window, crates/oxibonsai-model/src/layers/sliding_window.rs:173-189):
 //    the first `sinks` keys stay visible, the others while pos - key < window - sinks; chunks without a visible key
 //    are not walked.  window == 0: every key up to pos is visible.
-#define OXB_ATTN_MERGE_LDS_BYTES(heads_per) ((heads_per) * 65 * 4 + 12 + 256 * 16)  // LDS attn_merge_heads needs
-__device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t heads_per,
-                                                 float* sm, float* __restrict__ out);
+#define OXB_ATTN_MERGE_LDS_BYTES(heads, threads) ((heads) * 65 * 4 + 12 + (threads) * 16)  // LDS attn_merge_heads needs
+template <uint32_t NT>
+__device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t used, float* sm);
+__device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32_t b, uint32_t h_first, const float* kf);
+
+// Slots in use for a walk of n_walk chunks.  A second slot saves a chunk's time and costs a merge, and the two are about
+// equal (one fp16 sequence at 200, 128-position chunks: 7.6 us with one slot, 8.2 with two; six: 8.6 and 9.7): two
+// chunks stay with one workgroup.
+__device__ __forceinline__ uint32_t attn_slots_used(uint32_t n_walk, uint32_t n_splits) {
+    return n_walk <= 2 ? 1u : min(n_walk, n_splits);
+}
 
 // The workgroups of one (sequence, kv head) count themselves off once their slot results are written; the last one
 // to arrive merges the slots of the group's heads into the attention output, so that no second launch is needed.
@@ -245,60 +256,47 @@ __device__ __forceinline__ bool attn_last_arrival(const OxbAttnParams& p, uint32
     return *flag != 0u;
 }
 
-template <int HD, int KVM, bool OPT>  // OPT: a window and / or a paged cache may be in use (else neither costs anything)
-__global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p) {
+template <int HD, int KVM, uint32_t NW, bool OPT>  // NW: waves; OPT: a window and / or a paged cache may be in use (else neither costs anything)
+__global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParams p) {
+    constexpr uint32_t NT = 64 * NW, CH = 32 * NW;  // threads, KV positions of a chunk
     constexpr bool QC = KVM != OXB_KV_F16;
     constexpr int KS = HD / 32, NS = HD / 16, VSTR = HD + 8;
     constexpr int VPR = QC ? HD / 16 : HD / 8;  // 16-byte pieces per V row
     constexpr int VL = 32 * VPR / 64;           // pieces of the wave's 32-row V block per lane
     // V block per wave; after the loop the merge buffers.  Q * scale of the group's heads has an area of its own, so
     // that a wave whose Q operands are in registers starts staging V without waiting for the others.
-    __shared__ __attribute__((aligned(16))) _Float16 vs_all[4][32 * VSTR];
+    __shared__ __attribute__((aligned(16))) _Float16 vs_all[NW][32 * VSTR];
     __shared__ __attribute__((aligned(16))) _Float16 qs[2][16 * HD];  // fp16 hi and lo parts, as the B operands take them
     __shared__ uint32_t last_flag;
-    __shared__ __attribute__((aligned(16))) _Float16 kv_new[2][HD];  // the new position's K and V rows as stored (fp16 cache)
-    static_assert(sizeof(vs_all) >= OXB_ATTN_MERGE_LDS_BYTES(16), "the merge's slot weights and partial sums must fit in the V slices");
+    typedef typename std::conditional<QC, uint8_t, _Float16>::type cache_t;
+    __shared__ __attribute__((aligned(16))) cache_t kv_new[2][HD];  // the new position's K and V rows as stored
+    __shared__ float kv_new_scale[2];
+    static_assert(sizeof(vs_all) >= OXB_ATTN_MERGE_LDS_BYTES(16, NT), "the merge's slot weights and partial sums must fit in the V slices");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, qi = lane & 15u, g = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t slot = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const uint32_t G = p.nq / p.nkv, h0 = kvh * G, half = HD / 2;
     const uint32_t pos = p.pos[b], seq_len = pos + 1;
-    const uint32_t n_chunks = (seq_len + OXB_ATTN_CHUNK - 1) / OXB_ATTN_CHUNK;
-    if (slot >= n_chunks) return;  // never read by the merge
     // visible keys: [0, sink_n) and [lo, seq_len)
     const uint32_t window = OPT ? p.window : 0u;
     const uint32_t budget = window > p.sinks ? window - p.sinks : 0u;
     const uint32_t lo = window ? (seq_len > budget ? seq_len - budget : 0u) : 0u;
     const uint32_t sink_n = window ? min(p.sinks, seq_len) : 0u;
-    const uint32_t sink_chunks = (sink_n + OXB_ATTN_CHUNK - 1) / OXB_ATTN_CHUNK, lo_chunk = lo / OXB_ATTN_CHUNK;
-    auto next_needed = [&](uint32_t c) {  // first chunk >= c of this slot's walk that holds a visible key
-        if (c >= sink_chunks && c < lo_chunk) c += (lo_chunk - c + p.n_splits - 1) / p.n_splits * p.n_splits;
-        return c;
-    };
-    const bool owner = (pos / OXB_ATTN_CHUNK) % p.n_splits == slot;  // this workgroup stores the new position
-    const uint32_t first = next_needed(slot);
+    // the chunks that hold a visible key, in ascending order: `skip_at` of them, then a gap, then up to the new position's
+    const uint32_t lo_chunk = min(lo, pos) / CH, skip_at = min((sink_n + CH - 1) / CH, lo_chunk), gap = lo_chunk - skip_at;
+    const uint32_t n_walk = (seq_len + CH - 1) / CH - gap;
+    auto chunk_of = [&](uint32_t i) -> uint32_t { return OPT && i >= skip_at ? i + gap : i; };
+    const uint32_t used = attn_slots_used(n_walk, p.n_splits);
+    if (slot >= used) return;  // never read by the merge
+    const bool owner = (n_walk - 1) % used == slot;  // this workgroup stores the new position
     float* part = p.part + (((size_t)b * p.nq + h0) * p.n_splits + slot) * (HD + OXB_ATTN_PART_PAD);
     const size_t part_head = (size_t)p.n_splits * (HD + OXB_ATTN_PART_PAD);
     // slot results go out through agent-coherent stores: a workgroup of this same launch merges them
     const __amdgpu_buffer_rsrc_t r_out = make_rsrc(part, (uint32_t)(G * part_head * 4u));
     auto put = [&](size_t idx, float v) { buf_store_b32_coherent(r_out, (uint32_t)idx * 4u, v); };
-    if (first >= n_chunks && !owner) {  // nothing visible in this slot's chunks: an empty result for the merge
-        for (uint32_t i = tid; i < G * HD; i += 256) {
-            const uint32_t h = i / HD, d = i % HD;
-            put(h * part_head + d, 0.f);
-            if (d == 0) {
-                put(h * part_head + HD, -INFINITY);
-                put(h * part_head + HD + 1, 0.f);
-            }
-        }
-        if (attn_last_arrival(p, b, kvh, min(n_chunks, p.n_splits), &last_flag))
-            attn_merge_heads(p, b, h0, G, G, reinterpret_cast<float*>(&vs_all[0][0]), p.out_merged);
-        return;
-    }
     const float* qkv = p.qkv + (size_t)b * p.qkv_stride;
     const float* cs = p.cos_t + (size_t)pos * half;
     const float* sn = p.sin_t + (size_t)pos * half;
-    typedef typename std::conditional<QC, uint8_t, _Float16>::type cache_t;
     cache_t* Kc = reinterpret_cast<cache_t*>(p.k_cache);
     cache_t* Vc = reinterpret_cast<cache_t*>(p.v_cache);
     float* Ksc = p.k_scale;  // one scale per row
@@ -311,11 +309,11 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
     const bool paged = OPT && p.kv.page_table != nullptr;
     const uint32_t pshift = p.kv.page_shift, pmask = (1u << pshift) - 1u;
     const size_t row0 = paged ? ((size_t)(p.layer * p.nkv + kvh) * p.kv.n_pages) << pshift : kv_row(p.kv, b, p.layer, kvh, 0);
-    const uint32_t* tbl = paged ? p.kv.page_table + (size_t)b * p.kv.table_stride : nullptr;  // covers whole chunks
+    const uint32_t* tbl = paged ? p.kv.page_table + (size_t)b * p.kv.table_stride : nullptr;
     auto pages_of = [&](uint32_t chunk, uint32_t& pa, uint32_t& pb) {
         pa = pb = 0;
         if (!paged) return;
-        const uint32_t key0 = chunk * OXB_ATTN_CHUNK + 32 * wave, i0 = key0 >> pshift, i1 = (key0 + 16) >> pshift;
+        const uint32_t key0 = chunk * CH + 32 * wave, i0 = min(key0, seq_len - 1) >> pshift, i1 = min(key0 + 16, seq_len - 1) >> pshift;
         pa = (uint32_t)__builtin_amdgcn_readfirstlane((int)tbl[i0]);
         pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)tbl[i1]);
     };
@@ -333,7 +331,7 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
     float4 ksc0, ksc1, vsc0, vsc1;  // row scales of the lane's keys 4g .. 4g+3 and 16+4g .. 16+4g+3
     v4i vr[VL];
     auto load_k = [&](uint32_t chunk, uint32_t pa, uint32_t pb) {
-        const uint32_t key0 = chunk * OXB_ATTN_CHUNK + 32 * wave;
+        const uint32_t key0 = chunk * CH + 32 * wave;
         const size_t kr0 = row_of(min(key0 + qi, seq_len - 1), key0, pa, pb), kr1 = row_of(min(key0 + 16 + qi, seq_len - 1), key0, pa, pb);
 #pragma unroll
         for (int s = 0; s < KS; s++) {
@@ -351,7 +349,7 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
         }
     };
     auto load_v = [&](uint32_t chunk, uint32_t pa, uint32_t pb) {
-        const uint32_t key0 = chunk * OXB_ATTN_CHUNK + 32 * wave;
+        const uint32_t key0 = chunk * CH + 32 * wave;
 #pragma unroll
         for (int i = 0; i < VL; i++) {
             const uint32_t id = i * 64 + lane, col = id % VPR;
@@ -364,24 +362,18 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
         }
     };
 
-    // With an fp16 cache the rows of the first chunk are requested before anything else, so that their way from HBM
-    // overlaps the Q prologue.  In the workgroup that stores the new position that row is not in the cache yet (and
-    // rows past the end repeat it): it is patched in from LDS below, with the very values the cache receives.
-    // With a quantised cache there is no such patch: every workgroup requests early except the one whose first chunk
-    // holds the new position, which waits until its own stores of that row have landed.
-    constexpr bool EARLY = !QC;
-    const uint32_t pos_chunk = pos / OXB_ATTN_CHUNK;
-    const bool early = EARLY || !(owner && pos_chunk == first);  // (the same for the whole workgroup)
+    // The rows of the first chunk are requested before anything else, so that their way from HBM overlaps the Q prologue.
+    // The new position's row is not in the cache then (and rows past the end repeat it): in the chunk that holds it, it is
+    // patched in from LDS, with the very values the cache receives, so no workgroup waits for its own stores.
+    const uint32_t pos_walk = n_walk - 1;
     uint32_t na = 0, nb = 0;  // pages of the chunk whose rows are requested next
     auto request_first = [&]() {
-        if (first < n_chunks) {
-            uint32_t pa, pb;
-            pages_of(first, pa, pb);
-            load_k(first, pa, pb);
-            load_v(first, pa, pb);
-            const uint32_t second = next_needed(first + p.n_splits);
-            if (second < n_chunks) pages_of(second, na, nb);
-        }
+        uint32_t pa, pb;
+        const uint32_t first = chunk_of(slot);
+        pages_of(first, pa, pb);
+        load_k(first, pa, pb);
+        load_v(first, pa, pb);
+        if (slot + used < n_walk) pages_of(chunk_of(slot + used), na, nb);
     };
     // Inputs of the prologue, requested before the cache rows: loads return in issue order, so whatever the prologue
     // waits for must not queue behind the rows from HBM.  Lane d holds elements d and d + hd/2 of a head (the RoPE pair).
@@ -405,7 +397,9 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
         ss = wave_sum_f32(ss);
         return 1.0f / sqrtf(ss / (float)HD + p.eps);
     };
-    HeadIn q_in, cs_sn, qn, kv_in, kn;  // cs_sn: lo = cos, hi = sin; kv_in: the new K row (wave 0) or V row (wave 1) of the owner
+    // The owner's last two waves take the new K and V rows: up to NW - 2 heads have waves of their own.
+    constexpr uint32_t KW = NW - 2, VW = NW - 1;
+    HeadIn q_in, cs_sn, qn, kv_in, kn;  // cs_sn: lo = cos, hi = sin; kv_in: the new K row (wave KW) or V row (wave VW) of the owner
     {
 #pragma unroll
         for (int it = 0; it < KI; it++) {
@@ -415,18 +409,18 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
         }
         load_head(p.q_norm, qn);
         if (wave < G) load_head(qkv + (size_t)(h0 + wave) * HD, q_in);
-        if (owner && wave == 0) {
+        if (owner && wave == KW) {
             load_head(qkv + (size_t)(p.nq + kvh) * HD, kv_in);
             load_head(p.k_norm, kn);
-        } else if (owner && wave == 1) {
+        } else if (owner && wave == VW) {
             load_head(qkv + (size_t)(p.nq + p.nkv + kvh) * HD, kv_in);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (early) request_first();
+    request_first();
     __builtin_amdgcn_sched_barrier(0);
     // --- Q of the group's heads: RMSNorm over the head, RoPE on the pairs (d, d + hd/2), times 1/sqrt(hd) ---
-    for (uint32_t h = wave; h < G; h += 4) {
+    for (uint32_t h = wave; h < G; h += NW) {
         if (h != wave) load_head(qkv + (size_t)(h0 + h) * HD, q_in);
         const float inv = head_inv_rms(q_in);
 #pragma unroll
@@ -444,10 +438,10 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             }
         }
     }
-    // --- K and V of the new position, by the workgroup whose slot walks its chunk (wave 0 and wave 1) ---
+    // --- K and V of the new position, by the workgroup whose slot walks its chunk ---
     const size_t new_row = kv_row(p.kv, b, p.layer, kvh, pos);
     if (owner) {
-        if (wave == 0) {
+        if (wave == KW) {
             const float inv = head_inv_rms(kv_in);
             float klo[KI], khi[KI], mx = 0.f;
 #pragma unroll
@@ -465,22 +459,22 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             if constexpr (QC) {
                 mx = wave_max_f32(mx);
                 scale = kv_row_scale<KVM>(mx);
-                if (lane == 0) Ksc[new_row] = scale;
+                if (lane == 0) Ksc[new_row] = kv_new_scale[0] = scale;
             }
 #pragma unroll
             for (int it = 0; it < KI; it++) {
                 const uint32_t d = lane + 64 * it;
                 if (d < half) {
                     if constexpr (QC) {
-                        Kc[new_row * HD + d] = (uint8_t)kv_encode<KVM>(klo[it], scale);
-                        Kc[new_row * HD + d + half] = (uint8_t)kv_encode<KVM>(khi[it], scale);
+                        Kc[new_row * HD + d] = kv_new[0][d] = (uint8_t)kv_encode<KVM>(klo[it], scale);
+                        Kc[new_row * HD + d + half] = kv_new[0][d + half] = (uint8_t)kv_encode<KVM>(khi[it], scale);
                     } else {
                         Kc[new_row * HD + d] = kv_new[0][d] = (_Float16)klo[it];
                         Kc[new_row * HD + d + half] = kv_new[0][d + half] = (_Float16)khi[it];
                     }
                 }
             }
-        } else if (wave == 1) {
+        } else if (wave == VW) {
             float mx = 0.f;
 #pragma unroll
             for (int it = 0; it < KI; it++) mx = fmaxf(mx, fmaxf(fabsf(kv_in.lo[it]), fabsf(kv_in.hi[it])));
@@ -488,15 +482,15 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             if constexpr (QC) {
                 mx = wave_max_f32(mx);
                 scale = kv_row_scale<KVM>(mx);
-                if (lane == 0) Vsc[new_row] = scale;
+                if (lane == 0) Vsc[new_row] = kv_new_scale[1] = scale;
             }
 #pragma unroll
             for (int it = 0; it < KI; it++) {
                 const uint32_t d = lane + 64 * it;
                 if (d < half) {
                     if constexpr (QC) {
-                        Vc[new_row * HD + d] = (uint8_t)kv_encode<KVM>(kv_in.lo[it], scale);
-                        Vc[new_row * HD + d + half] = (uint8_t)kv_encode<KVM>(kv_in.hi[it], scale);
+                        Vc[new_row * HD + d] = kv_new[1][d] = (uint8_t)kv_encode<KVM>(kv_in.lo[it], scale);
+                        Vc[new_row * HD + d + half] = kv_new[1][d + half] = (uint8_t)kv_encode<KVM>(kv_in.hi[it], scale);
                     } else {
                         Vc[new_row * HD + d] = kv_new[1][d] = (_Float16)kv_in.lo[it];
                         Vc[new_row * HD + d + half] = kv_new[1][d + half] = (_Float16)kv_in.hi[it];
@@ -505,12 +499,7 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             }
         }
     }
-    // publishes qs and the LDS copy of the new rows.  The requested cache rows stay in flight across it, unless this
-    // workgroup will read the new position's rows back from the cache (requests after the prologue, or a walk of
-    // several chunks that ends in the new position's): then the stores must have landed first.
-    if (owner && !(EARLY && pos_chunk == first)) __syncthreads();
-    else lds_barrier();
-    if (!early) request_first();
+    lds_barrier();  // publishes qs and the LDS copy of the new rows; the requested cache rows stay in flight across it
 
     // B operands: lane (head = qi, g) holds the eight Q values that meet its K values in step s, as hi + lo: one
     // 16-byte LDS read each.  Columns past the group's heads repeat head 0; nothing of them is ever stored.
@@ -528,42 +517,59 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
     float m_run = -INFINITY, l_run = 0.f, u_run = QC ? 0.f : 1.f;  // u_run: the unit of O (largest V row scale so far)
     _Float16* vs = vs_all[wave];
 
-    for (uint32_t chunk = first; chunk < n_chunks;) {
-        const uint32_t key0 = chunk * OXB_ATTN_CHUNK + 32 * wave;
-        const uint32_t nxt = next_needed(chunk + p.n_splits);
-        const bool more = nxt < n_chunks;
-        // rows of the new position (and the repeats of it past the end) come from LDS where they were requested early
-        const bool patch = EARLY && owner && chunk == pos_chunk && chunk == first;
-        chunk = nxt;
+    for (uint32_t i = slot; i < n_walk;) {
+        const uint32_t key0 = chunk_of(i) * CH + 32 * wave;
+        const bool patch = i == pos_walk;  // (the last chunk of the owner's walk)
+        i += used;
+        const bool more = i < n_walk;
+        const uint32_t nxt = chunk_of(i);
         // stage the V block in the wave's LDS slice (the previous block's gathers were issued before: LDS runs in
         // order) and request the next chunk's
 #pragma unroll
-        for (int i = 0; i < VL; i++) {
-            const uint32_t id = i * 64 + lane;
+        for (int j = 0; j < VL; j++) {
+            const uint32_t id = j * 64 + lane;
             if constexpr (QC) {
                 uint32_t d[8];
-                kv_dec4<KVM>((uint32_t)vr[i].x, d[0], d[1]);
-                kv_dec4<KVM>((uint32_t)vr[i].y, d[2], d[3]);
-                kv_dec4<KVM>((uint32_t)vr[i].z, d[4], d[5]);
-                kv_dec4<KVM>((uint32_t)vr[i].w, d[6], d[7]);
+                v4i piece = vr[j];
+                if (patch && key0 + id / VPR >= pos) piece = *reinterpret_cast<const v4i*>(&kv_new[1][(id % VPR) * 16]);
+                kv_dec4<KVM>((uint32_t)piece.x, d[0], d[1]);
+                kv_dec4<KVM>((uint32_t)piece.y, d[2], d[3]);
+                kv_dec4<KVM>((uint32_t)piece.z, d[4], d[5]);
+                kv_dec4<KVM>((uint32_t)piece.w, d[6], d[7]);
                 _Float16* dst = vs + (id / VPR) * VSTR + (id % VPR) * 16;
                 *reinterpret_cast<v4i*>(dst) = (v4i){(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
                 *reinterpret_cast<v4i*>(dst + 8) = (v4i){(int)d[4], (int)d[5], (int)d[6], (int)d[7]};
             } else {
-                v4i piece = vr[i];
+                v4i piece = vr[j];
                 if (patch && key0 + id / VPR >= pos) piece = *reinterpret_cast<const v4i*>(&kv_new[1][(id % VPR) * 8]);
                 *reinterpret_cast<v4i*>(vs + (id / VPR) * VSTR + (id % VPR) * 8) = piece;
             }
         }
-        const float4 vc0 = vsc0, vc1 = vsc1;
+        float4 vc0 = vsc0, vc1 = vsc1;
+        auto patch_scale = [&](float4& a, uint32_t first_key, float v) {  // the scale of position `pos`, if it is one of the four
+            if (first_key == pos) a.x = v;
+            if (first_key + 1 == pos) a.y = v;
+            if (first_key + 2 == pos) a.z = v;
+            if (first_key + 3 == pos) a.w = v;
+        };
+        if (QC && patch) {
+            patch_scale(vc0, key0 + 4 * g, kv_new_scale[1]);
+            patch_scale(vc1, key0 + 16 + 4 * g, kv_new_scale[1]);
+        }
         if (more) load_v(nxt, na, nb);
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < KS; s++) {
             v8h_t a0, a1;
             if constexpr (QC) {
-                a0 = kv_dec8<KVM>(k0q[s]);
-                a1 = kv_dec8<KVM>(k1q[s]);
+                kvi2_t c0 = k0q[s], c1 = k1q[s];
+                if (patch) {
+                    const kvi2_t cn = *reinterpret_cast<const kvi2_t*>(&kv_new[0][(HD / 4) * g + 8 * s]);
+                    if (key0 + qi >= pos) c0 = cn;
+                    if (key0 + 16 + qi >= pos) c1 = cn;
+                }
+                a0 = kv_dec8<KVM>(c0);
+                a1 = kv_dec8<KVM>(c1);
             } else {
                 a0 = k0r[s];
                 a1 = k1r[s];
@@ -577,13 +583,16 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qh[s], s1, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, ql[s], s1, 0, 0, 0);
         }
-        const float4 kc0 = ksc0, kc1 = ksc1;
+        float4 kc0 = ksc0, kc1 = ksc1;
+        if (QC && patch) {
+            patch_scale(kc0, key0 + 4 * g, kv_new_scale[0]);
+            patch_scale(kc1, key0 + 16 + 4 * g, kv_new_scale[0]);
+        }
         if (more) {
             load_k(nxt, na, nb);
-            const uint32_t after = next_needed(nxt + p.n_splits);
-            if (after < n_chunks) pages_of(after, na, nb);  // used by the next iteration's requests
+            if (i + used < n_walk) pages_of(chunk_of(i + used), na, nb);  // used by the next iteration's requests
         }
-        // this wave's quarter of the chunk holds no visible key (past the end, or outside the window)
+        // this wave's part of the chunk holds no visible key (past the end, or outside the window)
         if (!(key0 < sink_n || max(key0, lo) < min(key0 + 32, seq_len))) continue;
         // this lane: head qi, keys key0 + 4g + v and key0 + 16 + 4g + v
         float sv[8];
@@ -658,12 +667,12 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             O[sl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, O[sl], 0, 0, 0);
         }
     }
-    // --- merge the four waves: lane (head = qi, g) holds O[head][16 sl + 4 g + v], m_run, l_run ---
+    // --- merge the waves: lane (head = qi, g) holds O[head][16 sl + 4 g + v], m_run, l_run ---
     __syncthreads();  // the V slices are dead: reuse them
-    static_assert(sizeof(vs_all) >= (4 * 16 * HD + 2 * 4 * 16) * sizeof(float), "merge buffers must fit in the V slices");
+    static_assert(sizeof(vs_all) >= (NW * 16 * HD + 2 * NW * 16) * sizeof(float), "merge buffers must fit in the V slices");
     float* mo = reinterpret_cast<float*>(&vs_all[0][0]);  // [wave][head 16][HD], then [wave][head 16] m, [wave][head 16] l
-    float* mm = mo + 4 * 16 * HD;
-    float* ml = mm + 4 * 16;
+    float* mm = mo + NW * 16 * HD;
+    float* ml = mm + NW * 16;
     if (qi < G) {
 #pragma unroll
         for (int sl = 0; sl < NS; sl++)
@@ -675,18 +684,25 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
         ml[wave * 16 + qi] = l_run;
     }
     __syncthreads();
-    for (uint32_t i = tid; i < G * HD; i += 256) {
+    const bool pack = p.pack_out != nullptr && G * HD == 512u;
+    float* keep = reinterpret_cast<float*>(&qs[0][0]);  // a single slot's outputs, for the quantiser
+    static_assert(sizeof(qs) >= 512 * sizeof(float), "room for them");
+    for (uint32_t i = tid; i < G * HD; i += NT) {
         const uint32_t h = i / HD, d = i % HD;
-        const float M = fmaxf(fmaxf(mm[h], mm[16 + h]), fmaxf(mm[32 + h], mm[48 + h]));
+        float M = mm[h];
+#pragma unroll
+        for (uint32_t w = 1; w < NW; w++) M = fmaxf(M, mm[w * 16 + h]);
         float o = 0.f, l = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
+        for (uint32_t w = 0; w < NW; w++) {
             const float wgt = mm[w * 16 + h] == -INFINITY ? 0.f : __expf(mm[w * 16 + h] - M);  // a wave that saw no key
             o = fmaf(mo[(w * 16 + h) * HD + d], wgt, o);
             l = fmaf(ml[w * 16 + h], wgt, l);
         }
-        if (p.out_single) {  // the only slot: what the merge would compute (weight 1, times 1 / sum)
-            p.out_single[((size_t)b * p.nq + h0 + h) * HD + d] = o * (l > 0.f ? 1.0f / l : 0.f);
+        if (used == 1) {  // the only slot: what the merge would compute (weight 1, times 1 / sum)
+            o *= l > 0.f ? 1.0f / l : 0.f;
+            p.out[((size_t)b * p.nq + h0 + h) * HD + d] = o;
+            if (pack) keep[i] = o;
             continue;
         }
         put(h * part_head + d, o);
@@ -695,34 +711,59 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(OxbAttnParams p)
             put(h * part_head + HD + 1, l);
         }
     }
-    if (p.out_single) return;
-    if (attn_last_arrival(p, b, kvh, min(n_chunks, p.n_splits), &last_flag))  // (the barrier inside also retires mo / mm / ml)
-        attn_merge_heads(p, b, h0, G, G, reinterpret_cast<float*>(&vs_all[0][0]), p.out_merged);
+    if (used == 1) {
+        if (pack) {
+            __syncthreads();
+            attn_pack_outputs(p, b, h0, keep);
+        }
+        return;
+    }
+    if (attn_last_arrival(p, b, kvh, used, &last_flag))  // (the barrier inside also retires mo / mm / ml)
+        attn_merge_heads<NT>(p, b, h0, G, used, reinterpret_cast<float*>(&vs_all[0][0]));
+}
+
+// One wave quantises the 512 outputs of a kv head's q heads (LDS) for the O projection: superblock h_first * hd / 512 of
+// vector b.
+__device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32_t b, uint32_t h_first, const float* kf) {
+    const uint32_t tid = threadIdx.x, e0 = h_first * p.hd;
+    if (tid >= 64) return;
+    float xe[2][4];
+    if (p.pack_fmt == OXB_FMT_Q1) {
+#pragma unroll
+        for (int pass = 0; pass < 2; pass++)
+#pragma unroll
+            for (int bb = 0; bb < 4; bb++) xe[pass][bb] = kf[gemv_pack_elem<OXB_FMT_Q1>(tid, pass, bb)];
+        gemv_pack_write<OXB_FMT_Q1>(xe, 0.f, tid, e0 / 512u, b, p.pack_n_sb, p.pack_nvg, p.pack_out);
+    } else {
+#pragma unroll
+        for (int pass = 0; pass < 2; pass++)
+#pragma unroll
+            for (int bb = 0; bb < 4; bb++) xe[pass][bb] = kf[gemv_pack_elem<OXB_FMT_TQ2>(tid, pass, bb)];
+        gemv_pack_write<OXB_FMT_TQ2>(xe, 0.f, tid, e0 / 512u, b, p.pack_n_sb, p.pack_nvg, p.pack_out);
+    }
 }
 
 // Merge the slot results of heads h_first .. h_first + nh - 1 of sequence b into the attention output
-// [batch][nq * hd] (fp32), the input of the O projection, by the 256 threads of a workgroup: per head one wave works
+// [batch][nq * hd] (fp32), the input of the O projection, by the NT threads of a workgroup: per head one wave works
 // out the softmax weights of the slots (one slot per lane); the weighted slot outputs of a group of four dimensions
 // are added by NPAR threads, thread j taking slots j, j + NPAR, ... in ascending order, and the NPAR sums meet in LDS
 // in thread order.  Every thread requests its first 16 slot outputs before the weights are worked out; NPAR is the
 // smallest of 1, 2, 4 that covers the slots in use with those requests (one round trip to memory for the whole merge),
-// as far as 256 threads allow for the heads' nh * hd / 4 groups.
-// sm: heads_per * 65 floats of LDS ([head][64] slot weights | [head] 1 / sum), then 256 float4 for the partial sums.
+// as far as the threads allow for the heads' nh * hd / 4 groups.
+// sm: nh * 65 floats of LDS ([head][64] slot weights | [head] 1 / sum), then NT float4 for the partial sums.
 // The slot results were written by other workgroups of this same launch: agent-coherent loads.
-__device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t heads_per,
-                                                 float* sm, float* __restrict__ out) {
+template <uint32_t NT>
+__device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t used, float* sm) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, hd = p.hd, qd = p.nq * hd;
     const uint32_t stride = hd + OXB_ATTN_PART_PAD;
     float* wts = sm;
-    float* inv_l = wts + heads_per * 64;
-    float4* sums = reinterpret_cast<float4*>(sm + ((heads_per * 65 + 3) & ~3u));
+    float* inv_l = wts + nh * 64;
+    float4* sums = reinterpret_cast<float4*>(sm + ((nh * 65 + 3) & ~3u));
     // The merged outputs once more, for the quantiser at the end: 128 groups of four, in the entries of `sums` that the
     // partial sums never use (those are written by threads tg and up, and with 128 groups tg >= 128).
     float4* keep = sums;
     const bool pack = p.pack_out != nullptr && nh * hd == 512u;
     const uint32_t e0 = h_first * hd;
-    const uint32_t n_chunks = (p.pos[b] + p.chunk) / p.chunk;  // chunks that hold positions 0..pos
-    const uint32_t used = n_chunks < p.n_splits ? n_chunks : p.n_splits;
     const float* part = p.part + (size_t)b * p.nq * p.n_splits * stride;
     const __amdgpu_buffer_rsrc_t r_part = make_rsrc(part, p.nq * p.n_splits * stride * 4u);
     auto ld4 = [&](const float* q) -> float4 {
@@ -732,9 +773,9 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
     auto ld1 = [&](const float* q) -> float { return buf_load_f32_coherent(r_part, (uint32_t)(q - part) * 4u); };
     const uint32_t groups = nh * hd / 4;
     // as few threads per group as keep all slots within the first 16 requests (more would only add the LDS step)
-    const uint32_t npar_max = groups <= 64 ? 4u : groups <= 128 ? 2u : 1u;
+    const uint32_t npar_max = groups <= NT / 4 ? 4u : groups <= NT / 2 ? 2u : 1u;
     const uint32_t npar = used <= 16u || npar_max == 1u ? 1u : (used <= 32u || npar_max == 2u ? 2u : 4u);
-    const uint32_t tg = 256u / npar, sh = tid / tg, egl = tid % tg;  // this thread: group egl (+ tg, ...), slots sh + npar u
+    const uint32_t tg = NT / npar, sh = tid / tg, egl = tid % tg;  // this thread: group egl (+ tg, ...), slots sh + npar u
     constexpr int PRE = 16;
     float4 pre[PRE];
     // the maxima and sums of the wave's first head are requested ahead of the slot outputs: loads return in issue
@@ -753,7 +794,7 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
             pre[u] = (egl < groups && sl < used) ? ld4(ph + (size_t)sl * stride) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
-    for (uint32_t hh = tid >> 6; hh < nh; hh += 4) {
+    for (uint32_t hh = tid >> 6; hh < nh; hh += NT / 64) {
         const float* ph = part + ((size_t)(h_first + hh) * p.n_splits + lane) * stride + hd;
         const bool first_head = hh == (tid >> 6);
         const float mv = first_head ? mv0 : (lane < used ? ld1(ph) : -INFINITY), lv = first_head ? lv0 : (lane < used ? ld1(ph + 1) : 0.f);
@@ -807,29 +848,13 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
         if (live && !sh) {
             const float il = inv_l[hh];
             acc.x *= il, acc.y *= il, acc.z *= il, acc.w *= il;
-            *reinterpret_cast<float4*>(out + (size_t)b * qd + e) = acc;
+            *reinterpret_cast<float4*>(p.out + (size_t)b * qd + e) = acc;
             if (pack) keep[eg] = acc;
         }
     }
-    if (pack) {  // (uniform) one wave quantises the 512 outputs for the O projection: superblock e0 / 512 of vector b
+    if (pack) {  // (uniform)
         __syncthreads();
-        if (tid < 64) {
-            const float* kf = reinterpret_cast<const float*>(keep);
-            float xe[2][4];
-            if (p.pack_fmt == OXB_FMT_Q1) {
-#pragma unroll
-                for (int pass = 0; pass < 2; pass++)
-#pragma unroll
-                    for (int bb = 0; bb < 4; bb++) xe[pass][bb] = kf[gemv_pack_elem<OXB_FMT_Q1>(tid, pass, bb)];
-                gemv_pack_write<OXB_FMT_Q1>(xe, 0.f, tid, e0 / 512u, b, p.pack_n_sb, p.pack_nvg, p.pack_out);
-            } else {
-#pragma unroll
-                for (int pass = 0; pass < 2; pass++)
-#pragma unroll
-                    for (int bb = 0; bb < 4; bb++) xe[pass][bb] = kf[gemv_pack_elem<OXB_FMT_TQ2>(tid, pass, bb)];
-                gemv_pack_write<OXB_FMT_TQ2>(xe, 0.f, tid, e0 / 512u, b, p.pack_n_sb, p.pack_nvg, p.pack_out);
-            }
-        }
+        attn_pack_outputs(p, b, h_first, reinterpret_cast<const float*>(keep));
     }
 }
 
@@ -913,26 +938,32 @@ hipError_t oxb_launch_qk_norm_rope_store(const OxbQkParams& p, uint32_t batch, h
 }
 
 hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStream_t st) {
-    if (p.chunk != OXB_ATTN_CHUNK || p.n_splits == 0 || p.n_splits > OXB_ATTN_MAX_SPLITS || p.nq % p.nkv || p.nq / p.nkv > 16 ||
-        !p.qkv || !p.q_norm || !p.k_norm || !p.cos_t || !p.sin_t || p.kv_mode > OXB_KV_FP8_E4M3 || (p.out_single && p.n_splits != 1) || (!p.out_single && (!p.done || !p.out_merged)) ||
-        (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale)) ||
-        (p.kv.page_table ? (p.kv.page_shift < 4 || p.kv.page_shift > 7) : (p.kv.row_stride % OXB_ATTN_CHUNK != 0 || p.kv.row_stride < p.max_seq)))
+    if (p.n_splits == 0 || p.n_splits > OXB_ATTN_MAX_SPLITS || p.nq % p.nkv || p.nq / p.nkv > 16 ||
+        !p.qkv || !p.q_norm || !p.k_norm || !p.cos_t || !p.sin_t || p.kv_mode > OXB_KV_FP8_E4M3 || !p.out || (p.n_splits > 1 && (!p.done || !p.part)) ||
+        (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale)) || (p.wide && (p.kv_mode == OXB_KV_F16 || p.hd > 128)) ||
+        (p.kv.page_table ? (p.kv.page_shift < 4 || p.kv.page_shift > 7) : (p.kv.row_stride % 128 != 0 || p.kv.row_stride < p.max_seq)))
         return hipErrorInvalidValue;
-    const dim3 grid(p.n_splits, p.nkv, batch), block(256);
+    const dim3 grid(p.n_splits, p.nkv, batch), block(p.wide ? 512 : 256);
     const bool opt = p.window != 0 || p.kv.page_table != nullptr;
     switch (p.hd) {
-#define OXB_ATTN_LAUNCH(HD_, KVM_)                                                                                   \
-    if (opt) hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, true>), grid, block, 0, st, p);                 \
-    else hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, false>), grid, block, 0, st, p);
-#define OXB_ATTN_CASE(HD_)                                         \
-    case HD_:                                                      \
-        if (p.kv_mode == OXB_KV_I8) {                              \
-            OXB_ATTN_LAUNCH(HD_, OXB_KV_I8)                        \
-        } else if (p.kv_mode == OXB_KV_FP8_E4M3) {                 \
-            OXB_ATTN_LAUNCH(HD_, OXB_KV_FP8_E4M3)                  \
-        } else {                                                   \
-            OXB_ATTN_LAUNCH(HD_, OXB_KV_F16)                       \
-        }                                                          \
+#define OXB_ATTN_LAUNCH(HD_, KVM_, NW_)                                                                              \
+    if (opt) hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, true>), grid, block, 0, st, p);            \
+    else hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, false>), grid, block, 0, st, p);
+#define OXB_ATTN_CASE(HD_)                                                                            \
+    case HD_:                                                                                         \
+        if (p.kv_mode == OXB_KV_F16) {                                                                \
+            OXB_ATTN_LAUNCH(HD_, OXB_KV_F16, 4)                                                       \
+        } else if constexpr (HD_ <= 128) { /* (eight waves of head dimension 256 exceed the LDS) */   \
+            if (p.kv_mode == OXB_KV_I8) {                                                             \
+                if (p.wide) { OXB_ATTN_LAUNCH(HD_, OXB_KV_I8, 8) } else { OXB_ATTN_LAUNCH(HD_, OXB_KV_I8, 4) }             \
+            } else {                                                                                  \
+                if (p.wide) { OXB_ATTN_LAUNCH(HD_, OXB_KV_FP8_E4M3, 8) } else { OXB_ATTN_LAUNCH(HD_, OXB_KV_FP8_E4M3, 4) } \
+            }                                                                                         \
+        } else if (p.kv_mode == OXB_KV_I8) {                                                          \
+            OXB_ATTN_LAUNCH(HD_, OXB_KV_I8, 4)                                                        \
+        } else {                                                                                      \
+            OXB_ATTN_LAUNCH(HD_, OXB_KV_FP8_E4M3, 4)                                                  \
+        }                                                                                             \
         break;
         OXB_ATTN_CASE(32)
         OXB_ATTN_CASE(64)

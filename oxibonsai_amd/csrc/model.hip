@@ -59,7 +59,8 @@ struct Model {
     uint32_t* d_table = nullptr;
     bool table_dirty = false;
     float *cos_t = nullptr, *sin_t = nullptr;
-    uint32_t chunk = 0, n_splits = 0;
+    uint32_t n_splits = 0;
+    bool attn_wide = false;
     // graph
     hipGraphExec_t graph_exec = nullptr;
     uint64_t checked_gen = 0;  // g_rt.weights_gen when every handle was last looked up
@@ -368,8 +369,7 @@ static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, co
     ap.window = m.window;
     ap.sinks = m.sinks;
     ap.part = m.attn_part;
-    ap.out_single = m.n_splits == 1 ? m.attn_out : nullptr;
-    ap.out_merged = m.attn_out;
+    ap.out = m.attn_out;
     ap.done = m.attn_done;
     ap.pos = m.pos;
     ap.nq = d.nq;
@@ -378,8 +378,8 @@ static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, co
     ap.max_seq = d.max_seq;
     ap.n_layers = d.n_layers;
     ap.layer = L;
-    ap.chunk = m.chunk;
     ap.n_splits = m.n_splits;
+    ap.wide = m.attn_wide ? 1u : 0u;
     ap.scale = 1.0f / sqrtf((float)d.hd);
     ap.pack_out = pack_for ? (uint32_t*)m.gpack_o.ptr : nullptr;  // the O projection's operands, written by the merging workgroups
     ap.pack_fmt = pack_for ? (uint32_t)pack_for->L.fmt : 0;
@@ -451,7 +451,7 @@ static int encode_decode_step(Model& m, bool with_lm_head) {
         // Where the q heads of a kv head are one superblock of the O projection's input and the batch's vectors are
         // quantised ahead of that GEMV, the attention kernel's merging workgroups do the quantising: no pack launch.
         const bool fuse_o = m.gpack_o.ptr && d.batch <= OXB_GEMV_PACKED_MAX_BATCH && d.batch >= gemv_packed_min_batch(qd) &&
-                            m.n_splits > 1 && (d.nq / d.nkv) * d.hd == 512u && m.gpack_o.cap >= oxb_gemv_pack_bytes(qd, d.batch);
+                            (d.nq / d.nkv) * d.hd == 512u && m.gpack_o.cap >= oxb_gemv_pack_bytes(qd, d.batch);
         OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm, fuse_o ? wo : nullptr));
         for (uint32_t b0 = 0; b0 < d.batch; b0 += chunk) {
             const uint32_t nb = (d.batch - b0) < chunk ? (d.batch - b0) : chunk;
@@ -643,17 +643,15 @@ int oxb_hip_free_f32(uint64_t id) {
     OXB_API_END
 }
 
-// Slots of the split-KV attention: about one workgroup (slot x kv head x sequence) per CU for the fp16 cache, two for a
-// quantised one (widening the codes adds arithmetic that a second resident workgroup hides), no more: every slot pays
-// the Q arithmetic and a merge, and walks its chunks with a prefetch.  Measured, 8B shape: four per CU are slower
-// everywhere (batch 8 at context 2048 by 12 %, batch 16 by 7 %, one sequence at context 32 000 by 3 %); two per CU
-// gain 4 % at batch 32 with the INT8 cache and lose 1-3 % with the fp16 cache.
-static uint32_t attn_slots(const Model& m, uint32_t kv_mode) {
+// Slots of the split-KV attention: at most one workgroup (slot x kv head x sequence) per CU where that is possible: a CU
+// with two of them is the one that the launch waits for, and every slot pays the Q arithmetic and a merge.  8B shape, us
+// per launch with the slots chosen here / one more: nine fp16 sequences at 1700 18.5 / 22.7, eleven 21.6 / 27.2, seventeen
+// 30.6 / 36.0, twenty-eight 39.6 / 40.8, 24 of INT8 at 500 13.4 / 16.3.
+static uint32_t attn_slots(const Model& m) {
     const oxb_model_desc& d = m.d;
-    uint32_t n = (d.max_seq + m.chunk - 1) / m.chunk;
-    const uint32_t per_cu = kv_mode == OXB_KV_F16 ? 1u : 2u;
-    const uint32_t want = (per_cu * g_rt.n_cus + d.nkv * d.batch - 1) / (d.nkv * d.batch);
-    if (n > want) n = want;
+    uint32_t n = (d.max_seq + OXB_ATTN_CHUNK_POSITIONS - 1) / OXB_ATTN_CHUNK_POSITIONS;
+    const uint32_t want = g_rt.n_cus / (d.nkv * d.batch);
+    if (n > want) n = want > 1 ? want : 1;
     if (const char* e = getenv("OXB_HIP_ATTN_SLOTS")) {  // measurement aid: a fixed slot count
         const long v = strtol(e, nullptr, 10);
         if (v > 0) n = (uint32_t)v < n ? (uint32_t)v : n;
@@ -662,13 +660,20 @@ static uint32_t attn_slots(const Model& m, uint32_t kv_mode) {
     return n;
 }
 
+// Eight waves per workgroup for one-byte rows where a slot may have to walk more than 512 positions, as long as a CU gets
+// one workgroup (two of them are slower than two with four waves: 40 INT8 sequences at 1300 38.8 against 34.8 us).
+static bool attn_wide(const Model& m, uint32_t kv_mode) {
+    const oxb_model_desc& d = m.d;
+    return kv_mode != OXB_KV_F16 && d.hd <= 128 && (uint64_t)d.nkv * d.batch * m.n_splits <= g_rt.n_cus && d.max_seq / m.n_splits > 512u;
+}
+
 // (Re)allocates the KV cache in the given storage form, contiguous (n_pages 0) or as a pool of n_pages pages of
 // page_size positions.  Row scales start at 0 so that a row never written reads as zeros.  A contiguous head holds a
-// whole number of attention chunks of rows, which keeps the kernels' 16-byte scale loads aligned and inside it.
+// multiple of 128 rows, which keeps the kernels' 16-byte scale loads aligned and inside it.
 static int alloc_kv_cache(Model& m, uint32_t kv_mode, uint32_t page_size, uint32_t n_pages) {
     const oxb_model_desc& d = m.d;
     free_kv_cache(m);
-    m.row_stride = (d.max_seq + OXB_ATTN_CHUNK_POSITIONS - 1) / OXB_ATTN_CHUNK_POSITIONS * OXB_ATTN_CHUNK_POSITIONS;
+    m.row_stride = (d.max_seq + 127u) / 128u * 128u;
     const size_t rows = n_pages ? (size_t)n_pages * d.n_layers * d.nkv * page_size : (size_t)d.batch * d.n_layers * d.nkv * m.row_stride;
     const size_t bytes = rows * d.hd * (kv_mode == OXB_KV_F16 ? 2 : 1);
     auto grab = [&](void** p, size_t n) -> int {
@@ -690,7 +695,7 @@ static int alloc_kv_cache(Model& m, uint32_t kv_mode, uint32_t page_size, uint32
         while ((1u << shift) < page_size) shift++;
         m.page_shift = shift;
         m.n_pages = n_pages;
-        m.table_stride = m.row_stride / page_size;   // whole attention chunks: the kernels look up every block of a chunk
+        m.table_stride = m.row_stride / page_size;
         m.h_table.assign((size_t)d.batch * m.table_stride, 0u);   // entries of unreserved blocks name page 0: never read
         m.seq_pages.assign(d.batch, {});
         m.free_pages.resize(n_pages);
@@ -731,12 +736,10 @@ int oxb_hip_model_create(const oxb_model_desc* desc, uint64_t* model) {
     int rc = check_model_handles(m);
     if (rc) return rc;
 
-    m.chunk = OXB_ATTN_CHUNK_POSITIONS;
-    m.n_splits = attn_slots(m, OXB_KV_F16);
-    const uint32_t max_slots = attn_slots(m, OXB_KV_I8);  // what any cache type may ask for: sizes the slot results
+    m.n_splits = attn_slots(m);
     const size_t B = d.batch;
     if ((rc = dev_alloc(m, (void**)&m.hidden, B * d.h * 4)) || (rc = dev_alloc(m, (void**)&m.qkv, B * qkv_rows * 4)) ||
-        (rc = dev_alloc(m, (void**)&m.attn_part, B * d.nq * max_slots * (d.hd + OXB_ATTN_PART_PAD) * 4)) ||
+        (rc = dev_alloc(m, (void**)&m.attn_part, B * d.nq * m.n_splits * (d.hd + OXB_ATTN_PART_PAD) * 4)) ||
         (rc = dev_alloc(m, (void**)&m.attn_out, B * qd * 4)) || (rc = dev_alloc(m, (void**)&m.gu, B * 2 * d.inter * 4)) ||
         (rc = dev_alloc(m, (void**)&m.act, B * d.inter * 4)) ||
         (rc = dev_alloc(m, (void**)&m.logits, B * (d.lm_head ? d.vocab : 1) * 4)) || (rc = dev_alloc(m, (void**)&m.tokens, B * 4)) ||
@@ -830,7 +833,7 @@ int oxb_hip_model_set_attention(uint64_t model, const oxb_attention_options* opt
             return rc;
         }
     }
-    m->n_splits = attn_slots(*m, m->kv_mode);
+    m->attn_wide = attn_wide(*m, m->kv_mode);
     m->window = opt->window_size;
     m->sinks = opt->sink_tokens;
     return OXB_HIP_OK;

@@ -214,6 +214,27 @@ def test_batched_decode_with_options_where_attention_packs_for_o(backend, mode, 
     assert _decode_parity(backend, PACKS_FOR_O, Q1, mode, window, sinks, 140, seed=91, batch=6, check_every=9)
 
 
+@pytest.mark.parametrize("mode,window,hd", [(KV_I8, 0, 128), (KV_FP8_E4M3, 0, 128), (KV_I8, 600, 64)])
+def test_long_walks_of_quantised_rows(backend, monkeypatch, mode, window, hd):
+    """More than 512 positions per slot: workgroups of eight waves, one to three chunks of 256 positions, two slots."""
+    monkeypatch.setenv("OXB_HIP_ATTN_SLOTS", "2")
+    cfg = dict(PACKS_FOR_O, hd=hd, max_seq=1280, fmt=Q1)
+    w = synth.make_model(cfg, 95)
+    gpu = HipModel(backend, cfg, w)
+    try:
+        gpu.set_attention(mode, window, 3 if window else 0)
+        rows = _rows(5, 1100, cfg["h"])
+        done = 0
+        for pos in (31, 255, 256, 511, 512, 767, 768, 1099):
+            gpu.prefill(rows[done:pos], done, want_logits=False)
+            got, _ = gpu.forward(rows[pos], pos)
+            done = pos
+            held = _oracle_on_device_cache(gpu, cfg, w, mode, window, 3 if window else 0, pos + 1)
+            assert parity_violations(np.ravel(got), held.forward(rows[pos], pos), 5e-3) == 0, pos
+    finally:
+        gpu.close()
+
+
 def test_sequences_at_different_positions_with_a_window(backend):
     """Two sequences of one batch, one far ahead of the other: every sequence masks by its own position."""
     cfg = dict(SMALL, fmt=Q1)
