@@ -301,7 +301,8 @@ int  oxb_hip_prefill_tokens(uint64_t model, uint64_t embedding, uint32_t seq, co
 /* ---- pinned host memory for results (no counterpart in the reference): a host output buffer that lies in such a block is
  * written by the device itself, without a copy through the library's staging.  Any host output parameter above may point
  * into one; freed blocks are kept for reuse up to 128 MiB, and at most 512 MiB are handed out at a time
- * (OXB_HIP_OUT_OF_MEMORY beyond: use ordinary memory).  Safe from any thread. */
+ * (OXB_HIP_OUT_OF_MEMORY beyond: use ordinary memory).  Safe from any thread.  The pages are shared with the device and
+ * not part of a child process that fork() makes: a child must not touch or free them. */
 int  oxb_hip_host_alloc(void** p, size_t n_bytes);
 int  oxb_hip_host_free(void* p);
 

@@ -10,7 +10,6 @@ would make exactly these calls through ``extern "C"``.
 from __future__ import annotations
 
 import ctypes as C
-import weakref
 
 import numpy as np
 
@@ -49,27 +48,10 @@ def _as_bytes(b) -> np.ndarray:
     return np.frombuffer(bytes(b), dtype=np.uint8)
 
 
-# Results from this size on lie in pinned memory: the device writes them there itself, where an ordinary array takes a
-# second copy on the host and, when it is new, a page fault every 4 KiB (19 MB of logits: 0.37 against 1.15 ms).
-_PINNED_FROM = 1 << 14
-
-
-def _result(shape) -> np.ndarray:
-    """An uninitialised float32 array for a call's output.  Its memory returns to the library's pool with the last
-    reference to it; where the pool is exhausted it is an ordinary array."""
-    n = 4
-    for d in shape:
-        n *= int(d)
-    if n >= _PINNED_FROM:
-        L = _lib.lib()
-        p = C.c_void_p()
-        if L.oxb_hip_host_alloc(C.byref(p), n) == 0:
-            buf = (C.c_float * (n // 4)).from_address(p.value)
-            weakref.finalize(buf, L.oxb_hip_host_free, p.value).atexit = False
-            return np.frombuffer(buf, dtype=np.float32).reshape(shape)
-    return np.empty(shape, dtype=np.float32)
-
-
+# Results are ordinary arrays: they own their memory (ndarray.resize works on them) and a forked child reads its own copy.
+# Memory of oxb_hip_host_alloc, which the device could write without the second copy on the host, offers neither - such
+# pages are shared with the device and left out of a child process.  It costs 0.35 ms for 19 MB of logits, page faults
+# of a new array included, and 20 us for 1.2 MB.
 def _rows_f32(a) -> np.ndarray:
     """`a` as a flat C-contiguous float32 array, itself where it is one already."""
     if type(a) is np.ndarray and a.dtype == np.float32 and a.flags.c_contiguous:
@@ -160,7 +142,7 @@ class NativeHipBackend:
         x = _rows_f32(input)
         if x.size != m * k:
             raise GpuError(5, f"invalid argument: input holds {x.size} values, {m * k} needed")
-        y = _result((m, n_rows))
+        y = np.empty((m, n_rows), dtype=np.float32)
         _check(self._lib.oxb_hip_gemm(int(handle), x.ctypes.data, y.ctypes.data, m, n_rows, k))
         return y
 
@@ -209,7 +191,7 @@ class NativeHipBackend:
         x = _rows_f32(input)
         if x.size < batch * k:
             raise GpuError(5, f"invalid argument: input holds {x.size} values, {batch * k} needed")
-        y = _result((batch, n_rows))
+        y = np.empty((batch, n_rows), dtype=np.float32)
         _check(self._lib.oxb_hip_gemv(int(handle), x.ctypes.data, y.ctypes.data, n_rows, k, batch))
         return y
 
@@ -217,7 +199,7 @@ class NativeHipBackend:
         """fp32 [n_rows x k] decoded on the device from the resident layout."""
         fmt, nr, k, nb = C.c_int(0), C.c_uint32(0), C.c_uint32(0), C.c_size_t(0)
         _check(self._lib.oxb_hip_weight_info(int(handle), C.byref(fmt), C.byref(nr), C.byref(k), C.byref(nb)))
-        out = _result((nr.value, k.value))
+        out = np.empty((nr.value, k.value), dtype=np.float32)
         _check(self._lib.oxb_hip_dequant(int(handle), _f32(out), out.size))
         return out
 

@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from .backend import GpuError, NativeHipBackend, _check, _result
+from .backend import GpuError, NativeHipBackend, _check
 from .synth import Q1
 
 
@@ -149,7 +149,7 @@ class Embedding:
 
     def rows(self, ids) -> np.ndarray:
         iv = np.ascontiguousarray(ids, dtype=np.uint32).reshape(-1)
-        out = _result((iv.size, self.h))
+        out = np.empty((iv.size, self.h), dtype=np.float32)
         _check(self._lib.oxb_hip_embedding_rows(self.id, iv.ctypes.data_as(_lib.u32p), iv.size, out.ctypes.data_as(_lib.f32p)))
         return out
 
@@ -232,7 +232,7 @@ class HipModel:
             pb, tb = np.zeros(self.batch, dtype=np.uint32), np.zeros(self.batch, dtype=np.uint32)
             io = self._io = (pb, tb, pb.ctypes.data, tb.ctypes.data)
         io[0][:] = pos      # a scalar, or one position per sequence
-        logits = _result((self.batch, self.cfg["vocab"])) if want_logits else None
+        logits = np.empty((self.batch, self.cfg["vocab"]), dtype=np.float32) if want_logits else None
         _check(self._lib.oxb_hip_decode(self.id, hv.ctypes.data, io[2], logits.ctypes.data if want_logits else None, io[3]))
         return logits, io[1].copy()
 
@@ -270,7 +270,7 @@ class HipModel:
         hidden: [n_tokens, h] embedding rows for positions pos_start.. -> (last-token logits [vocab] or None,
         greedy token of the last position).  Decode continues at pos_start + n_tokens."""
         hv = np.ascontiguousarray(hidden, dtype=np.float32).reshape(-1, self.cfg["h"])
-        logits = _result((self.cfg["vocab"],)) if want_logits else None
+        logits = np.empty(self.cfg["vocab"], dtype=np.float32) if want_logits else None
         token = np.empty(1, dtype=np.uint32)
         _check(self._lib.oxb_hip_prefill(self.id, seq, hv.ctypes.data_as(_lib.f32p), hv.shape[0], pos_start,
                                          logits.ctypes.data_as(_lib.f32p) if want_logits else None,
@@ -302,7 +302,7 @@ class HipModel:
     def prefill_tokens(self, embedding: Embedding, ids, pos_start: int = 0, seq: int = 0, want_logits: bool = True):
         """prefill() with the embedding rows gathered on the device from token ids."""
         iv = np.ascontiguousarray(ids, dtype=np.uint32).reshape(-1)
-        logits = _result((self.cfg["vocab"],)) if want_logits else None
+        logits = np.empty(self.cfg["vocab"], dtype=np.float32) if want_logits else None
         token = np.empty(1, dtype=np.uint32)
         _check(self._lib.oxb_hip_prefill_tokens(self.id, embedding.id, seq, iv.ctypes.data_as(_lib.u32p), iv.size, pos_start,
                                                 logits.ctypes.data_as(_lib.f32p) if want_logits else None,

@@ -1,6 +1,7 @@
 """Runtime behaviour of the native-hip library through the C ABI: calls from several host threads, device memory
 given back when handles and models are released (the reference serialises its CUDA graph singleton behind a Mutex,
 gpu_backend/cuda_graph/cudagraph_type.rs:18-32; weights live until freed, gpu_backend/mod.rs:445-472)."""
+import os
 import threading
 
 import numpy as np
@@ -44,6 +45,45 @@ def test_calls_from_several_threads_are_serialised(backend):
     for _, h, *_ in work:
         backend.free_weights(h)
     assert not errors, errors
+
+
+def _read_in_forked_child(a: np.ndarray) -> bytes:
+    """The first bytes of an array as a forked child sees them; a page the child does not have is an error of its write."""
+    view = memoryview(a.reshape(-1).view(np.uint8))[:2048]
+    r, w = os.pipe()
+    pid = os.fork()
+    if pid == 0:
+        try:
+            os.write(w, view)
+        finally:
+            os._exit(0)
+    os.close(w)
+    os.waitpid(pid, 0)
+    got = os.read(r, 4096)
+    os.close(r)
+    return got
+
+
+def test_results_are_arrays_of_their_own(backend):
+    # whatever their size, results own their memory, may be resized in place and can be read by a forked child
+    n, k, m = 1024, 512, 96
+    h = backend.upload_weights_raw(synth.make_blocks(Q1, 91, n, k), n, k)
+    x = synth.normal_f32(92, m * k).reshape(m, k)
+    cfg = dict(fmt=Q1, n_layers=1, h=128, inter=256, nq=4, nkv=2, hd=32, vocab=8192, max_seq=64, eps=1e-6, rope_theta=1e6)
+    gpu = HipModel(backend, cfg, synth.make_model(cfg, 93))
+    rows = synth.embedding_rows(94, range(8), cfg["h"]) * 50.0
+    try:
+        results = {"gemm": backend.gemm_cached(h, x, m, n, k), "gemv": backend.gemv_cached_batch(h, x[:8], n, k),
+                   "dequant": backend.dequant(h), "prefill": gpu.prefill(rows)[0], "decode": gpu.forward(rows[0], 8)[0]}
+        for name, y in results.items():
+            assert y.nbytes >= 32768 and y.flags.owndata and y.flags.c_contiguous and y.dtype == np.float32, name
+            assert _read_in_forked_child(y) == y.tobytes()[:2048], name
+            first = y.reshape(-1)[:4].copy()
+            y.resize((4,), refcheck=False)
+            assert np.array_equal(y, first), name
+    finally:
+        gpu.close()
+        backend.free_weights(h)
 
 
 def test_device_memory_returns_when_models_and_weights_go(backend):
