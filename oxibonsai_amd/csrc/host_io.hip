@@ -52,14 +52,13 @@ constexpr size_t kPoolOut = (size_t)512 << 20;  // result memory handed out at a
 constexpr size_t kPoolFree = (size_t)128 << 20; // ... and kept for reuse
 constexpr uint32_t kSyncEvery = 256;            // calls after which the stream is synchronised all the same (the runtime retires its commands there)
 
-struct Io {
+struct Staging {
     uint8_t *in = nullptr, *out = nullptr;
     size_t in_cap = 0, out_cap = 0, in_used = 0, out_used = 0;
     uint32_t *flag = nullptr, *arrived = nullptr, seq = 0, seq_begin = 0, calls = 0;
-    bool open = false;  // something may still be reading or writing the staging buffers
     struct Late { void* dst; size_t at, bytes; uint32_t seq; };
     std::vector<Late> late;  // results that wait in staging for the device
-} io;
+} st;
 
 int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two up to kStaging; nothing is in flight
     if (want > kStaging) want = kStaging;
@@ -79,15 +78,15 @@ int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two
 }
 
 int ensure_flag() {
-    if (io.flag) return OXB_HIP_OK;
-    if (hipHostMalloc((void**)&io.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&io.arrived, 4) != hipSuccess ||
-        hipMemset(io.arrived, 0, 4) != hipSuccess) {
+    if (st.flag) return OXB_HIP_OK;
+    if (hipHostMalloc((void**)&st.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&st.arrived, 4) != hipSuccess ||
+        hipMemset(st.arrived, 0, 4) != hipSuccess) {
         (void)hipGetLastError();
-        if (io.flag) (void)hipHostFree(io.flag);
-        io.flag = nullptr;
+        if (st.flag) (void)hipHostFree(st.flag);
+        st.flag = nullptr;
         return fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: completion flag");
     }
-    *io.flag = io.seq;
+    *st.flag = st.seq;
     return OXB_HIP_OK;
 }
 
@@ -96,8 +95,8 @@ int copy(const void* src, void* dst, size_t bytes, uint32_t* flag, uint32_t seq)
     const uint32_t grid = wgs < 1 ? 1u : wgs < OXB_IO_GRID ? (uint32_t)wgs : OXB_IO_GRID;
     const uintptr_t at = (uintptr_t)src | (uintptr_t)dst;
     if (at & 3) return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: a buffer of %zu bytes is not aligned to 4", bytes);
-    if (at & 15) hipLaunchKernelGGL(io_copy_kernel<uint32_t>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, io.arrived, flag, seq);
-    else hipLaunchKernelGGL(io_copy_kernel<uint4>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, io.arrived, flag, seq);
+    if (at & 15) hipLaunchKernelGGL(io_copy_kernel<uint32_t>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, st.arrived, flag, seq);
+    else hipLaunchKernelGGL(io_copy_kernel<uint4>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, st.arrived, flag, seq);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? OXB_HIP_OK : hip_fail(e, "kernel launch failed: io_copy");
 }
@@ -110,7 +109,7 @@ int sync_all(const char* what) {
 // Polls for a few milliseconds; a longer wait (or a stream in error, which never raises the flag) is the runtime's.
 int wait_for(uint32_t seq, const char* what) {
     const auto t0 = std::chrono::steady_clock::now();
-    for (uint32_t n = 1; (int32_t)(__atomic_load_n(io.flag, __ATOMIC_ACQUIRE) - seq) < 0; n++) {
+    for (uint32_t n = 1; (int32_t)(__atomic_load_n(st.flag, __ATOMIC_ACQUIRE) - seq) < 0; n++) {
         __builtin_ia32_pause();
         if ((n & 1023u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(4)) return sync_all(what);
     }
@@ -134,75 +133,75 @@ bool is_pinned(const void* p, size_t bytes) {
 
 }  // namespace
 
-int io_begin() {
+int IoCall::begin() {
     int rc = ensure_flag();
     if (rc) return rc;
-    if (io.open) {  // the call before ended in an error: whatever it left may still use the staging buffers
-        (void)hipDeviceSynchronize();
-        (void)hipMemset(io.arrived, 0, 4);
-    }
-    io.open = true;
-    io.in_used = io.out_used = 0;
-    io.seq_begin = io.seq;
-    io.late.clear();
+    open = true;
+    st.in_used = st.out_used = 0;
+    st.seq_begin = st.seq;
+    st.late.clear();
     return OXB_HIP_OK;
 }
 
-int io_upload(void* d_dst, const void* src, size_t bytes) {
+IoCall::~IoCall() {
+    if (open) (void)hipStreamSynchronize(g_rt.stream);
+}
+
+int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
     const uint8_t* s = (const uint8_t*)src;
     uint8_t* d = (uint8_t*)d_dst;
     if (((uintptr_t)s & 15) == 0 && is_pinned(s, bytes)) return copy(s, d, bytes, nullptr, 0);
     int rc;
-    if (io.in_used == 0 && (rc = staging(&io.in, &io.in_cap, bytes))) return rc;
+    if (st.in_used == 0 && (rc = staging(&st.in, &st.in_cap, bytes))) return rc;
     while (bytes) {
         const size_t n = bytes < kChunk ? bytes : kChunk;
-        if (io.in_used + n > io.in_cap) {  // every piece has been used once: wait for the device to be done with them
+        if (st.in_used + n > st.in_cap) {  // every piece has been used once: wait for the device to be done with them
             if ((rc = sync_all("input upload"))) return rc;
-            io.in_used = 0;
-            if ((rc = staging(&io.in, &io.in_cap, bytes))) return rc;
+            st.in_used = 0;
+            if ((rc = staging(&st.in, &st.in_cap, bytes))) return rc;
         }
-        memcpy(io.in + io.in_used, s, n);
-        if ((rc = copy(io.in + io.in_used, d, n, nullptr, 0))) return rc;
-        io.in_used += (n + 255) & ~(size_t)255;
+        memcpy(st.in + st.in_used, s, n);
+        if ((rc = copy(st.in + st.in_used, d, n, nullptr, 0))) return rc;
+        st.in_used += (n + 255) & ~(size_t)255;
         s += n, d += n, bytes -= n;
     }
     return OXB_HIP_OK;
 }
 
-int io_download(void* dst, const void* d_src, size_t bytes) {
-    if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, io.flag, ++io.seq);
+int IoCall::download(void* dst, const void* d_src, size_t bytes) {
+    if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, st.flag, ++st.seq);
     int rc;
-    if (io.out_used == 0 && (rc = staging(&io.out, &io.out_cap, bytes))) return rc;
+    if (st.out_used == 0 && (rc = staging(&st.out, &st.out_cap, bytes))) return rc;
     uint8_t* d = (uint8_t*)dst;
     const uint8_t* s = (const uint8_t*)d_src;
     while (bytes) {
         const size_t n = bytes < kChunk ? bytes : kChunk;
-        if (io.out_used + n > io.out_cap) {  // staging is full of results: hand them over first
+        if (st.out_used + n > st.out_cap) {  // staging is full of results: hand them over first
             if ((rc = sync_all("output download"))) return rc;
-            for (const Io::Late& l : io.late) memcpy(l.dst, io.out + l.at, l.bytes);
-            io.late.clear();
-            io.out_used = 0;
-            if ((rc = staging(&io.out, &io.out_cap, bytes))) return rc;
+            for (const Staging::Late& l : st.late) memcpy(l.dst, st.out + l.at, l.bytes);
+            st.late.clear();
+            st.out_used = 0;
+            if ((rc = staging(&st.out, &st.out_cap, bytes))) return rc;
         }
-        if ((rc = copy(s, io.out + io.out_used, n, io.flag, ++io.seq))) return rc;
-        io.late.push_back({d, io.out_used, n, io.seq});
-        io.out_used += (n + 255) & ~(size_t)255;
+        if ((rc = copy(s, st.out + st.out_used, n, st.flag, ++st.seq))) return rc;
+        st.late.push_back({d, st.out_used, n, st.seq});
+        st.out_used += (n + 255) & ~(size_t)255;
         s += n, d += n, bytes -= n;
     }
     return OXB_HIP_OK;
 }
 
-int io_finish(const char* what) {
+int IoCall::finish(const char* what) {
     int rc;
-    if (io.seq == io.seq_begin && (rc = sync_all(what))) return rc;  // nothing came back
-    for (const Io::Late& l : io.late) {  // one piece is copied on the host while the next ones cross the bus
+    if (st.seq == st.seq_begin && (rc = sync_all(what))) return rc;  // nothing came back
+    for (const Staging::Late& l : st.late) {  // one piece is copied on the host while the next ones cross the bus
         if ((rc = wait_for(l.seq, what))) return rc;
-        memcpy(l.dst, io.out + l.at, l.bytes);
+        memcpy(l.dst, st.out + l.at, l.bytes);
     }
-    io.late.clear();
-    if ((rc = wait_for(io.seq, what))) return rc;
-    if (++io.calls % kSyncEvery == 0 && (rc = sync_all(what))) return rc;
-    io.open = false;
+    st.late.clear();
+    if ((rc = wait_for(st.seq, what))) return rc;
+    if (++st.calls % kSyncEvery == 0 && (rc = sync_all(what))) return rc;
+    open = false;
     return OXB_HIP_OK;
 }
 
@@ -241,11 +240,11 @@ bool pinned_free(void* p) {
 }
 
 void io_shutdown() {  // results that a caller still holds stay
-    if (io.in) (void)hipHostFree(io.in);
-    if (io.out) (void)hipHostFree(io.out);
-    if (io.flag) (void)hipHostFree(io.flag);
-    if (io.arrived) (void)hipFree(io.arrived);
-    io = Io();
+    if (st.in) (void)hipHostFree(st.in);
+    if (st.out) (void)hipHostFree(st.out);
+    if (st.flag) (void)hipHostFree(st.flag);
+    if (st.arrived) (void)hipFree(st.arrived);
+    st = Staging();
     std::lock_guard<std::mutex> lk(pool.mu);
     for (auto& b : pool.free_blocks) (void)hipHostFree(b.second);
     pool.free_blocks.clear();

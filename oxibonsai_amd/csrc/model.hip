@@ -1085,16 +1085,17 @@ int oxb_hip_decode(uint64_t model, const float* hidden, const uint32_t* pos, flo
     for (uint32_t b = 0; b < d.batch; b++) OXB_TRY(kv_reserve(m, b, (uint64_t)pos[b] + 1));
     OXB_TRY(kv_sync_table(m));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    // (the previous call ended with a stream synchronisation, so the staging buffers are free)
+    IoCall io;
+    OXB_TRY(io.begin());
+    // (no call returns before its launches have read these buffers)
     memcpy(m.h_hidden, hidden, (size_t)d.batch * d.h * 4);
     memcpy(m.h_pos, pos, (size_t)d.batch * 4);
     // one kernel reads the pinned rows and positions; the step's last kernel leaves the token ids in pinned memory too
     OXB_TRY_HIP(oxb_launch_stage_in(m.h_hidden, d.batch * d.h, m.h_pos, d.batch, m.hidden, m.pos, st), "kernel launch failed: stage_in");
     OXB_TRY(run_decode_step(m));
     if (logits_or_null)
-        OXB_TRY(io_download(logits_or_null, m.logits, (size_t)d.batch * d.vocab * 4));
-    OXB_TRY(io_finish("decode"));
+        OXB_TRY(io.download(logits_or_null, m.logits, (size_t)d.batch * d.vocab * 4));
+    OXB_TRY(io.finish("decode"));
     if (token_out) memcpy(token_out, m.h_tokens, (size_t)d.batch * 4);
     return OXB_HIP_OK;
     OXB_API_END
@@ -1158,15 +1159,16 @@ int oxb_hip_decode_hidden(uint64_t model, const float* hidden, const uint32_t* p
     for (uint32_t b = 0; b < d.batch; b++) OXB_TRY(kv_reserve(m, b, (uint64_t)pos[b] + 1));
     OXB_TRY(kv_sync_table(m));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(m.hidden, hidden, (size_t)d.batch * d.h * 4));
-    OXB_TRY(io_upload(m.pos, pos, (size_t)d.batch * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(m.hidden, hidden, (size_t)d.batch * d.h * 4));
+    OXB_TRY(io.upload(m.pos, pos, (size_t)d.batch * 4));
     OXB_TRY(encode_decode_step(m, false));
     float* dst = m.gu;
     OXB_TRY_HIP(oxb_launch_rmsnorm(m.hidden, final_norm, d.h, d.batch, d.eps, dst, st), "kernel launch failed: rmsnorm");
     for (uint32_t b = 0; b < d.batch; b++)
-        OXB_TRY(io_download(normed_out + (size_t)b * d.h, dst + (size_t)b * d.h, (size_t)d.h * 4));
-    OXB_TRY(io_finish("decode_hidden"));
+        OXB_TRY(io.download(normed_out + (size_t)b * d.h, dst + (size_t)b * d.h, (size_t)d.h * 4));
+    OXB_TRY(io.finish("decode_hidden"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1212,12 +1214,13 @@ int oxb_hip_prefill(uint64_t model, uint32_t seq, const float* hidden, uint32_t 
     OXB_TRY(kv_sync_table(m));
     OXB_TRY(ensure_prefill_buffers(m, n_tokens));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(m.pf_hidden, hidden, (size_t)n_tokens * d.h * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(m.pf_hidden, hidden, (size_t)n_tokens * d.h * 4));
     OXB_TRY(encode_prefill(m, seq, n_tokens, pos_start));
     if (logits_or_null)
-        OXB_TRY(io_download(logits_or_null, m.logits + (size_t)seq * d.vocab, (size_t)d.vocab * 4));
-    OXB_TRY(io_finish("prefill"));
+        OXB_TRY(io.download(logits_or_null, m.logits + (size_t)seq * d.vocab, (size_t)d.vocab * 4));
+    OXB_TRY(io.finish("prefill"));
     if (token_out_or_null) *token_out_or_null = m.h_tokens[seq];
     return OXB_HIP_OK;
     OXB_API_END
@@ -1247,14 +1250,15 @@ int oxb_hip_attn_phase(int fmt, const float* hidden, const float* norm_w, float 
     float* d_norm = d_hidden + h;
     float* d_qkv = (float*)g_rt.ws_y.ptr;
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(d_hidden, hidden, (size_t)h * 4));
-    OXB_TRY(io_upload(d_norm, norm_w, (size_t)h * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(d_hidden, hidden, (size_t)h * 4));
+    OXB_TRY(io.upload(d_norm, norm_w, (size_t)h * 4));
     OXB_TRY(gemv_launch(*w, d_hidden, h, 1, d_qkv, rows, OXB_GEMV_PRO_RMSNORM, d_norm, eps, OXB_GEMV_STORE, nullptr));
-    OXB_TRY(io_download(q, d_qkv, (size_t)q_rows * 4));
-    OXB_TRY(io_download(k, d_qkv + q_rows, (size_t)k_rows * 4));
-    OXB_TRY(io_download(v, d_qkv + q_rows + k_rows, (size_t)k_rows * 4));
-    OXB_TRY(io_finish("attn_phase"));
+    OXB_TRY(io.download(q, d_qkv, (size_t)q_rows * 4));
+    OXB_TRY(io.download(k, d_qkv + q_rows, (size_t)k_rows * 4));
+    OXB_TRY(io.download(v, d_qkv + q_rows + k_rows, (size_t)k_rows * 4));
+    OXB_TRY(io.finish("attn_phase"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1278,13 +1282,14 @@ int oxb_hip_ffn_phase(int fmt, float* hidden, const float* attn_out, const float
     float* d_gu = (float*)g_rt.ws_y.ptr;
     float* d_act = d_gu + 2 * (size_t)inter;
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(d_hidden, hidden, (size_t)h * 4));
-    OXB_TRY(io_upload(d_norm, norm_w, (size_t)h * 4));
-    OXB_TRY(io_upload(d_attn, attn_out, (size_t)attn_k * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(d_hidden, hidden, (size_t)h * 4));
+    OXB_TRY(io.upload(d_norm, norm_w, (size_t)h * 4));
+    OXB_TRY(io.upload(d_attn, attn_out, (size_t)attn_k * 4));
     OXB_TRY(encode_ffn(d_hidden, d_attn, d_norm, eps, *wo, *wgu, *wdn, d_gu, d_act, h, inter, attn_k, 1, nullptr));
-    OXB_TRY(io_download(hidden, d_hidden, (size_t)h * 4));
-    OXB_TRY(io_finish("ffn_phase"));
+    OXB_TRY(io.download(hidden, d_hidden, (size_t)h * 4));
+    OXB_TRY(io.finish("ffn_phase"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1355,12 +1360,13 @@ int oxb_hip_embedding_rows(uint64_t embedding, const uint32_t* ids, uint32_t n, 
     OXB_TRY(g_rt.ws_x.ensure((size_t)n * 4));
     OXB_TRY(g_rt.ws_y.ensure((size_t)n * e->h * 4));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(g_rt.ws_x.ptr, ids, (size_t)n * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(g_rt.ws_x.ptr, ids, (size_t)n * 4));
     OXB_TRY_HIP(oxb_launch_embedding_gather(e->d, e->type, e->vocab, e->h, (const uint32_t*)g_rt.ws_x.ptr, n, (float*)g_rt.ws_y.ptr, st),
                 "kernel launch failed: embedding_gather");
-    OXB_TRY(io_download(out, g_rt.ws_y.ptr, (size_t)n * e->h * 4));
-    OXB_TRY(io_finish("embedding_rows"));
+    OXB_TRY(io.download(out, g_rt.ws_y.ptr, (size_t)n * e->h * 4));
+    OXB_TRY(io.finish("embedding_rows"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1405,15 +1411,16 @@ static int decode_tokens_impl(uint64_t model, uint64_t embedding, const uint32_t
     if (sampled && !rng_state) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: null rng_state");
     OXB_TRY(m.tok_hist.ensure((size_t)n_steps * d.batch * 4));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
+    IoCall io;
+    OXB_TRY(io.begin());
     if (sampled) {
         OXB_TRY(m.sample_ws.ensure(oxb_sample_ws_bytes(d.vocab, d.batch)));
         OXB_TRY(m.rng.ensure((size_t)d.batch * 8));
-        OXB_TRY(io_upload(m.rng.ptr, rng_state, (size_t)d.batch * 8));
+        OXB_TRY(io.upload(m.rng.ptr, rng_state, (size_t)d.batch * 8));
     }
     uint32_t* hist = (uint32_t*)m.tok_hist.ptr;
-    OXB_TRY(io_upload(m.tokens, tokens, (size_t)d.batch * 4));
-    OXB_TRY(io_upload(m.pos, pos, (size_t)d.batch * 4));
+    OXB_TRY(io.upload(m.tokens, tokens, (size_t)d.batch * 4));
+    OXB_TRY(io.upload(m.pos, pos, (size_t)d.batch * 4));
     for (uint32_t i = 0; i < n_steps; i++) {
         OXB_TRY_HIP(oxb_launch_embedding_gather(e->d, e->type, e->vocab, d.h, m.tokens, d.batch, m.hidden, st),
                     "kernel launch failed: embedding_gather");
@@ -1424,9 +1431,9 @@ static int decode_tokens_impl(uint64_t model, uint64_t embedding, const uint32_t
                         "kernel launch failed: sample");
         OXB_TRY_HIP(oxb_launch_token_step(m.tokens, hist + (size_t)i * d.batch, m.pos, d.batch, st), "kernel launch failed: token_step");
     }
-    OXB_TRY(io_download(tokens_out, hist, (size_t)n_steps * d.batch * 4));
-    if (sampled) OXB_TRY(io_download(rng_state, m.rng.ptr, (size_t)d.batch * 8));
-    OXB_TRY(io_finish("decode_tokens"));
+    OXB_TRY(io.download(tokens_out, hist, (size_t)n_steps * d.batch * 4));
+    if (sampled) OXB_TRY(io.download(rng_state, m.rng.ptr, (size_t)d.batch * 8));
+    OXB_TRY(io.finish("decode_tokens"));
     return OXB_HIP_OK;
 }
 
@@ -1454,11 +1461,12 @@ int oxb_hip_sum_in_order(const float* x, uint32_t n, float* sum_out) {
     float* d_x = (float*)g_rt.ws_y.ptr;
     float* d_sum = (float*)((uint8_t*)g_rt.ws_y.ptr + (((size_t)n * 4 + 255) & ~(size_t)255));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(d_x, x, (size_t)n * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(d_x, x, (size_t)n * 4));
     OXB_TRY_HIP(oxb_launch_sum_in_order(d_x, n, d_sum, st), "kernel launch failed: sum_in_order");
-    OXB_TRY(io_download(sum_out, d_sum, 4));
-    OXB_TRY(io_finish("sum_in_order"));
+    OXB_TRY(io.download(sum_out, d_sum, 4));
+    OXB_TRY(io.finish("sum_in_order"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1480,9 +1488,10 @@ int oxb_hip_sample_logits(const float* logits, uint32_t vocab, uint32_t batch, c
     uint64_t* d_rng = (uint64_t*)g_rt.ws_x.ptr;
     uint32_t* d_tok = (uint32_t*)(d_rng + batch);
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(d_logits, logits, lb));
-    OXB_TRY(io_upload(d_rng, rng_state, (size_t)batch * 8));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(d_logits, logits, lb));
+    OXB_TRY(io.upload(d_rng, rng_state, (size_t)batch * 8));
     if (params->temperature < 1e-6f) {
         OXB_TRY(g_rt.ws_aux.ensure((size_t)batch * OXB_ARGMAX_MAX_PARTS * 8));
         OXB_TRY_HIP(oxb_launch_argmax(d_logits, vocab, batch, d_tok, g_rt.ws_aux.ptr, st), "kernel launch failed: argmax");
@@ -1490,9 +1499,9 @@ int oxb_hip_sample_logits(const float* logits, uint32_t vocab, uint32_t batch, c
         OXB_TRY_HIP(oxb_launch_sample(d_logits, vocab, batch, params->temperature, params->top_k, params->top_p, d_rng, d_tok, d_ws, st),
                     "kernel launch failed: sample");
     }
-    OXB_TRY(io_download(tokens_out, d_tok, (size_t)batch * 4));
-    OXB_TRY(io_download(rng_state, d_rng, (size_t)batch * 8));
-    OXB_TRY(io_finish("sample_logits"));
+    OXB_TRY(io.download(tokens_out, d_tok, (size_t)batch * 4));
+    OXB_TRY(io.download(rng_state, d_rng, (size_t)batch * 8));
+    OXB_TRY(io.finish("sample_logits"));
     return OXB_HIP_OK;
     OXB_API_END
 }
@@ -1520,14 +1529,15 @@ int oxb_hip_prefill_tokens(uint64_t model, uint64_t embedding, uint32_t seq, con
     OXB_TRY(ensure_prefill_buffers(m, n_tokens));
     OXB_TRY(m.tok_ids.ensure((size_t)n_tokens * 4));
     hipStream_t st = g_rt.stream;
-    OXB_TRY(io_begin());
-    OXB_TRY(io_upload(m.tok_ids.ptr, ids, (size_t)n_tokens * 4));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(m.tok_ids.ptr, ids, (size_t)n_tokens * 4));
     OXB_TRY_HIP(oxb_launch_embedding_gather(e->d, e->type, e->vocab, d.h, (const uint32_t*)m.tok_ids.ptr, n_tokens, m.pf_hidden, st),
                 "kernel launch failed: embedding_gather");
     OXB_TRY(encode_prefill(m, seq, n_tokens, pos_start));
     if (logits_or_null)
-        OXB_TRY(io_download(logits_or_null, m.logits + (size_t)seq * d.vocab, (size_t)d.vocab * 4));
-    OXB_TRY(io_finish("prefill_tokens"));
+        OXB_TRY(io.download(logits_or_null, m.logits + (size_t)seq * d.vocab, (size_t)d.vocab * 4));
+    OXB_TRY(io.finish("prefill_tokens"));
     if (token_out_or_null) *token_out_or_null = m.h_tokens[seq];
     return OXB_HIP_OK;
     OXB_API_END

@@ -524,11 +524,12 @@ int oxb_hip_dequant(uint64_t id, float* out, size_t out_len) {
     if (!out || out_len < n) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: output holds %zu values, %zu needed", out_len, n);
     int rc = g_rt.ws_y.ensure(n * sizeof(float));
     if (rc) return rc;
-    if ((rc = io_begin())) return rc;
+    IoCall io;
+    if ((rc = io.begin())) return rc;
     hipError_t e = oxb_launch_dequant(w->L, w->d_codes, w->d_scales, (float*)g_rt.ws_y.ptr, g_rt.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch failed: dequant");
-    if ((rc = io_download(out, g_rt.ws_y.ptr, n * sizeof(float)))) return rc;
-    return io_finish("dequant");
+    if ((rc = io.download(out, g_rt.ws_y.ptr, n * sizeof(float)))) return rc;
+    return io.finish("dequant");
     OXB_API_END
 }
 
@@ -694,11 +695,12 @@ int oxb_hip_gemm(uint64_t id, const float* x, float* y, uint32_t m, uint32_t n_r
     const size_t xb = (size_t)m * k * sizeof(float), yb = (size_t)m * n_rows * sizeof(float);
     if ((rc = g_rt.ws_x.ensure(xb))) return rc;
     if ((rc = g_rt.ws_y.ensure(yb))) return rc;
-    if ((rc = io_begin()) || (rc = io_upload(g_rt.ws_x.ptr, x, xb))) return rc;
+    IoCall io;
+    if ((rc = io.begin()) || (rc = io.upload(g_rt.ws_x.ptr, x, xb))) return rc;
     rc = gemm_device(*w, (const float*)g_rt.ws_x.ptr, k, (float*)g_rt.ws_y.ptr, m, n_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_IDENT, nullptr, 0.f);
     if (rc) return rc;
-    if ((rc = io_download(y, g_rt.ws_y.ptr, yb))) return rc;
-    return io_finish("gemm");
+    if ((rc = io.download(y, g_rt.ws_y.ptr, yb))) return rc;
+    return io.finish("gemm");
     OXB_API_END
 }
 
@@ -766,11 +768,12 @@ int oxb_hip_gemv(uint64_t id, const float* x, float* y, uint32_t n_rows, uint32_
     const size_t xb = (size_t)batch * k * sizeof(float), yb = (size_t)batch * n_rows * sizeof(float);
     if ((rc = g_rt.ws_x.ensure(xb))) return rc;
     if ((rc = g_rt.ws_y.ensure(yb))) return rc;
-    if ((rc = io_begin()) || (rc = io_upload(g_rt.ws_x.ptr, x, xb))) return rc;
+    IoCall io;
+    if ((rc = io.begin()) || (rc = io.upload(g_rt.ws_x.ptr, x, xb))) return rc;
     rc = gemv_device(*w, (const float*)g_rt.ws_x.ptr, (float*)g_rt.ws_y.ptr, batch, n_rows, OXB_GEMV_STORE, nullptr);
     if (rc) return rc;
-    if ((rc = io_download(y, g_rt.ws_y.ptr, yb))) return rc;
-    return io_finish("gemv");
+    if ((rc = io.download(y, g_rt.ws_y.ptr, yb))) return rc;
+    return io.finish("gemv");
     OXB_API_END
 }
 

@@ -1,0 +1,212 @@
+// Checks of csrc/host_io.hip against the stand-in runtime of hip/hip_runtime.h; one check per run, named by argv[1].
+#include <chrono>
+#include <condition_variable>
+#include <cstdarg>
+#include <cstdio>
+#include <deque>
+#include <map>
+#include <thread>
+#include <vector>
+
+#include "../../include/oxb_hip.h"
+#include "../../oxibonsai_amd/csrc/host_io.h"
+#include "../../oxibonsai_amd/csrc/runtime_internal.h"
+
+thread_local dim3 blockIdx, threadIdx, gridDim;
+
+namespace fake {
+size_t syncs = 0, host_mallocs = 0, host_frees = 0, host_bytes = 0, host_bytes_limit = ~(size_t)0;
+static std::mutex mu;
+static std::condition_variable cv;
+static std::deque<std::function<void()>> queue, null_queue;
+static bool held = false, busy = false;
+static std::map<void*, size_t> host_blocks;
+
+static void device() {
+    std::unique_lock<std::mutex> lk(mu);
+    for (;;) {
+        cv.wait(lk, [] { return !held && !queue.empty(); });
+        auto f = std::move(queue.front());
+        queue.pop_front();
+        busy = true;
+        lk.unlock();
+        f();
+        lk.lock();
+        busy = false;
+        cv.notify_all();
+    }
+}
+void enqueue(std::function<void()> f) {
+    static bool started = (std::thread(device).detach(), true);
+    (void)started;
+    std::lock_guard<std::mutex> lk(mu);
+    queue.push_back(std::move(f));
+    cv.notify_all();
+}
+void hold() {
+    std::lock_guard<std::mutex> lk(mu);
+    held = true;
+}
+void release() {
+    std::lock_guard<std::mutex> lk(mu);
+    held = false;
+    cv.notify_all();
+}
+size_t pending() {
+    std::lock_guard<std::mutex> lk(mu);
+    return queue.size() + (busy ? 1 : 0);
+}
+static void drain() {
+    std::unique_lock<std::mutex> lk(mu);
+    cv.wait(lk, [] { return queue.empty() && !busy; });
+}
+}  // namespace fake
+
+hipError_t hipStreamSynchronize(hipStream_t) {
+    fake::syncs++;
+    fake::drain();
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() {
+    fake::drain();
+    for (auto& f : fake::null_queue) f();
+    fake::null_queue.clear();
+    return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t n) {
+    *p = malloc(n);
+    memset(*p, 0xCD, n);
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    fake::host_mallocs++;
+    if (fake::host_bytes + n > fake::host_bytes_limit) return hipErrorOutOfMemory;
+    *p = aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+    memset(*p, 0xCD, n);
+    fake::host_blocks[*p] = n;
+    fake::host_bytes += n;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+    fake::host_frees++;
+    fake::host_bytes -= fake::host_blocks.at(p);
+    fake::host_blocks.erase(p);
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipMemset(void* p, int v, size_t n) {
+    fake::null_queue.push_back([=] { memset(p, v, n); });
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
+    fake::enqueue([=] { memset(p, v, n); });
+    return hipSuccess;
+}
+
+namespace oxb {
+Runtime g_rt;
+std::recursive_mutex g_mu;
+int fail(int code, const char* fmt, ...) {
+    va_list ap;
+    va_start(ap, fmt);
+    vfprintf(stderr, fmt, ap);
+    fputc('\n', stderr);
+    va_end(ap);
+    return code;
+}
+int hip_fail(hipError_t, const char* what) { return fail(OXB_HIP_KERNEL_LAUNCH, "%s", what); }
+}  // namespace oxb
+
+using namespace oxb;
+
+#define CHECK(c)                                                        \
+    do {                                                                \
+        if (!(c)) {                                                     \
+            fprintf(stderr, "line %d: %s does not hold\n", __LINE__, #c); \
+            exit(1);                                                    \
+        }                                                               \
+    } while (0)
+
+static const size_t MiB = (size_t)1 << 20;
+
+static std::vector<uint8_t> bytes(size_t n, unsigned seed) {
+    std::vector<uint8_t> v(n);
+    for (size_t i = 0; i < n; i++) v[i] = (uint8_t)((i * 2654435761u + seed) >> 13);
+    return v;
+}
+
+// There and back through device memory: sizes around a piece, the staging buffer and its multiples, buffers that begin
+// off a 16-byte boundary, several buffers in one call.
+static void round_trip() {
+    const size_t sizes[] = {1, 4, 15, 16, 4096 + 4, 256 * 1024, MiB - 4, MiB, MiB + 20, 5 * MiB + 3, 32 * MiB, 32 * MiB + 8, 71 * MiB + 12};
+    std::vector<uint8_t> dev(80 * MiB + 64);
+    unsigned seed = 1;
+    for (size_t n : sizes)
+        for (size_t off : {(size_t)0, (size_t)1, (size_t)8}) {
+            std::vector<uint8_t> src = bytes(n + off, seed++), dst(n + off + 4, 0);
+            IoCall io;
+            CHECK(io.begin() == 0);
+            CHECK(io.upload(dev.data(), src.data() + off, n) == 0);
+            CHECK(io.download(dst.data() + off, dev.data(), n) == 0);
+            CHECK(io.finish("round trip") == 0);
+            CHECK(memcmp(dst.data() + off, src.data() + off, n) == 0 && dst[n + off] == 0);
+        }
+    IoCall io;
+    CHECK(io.begin() == 0);
+    std::vector<std::vector<uint8_t>> in, out;
+    const size_t part[] = {3 * MiB, 20 * MiB, 12, 15 * MiB + 4, 30 * MiB, 4};
+    size_t at = 0;
+    for (size_t n : part) {
+        in.push_back(bytes(n, (unsigned)n)), out.emplace_back(n);
+        CHECK(io.upload(dev.data() + at, in.back().data(), n) == 0);
+        if (at + (n + 15) / 16 * 16 < 40 * MiB) at += (n + 15) / 16 * 16;
+    }
+    at = 0;
+    CHECK(io.upload(dev.data(), in[4].data(), in[4].size()) == 0);
+    for (size_t i = 0; i < out.size(); i++) CHECK(io.download(out[i].data(), dev.data() + 64 * i, out[i].size()) == 0);
+    CHECK(io.finish("several buffers") == 0);
+    for (size_t i = 0; i < out.size(); i++) {
+        const size_t n = std::min(out[i].size(), in[4].size() - 64 * i);
+        CHECK(memcmp(out[i].data(), in[4].data() + 64 * i, n) == 0);
+    }
+}
+
+// A call that ends in an error between its copies and finish: the device is done with the caller's buffers.
+static void error_exit() {
+    uint8_t* src = (uint8_t*)pinned_alloc(64 * 1024);
+    uint8_t* dst = (uint8_t*)pinned_alloc(64 * 1024);
+    CHECK(src && dst);
+    std::vector<uint8_t> dev(64 * 1024);
+    {
+        IoCall first;  // (so that nothing below is a first-call clear)
+        CHECK(first.begin() == 0 && first.finish("nothing") == 0);
+    }
+    fake::hold();
+    std::thread later([] {
+        std::this_thread::sleep_for(std::chrono::milliseconds(50));
+        fake::release();
+    });
+    {
+        IoCall io;
+        CHECK(io.begin() == 0);
+        CHECK(io.upload(dev.data(), src, 64 * 1024) == 0);
+        CHECK(io.download(dst, dev.data(), 64 * 1024) == 0);
+    }
+    CHECK(fake::pending() == 0);
+    later.join();
+}
+
+int main(int argc, char** argv) {
+    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}};
+    for (const auto& c : checks)
+        if (argc == 2 && !strcmp(argv[1], c.name)) {
+            c.run();
+            fflush(nullptr);
+            _Exit(0);
+        }
+    return 2;
+}
