@@ -79,11 +79,13 @@ int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two
 
 int ensure_flag() {
     if (st.flag) return OXB_HIP_OK;
+    // (the counter is cleared in the stream whose kernels count on it: a clear in another one may come after them)
     if (hipHostMalloc((void**)&st.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&st.arrived, 4) != hipSuccess ||
-        hipMemset(st.arrived, 0, 4) != hipSuccess) {
+        hipMemsetAsync(st.arrived, 0, 4, g_rt.stream) != hipSuccess || hipStreamSynchronize(g_rt.stream) != hipSuccess) {
         (void)hipGetLastError();
         if (st.flag) (void)hipHostFree(st.flag);
-        st.flag = nullptr;
+        if (st.arrived) (void)hipFree(st.arrived);
+        st.flag = st.arrived = nullptr;
         return fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: completion flag");
     }
     *st.flag = st.seq;

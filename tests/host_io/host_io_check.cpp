@@ -200,8 +200,24 @@ static void error_exit() {
     later.join();
 }
 
+// The counter behind the completion flag is clear before the first kernel counts on it, whatever the null stream is doing:
+// the flag comes up by itself, from the first call on.
+static void first_call() {
+    std::vector<uint8_t> dev(4096), dst(4096);
+    for (int i = 0; i < 8; i++) {
+        IoCall io;
+        CHECK(io.begin() == 0);
+        const size_t before = fake::syncs;
+        CHECK(io.upload(dev.data(), dst.data(), 4096) == 0);
+        CHECK(io.download(dst.data(), dev.data(), 4096) == 0);
+        CHECK(io.finish("a call") == 0);
+        CHECK(fake::syncs == before);
+        if (i == 3) (void)hipDeviceSynchronize();
+    }
+}
+
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}, {"first_call", first_call}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.run();
