@@ -49,7 +49,7 @@ namespace {
 constexpr size_t kChunk = (size_t)1 << 20;      // host copy of one piece while the bus moves the one before
 constexpr size_t kStaging = (size_t)32 << 20;   // per direction; larger buffers take turns in it
 constexpr size_t kPoolOut = (size_t)512 << 20;  // result memory handed out at a time
-constexpr size_t kPoolFree = (size_t)128 << 20; // ... and kept for reuse
+constexpr size_t kPoolKept = (size_t)128 << 20; // ... and kept for reuse
 constexpr uint32_t kSyncEvery = 256;            // calls after which the stream is synchronised all the same (the runtime retires its commands there)
 
 struct Staging {
@@ -118,12 +118,33 @@ int wait_for(uint32_t seq, const char* what) {
     return OXB_HIP_OK;
 }
 
+// Blocks of pinned memory that are handed out, and those that wait to be: found by size, given back to the system oldest first.
 struct Pool {
+    struct Kept { uint8_t* p; uint64_t age; };
     std::mutex mu;
-    std::map<const uint8_t*, size_t> out;              // handed out: start -> size
-    std::multimap<size_t, uint8_t*> free_blocks;       // kept: size -> start
-    size_t out_bytes = 0, free_bytes = 0;
+    std::map<const uint8_t*, size_t> out;                        // handed out: start -> size
+    std::multimap<size_t, Kept> kept;                            // size -> block
+    std::map<uint64_t, std::multimap<size_t, Kept>::iterator> by_age;
+    uint64_t age = 0;
+    size_t out_bytes = 0, kept_bytes = 0;
+
+    uint8_t* take(std::multimap<size_t, Kept>::iterator it) {
+        uint8_t* p = it->second.p;
+        kept_bytes -= it->first;
+        by_age.erase(it->second.age);
+        kept.erase(it);
+        return p;
+    }
+    // What has to go so that no more than `limit` bytes are kept; freed by the caller, outside the lock (hipHostFree may
+    // wait for the device, and every call asks whether a buffer is pinned).
+    void trim(size_t limit, std::vector<uint8_t*>& gone) {
+        while (kept_bytes > limit) gone.push_back(take(by_age.begin()->second));
+    }
 } pool;
+
+void give_back(const std::vector<uint8_t*>& gone) {
+    for (uint8_t* p : gone) (void)hipHostFree(p);
+}
 
 bool is_pinned(const void* p, size_t bytes) {
     std::lock_guard<std::mutex> lk(pool.mu);
@@ -208,36 +229,55 @@ int IoCall::finish(const char* what) {
 }
 
 void* pinned_alloc(size_t bytes) {
+    if (!bytes) return nullptr;
     const size_t unit = bytes < kChunk ? (size_t)64 << 10 : kChunk, n = (bytes + unit - 1) / unit * unit;
-    std::lock_guard<std::mutex> lk(pool.mu);
-    uint8_t* p = nullptr;
-    auto it = pool.free_blocks.find(n);
-    if (it != pool.free_blocks.end()) {
-        p = it->second;
-        pool.free_blocks.erase(it);
-        pool.free_bytes -= n;
-    } else if (!bytes || pool.out_bytes + n > kPoolOut || hipHostMalloc((void**)&p, n, hipHostMallocCoherent) != hipSuccess) {
-        if (bytes) (void)hipGetLastError();
-        return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        // the smallest kept block that is large enough, unless it is more than twice as large
+        auto it = pool.kept.lower_bound(n);
+        if (it != pool.kept.end() && it->first <= 2 * n && pool.out_bytes + it->first <= kPoolOut) {
+            const size_t size = it->first;
+            uint8_t* p = pool.take(it);
+            pool.out[p] = size;
+            pool.out_bytes += size;
+            return p;
+        }
+        if (pool.out_bytes + n > kPoolOut) return nullptr;
+        pool.out_bytes += n;  // (room is taken before the lock goes)
     }
-    pool.out[p] = n;
-    pool.out_bytes += n;
+    uint8_t* p = nullptr;
+    hipError_t e = hipHostMalloc((void**)&p, n, hipHostMallocCoherent);
+    if (e != hipSuccess) {  // once more without what is kept
+        (void)hipGetLastError();
+        std::vector<uint8_t*> gone;
+        {
+            std::lock_guard<std::mutex> lk(pool.mu);
+            pool.trim(0, gone);
+        }
+        give_back(gone);
+        if (!gone.empty() && (e = hipHostMalloc((void**)&p, n, hipHostMallocCoherent)) != hipSuccess) (void)hipGetLastError();
+    }
+    std::lock_guard<std::mutex> lk(pool.mu);
+    if (e == hipSuccess) pool.out[p] = n;
+    else p = nullptr, pool.out_bytes -= n;
     return p;
 }
 
 bool pinned_free(void* p) {
-    std::lock_guard<std::mutex> lk(pool.mu);
-    auto it = pool.out.find((const uint8_t*)p);
-    if (it == pool.out.end()) return false;
-    const size_t n = it->second;
-    pool.out.erase(it);
-    pool.out_bytes -= n;
-    if (pool.free_bytes + n > kPoolFree) {
-        (void)hipHostFree(p);
-    } else {
-        pool.free_blocks.emplace(n, (uint8_t*)p);
-        pool.free_bytes += n;
+    std::vector<uint8_t*> gone;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        auto it = pool.out.find((const uint8_t*)p);
+        if (it == pool.out.end()) return false;
+        const size_t n = it->second;
+        pool.out.erase(it);
+        pool.out_bytes -= n;
+        pool.by_age[pool.age] = pool.kept.emplace(n, Pool::Kept{(uint8_t*)p, pool.age});
+        pool.age++;
+        pool.kept_bytes += n;
+        pool.trim(kPoolKept, gone);
     }
+    give_back(gone);
     return true;
 }
 
@@ -247,10 +287,12 @@ void io_shutdown() {  // results that a caller still holds stay
     if (st.flag) (void)hipHostFree(st.flag);
     if (st.arrived) (void)hipFree(st.arrived);
     st = Staging();
-    std::lock_guard<std::mutex> lk(pool.mu);
-    for (auto& b : pool.free_blocks) (void)hipHostFree(b.second);
-    pool.free_blocks.clear();
-    pool.free_bytes = 0;
+    std::vector<uint8_t*> gone;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        pool.trim(0, gone);
+    }
+    give_back(gone);
 }
 
 }  // namespace oxb

@@ -127,7 +127,7 @@ using namespace oxb;
     do {                                                                \
         if (!(c)) {                                                     \
             fprintf(stderr, "line %d: %s does not hold\n", __LINE__, #c); \
-            exit(1);                                                    \
+            fflush(nullptr), _Exit(1);                                                    \
         }                                                               \
     } while (0)
 
@@ -216,8 +216,56 @@ static void first_call() {
     }
 }
 
+// Blocks of sizes that come again or lie close by are reused, however much else is kept; what is kept stays within 128 MiB,
+// what is handed out within 512 MiB, and where memory runs out what is kept goes first.
+static void pool_of_results() {
+    std::vector<void*> all;
+    for (int i = 0; i < 128; i++) all.push_back(pinned_alloc(MiB));
+    for (void* p : all) CHECK(p && pinned_free(p));
+    CHECK(fake::host_mallocs == 128 && fake::host_frees == 0 && fake::host_bytes == 128 * MiB);
+    // another size while the pool is full: one new block, not one for every result
+    for (int i = 0; i < 100; i++) {
+        void* p = pinned_alloc(3 * MiB + 1);
+        CHECK(p && pinned_free(p));
+        CHECK(fake::host_bytes <= 128 * MiB);
+    }
+    CHECK(fake::host_mallocs == 129);
+    // ragged sizes: every result fits a block that is there
+    for (size_t n = 600 * 1024; n < MiB; n += 5 * 1024) {
+        void* p = pinned_alloc(n);
+        CHECK(p && pinned_free(p));
+    }
+    CHECK(fake::host_mallocs == 129);
+    // sizes that change for good: the old ones make room
+    all.clear();
+    for (int i = 0; i < 16; i++) all.push_back(pinned_alloc(8 * MiB));
+    for (void* p : all) CHECK(p && pinned_free(p));
+    CHECK(fake::host_bytes == 128 * MiB && fake::host_mallocs == 129 + 16);
+    for (int i = 0; i < 16; i++) all[i] = pinned_alloc(8 * MiB);
+    CHECK(fake::host_mallocs == 129 + 16);
+    for (void* p : all) CHECK(pinned_free(p));
+    CHECK(!pinned_free(all[0]) && !pinned_free(&all));
+    // the bound on what is handed out
+    all.clear();
+    for (int i = 0; i < 8; i++) all.push_back(pinned_alloc(64 * MiB));
+    for (void* p : all) CHECK(p);
+    CHECK(!pinned_alloc(1) && !pinned_alloc(0));
+    CHECK(pinned_free(all[7]));
+    CHECK((all[7] = pinned_alloc(1)) != nullptr);
+    for (void* p : all) CHECK(pinned_free(p));
+    CHECK(fake::host_bytes <= 128 * MiB);
+    // out of memory: what is kept is given up for the request
+    fake::host_bytes_limit = 100 * MiB;
+    void* p = pinned_alloc(90 * MiB);
+    CHECK(p && fake::host_bytes == 90 * MiB);
+    CHECK(!pinned_alloc(20 * MiB) && pinned_free(p));
+    CHECK((p = pinned_alloc(20 * MiB)) && pinned_free(p));
+    io_shutdown();
+    CHECK(fake::host_bytes == 0);
+}
+
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}, {"first_call", first_call}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}, {"first_call", first_call}, {"pool_of_results", pool_of_results}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.run();
