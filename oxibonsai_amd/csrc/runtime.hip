@@ -28,6 +28,9 @@ namespace oxb {
 
 thread_local std::string t_last_error;
 
+Runtime g_rt;
+std::recursive_mutex g_mu;
+
 int fail(int code, const char* fmt, ...) {
     char buf[512];
     va_list ap;
@@ -35,6 +38,9 @@ int fail(int code, const char* fmt, ...) {
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     t_last_error = buf;
+    // An error that is reported here is not left for the check behind the next launch, which asks for the last error of any
+    // call (a failed hipMalloc, above all).
+    if (g_rt.ready) (void)hipGetLastError();
     return code;
 }
 
@@ -42,9 +48,6 @@ int hip_fail(hipError_t e, const char* what) {
     int code = (e == hipErrorOutOfMemory) ? OXB_HIP_OUT_OF_MEMORY : OXB_HIP_KERNEL_LAUNCH;
     return fail(code, "%s: %s", what, hipGetErrorString(e));
 }
-
-Runtime g_rt;
-std::recursive_mutex g_mu;
 
 // Scratch of the allocation-free GEMM entry point (oxb_hip_gemm_dev_static): packed fp16 activations, per-row
 // exponents and multipliers, and the partial sums of a K split.  It lives in the code object, so the GPU the library

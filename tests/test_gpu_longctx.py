@@ -452,3 +452,26 @@ def test_page_pool_accounting(backend):
                 gpu.set_attention(KV_F16, 0, 0, **bad)
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("mode", [KV_F16])
+def test_failed_cache_change_leaves_the_model_decoding(backend, mode):
+    # a page pool that no device holds: the call fails and the model is back on the contiguous fp16 cache
+    cfg = dict(TINY, fmt=Q1, nq=8, nkv=8, hd=32, h=256, max_seq=8 * 512 + 64)
+    w = synth.make_model(cfg, 97)
+    gpu = HipModel(backend, cfg, w, batch=4)
+    cpu = oracle.OracleModel(cfg, w, kv_mode=oracle.KV_F16)
+    try:
+        gpu.set_attention(mode, 0, 0)
+        rows = synth.embedding_rows(98, range(12), cfg["h"]) * 50.0
+        gpu.forward(np.stack([rows[0]] * 4), 0)
+        with pytest.raises(GpuError) as e:
+            gpu.set_attention(mode, 0, 0, 128, (1 << 32) - 1)
+        assert e.value.kind == "OutOfMemory"
+        assert gpu.kv_pool().total_pages == 0
+        for pos in range(6):
+            got, _ = gpu.forward(np.stack([rows[pos]] * 4), pos)
+            want = cpu.forward(rows[pos], pos)
+            assert parity_violations(got[3], want) == 0, pos
+    finally:
+        gpu.close()
