@@ -704,6 +704,7 @@ static int alloc_kv_cache(Model& m, uint32_t kv_mode, uint32_t page_size, uint32
         OXB_TRY_HIP(hipMemset(m.d_table, 0, m.h_table.size() * 4), "page table clear");
     }
     m.kv_mode = kv_mode;
+    m.attn_wide = attn_wide(m, kv_mode);
     return OXB_HIP_OK;
 }
 
@@ -833,7 +834,6 @@ int oxb_hip_model_set_attention(uint64_t model, const oxb_attention_options* opt
             return rc;
         }
     }
-    m->attn_wide = attn_wide(*m, m->kv_mode);
     m->window = opt->window_size;
     m->sinks = opt->sink_tokens;
     return OXB_HIP_OK;

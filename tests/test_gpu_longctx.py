@@ -454,9 +454,11 @@ def test_page_pool_accounting(backend):
         gpu.close()
 
 
-@pytest.mark.parametrize("mode", [KV_F16])
+@pytest.mark.parametrize("mode", [KV_F16, KV_I8, KV_FP8_E4M3])
 def test_failed_cache_change_leaves_the_model_decoding(backend, mode):
-    # a page pool that no device holds: the call fails and the model is back on the contiguous fp16 cache
+    # a page pool that no device holds: the call fails and the model is back on the contiguous fp16 cache.  64 positions
+    # more than eight slots of 512: with one-byte rows this shape runs the decode attention's eight-wave form, which fp16 rows
+    # do not have.
     cfg = dict(TINY, fmt=Q1, nq=8, nkv=8, hd=32, h=256, max_seq=8 * 512 + 64)
     w = synth.make_model(cfg, 97)
     gpu = HipModel(backend, cfg, w, batch=4)
