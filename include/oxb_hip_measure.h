@@ -4,7 +4,7 @@
  * None of these stands in for an interface of the reference's kernel tier: a `NativeHipBackend` does not bind them.
  * They exist for the benchmark (per-kernel timings with HIP events on the stream the kernel runs on, as the reference
  * times its own kernels under CUDA_PROFILE / OXIBONSAI_PROFILE_GPU, KG/cuda_full_layer/mod.rs:339-344,
- * KG/metal_full_layer/functions.rs:17-35) and for one bit-exactness test of the sampler's in-order sum.
+ * KG/metal_full_layer/functions.rs:17-35) and for tests of single kernels: the prefill attention, the sampler's in-order sum.
  */
 #ifndef OXB_HIP_MEASURE_H
 #define OXB_HIP_MEASURE_H
@@ -33,6 +33,12 @@ int  oxb_hip_set_gemv_packed_min_batch(uint32_t n);
 /* Packs x once, then times `iters` prefill GEMM launches with events on the library's stream. */
 int  oxb_hip_profile_gemm(uint64_t id, const float* d_x, float* d_y, uint32_t m, uint32_t n_rows, uint32_t k,
                           uint32_t warmup, uint32_t iters, float* avg_us);
+/* The attention of one layer's prefill on its own: qkv [n_tokens][(nq + 2 nkv) hd] (host), as the layer's QKV product
+ * leaves it, is normed and rotated, its K and V rows go to the cache of sequence `seq` at pos_start .., and out
+ * [n_tokens][nq hd] (host) receives what the queries attend to.  Inside oxb_hip_prefill these values are rounded to fp16
+ * by the next product, which hides what this kernel's own precision is. */
+int  oxb_hip_model_prefill_attention(uint64_t model, uint32_t layer, uint32_t seq, const float* qkv, uint32_t n_tokens,
+                                     uint32_t pos_start, float* out);
 /* The f32 sum of x[0..n) taken element by element from 0, as the loop `sum += *v` of the reference's softmax does
  * (sampling.rs:126-130); all x >= 0.  The filter-off sampler depends on this order bit for bit; exposed so that it can
  * be checked on its own. */

@@ -58,6 +58,7 @@ _SIGNATURES = {
     "oxb_hip_model_set_lm_head": ([C.c_uint64, C.c_uint64, C.c_uint64, C.c_uint32], C.c_int),
     "oxb_hip_model_set_rope_rows": ([C.c_uint64, C.c_uint32, C.c_uint32, f32p, f32p], C.c_int),
     "oxb_hip_prefill": ([C.c_uint64, C.c_uint32, f32p, C.c_uint32, C.c_uint32, f32p, u32p], C.c_int),
+    "oxb_hip_model_prefill_attention": ([C.c_uint64, C.c_uint32, C.c_uint32, f32p, C.c_uint32, C.c_uint32, f32p], C.c_int),
     "oxb_hip_model_uses_graph": ([C.c_uint64], C.c_int),
     "oxb_hip_model_set_attention": ([C.c_uint64, C.c_void_p], C.c_int),
     "oxb_hip_model_get_attention": ([C.c_uint64, C.c_void_p], C.c_int),

@@ -497,6 +497,68 @@ static int ensure_prefill_buffers(Model& m, uint32_t rows) {
     return OXB_HIP_OK;
 }
 
+// QK-norm, RoPE and the store of M new K and V rows of one layer, then the causal attention of the M queries: qkv
+// [M][(nq + 2 nkv) hd] (raw projections) -> out [M][nq hd].
+static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t M, uint32_t pos_start, const float* qkv, const float* q_norm,
+                                    const float* k_norm, float* out) {
+    const oxb_model_desc& d = m.d;
+    hipStream_t st = g_rt.stream;
+    OxbQkParams qp;
+    qp.qkv = qkv;
+    qp.qkv_stride = (d.nq + 2 * d.nkv) * d.hd;
+    qp.q_norm = q_norm;
+    qp.k_norm = k_norm;
+    qp.cos_t = m.cos_t;
+    qp.sin_t = m.sin_t;
+    qp.pos = nullptr;
+    qp.pos_base = pos_start;
+    qp.seq = seq;
+    qp.q_rope = nullptr;  // the attention kernel norms and rotates Q itself
+    qp.k_cache = m.k_cache;
+    qp.v_cache = m.v_cache;
+    qp.k_scale = m.k_scale;
+    qp.v_scale = m.v_scale;
+    qp.kv_mode = m.kv_mode;
+    qp.kv = kv_layout(m);
+    qp.nq = d.nq;
+    qp.nkv = d.nkv;
+    qp.hd = d.hd;
+    qp.max_seq = d.max_seq;
+    qp.n_layers = d.n_layers;
+    qp.layer = L;
+    qp.eps = d.eps;
+    OXB_TRY_HIP(oxb_launch_qk_norm_rope_store(qp, M, st), "kernel launch failed: qk_norm_rope_store");
+    OxbPrefillAttnParams ap;
+    ap.qkv = qkv;
+    ap.qkv_stride = qp.qkv_stride;
+    ap.q_norm = q_norm;
+    ap.cos_t = m.cos_t;
+    ap.sin_t = m.sin_t;
+    ap.eps = d.eps;
+    ap.k_cache = m.k_cache;
+    ap.v_cache = m.v_cache;
+    ap.k_scale = m.k_scale;
+    ap.v_scale = m.v_scale;
+    ap.kv_mode = m.kv_mode;
+    ap.kv = kv_layout(m);
+    ap.seq = seq;
+    ap.layer = L;
+    ap.window = m.window;
+    ap.sinks = m.sinks;
+    ap.out = out;
+    ap.M = M;
+    ap.pos_start = pos_start;
+    ap.nq = d.nq;
+    ap.nkv = d.nkv;
+    ap.hd = d.hd;
+    ap.max_seq = d.max_seq;
+    ap.scale = 1.0f / sqrtf((float)d.hd);
+    OXB_TRY(m.pf_part.ensure(oxb_attn_prefill_part_bytes(ap, g_rt.n_cus)));
+    ap.part = (float*)m.pf_part.ptr;
+    OXB_TRY_HIP(oxb_launch_attn_prefill(ap, g_rt.n_cus, st), "kernel launch failed: attn_prefill");
+    return OXB_HIP_OK;
+}
+
 // All layers for M token rows of sequence `seq` at positions pos_start .. pos_start + M - 1: batched
 // projections on the matrix cores (RMSNorm and SwiGLU fused into the fp16 packer of the GEMM that consumes them), one causal attention launch per layer, KV written to the cache; then the
 // LM head and the greedy token for the last row.
@@ -518,59 +580,7 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
         const Weight* wdn = mat_ptr(ly.down, d.fmt, d.h, d.inter, "down", &rc);
         if (rc) return rc;
         OXB_TRY(gemm_device(*wqkv, m.pf_hidden, d.h, m.pf_qkv, M, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, nullptr, &sum));
-        OxbQkParams qp;
-        qp.qkv = m.pf_qkv;
-        qp.qkv_stride = qkv_rows;
-        qp.q_norm = q_norm;
-        qp.k_norm = k_norm;
-        qp.cos_t = m.cos_t;
-        qp.sin_t = m.sin_t;
-        qp.pos = nullptr;
-        qp.pos_base = pos_start;
-        qp.seq = seq;
-        qp.q_rope = nullptr;  // the attention kernel norms and rotates Q itself
-        qp.k_cache = m.k_cache;
-        qp.v_cache = m.v_cache;
-        qp.k_scale = m.k_scale;
-        qp.v_scale = m.v_scale;
-        qp.kv_mode = m.kv_mode;
-        qp.kv = kv_layout(m);
-        qp.nq = d.nq;
-        qp.nkv = d.nkv;
-        qp.hd = d.hd;
-        qp.max_seq = d.max_seq;
-        qp.n_layers = d.n_layers;
-        qp.layer = L;
-        qp.eps = d.eps;
-        OXB_TRY_HIP(oxb_launch_qk_norm_rope_store(qp, M, st), "kernel launch failed: qk_norm_rope_store");
-        OxbPrefillAttnParams ap;
-        ap.qkv = m.pf_qkv;
-        ap.qkv_stride = qkv_rows;
-        ap.q_norm = q_norm;
-        ap.cos_t = m.cos_t;
-        ap.sin_t = m.sin_t;
-        ap.eps = d.eps;
-        ap.k_cache = m.k_cache;
-        ap.v_cache = m.v_cache;
-        ap.k_scale = m.k_scale;
-        ap.v_scale = m.v_scale;
-        ap.kv_mode = m.kv_mode;
-        ap.kv = kv_layout(m);
-        ap.seq = seq;
-        ap.layer = L;
-        ap.window = m.window;
-        ap.sinks = m.sinks;
-        ap.out = m.pf_attn;
-        ap.M = M;
-        ap.pos_start = pos_start;
-        ap.nq = d.nq;
-        ap.nkv = d.nkv;
-        ap.hd = d.hd;
-        ap.max_seq = d.max_seq;
-        ap.scale = 1.0f / sqrtf((float)d.hd);
-        OXB_TRY(m.pf_part.ensure(oxb_attn_prefill_part_bytes(ap, g_rt.n_cus)));
-        ap.part = (float*)m.pf_part.ptr;
-        OXB_TRY_HIP(oxb_launch_attn_prefill(ap, g_rt.n_cus, st), "kernel launch failed: attn_prefill");
+        OXB_TRY(encode_prefill_attention(m, L, seq, M, pos_start, m.pf_qkv, q_norm, k_norm, m.pf_attn));
         OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr, &sum));
         // SwiGLU in the epilogue of the gate || up product: the activation [M][inter] is all that is written
         OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, nullptr, &sum));
@@ -1223,6 +1233,35 @@ int oxb_hip_prefill(uint64_t model, uint32_t seq, const float* hidden, uint32_t 
     OXB_TRY(io.finish("prefill"));
     if (token_out_or_null) *token_out_or_null = m.h_tokens[seq];
     return OXB_HIP_OK;
+    OXB_API_END
+}
+
+int oxb_hip_model_prefill_attention(uint64_t model, uint32_t layer, uint32_t seq, const float* qkv, uint32_t n_tokens, uint32_t pos_start,
+                                    float* out) {
+    OXB_API_BEGIN
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    Model* mp = find_model(model);
+    if (!mp) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: unknown model %llu", (unsigned long long)model);
+    Model& m = *mp;
+    const oxb_model_desc& d = m.d;
+    if (!qkv || !out || n_tokens == 0) return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: null buffer or no tokens");
+    if (layer >= d.n_layers || seq >= d.batch || (uint64_t)pos_start + n_tokens > d.max_seq)
+        return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: layer %u, sequence %u, positions %u..%llu out of range", layer, seq, pos_start,
+                    (unsigned long long)pos_start + n_tokens - 1);
+    if (m.checked_gen != g_rt.weights_gen) OXB_TRY(check_model_handles(m));
+    int rc = OXB_HIP_OK;
+    const float* q_norm = vec_ptr(m.layers[layer].q_norm, d.hd, "q_norm", &rc);
+    const float* k_norm = vec_ptr(m.layers[layer].k_norm, d.hd, "k_norm", &rc);
+    if (rc) return rc;
+    OXB_TRY(kv_reserve(m, seq, (uint64_t)pos_start + n_tokens));
+    OXB_TRY(kv_sync_table(m));
+    OXB_TRY(ensure_prefill_buffers(m, n_tokens));
+    IoCall io;
+    OXB_TRY(io.begin());
+    OXB_TRY(io.upload(m.pf_qkv, qkv, (size_t)n_tokens * (d.nq + 2 * d.nkv) * d.hd * 4));
+    OXB_TRY(encode_prefill_attention(m, layer, seq, n_tokens, pos_start, m.pf_qkv, q_norm, k_norm, m.pf_attn));
+    OXB_TRY(io.download(out, m.pf_attn, (size_t)n_tokens * d.nq * d.hd * 4));
+    return io.finish("prefill_attention");
     OXB_API_END
 }
 

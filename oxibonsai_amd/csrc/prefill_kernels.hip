@@ -29,8 +29,11 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 //                                               scores keep fp32-level accuracy)
 //   O^T[d][q]   += sum_key V[key][d] P[q][key]  B = the lane's own 8 probabilities of 32 keys,
 //                                               A = V gathered for exactly those 8 keys (two transposing LDS reads)
-// Lane (q = lane % 16, g = lane / 16) holds keys {4g..4g+3} and {16+4g..16+4g+3} of every 32 keys.  The sum of the
-// probabilities is one more MFMA, against an operand of ones: it adds the same rounded values the numerator adds.
+// Lane (q = lane % 16, g = lane / 16) holds keys {4g..4g+3} and {16+4g..16+4g+3} of every 32 keys, and sums their
+// probabilities in fp32 as they are before the rounding to fp16 that the second product needs.  They are relative to the
+// row's running maximum itself, so that the largest is exactly 1: against float64, 16 000 keys, the output is 5e-7 off where one
+// key lies 12 above the rest, 4e-5 with scores of spread 3.  (Summing the rounded values on the matrix cores, relative to a
+// power of two that follows the maximum at a distance, gives 2e-5 and 1.7e-4.)
 //
 // The four waves of a workgroup walk the same keys and values: they take `hpw` q heads of ONE kv head (4, 2 or 1,
 // whatever divides the group) times 4 / hpw consecutive runs of QT query tiles.  Each block of KB keys (K and V) is
@@ -39,11 +42,10 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // XOR with the row number, which keeps both kinds of read free of bank conflicts.
 //
 // What bounds it: the SIMDs' issue slots.  With 16 queries per wave and 32-key blocks the kernel issued about 200 vector
-// instructions around 24 MFMAs per block (94 us per layer for 2048 tokens of the 8B shape, 201 us for 301 tokens behind
-// 6000 INT8 positions).  Two query tiles per wave halve the LDS reads per MFMA; a running maximum that is replaced only
-// when a score exceeds it by more than 8 (powers of two: the result does not depend on when) takes the rescaling of the
-// accumulators out of nearly every block; the visibility tests run only in blocks that some query of the wave sees in part:
-// 77 us and 76 us per layer for the two.
+// instructions around 24 MFMAs per block.  Two query tiles per wave halve the LDS reads per MFMA; the accumulators of a tile
+// are rescaled only in blocks that bring a new maximum for one of its 16 queries; the visibility tests run only in blocks that
+// some query of the wave sees in part.  Per layer of the 8B shape, in a kernel trace: 90 us for 2048 tokens, 86 us (and 9 for
+// the merge) for 301 tokens behind 6000 INT8 positions.
 //
 // Options as in the decode attention: quantised cache rows (template KVM; the codes are widened to exact fp16
 // numbers on their way into LDS, V already multiplied by its row scale there, the K row scale multiplies the
@@ -65,7 +67,6 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
     constexpr int PPR = HD / 8;                                      // 16-byte pieces of an LDS row
     constexpr int RB = PPR >= 16 ? 1 : 16 / PPR, PM = (PPR < 16 ? PPR : 16) - 1;  // rows per 256 bytes; mask of the permutation
     constexpr int NI = QC ? (RPW * HD / 16 + 63) / 64 : RPW * PPR / 64;  // 16-byte pieces per lane and block, of K and of V
-    constexpr float LAZY = 8.0f;
     __shared__ __attribute__((aligned(16))) _Float16 ks0[KB * HD], ks1[KB * HD], vs0[KB * HD], vs1[KB * HD];
     __shared__ __attribute__((aligned(16))) float kscale0[KB], kscale1[KB];  // K row scales of the block (quantised cache)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, qi = lane & 15u, g = lane >> 4;
@@ -245,18 +246,14 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
     // of 16 rows, where the permutation is the same.
     const uint32_t k_at = (qi * PPR + (g ^ ((qi / RB) & PM))) * 8;
     const uint32_t v_row = 4 * g + (qi >> 2), v_at = (v_row * PPR + (((qi >> 1) & 1u) ^ ((v_row / RB) & PM))) * 8 + (qi & 1u) * 4;
-    v8h ones;
-#pragma unroll
-    for (int e = 0; e < 8; e++) ones[e] = (_Float16)1.0f;
-
-    v4f O[QT][NS], lsum[QT];
-    float m_ref[QT];
+    v4f O[QT][NS];
+    float m_run[QT], lsum[QT];  // running maximum of the tile's queries; this lane's share of the sum of their probabilities
 #pragma unroll
     for (int t = 0; t < QT; t++) {
 #pragma unroll
         for (int i = 0; i < NS; i++) O[t][i] = (v4f){0.f, 0.f, 0.f, 0.f};
-        lsum[t] = (v4f){0.f, 0.f, 0.f, 0.f};
-        m_ref[t] = -INFINITY;
+        lsum[t] = 0.f;
+        m_run[t] = -INFINITY;
     }
     auto block = [&](const _Float16* kb, const _Float16* vb, const float* ksc, uint32_t blk_key0) {
         uint32_t ka = k_at, va = v_at;
@@ -323,37 +320,31 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
                             S[t][kt][v] = vis ? S[t][kt][v] : -INFINITY;
                         }
             }
-            float mx[QT];
-            bool grow = false;
+            v8h P[QT];
 #pragma unroll
             for (int t = 0; t < QT; t++) {
                 const float m0 = max_raw(max_raw(S[t][0][0], S[t][0][1]), max_raw(S[t][0][2], S[t][0][3]));
                 const float m1 = max_raw(max_raw(S[t][1][0], S[t][1][1]), max_raw(S[t][1][2], S[t][1][3]));
-                mx[t] = max_rows4_raw(max_raw(m0, m1));
-                grow |= mx[t] > m_ref[t] + LAZY;
-            }
-            if (__builtin_amdgcn_ballot_w64(grow)) {
-#pragma unroll
-                for (int t = 0; t < QT; t++) {
-                    // a whole number: the factors are powers of two and leave every bit of the sums as it is
-                    const float m_new = mx[t] > m_ref[t] ? ceilf(mx[t]) : m_ref[t];
-                    const float alpha = m_ref[t] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
-                    m_ref[t] = m_new;
+                const float mx = max_rows4_raw(max_raw(m0, m1));
+                if (__builtin_amdgcn_ballot_w64(mx > m_run[t])) {  // a new maximum for some query of the tile
+                    const float m_new = max_raw(m_run[t], mx);
+                    const float alpha = m_run[t] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[t] - m_new);
+                    m_run[t] = m_new;
 #pragma unroll
                     for (int sl = 0; sl < NS; sl++)
 #pragma unroll
                         for (int v = 0; v < 4; v++) O[t][sl][v] *= alpha;
-#pragma unroll
-                    for (int v = 0; v < 4; v++) lsum[t][v] *= alpha;
+                    lsum[t] *= alpha;
                 }
-            }
-            v8h P[QT];
-#pragma unroll
-            for (int t = 0; t < QT; t++) {
                 // (a query that has seen nothing yet keeps its empty state: every probability 0)
-                const float m = m_ref[t] == -INFINITY ? 0.f : m_ref[t];
+                const float m = m_run[t] == -INFINITY ? 0.f : m_run[t];
+                float pe[8];
 #pragma unroll
-                for (int e = 0; e < 8; e++) P[t][e] = (_Float16)__builtin_amdgcn_exp2f(S[t][e >> 2][e & 3] - m);
+                for (int e = 0; e < 8; e++) {
+                    pe[e] = __builtin_amdgcn_exp2f(S[t][e >> 2][e & 3] - m);
+                    P[t][e] = (_Float16)pe[e];
+                }
+                lsum[t] += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
             }
             v8h V2[NS - NV];
 #pragma unroll
@@ -364,8 +355,6 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
 #pragma unroll
                 for (int t = 0; t < QT; t++)
                     O[t][sl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl < NV ? V[sl < NV ? sl : 0] : V2[sl < NV ? 0 : sl - NV], P[t], O[t][sl], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < QT; t++) lsum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, P[t], lsum[t], 0, 0, 0);
         }
     };
     if (i0 < i1) {
@@ -384,8 +373,8 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
 #pragma unroll
     for (int t = 0; t < QT; t++) {
         const uint32_t tok = t_first + t * 16 + qi;
+        const float l = sum_rows4(lsum[t]);
         if (tok >= p.M) continue;
-        const float l = lsum[t][0];
         if (gridDim.y == 1) {
             const float inv = l > 0.f ? 1.0f / l : 0.f;
             float* o = p.out + ((size_t)tok * p.nq + head) * HD + 4 * g;
@@ -394,7 +383,7 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
                 *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[t][sl][0] * inv, O[t][sl][1] * inv, O[t][sl][2] * inv, O[t][sl][3] * inv);
         } else {
             const size_t at = ((size_t)blockIdx.y * p.M + tok) * p.nq + head;
-            if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_ref[t], l);
+            if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_run[t], l);
             if (!(l == 0.f)) {  // (an empty run is left out of the merge)
                 float* o = p.part + (size_t)gridDim.y * p.M * p.nq * 2 + at * HD + 4 * g;
 #pragma unroll

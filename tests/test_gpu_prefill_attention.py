@@ -1,0 +1,165 @@
+"""The prefill's attention kernel on its own (oxb_hip_model_prefill_attention), against softmax(q K^T / sqrt(hd)) V in
+float64 over the cache rows that the device stored.
+
+What the kernel rounds, element by element of the output: every probability to fp16 (2^-11 of it), every V value of a
+quantised cache twice (the row scale to fp16, the product to fp16), and the scores to fp32 accuracy (q enters as fp16 hi +
+lo, 2^-22 of it; sums of hd products).  With sum(p |v|) for one output element, p the float64 probabilities,
+
+    |out - want| <= (2^-11 + 2 * 2^-11 [quantised] + 2^-15) sum(p |v|) + n_keys 2^-25 max|v| / sum
+
+where the last term covers probabilities below fp16's smallest normal number (a quantum of 2^-24, sum: in units of the
+largest probability)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import Q1
+from oracle import oracle
+from oxibonsai_amd import _lib, synth
+from oxibonsai_amd.backend import _check
+from oxibonsai_amd.model import KV_F16, KV_FP8_E4M3, KV_I8, HipModel
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(backend, nq, nkv, hd, max_seq, q_norm=None, seed=1, batch=1):
+    h = 128
+    cfg = dict(fmt=Q1, n_layers=2, h=h, inter=256, nq=nq, nkv=nkv, hd=hd, vocab=32, max_seq=max_seq, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, seed)
+    if q_norm is not None:
+        for layer in w["layers"]:
+            layer["q_norm"], layer["k_norm"] = np.full(hd, q_norm, np.float32), np.ones(hd, np.float32)
+    return HipModel(backend, cfg, w, batch=batch), w
+
+
+def _attend(gpu, layer, seq, qkv, pos):
+    cfg = gpu.cfg
+    qkv = np.ascontiguousarray(qkv, dtype=np.float32)
+    out = np.full((qkv.shape[0], cfg["nq"] * cfg["hd"]), np.nan, dtype=np.float32)
+    _check(_lib.lib().oxb_hip_model_prefill_attention(gpu.id, layer, seq, qkv.ctypes.data_as(_lib.f32p), qkv.shape[0], pos, out.ctypes.data_as(_lib.f32p)))
+    return out.reshape(qkv.shape[0], cfg["nq"], cfg["hd"])
+
+
+def _rows(gpu, layer, head, n, seq):
+    """The device's own cache rows as float64 values."""
+    mode = gpu.attention().kv_dtype
+    k, v, ks, vs = gpu.read_kv(layer, head, 0, n, seq)
+    if mode == KV_F16:
+        return k.astype(np.float64), v.astype(np.float64)
+    val = (lambda c: c.view(np.int8).astype(np.float64)) if mode == KV_I8 else (lambda c: oracle.fp8_decode(np.arange(256, dtype=np.uint8)).astype(np.float64)[c])
+    return val(k) * ks[:, None].astype(np.float64), val(v) * vs[:, None].astype(np.float64)
+
+
+def _queries(cfg, w, layer, qkv, cos, sin):
+    """Q in float64: per-head RMSNorm, rotation of the pairs (d, d + hd/2), log2 e / sqrt(hd)."""
+    M, nq, hd = qkv.shape[0], cfg["nq"], cfg["hd"]
+    q = qkv[:, :nq * hd].astype(np.float64).reshape(M, nq, hd)
+    q = q / np.sqrt((q * q).mean(-1, keepdims=True) + cfg["eps"]) * w["layers"][layer]["q_norm"].astype(np.float64)
+    a, b = q[..., :hd // 2], q[..., hd // 2:]
+    c, s = cos[:, None, :].astype(np.float64), sin[:, None, :].astype(np.float64)
+    return np.concatenate([a * c - b * s, a * s + b * c], axis=-1) * (np.log2(np.e) / np.sqrt(hd))
+
+
+def _visible(pos, n, window, sinks):
+    key, qp = np.arange(n)[None, :], pos[:, None]
+    return (key <= qp) & ((window == 0) | (key < sinks) | (qp - key < max(window - sinks, 0)))
+
+
+# (queries, first position, q heads, kv heads, head_dim, cache, window, sinks, page size): what the launcher makes of them is
+# noted as query tiles per wave, runs of keys x blocks per run.
+CASES = [
+    (7, 0, 2, 1, 128, KV_F16, 0, 0, 0),           # one tile, a single block
+    (130, 0, 8, 2, 64, KV_F16, 0, 0, 0),          # two tiles, 3 x 1
+    (5, 1200, 1, 1, 128, KV_F16, 0, 0, 0),        # one tile, 19 x 1: an odd number (19 x 5 x 1) of rows of sums
+    (7, 1500, 3, 3, 128, KV_F16, 0, 0, 16),       # one tile, 24 x 1, paged
+    (49, 3001, 2, 2, 64, KV_F16, 0, 0, 32),       # two tiles (the fewest queries that take two), 24 x 2, paged
+    (48, 3001, 4, 2, 128, KV_F16, 0, 0, 0),       # one tile (the most), 24 x 2
+    (64, 4000, 4, 2, 128, KV_F16, 0, 0, 0),       # two tiles, 32 x 2
+    (331, 768, 4, 2, 128, KV_I8, 0, 0, 0),        # two tiles, blocks of 32 keys, 7 x 5
+    (331, 768, 4, 2, 128, KV_FP8_E4M3, 0, 0, 16),
+    (33, 2900, 4, 1, 32, KV_I8, 0, 0, 64),        # one tile, 23 x 2: half a wave fetches all pieces of a block
+    (100, 3000, 4, 1, 32, KV_FP8_E4M3, 0, 0, 0),  # two tiles, 25 x 2
+    (3, 2300, 5, 1, 128, KV_I8, 0, 0, 128),       # five heads: one per workgroup
+    (21, 1000, 2, 1, 256, KV_F16, 0, 0, 0),       # 32 x 1
+    (17, 900, 2, 2, 256, KV_I8, 0, 0, 16),        # 29 x 1
+    (90, 2100, 8, 2, 64, KV_F16, 700, 5, 0),      # a window: 15 x 1, runs that some queries see nothing of
+    (50, 2500, 4, 2, 128, KV_I8, 1200, 70, 16),   # 15 x 3, sinks across a block's edge, paged
+    (40, 2500, 4, 2, 64, KV_FP8_E4M3, 64, 64, 32),  # nothing visible but the sinks
+]
+
+
+@pytest.mark.parametrize("M,start,nq,nkv,hd,mode,window,sinks,page", CASES)
+def test_prefill_attention_matches_float64(backend, M, start, nq, nkv, hd, mode, window, sinks, page):
+    max_seq, layer, seq = start + M + 9, 1, 1
+    gpu, w = _model(backend, nq, nkv, hd, max_seq, batch=2)
+    g = np.random.default_rng([M, start, hd, mode])
+    try:
+        if mode != KV_F16 or window or page:
+            gpu.set_attention(mode, window, sinks, page, 2 * -(-max_seq // page) if page else 0)
+        ang = g.uniform(0, 2 * np.pi, (max_seq, hd // 2)).astype(np.float32)
+        cos, sin = np.cos(ang), np.sin(ang)
+        gpu.set_rope_rows(0, cos, sin)
+        qkv = g.standard_normal((start + M, (nq + 2 * nkv) * hd)).astype(np.float32)
+        if start:
+            gpu.kv_reserve(0, 17)                 # (another sequence's pages in between)
+            _attend(gpu, layer, seq, qkv[:start], 0)
+        got = _attend(gpu, layer, seq, qkv[start:], start)
+        n = start + M
+        q = _queries(gpu.cfg, w, layer, qkv[start:], cos[start:n], sin[start:n])
+        vis = _visible(np.arange(start, n), n, window, sinks)
+        worst = 0.0
+        for kvh in range(nkv):
+            K, V = _rows(gpu, layer, kvh, n, seq)
+            for hh in range(nq // nkv):
+                s = np.where(vis, q[:, kvh * (nq // nkv) + hh] @ K.T, -np.inf)
+                p = np.exp2(s - s.max(1, keepdims=True))
+                total = p.sum(1, keepdims=True)
+                want, size = p @ V / total, p @ np.abs(V) / total
+                bound = ((3 if mode != KV_F16 else 1) * 2.0**-11 + 2.0**-15) * size + n * 2.0**-25 * np.abs(V).max() / total
+                worst = max(worst, float((np.abs(got[:, kvh * (nq // nkv) + hh] - want) / bound).max()))
+        assert worst <= 1.0, worst
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("shape", ["spread", "sink", "far sink", "late peak"])
+@pytest.mark.parametrize("M", [16, 64])
+def test_prefill_attention_weights_are_relative_to_the_row_maximum(backend, M, shape):
+    # Against float64 the kernel is as good as probabilities rounded to fp16 relative to the row's own maximum, over their
+    # unrounded sum: the largest weight is exactly 1, which an attention sink (one key 12 or 17 above 16 000 others) lives on.
+    # The comparison allows a quarter more, and 3e-6 for sums of 16 000 fp32 terms.
+    nq, nkv, hd, n = 4, 2, 128, 16000 + M
+    c = {"spread": 3.0, "sink": 12.0 / 11.2, "far sink": 17.0 / 11.2, "late peak": 6.0 / 11.2}[shape]
+    gpu, w = _model(backend, nq, nkv, hd, n, q_norm=c)
+    g = np.random.default_rng([M, len(shape)])
+    try:
+        gpu.set_rope_rows(0, np.ones((n, hd // 2), np.float32), np.zeros((n, hd // 2), np.float32))
+        x = g.standard_normal((n, nq + 2 * nkv, hd)).astype(np.float32)
+        if shape != "spread":
+            u = g.standard_normal(hd)
+            u /= np.linalg.norm(u)
+            k = x[:, nq:nq + nkv]
+            k -= (k @ u)[..., None] * u
+            k[9000 if shape == "late peak" else 0] = u * 11.0
+            x[:, :nq] = 11.0 * u + 0.12 * x[:, :nq]
+        qkv = x.reshape(n, -1)
+        _attend(gpu, 0, 0, qkv[:16000], 0)
+        got = _attend(gpu, 0, 0, qkv[16000:], 16000)
+        q = _queries(gpu.cfg, w, 0, qkv[16000:], np.ones((M, hd // 2)), np.zeros((M, hd // 2)))
+        vis = _visible(np.arange(16000, n), n, 0, 0)
+        err = ref = size = 0.0
+        for h in range(nq):
+            K, V = _rows(gpu, 0, h // (nq // nkv), n, 0)
+            s = np.where(vis, q[:, h] @ K.T, -np.inf)
+            p = np.exp2(s - s.max(1, keepdims=True))
+            want = p @ V / p.sum(1, keepdims=True)
+            rounded = p.astype(np.float16).astype(np.float64) @ V / p.sum(1, keepdims=True)
+            err += ((got[:, h] - want)**2).sum()
+            ref += ((rounded - want)**2).sum()
+            size += (want**2).sum()
+        err, ref = np.sqrt(err / size), np.sqrt(ref / size)
+        print(f"{shape}, {M} queries: {err:.2e} off float64, weights rounded against the maximum {ref:.2e}")
+        assert err <= 1.25 * ref + 3e-6, (err, ref)
+    finally:
+        gpu.close()
