@@ -56,6 +56,9 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // walk into runs of p.blocks_per_split blocks, each run leaves its un-normalised sums in p.part, and
 // attn_prefill_merge_kernel adds them in order.
 // ---------------------------------------------------------------------------
+// p.part: maximum and sum of every (run, query, head), then from a 16-byte boundary on their outputs.
+__host__ __device__ constexpr size_t pf_part_head(size_t n_splits, size_t rows) { return (n_splits * rows * 2 + 3) & ~(size_t)3; }
+
 // Keys per block: 64, or 32 where the LDS (4 x KB x 2 HD bytes) or the registers that hold a block of codes leave no room.
 constexpr int pf_block_keys(int hd, bool quantised) { return hd == 256 || (hd == 128 && quantised) ? 32 : 64; }
 
@@ -385,7 +388,7 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
             const size_t at = ((size_t)blockIdx.y * p.M + tok) * p.nq + head;
             if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_run[t], l);
             if (!(l == 0.f)) {  // (an empty run is left out of the merge)
-                float* o = p.part + (size_t)gridDim.y * p.M * p.nq * 2 + at * HD + 4 * g;
+                float* o = p.part + pf_part_head(gridDim.y, (size_t)p.M * p.nq) + at * HD + 4 * g;
 #pragma unroll
                 for (int sl = 0; sl < NS; sl++)
                     *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[t][sl][0], O[t][sl][1], O[t][sl][2], O[t][sl][3]);
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
     const uint32_t i = blockIdx.x * 256 + threadIdx.x, row = i / hd4, c = i % hd4;
     if (row >= rows) return;
     const float2* ml = reinterpret_cast<const float2*>(part);
-    const float4* po = reinterpret_cast<const float4*>(part + (size_t)n_splits * rows * 2);
+    const float4* po = reinterpret_cast<const float4*>(part + pf_part_head(n_splits, rows));
     float m = -INFINITY;
     for (uint32_t s = 0; s < n_splits; s++) {
         const float2 v = ml[(size_t)s * rows + row];
@@ -449,7 +452,8 @@ static OxbPrefillAttnPlan plan_attn(const OxbPrefillAttnParams& p, uint32_t n_cu
 
 size_t oxb_attn_prefill_part_bytes(const OxbPrefillAttnParams& p, uint32_t n_cus) {
     const OxbPrefillAttnPlan pl = plan_attn(p, n_cus);
-    return pl.n_splits > 1 ? (size_t)pl.n_splits * p.M * p.nq * (p.hd + 2) * sizeof(float) : 0;
+    const size_t rows = (size_t)p.M * p.nq;
+    return pl.n_splits > 1 ? (pf_part_head(pl.n_splits, rows) + pl.n_splits * rows * p.hd) * sizeof(float) : 0;
 }
 
 hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipStream_t st) {
