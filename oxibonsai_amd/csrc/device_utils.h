@@ -68,6 +68,8 @@ __device__ __forceinline__ float wave_max_f32(float v) {
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 #define OXB_OOB 0xFFFFFFF0u
+// The same where a constant is added to the offset: OXB_OOB plus 16 is 0, the first element.  (Buffers end below it.)
+#define OXB_OOB_BASE 0x7FFF0000u
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(512) void gemv_kernel(const OxbGemvParams p) {
 #pragma unroll
             for (int pass = 0; pass < 2; pass++) {
                 const uint32_t blk = (sb0 + i) * 4 + pass * 2 + blh;
-                const uint32_t off = i < sb_lim ? blk * 512u + koff : OXB_OOB;  // beyond k the buffer returns 0
+                const uint32_t off = i < sb_lim ? blk * 512u + koff : OXB_OOB_BASE;  // beyond k the buffer returns 0
 #pragma unroll
                 for (int bb = 0; bb < 4; bb++) {
                     xe[i][pass][bb] = __uint_as_float(buf_load_b32(r_x, off + KS * 4u * bb));
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(512) void gemv_f4_kernel(const OxbGemvParams p) {
     float xe[NSBW][8], we[NSBW][8];
 #pragma unroll
     for (int i = 0; i < NSBW; i++) {
-        const uint32_t off = i < sb_lim ? (sb0 + i) * 2048u + koff : OXB_OOB;  // beyond k the buffer returns 0
+        const uint32_t off = i < sb_lim ? (sb0 + i) * 2048u + koff : OXB_OOB_BASE;  // beyond k the buffer returns 0
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             xe[i][e] = __uint_as_float(buf_load_b32(r_x, off + XS * e));
@@ -1136,7 +1136,7 @@ static hipError_t launch_gemv_packed2_t(const OxbGemvParams& p, const GemvPlan& 
 static bool check_gemv_args(const OxbGemvParams& p) {
     if (p.nvec == 0 || p.nvec > (p.xq ? OXB_GEMV_PACKED_MAX_BATCH : OXB_GEMV_MAX_BATCH)) return false;
     if (p.xq && (p.nvg != (p.nvec + 3) / 4 || p.xq_bytes < oxb_gemv_pack_dwords(p.n_sb, p.nvg) * 4)) return false;
-    if (p.codes_bytes >= 0x7FFFFFFFull || (uint64_t)p.k * 4 >= 0x7FFFFFFFull) return false;
+    if (p.codes_bytes >= 0x7FFFFFFFull || (uint64_t)p.k * 4 >= OXB_OOB_BASE) return false;
     if (p.pro != OXB_GEMV_PRO_F32 && p.pro != OXB_GEMV_PRO_RMSNORM) return false;
     if (p.pro == OXB_GEMV_PRO_RMSNORM && !p.norm_w) return false;
     if (p.epi == OXB_GEMV_RESIDUAL && !p.residual) return false;

@@ -252,3 +252,36 @@ def test_batch_attn_phase(backend, fmt, h):
         assert np.max(np.abs(got - want)) < 2e-5 * float(np.max(np.abs(want)))
     finally:
         backend.free_weights(hd)
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("h", [4352, 4480, 4608, 8320, 8704, 10240, 16896])
+def test_rms_of_rows_that_do_not_fill_the_waves(backend, fmt, h):
+    """Rows of 9, 17 or 20 superblocks of 512 leave one or two of the two or three that each wave takes without values
+    (16896: in the second, accumulating launch); nothing of the row may be counted for them.  One vector through the QKV
+    product, then three sequences of a model whose products quantise their vectors in every workgroup."""
+    from oxibonsai_amd.model import batch_attn_phase
+    qr, kr = 128, 64
+    a = synth.make_blocks(fmt, 0xA87 + fmt, qr + 2 * kr, h)
+    x = synth.normal_f32(0xA88, h)
+    nw = (1.0 + synth.normal_f32(0xA89, h, 0.02)).astype(np.float32)
+    hd = _upload(backend, fmt, a)
+    try:
+        got = np.concatenate(batch_attn_phase(backend, fmt, x, nw, 1e-6, hd, qr, kr, h))
+        want = oracle.gemv(fmt, a, oracle.rms_norm(x, nw, 1e-6), qr + 2 * kr, h)
+        assert np.max(np.abs(got - want)) < 2e-5 * float(np.max(np.abs(want)))
+    finally:
+        backend.free_weights(hd)
+    cfg = dict(fmt=fmt, n_layers=1, h=h, inter=256, nq=2, nkv=2, hd=64, vocab=64, max_seq=16, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 0xA8A)
+    gpu = HipModel(backend, cfg, w, batch=3)
+    rows = synth.embedding_rows(0xA8B, range(3), h) * 50.0
+    assert _lib.lib().oxb_hip_set_gemv_packed_min_batch(0) == 0
+    try:
+        got, _ = gpu.forward(rows, 0)
+        for b in range(3):
+            want = oracle.OracleModel(cfg, w, kv_f16=True).forward(rows[b], 0)
+            assert np.max(np.abs(got[b] - want)) < 1e-3 * float(np.max(np.abs(want))), b
+    finally:
+        assert _lib.lib().oxb_hip_set_gemv_packed_min_batch(1) == 0
+        gpu.close()
