@@ -1003,7 +1003,9 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
     }
     // Four rows per workgroup, two where four would leave half the CUs idle; eight for long rows where each CU has a
     // workgroup all the same (2048 rows of 12288: 25 us against 28 with four and 36 with two; of 4096: 11, 10 and 12).
-    const uint32_t rpw = OP == OXB_PACK_IDENT && k > 8192 && M_pad >= 2048 ? 8 : M_pad >= 512 ? 4 : 2, per_lane = (nblk_pad * 4 * rpw + 63) / 64;  // pieces of four values per lane
+    // Long rows with sums to add: two, or the registers of the planes spill (600 rows of 10240 33 us against 60, 1700 of 8320
+    // 60 against 100).
+    const uint32_t rpw = OP == OXB_PACK_IDENT && k > 8192 && M_pad >= 2048 ? 8 : M_pad >= 512 && !(SUM && k > 8192) ? 4 : 2, per_lane = (nblk_pad * 4 * rpw + 63) / 64;  // pieces of four values per lane
 #define OXB_WIDE_CASE(RPW, NI)                                                                                                     \
     if (rpw == RPW && per_lane <= NI) {                                                                                            \
         if (fmt == OXB_FMT_Q1)                                                                                                     \
@@ -1014,7 +1016,9 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
                                k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                            \
         return;                                                                                                                    \
     }
-    OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16) OXB_WIDE_CASE(4, 24) OXB_WIDE_CASE(2, 4) OXB_WIDE_CASE(2, 8) OXB_WIDE_CASE(2, 12)
+    OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16)
+    if constexpr (!SUM) { OXB_WIDE_CASE(4, 24) }
+    OXB_WIDE_CASE(2, 4) OXB_WIDE_CASE(2, 8) OXB_WIDE_CASE(2, 12)
     if constexpr (OP == OXB_PACK_IDENT) { OXB_WIDE_CASE(8, 48) }
     // (rows of more than 12288 values take two launches)
 #undef OXB_WIDE_CASE
