@@ -33,6 +33,11 @@ int  oxb_hip_set_gemv_packed_min_batch(uint32_t n);
 /* Packs x once, then times `iters` prefill GEMM launches with events on the library's stream. */
 int  oxb_hip_profile_gemm(uint64_t id, const float* d_x, float* d_y, uint32_t m, uint32_t n_rows, uint32_t k,
                           uint32_t warmup, uint32_t iters, float* avg_us);
+/* Which kernel a GEMM of m rows runs on (no GPU needed): swiglu != 0 for the gate || up product, sum_later != 0 for a residual
+ * product whose K slices the next pack may add, n_cus compute units.  plan[0..5] = narrow kernel (1) or wide (0), row
+ * tiles per workgroup (narrow) or wave (wide), row tiles per workgroup (wide), token tiles of 16, K slices, superblocks per
+ * slice. */
+int  oxb_hip_gemm_plan(int fmt, uint32_t m, uint32_t n_rows, uint32_t k, int swiglu, int sum_later, uint32_t n_cus, uint32_t plan[6]);
 /* The attention of one layer's prefill on its own: qkv [n_tokens][(nq + 2 nkv) hd] (host), as the layer's QKV product
  * leaves it, is normed and rotated, its K and V rows go to the cache of sequence `seq` at pos_start .., and out
  * [n_tokens][nq hd] (host) receives what the queries attend to.  Inside oxb_hip_prefill these values are rounded to fp16

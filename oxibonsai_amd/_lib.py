@@ -43,6 +43,7 @@ _SIGNATURES = {
     "oxb_hip_gemm_dev_static": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_profile_gemm": ([C.c_uint64, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32,
                               C.c_uint32, C.c_uint32, f32p], C.c_int),
+    "oxb_hip_gemm_plan": ([C.c_int, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int, C.c_int, C.c_uint32, u32p], C.c_int),
     "oxb_hip_gemv_q1_g128": ([u8p, C.c_size_t, f32p, C.c_size_t, f32p, C.c_size_t, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_gemv_tq2_g128": ([u8p, C.c_size_t, f32p, C.c_size_t, f32p, C.c_size_t, C.c_uint32, C.c_uint32], C.c_int),
     "oxb_hip_ffn_phase": ([C.c_int, f32p, f32p, f32p, C.c_float, C.c_uint64, C.c_uint64, C.c_uint64, C.c_uint32,

@@ -45,6 +45,10 @@ struct OxbPackSum { const float* part; uint32_t n; size_t plane; };
 bool oxb_pack_can_sum(uint32_t k, uint32_t M);
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
                               uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr);
+// What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16, or the wide one
+// with rt row tiles per wave, tpw per workgroup, 16 ct tokens per tile; K in ksplit slices of sb_per_split superblocks.
+struct OxbGemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };
+OxbGemmPlan oxb_gemm_plan(int fmt, const OxbGemmParams& p, uint32_t n_cus);
 // Number of K slices the launcher will use for this shape (1: no workspace needed).
 uint32_t oxb_gemm_ksplit(int fmt, const OxbGemmParams& p, uint32_t n_cus);
 hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st);

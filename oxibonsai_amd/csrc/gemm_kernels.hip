@@ -817,7 +817,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
         // One lane offset; step and block go into the wave-uniform part, the token tile into the instruction's constant.
         const uint32_t b_off = (4u * g * p.M_pad + r) * 16u;
         auto load_b = [&](uint32_t blk, int s, v8h (&dst)[CT]) {
-            const uint32_t at = blk < blk_end ? b_off : 0x7FFFF000u;  // (past the slice: out of range, a constant may still be added)
+            const uint32_t at = blk < blk_end ? b_off : OXB_OOB_BASE;  // (past the slice)
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) dst[ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, at + ct * 256u, blk * blk_stride + s * p.M_pad * 16u));
         };
@@ -1063,17 +1063,13 @@ static hipError_t launch_gemm_case(const OxbGemmParams& p, uint32_t grid, hipStr
     return hipGetLastError();
 }
 
-// What the launcher runs: the narrow kernel with rt row tiles per workgroup, or the wide one with rt row tiles per wave, tpw
-// per workgroup, 16 ct tokens per tile and K in ksplit slices of sb_per_split superblocks.
-struct GemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };
-
 // Time of a wide plan in us, from 19 000 measured (shape, tokens, plan) triples - both formats, 1280 .. 24576 rows, K 1280 ..
 // 12288, 33 .. 2048 tokens - whose best plan it names within 2 % on average (the rule before it, 128-token tiles by rounds
 // of workgroups: 12 %).  Per 128-weight block a workgroup alone on its CU needs `lone`, a latency; workgroups that share
 // one need `busy` each, a rate.  More tokens per tile amortise the expansion of the weights, more row tiles the reading of
 // the token tile out of LDS; small tiles make more workgroups and less padding.
-static float wide_cost(bool tq2, const OxbGemmParams& p, const GemmPlan& g, uint32_t n_cus) {
-    // [format][ct = 4, 5, 8][rt - 1]; rt = 5 goes with ct = 8 only
+static float wide_cost(bool tq2, const OxbGemmParams& p, const OxbGemmPlan& g, uint32_t n_cus) {
+    // [format][ct = 4, 5, 8][rt - 1]; rt = 5 goes with ct = 8 only, rt = 1 not with it (smaller token tiles always beat it)
     static const float lone_us[2][3][5] = {{{0.34f, 0.50f, 0.68f, 0.82f}, {0.40f, 0.59f, 0.81f, 0.96f}, {0.66f, 0.86f, 1.18f, 1.42f, 1.69f}},
                                            {{0.39f, 0.59f, 0.85f, 1.05f}, {0.45f, 0.70f, 0.96f, 1.19f}, {0.69f, 0.99f, 1.30f, 1.60f, 1.83f}}};
     static const float busy_us[2][3][5] = {{{0.25f, 0.41f, 0.58f, 0.77f}, {0.31f, 0.51f, 0.70f, 0.92f}, {0.54f, 0.83f, 1.09f, 1.42f, 1.69f}},
@@ -1109,14 +1105,14 @@ static float narrow_cost(bool tq2, const OxbGemmParams& p, uint32_t rt, uint32_t
 
 // The narrow kernel up to OXB_GEMM_NARROW_MAX_M token rows (the wide one would spend its time on barriers and padding),
 // the cheaper of the two up to 128, the wide one beyond.
-static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
+OxbGemmPlan oxb_gemm_plan(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
     const bool tq2 = fmt == OXB_FMT_TQ2, sw = p.mode == OXB_GEMM_SWIGLU;
-    GemmPlan best = {true, 0, 0, 0, 1, p.n_sb};
+    OxbGemmPlan best = {true, 0, 0, 0, 1, p.n_sb};
     float best_us = 1e30f;
     if (p.M <= 128) {
         // row tiles per workgroup: as many as the registers hold next to the token tiles (six: Q1 only), two or more with SWIGLU
         static const uint32_t choices[4] = {1, 2, 4, 6};
-        const uint32_t ct = (p.M + 15) / 16, most = ct <= 2 && !tq2 ? 6 : ct <= 4 ? 4 : ct <= 7 ? 2 : 1;
+        const uint32_t ct = best.ct = (p.M + 15) / 16, most = ct <= 2 && !tq2 ? 6 : ct <= 4 ? 4 : ct <= 7 ? 2 : 1;
         for (uint32_t rt : choices) {
             if (rt > most || (sw && rt == 1)) continue;
             // K in slices where the next pack adds them anyway: with few row tiles they fill the chip, and a workgroup takes in
@@ -1137,9 +1133,9 @@ static GemmPlan plan_gemm(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
         const uint32_t spk = (p.n_sb + ks - 1) / ks;
         if ((p.n_sb + spk - 1) / spk != ks) continue;  // same slices as a smaller count
         for (uint32_t ct : cts)
-            for (uint32_t rt = 1; rt <= (ct == 8 ? 5u : 4u); rt++) {
+            for (uint32_t rt = ct == 8 ? 2 : 1; rt <= (ct == 8 ? 5u : 4u); rt++) {
                 if (sw && rt != 2 && rt != 3) continue;  // a gate and an up tile per wave, or three tiles of either kind
-                const GemmPlan g = {false, rt, 4 * rt, ct, ks, spk};
+                const OxbGemmPlan g = {false, rt, 4 * rt, ct, ks, spk};
                 const float us = wide_cost(tq2, p, g, n_cus);
                 if (us < best_us) best_us = us, best = g;
             }
@@ -1175,7 +1171,7 @@ static hipError_t launch_gemm_narrow(int fmt, OxbGemmParams p, uint32_t rt, hipS
 
 uint32_t oxb_gemm_ksplit(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
     if (p.M == 0 || p.n_rows == 0 || p.n_sb == 0) return 1;
-    return plan_gemm(fmt, p, n_cus).ksplit;
+    return oxb_gemm_plan(fmt, p, n_cus).ksplit;
 }
 
 hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t st) {
@@ -1183,7 +1179,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     if (p.n_sb == 0 || (uint64_t)p.n_tiles * p.n_sb * 2048ull >= 0xFFFFFFF0ull) return hipErrorInvalidValue;
     if (p.mode == OXB_GEMM_SWIGLU && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // whole gate and up row tiles
     p.M_pad = (p.M + 15u) / 16u * 16u;
-    const GemmPlan plan = plan_gemm(fmt, p, n_cus);
+    const OxbGemmPlan plan = oxb_gemm_plan(fmt, p, n_cus);
     p.ksplit = plan.ksplit;
     p.sb_per_split = plan.sb_per_split;
     if (p.ksplit > 1 && !p.part) return hipErrorInvalidValue;
@@ -1196,7 +1192,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
 #define OXB_GEMM_CASE(R, C)                                                                        \
     if (plan.rt == R && plan.ct == C)                                                              \
         err = fmt == OXB_FMT_Q1 ? launch_gemm_case<OXB_FMT_Q1, R, C>(p, grid, st) : launch_gemm_case<OXB_FMT_TQ2, R, C>(p, grid, st);
-    OXB_GEMM_CASE(1, 8) OXB_GEMM_CASE(2, 8) OXB_GEMM_CASE(3, 8) OXB_GEMM_CASE(4, 8) OXB_GEMM_CASE(5, 8)
+    OXB_GEMM_CASE(2, 8) OXB_GEMM_CASE(3, 8) OXB_GEMM_CASE(4, 8) OXB_GEMM_CASE(5, 8)
     OXB_GEMM_CASE(1, 5) OXB_GEMM_CASE(2, 5) OXB_GEMM_CASE(3, 5) OXB_GEMM_CASE(4, 5)
     OXB_GEMM_CASE(1, 4) OXB_GEMM_CASE(2, 4) OXB_GEMM_CASE(3, 4) OXB_GEMM_CASE(4, 4)
 #undef OXB_GEMM_CASE

@@ -760,6 +760,23 @@ int oxb_hip_profile_gemm(uint64_t id, const float* d_x, float* d_y, uint32_t m, 
     OXB_API_END
 }
 
+int oxb_hip_gemm_plan(int fmt, uint32_t m, uint32_t n_rows, uint32_t k, int swiglu, int sum_later, uint32_t n_cus, uint32_t plan[6]) {
+    OXB_API_BEGIN
+    if ((fmt != OXB_FMT_Q1 && fmt != OXB_FMT_TQ2) || !m || !n_rows || !k || k % OXB_QK != 0 || !n_cus || !plan || (swiglu && (n_rows & 31u)))
+        return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: no such GEMM");
+    const OxbLayout L = oxb_make_layout((uint32_t)fmt, n_rows, k);
+    OxbGemmParams p;
+    memset(&p, 0, sizeof p);
+    p.n_rows = n_rows, p.n_tiles = L.n_tiles, p.n_sb = L.n_sb, p.M = m, p.ldy = n_rows;
+    p.mode = swiglu ? OXB_GEMM_SWIGLU : sum_later ? OXB_GEMM_RESIDUAL : OXB_GEMM_STORE;
+    p.sum_later = sum_later && !swiglu;
+    const OxbGemmPlan g = oxb_gemm_plan(fmt, p, n_cus);
+    const uint32_t out[6] = {g.narrow ? 1u : 0u, g.rt, g.tpw, g.ct, g.ksplit, g.sb_per_split};
+    memcpy(plan, out, sizeof out);
+    return OXB_HIP_OK;
+    OXB_API_END
+}
+
 int oxb_hip_gemv(uint64_t id, const float* x, float* y, uint32_t n_rows, uint32_t k, uint32_t batch) {
     OXB_API_BEGIN
     std::lock_guard<std::recursive_mutex> lk(g_mu);

@@ -111,6 +111,59 @@ def parity_violations(a: np.ndarray, b: np.ndarray, tol: float = 1e-3) -> int:
 from oxibonsai_amd.gguf import GGUF_F16, GGUF_F32, GGUF_MAGIC, GGUF_Q1, GGUF_TQ2, gguf_bytes, model_gguf  # noqa: E402,F401
 
 
+# Products (format, token rows, rows, k) that between them run every form of the two GEMM kernels that the launcher picks on
+# 256 compute units: (narrow, row tiles, token tiles, K in slices).  Token rows and rows off the tiles' multiples, K of an
+# odd number of half superblocks.  tests/test_host.py holds the list to the launcher's own plans.
+GEMM_FORMS = {
+    (Q1, 1, 1, 1, False): (1, 20, 896), (TQ2, 1, 1, 1, False): (5, 31, 640),
+    (Q1, 1, 1, 2, False): (19, 17, 640), (TQ2, 1, 1, 2, False): (31, 19, 640),
+    (Q1, 1, 1, 3, False): (36, 20, 640), (TQ2, 1, 1, 3, False): (33, 20, 640),
+    (Q1, 1, 1, 4, False): (57, 17, 640), (TQ2, 1, 1, 4, False): (53, 19, 640),
+    (Q1, 1, 1, 5, False): (65, 17, 640), (TQ2, 1, 1, 5, False): (79, 17, 640),
+    (Q1, 1, 1, 6, False): (89, 17, 640), (TQ2, 1, 1, 6, False): (84, 18, 640),
+    (Q1, 1, 1, 7, False): (104, 17, 640), (TQ2, 1, 1, 7, False): (103, 18, 640),
+    (Q1, 1, 1, 8, False): (126, 17, 640), (TQ2, 1, 1, 8, False): (118, 17, 640),
+    (Q1, 1, 2, 1, False): (1, 4202, 1152), (TQ2, 1, 2, 1, False): (1, 4120, 1152),
+    (Q1, 1, 2, 2, False): (17, 4163, 640), (TQ2, 1, 2, 2, False): (17, 4131, 640),
+    (Q1, 1, 2, 3, False): (33, 4165, 640), (TQ2, 1, 2, 3, False): (33, 4137, 640),
+    (Q1, 1, 2, 4, False): (50, 4133, 640), (TQ2, 1, 2, 4, False): (49, 4150, 640),
+    (Q1, 1, 2, 5, False): (66, 4119, 640), (TQ2, 1, 2, 5, False): (65, 4115, 640),
+    (Q1, 1, 2, 6, False): (81, 4183, 640), (TQ2, 1, 2, 6, False): (82, 4169, 640),
+    (Q1, 1, 2, 7, False): (98, 4188, 640), (TQ2, 1, 2, 7, False): (97, 4109, 640),
+    (Q1, 1, 4, 1, False): (1, 12368, 12032),
+    (Q1, 1, 4, 2, False): (17, 8220, 640), (TQ2, 1, 4, 2, False): (17, 12454, 640),
+    (Q1, 1, 4, 3, False): (34, 8242, 640), (TQ2, 1, 4, 3, False): (33, 8342, 640),
+    (Q1, 1, 4, 4, False): (50, 8194, 640), (TQ2, 1, 4, 4, False): (49, 8205, 640),
+    (Q1, 1, 6, 1, False): (1, 20605, 640), (Q1, 1, 6, 2, False): (17, 16440, 640),
+    (Q1, 0, 1, 4, False): (142, 19, 640), (TQ2, 0, 1, 4, False): (143, 27, 640),
+    (Q1, 0, 1, 4, True): (209, 20, 1152), (TQ2, 0, 1, 4, True): (136, 20, 1408),
+    (Q1, 0, 1, 5, False): (129, 5557, 640), (TQ2, 0, 1, 5, False): (130, 5602, 640),
+    (Q1, 0, 1, 5, True): (152, 1368, 1664), (TQ2, 0, 1, 5, True): (139, 1364, 1664),
+    (Q1, 0, 2, 4, False): (81, 24659, 640), (TQ2, 0, 2, 4, False): (81, 24716, 640),
+    (Q1, 0, 2, 5, False): (65, 16607, 640), (TQ2, 0, 2, 5, False): (409, 10828, 640),
+    (TQ2, 0, 2, 8, False): (670, 10827, 640),
+    (Q1, 0, 3, 4, False): (82, 16388, 640), (TQ2, 0, 3, 4, False): (260, 16406, 640),
+    (Q1, 0, 3, 4, True): (204, 2708, 5120),
+    (Q1, 0, 3, 5, False): (129, 16613, 640), (TQ2, 0, 3, 5, False): (129, 16504, 640),
+    (Q1, 0, 3, 5, True): (65, 16808, 5120), (TQ2, 0, 3, 5, True): (65, 16600, 5120),
+    (Q1, 0, 3, 8, False): (482, 21307, 640), (TQ2, 0, 3, 8, False): (161, 22026, 640),
+    (Q1, 0, 4, 4, False): (257, 24918, 640), (TQ2, 0, 4, 4, False): (259, 24620, 640),
+    (Q1, 0, 4, 5, False): (195, 16463, 640), (TQ2, 0, 4, 5, False): (131, 24665, 640),
+    (Q1, 0, 4, 8, False): (241, 24663, 640), (TQ2, 0, 4, 8, False): (193, 24728, 640),
+    (Q1, 0, 5, 8, False): (322, 24695, 640), (TQ2, 0, 5, 8, False): (327, 21773, 640),
+}
+
+
+def gemm_plan(fmt: int, m: int, n: int, k: int, swiglu: bool = False, sum_later: bool = False, n_cus: int = 256):
+    """(narrow, row tiles, row tiles per workgroup, token tiles, K slices, superblocks per slice) of a GEMM's launch."""
+    import ctypes as C
+
+    from oxibonsai_amd import _lib
+    plan = (C.c_uint32 * 6)()
+    assert _lib.lib().oxb_hip_gemm_plan(fmt, m, n, k, swiglu, sum_later, n_cus, plan) == 0
+    return tuple(plan)
+
+
 class DeviceBuffer:
     """A device allocation made through the HIP runtime the library itself links (libamdhip64.so.7), for the
     entry points that take device pointers; no second runtime (torch ships its own) enters the process."""

@@ -7,7 +7,7 @@ Inputs that are exact in fp16 must give bit-exact results, which pins the k orde
 import numpy as np
 import pytest
 
-from helpers import Q1, TQ2, dense_f64, parity_violations, q1_block, tq2_block
+from helpers import GEMM_FORMS, Q1, TQ2, dense_f64, parity_violations, q1_block, tq2_block
 from oracle import oracle
 from oxibonsai_amd import GpuError, synth
 
@@ -56,6 +56,16 @@ def test_gemm_matches_oracle(backend, fmt, shape):
     want = oracle.gemm(fmt, a, x, m, n, k)
     assert got.shape == (m, n)
     assert parity_violations(got, want, GEMM_REL_TOL) == 0
+    _check_against_truth(got, dense_f64(fmt, a, n, k), x)
+
+
+@pytest.mark.parametrize("form", GEMM_FORMS, ids=lambda f: "-".join(str(int(v)) for v in f))
+def test_gemm_every_form_of_both_kernels(backend, form):
+    # outputs within the bound that rounding the activations to fp16 implies, for every form that the launcher picks
+    fmt, (m, n, k) = form[0], GEMM_FORMS[form]
+    a = synth.make_blocks(fmt, 9100 + m + n, n, k)
+    x = synth.normal_f32(9101 + n, m * k).reshape(m, k)
+    got = _gemm(backend, fmt, a, x, m, n, k)
     _check_against_truth(got, dense_f64(fmt, a, n, k), x)
 
 

@@ -10,7 +10,7 @@ cache the prefill wrote, which checks the stored keys and values."""
 import numpy as np
 import pytest
 
-from helpers import Q1, TQ2, parity_violations
+from helpers import Q1, TQ2, gemm_plan, parity_violations
 from oracle import oracle
 from oxibonsai_amd import GpuError, synth
 from oxibonsai_amd.model import HipModel
@@ -26,8 +26,8 @@ WIDE = dict(n_layers=1, h=256, inter=512, nq=2, nkv=2, hd=256, vocab=64, max_seq
 G4_HD32 = dict(n_layers=2, h=128, inter=256, nq=4, nkv=1, hd=32, vocab=64, max_seq=200, eps=1e-6, rope_theta=1e4)
 G4_HD256 = dict(n_layers=1, h=1024, inter=512, nq=4, nkv=1, hd=256, vocab=64, max_seq=96, eps=1e-6, rope_theta=1e6)
 G8_HD128 = dict(n_layers=1, h=1024, inter=512, nq=8, nkv=1, hd=128, vocab=64, max_seq=160, eps=1e-6, rope_theta=1e6)
-# an FFN wide enough (392 gate tiles x 4 token tiles of 128) for the gate || up GEMM to take three row tiles per wave, gate
-# and up tiles in different waves; 392 = 65 x 6 + 2 and 500 = 3 x 128 + 116: the last workgroups are partly empty
+# an FFN wide enough (392 gate tiles x 7 token tiles of 80) for the gate || up GEMM to take three row tiles per wave, gate
+# and up tiles in different waves; 392 = 65 x 6 + 2 and 500 = 6 x 80 + 20: the last workgroups are partly empty
 LONG_FFN = dict(n_layers=1, h=256, inter=6272, nq=4, nkv=2, hd=64, vocab=64, max_seq=520, eps=1e-6, rope_theta=1e6)
 
 
@@ -70,6 +70,50 @@ def test_prefill_matches_sequential_oracle(backend, fmt, cfg, n):
             want = cpu.forward(r, n + step)
             g, t = gpu.forward(r, n + step)
             _check(g[0], want, int(t[0]))
+    finally:
+        gpu.close()
+
+
+# (format, hidden, inter, q heads, kv heads, head_dim, tokens; the gate || up product's form: narrow kernel, row tiles, token
+# tiles; K slices of the down product, whose sums the next layer's pack adds): the forms of the SwiGLU product ...
+SWIGLU_FORMS = [(fmt, 640, 384, 4, 2, 64, m, (1, 2, -(-m // 16)), None) for fmt in (Q1, TQ2) for m in (9, 19, 34, 49, 67, 82, 97)]
+SWIGLU_FORMS += [(fmt, 256, 4224, 4, 2, 64, m, (1, 4, -(-m // 16)), None) for fmt in (Q1, TQ2) for m in (19, 34, 49)]
+SWIGLU_FORMS += [(fmt, 256, inter, 4, 2, 64, m, form, None) for fmt in (Q1, TQ2) for m, inter, form in
+                 ((115, 384, (0, 2, 4)), (67, 8320, (0, 2, 5)), (82, 8320, (0, 3, 4)), (129, 8320, (0, 3, 5)))]
+SWIGLU_FORMS += [(Q1, 640, 8320, 4, 2, 64, 1, (1, 6, 1), None), (Q1, 256, 8320, 4, 2, 64, 19, (1, 6, 2), None), (Q1, 256, 10496, 4, 2, 64, 500, (0, 3, 8), None),
+                 (TQ2, 256, 12416, 4, 2, 64, 250, (0, 2, 8), None), (TQ2, 256, 11008, 4, 2, 64, 161, (0, 3, 8), None)]
+# ... and the packs that add a residual product's K slices: up to 64 rows one to four items per thread, beyond two or four
+# rows per workgroup with rows of up to 4096, 8192 and 12288 values
+SUM_PACKS = [(Q1, 1024, 4096, 16, 4, 128, 40, None, 4), (TQ2, 4096, 4096, 4, 2, 64, 64, None, 2), (Q1, 4352, 4608, 4, 2, 64, 40, None, 3),
+             (Q1, 1024, 4096, 16, 4, 128, 100, None, 4), (TQ2, 4096, 4096, 4, 2, 64, 130, None, 4), (TQ2, 4352, 4608, 4, 2, 64, 66, None, 3),
+             (Q1, 8320, 3072, 4, 2, 64, 66, None, 3), (TQ2, 1024, 4096, 16, 4, 128, 520, None, 4), (TQ2, 4352, 4608, 4, 2, 64, 600, None, 3),
+             (TQ2, 10240, 9216, 4, 2, 64, 600, None, 3)]
+
+
+@pytest.mark.parametrize("fmt,h,inter,nq,nkv,hd,n,form,slices", SWIGLU_FORMS + SUM_PACKS)
+def test_prefill_rows_match_the_oracle(backend, fmt, h, inter, nq, nkv, hd, n, form, slices):
+    """Every token's K and V rows of the second layer - behind all products of the first one - and the last token's logits.
+    About six roundings of activations to fp16 (2^-11 / sqrt 3 in the root mean square each) lie in front of a row, and one
+    of the row itself: 7e-4; three times that is allowed for any single row."""
+    narrow, rt, _, ct, _, _ = gemm_plan(fmt, n, 2 * inter, h, swiglu=True)
+    assert form in (None, (narrow, rt, ct))
+    assert slices in (None, gemm_plan(fmt, n, h, inter, sum_later=True)[4])
+    cfg = dict(fmt=fmt, n_layers=2, h=h, inter=inter, nq=nq, nkv=nkv, hd=hd, vocab=64, max_seq=n + 4, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 300 + n)
+    rows = _rows(21, n, h)
+    cpu = oracle.OracleModel(cfg, w, kv_f16=True, simd=True)
+    want = cpu.forward_batch(rows, 0)
+    gpu = HipModel(backend, cfg, w)
+    try:
+        got, tok = gpu.prefill(rows)
+        worst = 0.0
+        for head in range(nkv):
+            for a, b in zip(gpu.read_kv(1, head, 0, n)[:2], cpu.cache_rows(1, head, 0, n)):
+                d = a.astype(np.float64) - b
+                worst = max(worst, float(np.sqrt(np.mean(d * d, axis=1) / np.mean(b.astype(np.float64) ** 2, axis=1)).max()))
+        print(f"worst row {worst:.2e}, logits {np.max(np.abs(got - want)):.2e} off, largest {np.max(np.abs(want)):.2e}")
+        assert worst <= 2.1e-3, worst
+        _check(got, want, tok)
     finally:
         gpu.close()
 

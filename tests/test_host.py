@@ -9,7 +9,7 @@ import pytest
 
 import kernel_model
 import oxibonsai_amd as ox
-from helpers import Q1, TQ2, block, cross_tier_q1, dense_f64, metal_tq2, simd_parity_tq2
+from helpers import GEMM_FORMS, Q1, TQ2, block, cross_tier_q1, dense_f64, gemm_plan, metal_tq2, simd_parity_tq2
 from oracle import oracle
 from oxibonsai_amd import _lib, synth
 
@@ -26,6 +26,26 @@ def test_library_exports_every_declared_symbol():
     missing = [s for s in sorted(declared) if not hasattr(L, s)]
     assert not missing, missing
     assert declared == set(_lib._SIGNATURES), declared ^ set(_lib._SIGNATURES)
+
+
+def test_gemm_forms_cover_what_the_launcher_picks():
+    # the list that the GPU tests run, against the launcher's own plans: every entry is what it says, and a sweep over sizes
+    # meets no form that the list lacks
+    def form(fmt, m, n, k):
+        narrow, rt, _, ct, ksplit, _ = gemm_plan(fmt, m, n, k)
+        return (fmt, narrow, rt, ct, ksplit > 1)
+
+    for key, shape in GEMM_FORMS.items():
+        assert form(key[0], *shape) == key, (key, shape, gemm_plan(key[0], *shape))
+    g = np.random.default_rng(12)
+    seen = set()
+    for m, n, k in zip(*(np.exp(g.uniform(0, np.log(hi), 60000)).astype(int) + lo for lo, hi in ((1, 3000), (1, 152000), (1, 100)))):
+        for fmt in (Q1, TQ2):
+            seen.add(form(fmt, int(m), int(n), 128 * int(k))[:4])      # (K in slices is the same code)
+    assert seen <= {f[:4] for f in GEMM_FORMS}, seen - {f[:4] for f in GEMM_FORMS}
+    for bad in ((2, 4, 16, 128), (Q1, 0, 16, 128), (Q1, 4, 16, 100), (TQ2, 4, 0, 128)):
+        plan = (C.c_uint32 * 6)()
+        assert _lib.lib().oxb_hip_gemm_plan(*bad, 0, 0, 256, plan) == 5
 
 
 def test_static_library_is_built():
