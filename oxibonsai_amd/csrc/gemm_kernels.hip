@@ -780,8 +780,8 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 
 template <int FMT, int RT, int CT>
 __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(const OxbGemmParams p) {
-    // The partial sums meet in LDS in passes of PT row tiles (all of them up to four; pairs beyond, so that the
-    // array stays within 64 KB): in SWIGLU mode a pass holds gate tiles and the up tiles of the same rows.
+    // The partial sums meet in LDS in passes of PT row tiles: all of them where that takes 64 KB at most, else pairs (48 KB with
+    // three token tiles to 112 with seven): in SWIGLU mode a pass holds gate tiles and the up tiles of the same rows.
     constexpr int PT = RT * CT <= 8 || RT == 1 ? RT : 2, NPASS = RT / PT;
     static_assert(RT % PT == 0, "row tiles per pass");
     constexpr int D = CT <= 2 && RT <= 4 ? 8 : 4;  // steps of B operands in registers (16 D CT registers)
@@ -1001,8 +1001,8 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
         if constexpr (!SUM) { OXB_ROWS_CASE(6) OXB_ROWS_CASE(8) }
 #undef OXB_ROWS_CASE
     }
-    // Four rows per workgroup, two where four would leave half the CUs idle; eight for long rows where each CU has a
-    // workgroup all the same (2048 rows of 12288: 25 us against 28 with four and 36 with two; of 4096: 11, 10 and 12).
+    // Four rows per workgroup, two where four would leave half the CUs idle; eight for long rows where each of 256 CUs has
+    // a workgroup all the same (2048 rows of 12288: 25 us against 28 with four and 36 with two; of 4096: 11, 10 and 12).
     // Long rows with sums to add: two, or the registers of the planes spill (600 rows of 10240 33 us against 60, 1700 of 8320
     // 60 against 100).
     const uint32_t rpw = OP == OXB_PACK_IDENT && k > 8192 && M_pad >= 2048 ? 8 : M_pad >= 512 && !(SUM && k > 8192) ? 4 : 2, per_lane = (nblk_pad * 4 * rpw + 63) / 64;  // pieces of four values per lane

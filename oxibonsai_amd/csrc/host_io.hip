@@ -50,7 +50,9 @@ constexpr size_t kChunk = (size_t)1 << 20;      // host copy of one piece while 
 constexpr size_t kStaging = (size_t)32 << 20;   // per direction; larger buffers take turns in it
 constexpr size_t kPoolOut = (size_t)512 << 20;  // result memory handed out at a time
 constexpr size_t kPoolKept = (size_t)128 << 20; // ... and kept for reuse
-constexpr uint32_t kSyncEvery = 256;            // calls after which the stream is synchronised all the same (the runtime retires its commands there)
+// Calls after which the stream is synchronised all the same, for the runtime to retire its commands (host to host, 1024 x 2048
+// GEMV: 17.5 us at the median, 40 to 85 for one call in 256, 17.9 on average).
+constexpr uint32_t kSyncEvery = 256;
 
 struct Staging {
     uint8_t *in = nullptr, *out = nullptr;

@@ -59,13 +59,13 @@ hipError_t oxb_launch_qk_norm_rope_store(const OxbQkParams& p, uint32_t batch, h
 #define OXB_ATTN_MAX_SPLITS 64        // slots the KV sequence is split over; slot s walks chunks s, s + n_splits, ...
 #define OXB_ATTN_PART_PAD 4           // floats after the hd outputs of a slot: maximum, sum, 2 unused (16-byte rows)
 // QK-norm, RoPE, KV store of the new position, split-KV attention (at most 16 q heads per kv head) into p.part and
-// the merge of the slots into the fp32 attention output p.out_merged [batch][nq * hd], all in one launch.
+// the merge of the slots into the fp32 attention output p.out [batch][nq * hd], all in one launch.
 hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStream_t st);
 // out[v] = w * x[v] / sqrt(mean(x[v]^2) + eps) for nvec vectors of n values; d_w == nullptr copies.
 hipError_t oxb_launch_rmsnorm(const float* d_x, const float* d_w, uint32_t n, uint32_t nvec, float eps, float* d_out, hipStream_t st);
 // d_ws: batch * OXB_ARGMAX_MAX_PARTS * 8 bytes of scratch for the per-span maxima.
 #define OXB_ARGMAX_MAX_PARTS 256u
-// host_copy_or_null: pinned host memory that receives the token ids too (readable after the stream is synchronised)
+// host_copy_or_null: pinned host memory that receives the token ids too (readable once a later launch of the stream has been seen to end)
 hipError_t oxb_launch_argmax(const float* d_logits, uint32_t n, uint32_t batch, uint32_t* d_out, void* d_ws, hipStream_t st,
                              uint32_t* host_copy_or_null = nullptr);
 // hidden rows (n_floats, a multiple of 4) and positions from pinned host memory to their device buffers, one launch

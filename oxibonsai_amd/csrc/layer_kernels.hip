@@ -206,8 +206,9 @@ hipError_t oxb_launch_kv_quantize_rows(int kv_mode, const float* d_x, uint32_t n
 //   O^T[d][head]  += sum_key V[key][d] P[head][key]  A = V gathered from the wave's LDS copy of the block,
 //                                                    B = the lane's own probabilities as fp16 hi + lo
 // so scores and weighted sums keep fp32-level accuracy.  Every wave runs its own online softmax; the results
-// meet in LDS.  The workgroup whose slot holds the new position computes K (norm + RoPE) and V of that position,
-// stores them to the cache and, after a barrier, reads them back like any other row.
+// meet in LDS.  The workgroup whose slot holds the new position computes K (norm + RoPE) and V of that position, stores
+// them to the cache and leaves a copy in LDS, as stored, which takes the row's place in the chunk that holds it: nothing waits
+// for the stores.
 // ---------------------------------------------------------------------------
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 
@@ -219,7 +220,7 @@ typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 //    contiguous quarter of a K row (hd / 4 bytes), so the Q operand follows that order.
 //    Eight waves widen the codes of one CU's walk twice as fast as four, but cost 1 us more to start, to meet and to
 //    merge; fp16 rows, which need no widening, are limited by the requests in flight either way: four waves, except for
-//    long walks of quantised rows (model.hip: attn_slots).  8B shape, us per launch with 4 / 8 waves: one FP8 sequence at
+//    long walks of quantised rows (model.hip: attn_wide).  8B shape, us per launch with 4 / 8 waves: one FP8 sequence at
 //    32 000 28.2 / 22.4, at 8 000 13.5 / 14.0; 32 of INT8 at 2048 35.8 / 33.0, at 500 13.0 / 13.3; one of fp16 at 700
 //    8.7 / 10.8, at 20 000 21.0 / 22.5.
 //  * sliding window with attention sinks (is_in_window, crates/oxibonsai-model/src/layers/sliding_window.rs:173-189):
@@ -232,7 +233,8 @@ __device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32
 
 // Slots in use for a walk of n_walk chunks.  A second slot saves a chunk's time and costs a merge, and the two are about
 // equal (one fp16 sequence at 200, 128-position chunks: 7.6 us with one slot, 8.2 with two; six: 8.6 and 9.7): two
-// chunks stay with one workgroup.
+// chunks stay with one workgroup, also where eight waves make them 256 positions each (INT8 at 350: one sequence
+// 9.5 and 9.7, four 10.2 and 10.5; FP8, eight at 500: 10.6 and 11.3).
 __device__ __forceinline__ uint32_t attn_slots_used(uint32_t n_walk, uint32_t n_splits) {
     return n_walk <= 2 ? 1u : min(n_walk, n_splits);
 }

@@ -655,8 +655,10 @@ int oxb_hip_free_f32(uint64_t id) {
 
 // Slots of the split-KV attention: at most one workgroup (slot x kv head x sequence) per CU where that is possible: a CU
 // with two of them is the one that the launch waits for, and every slot pays the Q arithmetic and a merge.  8B shape, us
-// per launch with the slots chosen here / one more: nine fp16 sequences at 1700 18.5 / 22.7, eleven 21.6 / 27.2, seventeen
-// 30.6 / 36.0, twenty-eight 39.6 / 40.8, 24 of INT8 at 500 13.4 / 16.3.
+// per launch with the slots chosen here / one more: nine fp16 sequences at 1700 18.5 / 22.7, eleven 21.6 / 27.2.  Seventeen,
+// 24 and 31 sequences, where one slot leaves up to half the CUs idle and two put two workgroups on some: fp16 at 500
+// 11.3 / 15.0, 11.8 / 15.7, 14.0 / 17.7, at 16 000 212 / 279, 268 / 300, 344 / 350; INT8 (one slot of eight waves, two of
+// four) at 500 10.9 / 14.8, 11.4 / 15.0, 12.1 / 15.4, at 16 000 155 / 170, 177 / 186, 208 / 216.
 static uint32_t attn_slots(const Model& m) {
     const oxb_model_desc& d = m.d;
     uint32_t n = (d.max_seq + OXB_ATTN_CHUNK_POSITIONS - 1) / OXB_ATTN_CHUNK_POSITIONS;
@@ -671,7 +673,11 @@ static uint32_t attn_slots(const Model& m) {
 }
 
 // Eight waves per workgroup for one-byte rows where a slot may have to walk more than 512 positions, as long as a CU gets
-// one workgroup (two of them are slower than two with four waves: 40 INT8 sequences at 1300 38.8 against 34.8 us).
+// one workgroup (two of them are slower than two with four waves: 40 INT8 sequences at 1300 38.8 against 34.8 us).  What
+// counts is the walk, but the form is part of the captured step, so the rule goes by the longest walk that the model allows:
+// while a long context is still short the other form would do better.  INT8, 8B shape, us per launch with eight / four waves, one
+// sequence in 32 slots: at 500 10.1 / 8.9, at 2000 11.4 / 9.9, 8000 13.8 / 13.8, 16 000 16.8 / 17.4, 32 000 22.0 / 24.2; eight in
+// four slots: at 500 11.4 / 9.9, 2000 15.6 / 15.8, 8000 31.2 / 38.0; 32 in one: at 500 11.9 / 12.4, 2000 28.6 / 34.6.
 static bool attn_wide(const Model& m, uint32_t kv_mode) {
     const oxb_model_desc& d = m.d;
     return kv_mode != OXB_KV_F16 && d.hd <= 128 && (uint64_t)d.nkv * d.batch * m.n_splits <= g_rt.n_cus && d.max_seq / m.n_splits > 512u;
