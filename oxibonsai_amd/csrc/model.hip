@@ -103,6 +103,12 @@ static int dev_alloc(Model& m, void** p, size_t bytes) {
     return OXB_HIP_OK;
 }
 
+// Zeros, complete when this returns: the null stream that clears has no order with the library's own.
+static hipError_t clear_now(void* p, size_t bytes) {
+    const hipError_t e = hipMemset(p, 0, bytes);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+
 static void free_kv_cache(Model& m) {
     void* bufs[5] = {m.k_cache, m.v_cache, m.k_scale, m.v_scale, m.d_table};
     for (void* p : bufs)
@@ -264,7 +270,7 @@ static int size_gemm_workspaces(Model& m) {
         if (d.batch <= OXB_GEMV_PACKED_MAX_BATCH && !m.gpack_o.ptr) {
             const size_t n = oxb_gemv_pack_bytes(d.nq * d.hd, d.batch);
             if ((rc = m.gpack_o.ensure(n))) return rc;
-            OXB_TRY_HIP(hipMemset(m.gpack_o.ptr, 0, n), "pack buffer clear");  // (at creation, like the cache's scales: never inside a capture)
+            OXB_TRY_HIP(clear_now(m.gpack_o.ptr, n), "pack buffer clear");  // (at creation, like the cache's scales: never inside a capture)
         }
     }
     if (d.batch < OXB_DECODE_GEMM_MIN_BATCH) return OXB_HIP_OK;
@@ -703,8 +709,8 @@ static int alloc_kv_cache(Model& m, uint32_t kv_mode, uint32_t page_size, uint32
         const size_t sb = rows * sizeof(float);
         OXB_TRY(grab((void**)&m.k_scale, sb));
         OXB_TRY(grab((void**)&m.v_scale, sb));
-        OXB_TRY_HIP(hipMemset(m.k_scale, 0, sb), "scale clear");
-        OXB_TRY_HIP(hipMemset(m.v_scale, 0, sb), "scale clear");
+        OXB_TRY_HIP(clear_now(m.k_scale, sb), "scale clear");
+        OXB_TRY_HIP(clear_now(m.v_scale, sb), "scale clear");
     }
     if (n_pages) {
         uint32_t shift = 0;
@@ -717,7 +723,7 @@ static int alloc_kv_cache(Model& m, uint32_t kv_mode, uint32_t page_size, uint32
         m.free_pages.resize(n_pages);
         for (uint32_t i = 0; i < n_pages; i++) m.free_pages[i] = n_pages - 1 - i;   // page 0 is handed out first
         OXB_TRY(grab((void**)&m.d_table, m.h_table.size() * 4));
-        OXB_TRY_HIP(hipMemset(m.d_table, 0, m.h_table.size() * 4), "page table clear");
+        OXB_TRY_HIP(clear_now(m.d_table, m.h_table.size() * 4), "page table clear");
     }
     m.kv_mode = kv_mode;
     m.attn_wide = attn_wide(m, kv_mode);
@@ -774,7 +780,7 @@ int oxb_hip_model_create(const oxb_model_desc* desc, uint64_t* model) {
             return fail(OXB_HIP_OUT_OF_MEMORY, "out of host memory: pinned staging of %zu bytes", B * d.h * 4);
         }
         m.h_tokens = m.h_pos + B;
-        e = hipMemset(m.attn_done, 0, B * d.nkv * 4);
+        e = clear_now(m.attn_done, B * d.nkv * 4);
         if (e != hipSuccess) {
             free_model(m);
             return hip_fail(e, "counter clear");
