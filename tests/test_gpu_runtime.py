@@ -86,6 +86,70 @@ def test_results_are_arrays_of_their_own(backend):
         backend.free_weights(h)
 
 
+def test_pinned_buffers_of_the_caller(backend):
+    # inputs and outputs in memory of oxb_hip_host_alloc, which the device reads and writes itself where they lie on a
+    # 16-byte boundary: the same values as through ordinary arrays, in either place, and nothing beside them
+    import ctypes as C
+
+    from oxibonsai_amd import _lib
+    lib = _lib.lib()
+
+    def block(n_bytes):
+        p = C.c_void_p()
+        assert lib.oxb_hip_host_alloc(C.byref(p), n_bytes) == 0
+        return p.value, np.frombuffer((C.c_uint8 * n_bytes).from_address(p.value), dtype=np.uint8)
+
+    n, k, m = 1021, 640, 45
+    w = backend.upload_weights_raw(synth.make_blocks(Q1, 95, n, k), n, k)
+    x = synth.normal_f32(96, m * k)
+    want, want1 = backend.gemm_cached(w, x, m, n, k), backend.gemv_q1_g128_cached(w, x[:k], n, k)
+    p_in, a_in = block(x.nbytes + 64)
+    p_out, a_out = block(want.nbytes + 64)
+    try:
+        for off_in in (0, 4, 16):
+            for off_out in (0, 12, 32):
+                a_out[:] = 0xEE
+                a_in[off_in:off_in + x.nbytes] = x.view(np.uint8)
+                assert lib.oxb_hip_gemm(int(w), p_in + off_in, p_out + off_out, m, n, k) == 0
+                assert np.array_equal(a_out[off_out:off_out + want.nbytes], want.reshape(-1).view(np.uint8)), (off_in, off_out)
+                assert (a_out[:off_out] == 0xEE).all() and (a_out[off_out + want.nbytes:] == 0xEE).all()
+                assert lib.oxb_hip_gemv(int(w), p_in + off_in, p_out + off_out, n, k, 1) == 0
+                assert np.array_equal(a_out[off_out:off_out + want1.nbytes], want1.view(np.uint8)), (off_in, off_out)
+    finally:
+        backend.free_weights(w)
+    del a_in, a_out
+    assert lib.oxb_hip_host_free(p_in) == 0 and lib.oxb_hip_host_free(p_out) == 0
+    assert lib.oxb_hip_host_free(p_in) == 5 and lib.oxb_hip_host_free(None) == 5           # OXB_HIP_INVALID_ARGUMENT
+    # at most 512 MiB at a time
+    held = []
+    for _ in range(8):
+        p = C.c_void_p()
+        assert lib.oxb_hip_host_alloc(C.byref(p), 64 << 20) == 0
+        held.append(p.value)
+    p = C.c_void_p()
+    assert lib.oxb_hip_host_alloc(C.byref(p), 1) == 2 and not p.value                      # OXB_HIP_OUT_OF_MEMORY
+    for q in held:
+        assert lib.oxb_hip_host_free(q) == 0
+
+
+@pytest.mark.parametrize("fmt,n,k", [(Q1, 4100, 4096), (TQ2, 2051, 8192)])
+def test_results_beyond_the_staging_buffer(backend, fmt, n, k):
+    # 64 MiB and a little of dequantised values out, 37 MiB of activations in: both take turns in the 32 MiB of staging.  The
+    # single rows run on another form of the GEMM: the same products, summed in fp32 in another order.
+    a = synth.make_blocks(fmt, 97, n, k)
+    w = backend.upload_weights_raw(a, n, k) if fmt == Q1 else backend.upload_weights_ternary(a, n, k)
+    try:
+        assert np.array_equal(backend.dequant(w).reshape(-1).view(np.uint32), oracle.dequant(fmt, a).view(np.uint32))
+        m = (37 << 20) // (4 * k)
+        x = synth.normal_f32(98, m * k).reshape(m, k)
+        got = backend.gemm_cached(w, x, m, n, k)
+        for i in (0, m // 2, m - 1):    # rows from either side of the hand-overs, against products of their own
+            part = backend.gemm_cached(w, x[i:i + 1], 1, n, k)[0]
+            assert np.max(np.abs(got[i] - part)) <= 2e-6 * k**0.5 * np.max(np.abs(part)), i
+    finally:
+        backend.free_weights(w)
+
+
 def test_device_memory_returns_when_models_and_weights_go(backend):
     cfg = dict(fmt=TQ2, n_layers=2, h=512, inter=1024, nq=8, nkv=2, hd=64, vocab=1000, max_seq=2048, eps=1e-6, rope_theta=1e6)
     w = synth.make_model(cfg, 5)
