@@ -81,9 +81,9 @@ int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two
 
 int ensure_flag() {
     if (st.flag) return OXB_HIP_OK;
-    // (the counter is cleared in the stream whose kernels count on it: a clear in another one may come after them)
+    // (the null stream that clears has no order with the stream whose kernels count on it: the clear is waited for)
     if (hipHostMalloc((void**)&st.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&st.arrived, 4) != hipSuccess ||
-        hipMemsetAsync(st.arrived, 0, 4, g_rt.stream) != hipSuccess || hipStreamSynchronize(g_rt.stream) != hipSuccess) {
+        hipMemset(st.arrived, 0, 4) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
         (void)hipGetLastError();
         if (st.flag) (void)hipHostFree(st.flag);
         if (st.arrived) (void)hipFree(st.arrived);

@@ -39,14 +39,13 @@ size_t pending();            // work not finished yet
 extern size_t syncs, host_mallocs, host_frees, host_bytes, host_bytes_limit;
 }  // namespace fake
 
-hipError_t hipStreamSynchronize(hipStream_t);
+hipError_t hipStreamSynchronize(hipStream_t);  // nullptr: the null stream
 hipError_t hipDeviceSynchronize();
 hipError_t hipMalloc(void** p, size_t n);
 hipError_t hipFree(void* p);
 hipError_t hipHostMalloc(void** p, size_t n, unsigned flags);
 hipError_t hipHostFree(void* p);
-hipError_t hipMemset(void* p, int v, size_t n);                  // on the null stream: no order with the stream in use
-hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t);
+hipError_t hipMemset(void* p, int v, size_t n);  // on the null stream, which has no order with the others: done when that is waited for
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char* hipGetErrorString(hipError_t) { return "error"; }
 
