@@ -14,7 +14,8 @@ struct OxbGemmParams {
     const uint32_t* codes;   // resident codes section
     const uint16_t* scales;  // resident scales section
     const uint32_t* xh;      // packed fp16 activations (oxb_launch_xh_pack)
-    const int32_t* xsh;      // [M] exponent that undoes the row scaling, INT32_MIN for a non-finite row
+    const int32_t* xsh;      // [M] exponent that undoes the row scaling, INT32_MIN for a non-finite row; null: x_exp for all rows
+    int32_t x_exp;
     float* y;                // [M][ldy]
     const float* residual;   // [M][ldy], mode RESIDUAL only
     uint32_t n_rows, n_tiles, n_sb;
@@ -27,6 +28,13 @@ struct OxbGemmParams {
     float* part;             // [ksplit][M][ldy] partial sums, needed when oxb_gemm_ksplit(...) > 1
     uint32_t codes_bytes, scales_bytes, xh_bytes;  // buffer extents (loads beyond them read 0)
     int mode;
+    // Mode SWIGLU, optional: instead of y the packed activations of the product that follows (n_rows / 2 values a row, a multiple
+    // of 128; its format is this matrix's) and their exponents.  norm: |a|_2 < 2^norm of every row (oxb_launch_xh_pack),
+    // w_exp: the 2-norm of every row of the matrix is below 2^w_exp.
+    uint32_t* xh_out;
+    int32_t* xsh_out;
+    const int32_t* norm;
+    int32_t w_exp;
     bool no_split;           // keep K in one piece (a caller without room for partial sums)
     bool sum_later;          // mode RESIDUAL: with K in slices leave the sums in `part`, the next pack of y adds them (OxbPackSum)
 };
@@ -44,7 +52,10 @@ enum { OXB_PACK_IDENT = 0, OXB_PACK_RMSNORM = 1 };
 struct OxbPackSum { const float* part; uint32_t n; size_t plane; };
 bool oxb_pack_can_sum(uint32_t k, uint32_t M);
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
-                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr);
+                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr,
+                              int32_t* d_norm = nullptr);  // d_norm (RMSNORM): [M] exponents, the 2-norm of a row's activations is below 2^norm
+// Largest sum of squared scales of a row, as float bits, joined by maximum with what *d_out holds.
+hipError_t oxb_launch_row_norm(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t* d_out, hipStream_t st);
 // What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16, or the wide one
 // with rt row tiles per wave, tpw per workgroup, 16 ct tokens per tile; K in ksplit slices of sb_per_split superblocks.
 struct OxbGemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };

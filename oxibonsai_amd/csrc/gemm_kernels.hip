@@ -26,6 +26,7 @@
 #include "device_utils.h"
 #include "gemm_kernels.h"
 #include "layout.h"
+#include "operand_device.h"
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
@@ -47,12 +48,16 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     const v2h h = {(_Float16)a, (_Float16)b};
     return __builtin_bit_cast(uint32_t, h);
 }
+__device__ __forceinline__ float sum_sq(const float4& a, float s) { return fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, fmaf(a.w, a.w, s)))); }
 __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
-// Multiplier and exponent of one token row from its sum of squares, its largest |a| before the producer's scalar and
-// whether it holds something non-finite.
+// What the packer says about one token row: its multiplier, the exponent that undoes the power of two, and (RMSNORM) an
+// exponent above the 2-norm of its activations, |a|_2 < 2^norm.
+struct RowScale { float mul; int32_t xsh, norm; };
+// ... from the row's sum of squares, that of its |a| before the producer's scalar, the largest of those and whether it holds
+// something non-finite.
 template <int OP>
-__device__ __forceinline__ void row_scale(float ss, float mx, int bad, uint32_t k, float eps, float* mul_out, int32_t* xsh_out) {
+__device__ __forceinline__ RowScale row_scale(float ss, float sa, float mx, int bad, uint32_t k, float eps) {
     float scalar = 1.0f;
     if (OP == OXB_PACK_RMSNORM) {
         scalar = 1.0f / sqrtf(ss / (float)k + eps);
@@ -62,22 +67,27 @@ __device__ __forceinline__ void row_scale(float ss, float mx, int bad, uint32_t 
     int E = 0;
     if (mx > 0.0f) (void)frexpf(mx, &E);  // mx = f * 2^E, f in [0.5, 1)
     const int shift = mx > 0.0f ? 15 - E : 0;
-    *mul_out = bad ? 0.0f : ldexpf(scalar, shift);
-    *xsh_out = bad ? INT32_MIN : -shift;
+    int N = -64;
+    if (OP == OXB_PACK_RMSNORM) {
+        // (a sum of squares that overflows comes from values whose norm the products' fp32 sums could not hold either)
+        const float norm = sqrtf(sa) * scalar;
+        if (norm > 0.0f) (void)frexpf(fminf(norm, 3.402823466e38f), &N);
+        N = N < -64 ? -64 : N;
+    }
+    return {bad ? 0.0f : ldexpf(scalar, shift), bad ? INT32_MIN : -shift, bad ? 0 : N};
 }
 
-// Multiplier and exponent of one token row from the threads' partial results (sum of squares of x, largest |a|,
-// non-finite seen); all 256 threads of the workgroup call it, thread 0 gets the result.
+// The threads' partial results (sums of squares of x and of a, largest |a|, non-finite seen) joined; all 256 threads of the
+// workgroup call it, thread 0 gets the result.
+struct RowRed { float s[4], a[4], m[4]; int b[4]; };
 template <int OP>
-__device__ __forceinline__ void row_finish(float ss, float mx, int bad, uint32_t k, float eps, float* red_s, float* red_m,
-                                           int* red_b, float* mul_out, int32_t* xsh_out);
+__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, RowRed& red);
 
 // The same with the pass over the row in front: a float4 per thread and step, in row order.
 template <int OP>
-__device__ __forceinline__ void row_stats(const float* __restrict__ xr, const float* __restrict__ w, uint32_t k, float eps,
-                                          float* red_s, float* red_m, int* red_b, float* mul_out, int32_t* xsh_out) {
+__device__ __forceinline__ RowScale row_stats(const float* __restrict__ xr, const float* __restrict__ w, uint32_t k, float eps, RowRed& red) {
     const uint32_t tid = threadIdx.x;
-    float ss = 0.f, mx = 0.f;
+    float ss = 0.f, sa = 0.f, mx = 0.f;
     int bad = 0;
     for (uint32_t i = tid * 4; i < k; i += 1024) {
         const float4 v = *reinterpret_cast<const float4*>(xr + i);
@@ -86,39 +96,38 @@ __device__ __forceinline__ void row_stats(const float* __restrict__ xr, const fl
             const float4 g = *reinterpret_cast<const float4*>(w + i);
             ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
             a = make_float4(g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
+            sa = sum_sq(a, sa);
         }
         bad |= !(fabsf(a.x) <= 3.402823466e38f) | !(fabsf(a.y) <= 3.402823466e38f) | !(fabsf(a.z) <= 3.402823466e38f) |
                !(fabsf(a.w) <= 3.402823466e38f);
         mx = fmaxf(fmaxf(mx, fmaxf(fabsf(a.x), fabsf(a.y))), fmaxf(fabsf(a.z), fabsf(a.w)));
     }
-    row_finish<OP>(ss, mx, bad, k, eps, red_s, red_m, red_b, mul_out, xsh_out);
+    return row_finish<OP>(ss, sa, mx, bad, k, eps, red);
 }
 
 template <int OP>
-__device__ __forceinline__ void row_finish(float ss, float mx, int bad, uint32_t k, float eps, float* red_s, float* red_m,
-                                           int* red_b, float* mul_out, int32_t* xsh_out) {
+__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, RowRed& red) {
     const uint32_t tid = threadIdx.x;
-    ss = wave_sum_f32(ss);  // DPP and lane swaps: no trips through the LDS pipeline
+    if (OP == OXB_PACK_RMSNORM) ss = wave_sum_f32(ss), sa = wave_sum_f32(sa);  // DPP and lane swaps: no trips through the LDS pipeline
     mx = wave_max_f32(mx);
     bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
-    if ((tid & 63u) == 0) red_s[tid >> 6] = ss, red_m[tid >> 6] = mx, red_b[tid >> 6] = bad;
+    if ((tid & 63u) == 0) red.s[tid >> 6] = ss, red.a[tid >> 6] = sa, red.m[tid >> 6] = mx, red.b[tid >> 6] = bad;
     __syncthreads();
-    if (tid == 0)
-        row_scale<OP>(red_s[0] + red_s[1] + red_s[2] + red_s[3], fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3])),
-                      red_b[0] | red_b[1] | red_b[2] | red_b[3], k, eps, mul_out, xsh_out);
+    if (tid) return {0.f, 0, 0};
+    return row_scale<OP>(red.s[0] + red.s[1] + red.s[2] + red.s[3], red.a[0] + red.a[1] + red.a[2] + red.a[3],
+                         fmaxf(fmaxf(red.m[0], red.m[1]), fmaxf(red.m[2], red.m[3])), red.b[0] | red.b[1] | red.b[2] | red.b[3], k, eps);
 }
 
 template <int OP>
 __global__ __launch_bounds__(256) void row_stats_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                          uint32_t ldx, uint32_t k, float eps, float* __restrict__ rowmul,
-                                                         int32_t* __restrict__ xsh) {
-    __shared__ float red_s[4], red_m[4];
-    __shared__ int red_b[4];
+                                                         int32_t* __restrict__ xsh, int32_t* __restrict__ norm) {
+    __shared__ RowRed red;
     const uint32_t m = blockIdx.x;
-    float mul = 0.f;
-    int32_t e = 0;
-    row_stats<OP>(x + (size_t)m * ldx, w, k, eps, red_s, red_m, red_b, &mul, &e);
-    if (threadIdx.x == 0) rowmul[m] = mul, xsh[m] = e;
+    const RowScale r = row_stats<OP>(x + (size_t)m * ldx, w, k, eps, red);
+    if (threadIdx.x) return;
+    rowmul[m] = r.mul, xsh[m] = r.xsh;
+    if (norm) norm[m] = r.norm;
 }
 
 // The eight activations of token row xr that chunk c = 4g + s of block blk holds, scaled by mul, as four fp16 pairs.
@@ -163,9 +172,8 @@ __device__ __forceinline__ float4 add4(const float4& a, const float4& b) { retur
 template <int FMT, int OP, int NI, bool SUM>
 __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float* __restrict__ w, uint32_t ldx,
                                                             uint32_t k, float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh, const OxbPackSum sum) {
-    __shared__ float red_s[4], red_m[4];
-    __shared__ int red_b[4];
+                                                            int32_t* __restrict__ xsh, int32_t* __restrict__ norm, uint4* __restrict__ xh, const OxbPackSum sum) {
+    __shared__ RowRed red;
     __shared__ float mul_s;
     const uint32_t m = blockIdx.x, tid = threadIdx.x, n_items = nblk_pad * 16;
     if (m >= M) {  // uniform over the workgroup
@@ -225,7 +233,7 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
             }
         }
     }
-    float ss = 0.f, mx = 0.f;
+    float ss = 0.f, sa = 0.f, mx = 0.f;
     int bad = 0;
 #pragma unroll
     for (int it = 0; it < NI; it++) {
@@ -236,6 +244,7 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
             ss = fmaf(q.x, q.x, fmaf(q.y, q.y, fmaf(q.z, q.z, fmaf(q.w, q.w, ss))));
             p = make_float4(wa[it].x * p.x, wa[it].y * p.y, wa[it].z * p.z, wa[it].w * p.w);
             q = make_float4(wb[it].x * q.x, wb[it].y * q.y, wb[it].z * q.z, wb[it].w * q.w);
+            sa = sum_sq(q, sum_sq(p, sa));
         }
         const float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -244,12 +253,13 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
             mx = fmaxf(mx, fabsf(v[e]));
         }
     }
-    float mul = 0.f;
-    int32_t e = 0;
-    row_finish<OP>(ss, mx, bad, k, eps, red_s, red_m, red_b, &mul, &e);
-    if (tid == 0) mul_s = mul, xsh[m] = e;
+    const RowScale rs = row_finish<OP>(ss, sa, mx, bad, k, eps, red);
+    if (tid == 0) {
+        mul_s = rs.mul, xsh[m] = rs.xsh;
+        if (OP == OXB_PACK_RMSNORM && norm) norm[m] = rs.norm;
+    }
     __syncthreads();
-    mul = mul_s;
+    const float mul = mul_s;
 #pragma unroll
     for (int it = 0; it < NI; it++) {
         const uint32_t id = it * 256 + tid;
@@ -271,13 +281,13 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
 template <int FMT, int OP, int RPW, int NI, bool SUM>
 __global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float* __restrict__ w, uint32_t ldx, uint32_t k,
                                                             float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, uint4* __restrict__ xh, const OxbPackSum sum) {
+                                                            int32_t* __restrict__ xsh, int32_t* __restrict__ norm, uint4* __restrict__ xh, const OxbPackSum sum) {
     constexpr int WPR = 8 / RPW, SEG = NI <= 16 ? NI : NI == 48 ? 16 : 12;
     static_assert(NI % SEG == 0, "whole segments");
     constexpr uint32_t VALS = SEG * 256 * WPR, STR = VALS + 16;  // values of a row in a segment; LDS row stride (32 bytes of padding spread the rows over the banks)
     constexpr int WG = OP == OXB_PACK_RMSNORM && NI > 16 ? 4 : SEG;  // norm weights requested at a time (registers)
     __shared__ __attribute__((aligned(16))) _Float16 rows[RPW * STR];
-    __shared__ float red_s[8], red_m[8];
+    __shared__ float red_s[8], red_a[8], red_m[8];
     __shared__ int red_b[8];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, m0 = blockIdx.x * RPW;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), wr = wave / WPR, part = wave % WPR, m = m0 + wr;
@@ -303,7 +313,7 @@ __global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float
             if (at_of(i) < k) *reinterpret_cast<float4*>(xr + at_of(i)) = a[i];
         }
     }
-    float ss = 0.f, mx = 0.f;
+    float ss = 0.f, sa = 0.f, mx = 0.f;
     int bad = 0;
 #pragma unroll
     for (int i0 = 0; i0 < NI; i0 += WG) {
@@ -319,27 +329,29 @@ __global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float
                 ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
                 const float4 q = g[OP == OXB_PACK_RMSNORM ? i : 0];
                 v = make_float4(q.x * v.x, q.y * v.y, q.z * v.z, q.w * v.w);
+                sa = sum_sq(v, sa);
             }
             bad |= !(fabsf(v.x) <= 3.402823466e38f) | !(fabsf(v.y) <= 3.402823466e38f) | !(fabsf(v.z) <= 3.402823466e38f) |
                    !(fabsf(v.w) <= 3.402823466e38f);
             mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
         }
     }
-    ss = wave_sum_f32(ss);
+    if (OP == OXB_PACK_RMSNORM) ss = wave_sum_f32(ss), sa = wave_sum_f32(sa);
     mx = wave_max_f32(mx);
     bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
     if constexpr (WPR > 1) {  // the row's waves, added in wave order
-        if (lane == 0) red_s[wave] = ss, red_m[wave] = mx, red_b[wave] = bad;
+        if (lane == 0) red_s[wave] = ss, red_a[wave] = sa, red_m[wave] = mx, red_b[wave] = bad;
         __syncthreads();
-        ss = red_s[wr * WPR], mx = red_m[wr * WPR], bad = red_b[wr * WPR];
+        ss = red_s[wr * WPR], sa = red_a[wr * WPR], mx = red_m[wr * WPR], bad = red_b[wr * WPR];
 #pragma unroll
-        for (int i = 1; i < WPR; i++) ss += red_s[wr * WPR + i], mx = fmaxf(mx, red_m[wr * WPR + i]), bad |= red_b[wr * WPR + i];
+        for (int i = 1; i < WPR; i++) ss += red_s[wr * WPR + i], sa += red_a[wr * WPR + i], mx = fmaxf(mx, red_m[wr * WPR + i]), bad |= red_b[wr * WPR + i];
     }
-    float mul;
-    int32_t e;
-    row_scale<OP>(ss, mx, bad, k, eps, &mul, &e);
-    if (!live) mul = 0.f;
-    else if (part == 0 && lane == 0) xsh[m] = e;
+    const RowScale rs = row_scale<OP>(ss, sa, mx, bad, k, eps);
+    const float mul = live ? rs.mul : 0.f;
+    if (live && part == 0 && lane == 0) {
+        xsh[m] = rs.xsh;
+        if (OP == OXB_PACK_RMSNORM && norm) norm[m] = rs.norm;
+    }
 #pragma unroll
     for (int i0 = 0; i0 < NI; i0 += SEG) {
         if (i0) __syncthreads();  // the segment before has been read
@@ -530,6 +542,22 @@ __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A
     }
 }
 
+// Exponent that undoes the scaling of token row m, INT32_MIN for a row that holds something non-finite.
+__device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) { return p.xsh ? p.xsh[m] : p.x_exp; }
+
+// SWIGLU with the next product's operand as the output: |gate|, |up| < 2^(w_exp + norm) (Cauchy-Schwarz; a factor of two is
+// left for the roundings), so silu(gate) up 2^shift lies below 2^15.
+__device__ __forceinline__ int swiglu_shift(const OxbGemmParams& p, uint32_t m) { return 14 - 2 * (p.w_exp + p.norm[m]); }
+
+// What else the operand of n_rows / 2 values a row needs: the rows' exponents, and zeros in the blocks up to a whole superblock.
+// By one workgroup for `rows` rows from m0 on.
+__device__ __forceinline__ void finish_operand(const OxbGemmParams& p, uint32_t m0, uint32_t rows, uint32_t tid, uint32_t threads) {
+    for (uint32_t j = tid; j < rows && m0 + j < p.M; j += threads) p.xsh_out[m0 + j] = -swiglu_shift(p, m0 + j);
+    const uint32_t blocks = p.n_rows / 256u, pad = ((blocks + 3u) & ~3u) - blocks;
+    for (uint32_t i = tid; i < pad * 16u * rows; i += threads)
+        reinterpret_cast<uint4*>(p.xh_out)[(size_t)(blocks * 16u + i / rows) * p.M_pad + m0 + i % rows] = make_uint4(0, 0, 0, 0);
+}
+
 template <int FMT, int RT, int CT>
 __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_kernel(const OxbGemmParams p) {
     constexpr int BM = 16 * CT;
@@ -545,11 +573,9 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
     const uint32_t sb0 = ks * p.sb_per_split, sb1 = min(sb0 + p.sb_per_split, p.n_sb);
     // row tiles: the workgroup's [wg_t0, wg_t1), split evenly over the four waves
     const uint32_t wg_t0 = n_g * p.tpw, wg_t1 = min(wg_t0 + p.tpw, p.n_tiles);
-    // SWIGLU mode (the matrix is gate || up).  Even RT: the tile sequence interleaves gate tile j and up tile j, and
-    // every wave starts on a gate tile (the launcher gives it an even count), so accumulators 2q and 2q+1 hold both
-    // factors of 16 output rows.  Odd RT (three tiles per wave, the count that still runs two workgroups per CU): waves 0
-    // and 1 take RT gate tiles each, waves 2 and 3 the up tiles of the same rows; the up factors cross over through the
-    // LDS stages once the K loop is done.
+    // SWIGLU mode (the matrix is gate || up).  Two tiles per wave: a gate tile and the up tile of the same rows.  Three (the
+    // count that still runs two workgroups per CU): waves 0 and 1 take three gate tiles each, waves 2 and 3 the up tiles of
+    // the same rows.  The factors meet in the LDS stages once the K loop is done.
     const bool sw = p.mode == OXB_GEMM_SWIGLU;
     constexpr bool SPLIT = RT == 3;  // (of the SWIGLU mode; other odd counts are never launched in it)
     auto tile_of = [&](uint32_t u) -> uint32_t { return sw ? ((u & 1u) ? p.n_tiles / 2 + (u >> 1) : (u >> 1)) : u; };
@@ -674,80 +700,83 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 
     // epilogue: lane holds rows 4g..4g+3 of the row tile for token 16ct + r
     const bool vec_ok = (p.ldy & 3u) == 0;
-    if (sw && SPLIT) {
-        // The K loop ended behind a barrier with no stage load in flight: both stages are free.  Up waves leave their
-        // factors (already scaled back by the row's power of two) in the stage of their half, tile by tile as
-        // [rt][ct][lane] float4; the gate waves of the same half pick them up.
-        float4* ex = reinterpret_cast<float4*>((wave & 1u) ? xs1 : xs0);
-        static_assert(!SPLIT || (size_t)RT * CT * 64 * 16 <= sizeof(xs0), "the up factors of a wave fit a stage");
-        if (wave >> 1) {
+    if constexpr (RT == 2 || RT == 3) {  // (the counts that are launched in SWIGLU mode)
+        if (sw) {
+            // The K loop ended behind a barrier with no stage load in flight: both stages are free.  Half of the token tiles at
+            // a time the waves leave their factors there (already scaled back by the row's power of two), tile by tile as
+            // [tile][ct][lane] float4, gate in the first stage and up in the second, and then take pairs of gate tiles in
+            // turn: two tiles are 32 output rows, whole pieces of the next product's operand.
+            constexpr int CH = (CT + 1) / 2, TILES = SPLIT ? 2 * RT : 4;  // token tiles a pass, gate tiles of the workgroup
+            static_assert((size_t)TILES * CH * 64 * 16 <= sizeof(xs0), "the factors of half the token tiles fit the stages");
+            const uint32_t half_tiles = p.n_tiles / 2, g_first = n_g * TILES;
+            float4* const gx = reinterpret_cast<float4*>(xs0);
+            float4* const ux = reinterpret_cast<float4*>(xs1);
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++) {
-                const uint32_t m = m0 + ct * 16 + r;
-                const int e = m < p.M ? p.xsh[m] : 0;
+            for (int ps = 0; ps < 2; ps++) {
+                if (ps) __syncthreads();
 #pragma unroll
-                for (int rt = 0; rt < RT; rt++) {
-                    float u[4];
+                for (int ci = 0; ci < CH; ci++) {
+                    const int ct = ps * CH + ci;
+                    if (ct >= CT) continue;
+                    const uint32_t m = m0 + ct * 16 + r;
+                    const int e = m < p.M ? row_exp(p, m) : 0;
 #pragma unroll
-                    for (int v = 0; v < 4; v++) u[v] = e == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(acc[rt][ct][v], e);
-                    ex[(rt * CT + ct) * 64 + lane] = make_float4(u[0], u[1], u[2], u[3]);
+                    for (int rt = 0; rt < RT; rt++) {
+                        float o[4];
+#pragma unroll
+                        for (int v = 0; v < 4; v++) o[v] = e == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(acc[rt][ct < CT ? ct : 0][v], e);
+                        const uint32_t slot = SPLIT ? (wave & 1u) * RT + rt : wave;
+                        (( SPLIT ? wave >> 1 : (uint32_t)rt) ? ux : gx)[(slot * CH + ci) * 64 + lane] = make_float4(o[0], o[1], o[2], o[3]);
+                    }
+                }
+                __syncthreads();
+                for (uint32_t u = wave; u < TILES / 2 * CH; u += 4) {
+                    const uint32_t pr = u / CH, ci = u % CH, ct = ps * CH + ci, m = m0 + ct * 16 + r;
+                    if (ct >= CT || m >= p.M) continue;
+                    auto four = [&](uint32_t t, uint32_t ln) -> float4 {  // rows 4g..4g+3 of tile 2 pr + t for lane ln = 16 g + r
+                        const uint32_t at = ((2 * pr + t) * CH + ci) * 64 + ln;
+                        const float4 a = gx[at], b = ux[at];
+                        return make_float4(silu_mul(a.x, b.x), silu_mul(a.y, b.y), silu_mul(a.z, b.z), silu_mul(a.w, b.w));
+                    };
+                    if (p.xh_out) {
+                        if (g_first + 2 * pr >= half_tiles) continue;  // (whole blocks of 128 rows: pairs are complete)
+                        const OxbOperandOut out = {(_Float16*)p.xh_out, FMT, p.M_pad, swiglu_shift(p, m)};
+                        // lane 16 s + r writes piece s of the 32 rows
+                        const uint32_t k0 = (g_first + 2 * pr) * 16;
+                        if constexpr (FMT == OXB_FMT_Q1) operand_store8(out, k0 + 4 * g, m, four(0, lane), four(1, lane));
+                        else operand_store8(out, k0 + 16 * (g >> 1) + 4 * (g & 1u), m, four(g >> 1, (g & 1u) * 16 + r), four(g >> 1, ((g & 1u) + 2) * 16 + r));
+                        continue;
+                    }
+#pragma unroll
+                    for (uint32_t t = 0; t < 2; t++) {
+                        const uint32_t tile = g_first + 2 * pr + t, n = tile * 16 + 4 * g;
+                        if (tile >= half_tiles) continue;
+                        const float4 o = four(t, lane);
+                        float* yr = p.y + (size_t)m * p.ldy + n;
+                        if (vec_ok) *reinterpret_cast<float4*>(yr) = o;
+                        else yr[0] = o.x, yr[1] = o.y, yr[2] = o.z, yr[3] = o.w;
+                    }
                 }
             }
+            if (p.xh_out && n_g == 0) finish_operand(p, m0, min((uint32_t)BM, p.M_pad - m0), tid, OXB_GEMM_THREADS);
+            return;
         }
-        __syncthreads();
-        if (wave >> 1) return;
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) {
-            const uint32_t m = m0 + ct * 16 + r;
-            if (m >= p.M) continue;
-            const int e = p.xsh[m];
-            float* yr = p.y + (size_t)m * p.ldy;
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                if ((uint32_t)rt >= n_valid) continue;
-                const uint32_t n = (t0 + rt) * 16 + 4 * g, n_lim = p.n_rows / 2;
-                const float4 u = ex[(rt * CT + ct) * 64 + lane];
-                const float uu[4] = {u.x, u.y, u.z, u.w};
-                float o[4];
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    o[v] = silu_mul(e == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(acc[rt][ct][v], e), uu[v]);
-                if (vec_ok && n + 3 < n_lim) {
-                    *reinterpret_cast<float4*>(yr + n) = make_float4(o[0], o[1], o[2], o[3]);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        if (n + v < n_lim) yr[n + v] = o[v];
-                }
-            }
-        }
-        return;
     }
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) {
         const uint32_t m = m0 + ct * 16 + r;
         if (m >= p.M) continue;
-        const int e = p.xsh[m];
+        const int e = row_exp(p, m);
         // with K split over workgroups, slice ks writes its partial sums to plane ks of the workspace
         float* yr = p.ksplit > 1 ? p.part + ((size_t)ks * p.M + m) * p.ldy : p.y + (size_t)m * p.ldy;
         const float* rr = (p.mode == OXB_GEMM_RESIDUAL && p.ksplit == 1) ? p.residual + (size_t)m * p.ldy : nullptr;
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             if ((uint32_t)rt >= n_valid) continue;
-            if (sw && (rt & 1)) continue;  // the up factor: consumed with its gate tile
-            const uint32_t n = sw ? ((t0 + rt) >> 1) * 16 + 4 * g : (t0 + rt) * 16 + 4 * g;
-            const uint32_t n_lim = sw ? p.n_rows / 2 : p.n_rows;
+            const uint32_t n = (t0 + rt) * 16 + 4 * g, n_lim = p.n_rows;
             float o[4];
 #pragma unroll
             for (int v = 0; v < 4; v++) o[v] = e == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(acc[rt][ct][v], e);
-            if (sw) {
-                constexpr int ru = RT > 1 ? 1 : 0;  // (RT = 1 is never launched in this mode)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const float u = e == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(acc[rt + ru < RT ? rt + ru : rt][ct][v], e);
-                    o[v] = silu_mul(o[v], u);
-                }
-            }
             if (vec_ok && n + 3 < n_lim) {
                 if (rr) {
                     const float4 q4 = *reinterpret_cast<const float4*>(rr + n);
@@ -926,7 +955,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
         const uint32_t q = idx / CT, ct = idx % CT, m = ct * 16 + r;
         const uint32_t rt = (uint32_t)pass_rt(ps, (int)q);
         if (!valid((int)rt) || m >= p.M) continue;
-        const int e = p.xsh[m];
+        const int e = row_exp(p, m);
         float o[4];
         total(idx, o, e);
         if (sw) {  // y[m][row] = silu(gate) * up, rows counted within the gate half
@@ -934,6 +963,10 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
             total((q + q_up) * CT + ct, u, e);
 #pragma unroll
             for (int v = 0; v < 4; v++) o[v] = silu_mul(o[v], u[v]);
+            if (p.xh_out) {
+                operand_store4({(_Float16*)p.xh_out, FMT, p.M_pad, swiglu_shift(p, m)}, (t0 + rt) * 16 + 4 * g, m, o[0], o[1], o[2], o[3]);
+                continue;
+            }
         }
         // (with K split over workgroups, slice ks writes its partial sums to plane ks of the workspace)
         float* yr = p.ksplit > 1 ? p.part + ((size_t)ks * p.M + m) * p.ldy : p.y + (size_t)m * p.ldy;
@@ -952,6 +985,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
         }
     }
     }
+    if (sw && p.xh_out && ng == 0) finish_operand(p, 0, p.M_pad, tid, OXB_GEMM_NARROW_THREADS);
 }
 
 // y = (residual +) the K slices' partial sums, added in slice order (deterministic): where no pack of the result follows.
@@ -972,9 +1006,32 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     reinterpret_cast<float4*>(y)[i] = a;
 }
 
+// Largest sum of squares of the fp16 scales of a row among row tiles [t0, t1), one workgroup per tile; 128 times that bounds the
+// square of every row's 2-norm (weights are +-d or 0).  The maximum of non-negative floats is that of their bits.
+__global__ __launch_bounds__(256) void row_norm_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t t0, uint32_t* __restrict__ out) {
+    __shared__ float part[16][17];
+    const uint32_t tid = threadIdx.x, r = tid & 15u, j = tid >> 4;
+    const _Float16* s = reinterpret_cast<const _Float16*>(scales) + (size_t)(t0 + blockIdx.x) * n_sb * 64u + r * 4u;
+    float a = 0.f;
+    for (uint32_t sb = j; sb < n_sb; sb += 16)
+        for (int q = 0; q < 4; q++) a = fmaf((float)s[sb * 64u + q], (float)s[sb * 64u + q], a);
+    part[j][r] = a;
+    __syncthreads();
+    if (tid < 16) {
+        for (int i = 1; i < 16; i++) a += part[i][tid];
+        atomicMax(out, a == a ? __float_as_uint(a) : 0x7F800000u);  // (a NaN scale: no bound)
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers.
 // ---------------------------------------------------------------------------
+hipError_t oxb_launch_row_norm(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t* d_out, hipStream_t st) {
+    const uint32_t t0 = row0 / 16, t1 = (row0 + n_rows + 15) / 16;
+    hipLaunchKernelGGL(row_norm_kernel, dim3(t1 - t0), dim3(256), 0, st, d_scales, n_sb, t0, d_out);
+    return hipGetLastError();
+}
+
 size_t oxb_xh_bytes(uint32_t k, uint32_t M) {
     const size_t nblk_pad = ((k + 511u) / 512u) * 4u, M_pad = (M + 15u) / 16u * 16u;
     return nblk_pad * 16 * M_pad * 16;
@@ -984,17 +1041,17 @@ size_t oxb_xh_bytes(uint32_t k, uint32_t M) {
 
 template <int OP, bool SUM>
 static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, uint32_t k, uint32_t M, uint32_t M_pad,
-                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, const OxbPackSum& sum, hipStream_t st) {
+                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, int32_t* d_norm, const OxbPackSum& sum, hipStream_t st) {
     const uint32_t per_thread = (nblk_pad * 16 + 255) / 256;  // items of a row per thread of the one-launch packer
     if (M <= OXB_PACK_ROWS_MAX && per_thread <= 8) {
 #define OXB_ROWS_CASE(NI)                                                                                                      \
     if (per_thread <= NI) {                                                                                                    \
         if (fmt == OXB_FMT_Q1)                                                                                                 \
             hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_Q1, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                                   \
+                               M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         else                                                                                                                   \
             hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_TQ2, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                                   \
+                               M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         return;                                                                                                                \
     }
         OXB_ROWS_CASE(1) OXB_ROWS_CASE(2) OXB_ROWS_CASE(4)
@@ -1010,10 +1067,10 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
     if (rpw == RPW && per_lane <= NI) {                                                                                            \
         if (fmt == OXB_FMT_Q1)                                                                                                     \
             hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_Q1, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                            \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
         else                                                                                                                       \
             hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_TQ2, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, reinterpret_cast<uint4*>(d_xh), sum);                            \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
         return;                                                                                                                    \
     }
     OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16)
@@ -1023,7 +1080,7 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
     // (rows of more than 12288 values take two launches)
 #undef OXB_WIDE_CASE
     if constexpr (!SUM) {
-        hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh);
+        hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh, d_norm);
         const dim3 grid(M_pad / 16, nblk_pad < 16 ? nblk_pad : 16);
         if (fmt == OXB_FMT_Q1)
             hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_Q1, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
@@ -1037,7 +1094,7 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
 bool oxb_pack_can_sum(uint32_t k, uint32_t M) { return k <= (M <= OXB_PACK_ROWS_MAX ? 8192u : 12288u) && (k % OXB_QK) == 0; }
 
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
-                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum) {
+                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum, int32_t* d_norm) {
     if (M == 0 || k == 0 || (k % OXB_QK) != 0 || (ldx & 3u) != 0) return hipErrorInvalidValue;
     if (op == OXB_PACK_RMSNORM && !d_w) return hipErrorInvalidValue;
     const uint32_t nblk_pad = ((k + 511u) / 512u) * 4u, M_pad = (M + 15u) / 16u * 16u;
@@ -1045,13 +1102,13 @@ hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_
     float* x = const_cast<float*>(d_x);  // (written with `sum` only)
     if (sum && sum->n > 1) {
         if (op != OXB_PACK_RMSNORM || !oxb_pack_can_sum(k, M) || ldx != k) return hipErrorInvalidValue;
-        launch_pack_op<OXB_PACK_RMSNORM, true>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, *sum, st);
+        launch_pack_op<OXB_PACK_RMSNORM, true>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, *sum, st);
         return hipGetLastError();
     }
     const OxbPackSum none = {nullptr, 0, 0};
     switch (op) {
-        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, none, st); break;
-        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, none, st); break;
+        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, none, st); break;
+        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, none, st); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1178,6 +1235,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     if (p.M == 0 || p.n_rows == 0) return hipSuccess;
     if (p.n_sb == 0 || (uint64_t)p.n_tiles * p.n_sb * 2048ull >= 0xFFFFFFF0ull) return hipErrorInvalidValue;
     if (p.mode == OXB_GEMM_SWIGLU && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // whole gate and up row tiles
+    if (p.xh_out && (p.mode != OXB_GEMM_SWIGLU || (p.n_rows & 255u) != 0 || !p.xsh_out || !p.norm)) return hipErrorInvalidValue;  // whole blocks
     p.M_pad = (p.M + 15u) / 16u * 16u;
     const OxbGemmPlan plan = oxb_gemm_plan(fmt, p, n_cus);
     p.ksplit = plan.ksplit;

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "kv_quant_device.h"
+#include "operand_device.h"
 
 struct OxbQkParams {
     const float* qkv;      // [batch][qkv_stride]: q heads | k heads | v heads
@@ -47,6 +48,8 @@ struct OxbAttnParams {
     // pack_fmt = the O weight's format.
     uint32_t* pack_out;                  // nullptr = off
     uint32_t pack_fmt, pack_n_sb, pack_nvg;
+    // Optional: the outputs as the packed activations of the O projection's GEMM instead of p.out.
+    OxbOperandOut op;
 };
 
 // n_rows rows of n values -> one-byte codes [n_rows][n] and a scale per row (kv_mode: OXB_KV_I8 or OXB_KV_FP8_E4M3).

@@ -703,7 +703,8 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         }
         if (used == 1) {  // the only slot: what the merge would compute (weight 1, times 1 / sum)
             o *= l > 0.f ? 1.0f / l : 0.f;
-            p.out[((size_t)b * p.nq + h0 + h) * HD + d] = o;
+            if (p.op.xh) p.op.xh[oxb_operand_index(p.op.fmt, (h0 + h) * HD + d, b, p.op.M_pad)] = (_Float16)ldexpf(o, p.op.shift);
+            else p.out[((size_t)b * p.nq + h0 + h) * HD + d] = o;
             if (pack) keep[i] = o;
             continue;
         }
@@ -850,7 +851,8 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
         if (live && !sh) {
             const float il = inv_l[hh];
             acc.x *= il, acc.y *= il, acc.z *= il, acc.w *= il;
-            *reinterpret_cast<float4*>(p.out + (size_t)b * qd + e) = acc;
+            if (p.op.xh) operand_store4(p.op, e, b, acc.x, acc.y, acc.z, acc.w);
+            else *reinterpret_cast<float4*>(p.out + (size_t)b * qd + e) = acc;
             if (pack) keep[eg] = acc;
         }
     }

@@ -80,6 +80,11 @@ struct Model {
                         // nothing else writes it, so the slots of a last vector group's absent vectors stay zero vectors
     // a model loaded from a file owns the weights it uploaded
     std::vector<uint64_t> owned_mats, owned_vecs;
+    // Bounds for the products that hand their operands on (GemmFlow): every gate and up row's 2-norm is below 2^gate_up, every
+    // value row of the cache below 2^value; NO_BOUND where there is none that helps.
+    struct Bounds { int32_t gate_up, value; };
+    std::vector<Bounds> bounds;
+    DevBuf norm_buf;
     DevBuf tok_hist, tok_ids;  // token history of the on-device generation loop; prompt ids of a token prefill
     DevBuf sample_ws, rng;     // sampler scratch and per-sequence xorshift64 states
 };
@@ -144,6 +149,7 @@ static void free_model(Model& m) {
     m.tok_ids.release();
     m.sample_ws.release();
     m.rng.release();
+    m.norm_buf.release();
 }
 
 void shutdown_models() {
@@ -234,6 +240,75 @@ static int encode_ffn(float* hidden, const float* attn_out, const float* ffn_nor
 // Sequences per pass of the GEMV-based step: all of them up to eight.
 static uint32_t decode_chunk(uint32_t batch) { return batch <= OXB_GEMV_PACKED_MAX_BATCH ? batch : OXB_GEMV_PACKED_MAX_BATCH; }
 
+// Exponent E with sqrt(128 norm2) * by < 2^E.
+constexpr int32_t NO_BOUND = 1000;
+static int32_t bound_exp(float norm2, double by) {
+    const double b = std::sqrt(128.0 * (double)norm2) * by;
+    int e = 0;
+    if (!std::isfinite(b)) return NO_BOUND;
+    if (b > 0.0) (void)std::frexp(b, &e);
+    return e < -50 ? -50 : e > 50 ? NO_BOUND : e;
+}
+
+// Bounds of every layer, from the scales of gate || up and of the value rows of Q || K || V: |W a| <= |W row|_2 |a|_2, and the
+// normalised rows of a layer's input have |a|_2 <= max |norm weight| sqrt(h).  A matrix is looked at once.
+static int find_bounds(Model& m) {
+    const oxb_model_desc& d = m.d;
+    const uint32_t v0 = (d.nq + d.nkv) * d.hd;
+    std::vector<Weight*> todo;
+    for (const oxb_layer_ids& ly : m.layers) {
+        Weight *gu = find_weight(ly.gate_up), *qkv = find_weight(ly.qkv);
+        if (gu->norm2 < 0.f || gu->norm_row0 != 0) gu->norm_row0 = 0, gu->norm2 = -1.f, todo.push_back(gu);
+        if (qkv->norm2 < 0.f || qkv->norm_row0 != v0) qkv->norm_row0 = v0, qkv->norm2 = -1.f, todo.push_back(qkv);
+    }
+    if (!todo.empty()) {
+        OXB_TRY(m.norm_buf.ensure(todo.size() * sizeof(float)));
+        OXB_TRY_HIP(clear_now(m.norm_buf.ptr, todo.size() * sizeof(float)), "norm buffer clear");
+        for (size_t i = 0; i < todo.size(); i++) {
+            const Weight& w = *todo[i];
+            OXB_TRY_HIP(oxb_launch_row_norm(w.d_scales, w.L.n_sb, w.norm_row0, w.L.n_rows - w.norm_row0, (uint32_t*)m.norm_buf.ptr + i, g_rt.stream),
+                        "kernel launch failed: row_norm");
+        }
+        std::vector<float> h(todo.size());
+        OXB_TRY_HIP(hipMemcpyAsync(h.data(), m.norm_buf.ptr, h.size() * sizeof(float), hipMemcpyDeviceToHost, g_rt.stream), "norm download");
+        OXB_TRY_HIP(hipStreamSynchronize(g_rt.stream), "norm download");
+        for (size_t i = 0; i < todo.size(); i++) todo[i]->norm2 = h[i];
+    }
+    m.bounds.resize(m.layers.size(), {NO_BOUND, -NO_BOUND});
+    for (size_t L = 0; L < m.layers.size(); L++) {
+        const oxb_layer_ids& ly = m.layers[L];
+        m.bounds[L].gate_up = bound_exp(find_weight(ly.gate_up)->norm2, 1.0);
+        // (rows that an earlier matrix wrote may still be in the cache: the bound only grows)
+        const int32_t v = bound_exp(find_weight(ly.qkv)->norm2, (double)g_rt.vectors[ly.attn_norm].absmax * std::sqrt((double)d.h));
+        if (v > m.bounds[L].value) m.bounds[L].value = v;
+    }
+    return OXB_HIP_OK;
+}
+
+// Whether the attention of layer L leaves the O projection's operand, and gate || up that of the down projection.
+static bool attn_hands_on(const Model& m, uint32_t L) { return m.bounds[L].value < NO_BOUND && (m.d.nq * m.d.hd) % 512u == 0; }
+static GemmFlow flow_gate_up(const Model& m, uint32_t L) {
+    GemmFlow f;
+    f.out = m.bounds[L].gate_up < NO_BOUND && m.d.inter % OXB_QK == 0;
+    f.w_exp = m.bounds[L].gate_up;
+    return f;
+}
+static GemmFlow flow_down(const Model& m, uint32_t L) {
+    GemmFlow f;
+    if (flow_gate_up(m, L).out) f.in = GemmFlow::SWIGLU;
+    return f;
+}
+// (the bound leaves a factor of two below 2^15 for the roundings on the way)
+static GemmFlow flow_o(const Model& m, uint32_t L, const GemmWorkspace& ws, uint32_t M, OxbOperandOut* op) {
+    GemmFlow f;
+    *op = {nullptr, (uint32_t)m.d.fmt, (M + 15u) / 16u * 16u, 14 - m.bounds[L].value};
+    if (!attn_hands_on(m, L)) return f;
+    op->xh = (_Float16*)ws.xh.ptr;
+    f.in = GemmFlow::ATTENTION;
+    f.x_exp = -op->shift;
+    return f;
+}
+
 // Looks every handle of the model up with the shape the model needs (which also binds a weight that was uploaded
 // without one).  Run at creation and again whenever a weight or vector was replaced or freed since, before a decode
 // step is captured: inside the capture nothing may allocate.
@@ -254,6 +329,7 @@ static int check_model_handles(Model& m) {
     }
     if (!rc && d.final_norm) vec_ptr(d.final_norm, d.h, "final_norm", &rc);
     if (!rc && d.lm_head) mat_ptr(d.lm_head, d.fmt, d.vocab, d.h, "lm_head", &rc);
+    if (!rc) rc = find_bounds(m);
     if (!rc) m.checked_gen = g_rt.weights_gen;
     return rc;
 }
@@ -297,7 +373,8 @@ static int size_gemm_workspaces(Model& m) {
         if (oxb_gemm_ksplit((int)w->L.fmt, gp, g_rt.n_cus) > 1 && b > part_bytes) part_bytes = b;
     }
     int rc;
-    if ((rc = m.gws.xh.ensure(oxb_xh_bytes(kx, d.batch))) || (rc = m.gws.xsh.ensure(((size_t)d.batch + 16) * 4)) ||
+    if ((rc = m.gws.xh2.ensure(oxb_xh_bytes(d.inter, d.batch))) || (rc = m.gws.xsh2.ensure(((size_t)d.batch + 16) * 4)) ||
+        (rc = m.gws.norm.ensure(((size_t)d.batch + 16) * 4)) || (rc = m.gws.xh.ensure(oxb_xh_bytes(kx, d.batch))) || (rc = m.gws.xsh.ensure(((size_t)d.batch + 16) * 4)) ||
         (rc = m.gws.rowmul.ensure(((size_t)d.batch + 16) * 4)) || (part_bytes && (rc = m.gws.part.ensure(part_bytes))))
         return rc;
     return OXB_HIP_OK;
@@ -356,9 +433,11 @@ static int kv_sync_table(Model& m) {
 // slot results in m.attn_part and the parameters the merge needs in *ap.
 // One launch: QK-norm, RoPE, the store of the new rows, attention over the cache and the merge of the KV slots into
 // m.attn_out (with a single slot per sequence the kernel writes its output directly).
-static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, const float* k_norm, const Weight* pack_for = nullptr) {
+static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, const float* k_norm, const Weight* pack_for = nullptr,
+                                   const OxbOperandOut* op = nullptr) {
     const oxb_model_desc& d = m.d;
     OxbAttnParams ap;
+    ap.op = op ? *op : OxbOperandOut{nullptr, 0, 0, 0};
     ap.qkv = m.qkv;
     ap.qkv_stride = (d.nq + 2 * d.nkv) * d.hd;
     ap.q_norm = q_norm;
@@ -414,11 +493,13 @@ static int encode_decode_step_gemm(Model& m) {
         const Weight* wdn = mat_ptr(ly.down, d.fmt, d.h, d.inter, "down", &rc);
         if (rc) return rc;
         OXB_TRY(gemm_device(*wqkv, m.hidden, d.h, m.qkv, B, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, &m.gws, &sum));
-        OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm));
-        OXB_TRY(gemm_device(*wo, m.attn_out, qd, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum));
-        // SwiGLU in the epilogue of the gate || up product
-        OXB_TRY(gemm_device(*wgu, m.hidden, d.h, m.gu, B, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, &m.gws, &sum));
-        OXB_TRY(gemm_device(*wdn, m.gu, d.inter, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum));
+        // the attention and the SwiGLU epilogue of gate || up leave the next product's operand: two packs a layer, not four
+        OxbOperandOut op;
+        const GemmFlow fo = flow_o(m, L, m.gws, B, &op);
+        OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm, nullptr, &op));
+        OXB_TRY(gemm_device(*wo, m.attn_out, qd, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum, fo));
+        OXB_TRY(gemm_device(*wgu, m.hidden, d.h, m.gu, B, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, &m.gws, &sum, flow_gate_up(m, L)));
+        OXB_TRY(gemm_device(*wdn, m.gu, d.inter, m.hidden, B, d.h, OXB_GEMM_RESIDUAL, m.hidden, OXB_PACK_IDENT, nullptr, 0.f, &m.gws, &sum, flow_down(m, L)));
     }
     const float* final_norm = vec_ptr(d.final_norm, d.h, "final_norm", &rc);
     const Weight* lm = mat_ptr(d.lm_head, d.fmt, d.vocab, d.h, "lm_head", &rc);
@@ -506,7 +587,7 @@ static int ensure_prefill_buffers(Model& m, uint32_t rows) {
 // QK-norm, RoPE and the store of M new K and V rows of one layer, then the causal attention of the M queries: qkv
 // [M][(nq + 2 nkv) hd] (raw projections) -> out [M][nq hd].
 static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t M, uint32_t pos_start, const float* qkv, const float* q_norm,
-                                    const float* k_norm, float* out) {
+                                    const float* k_norm, float* out, const OxbOperandOut* op = nullptr) {
     const oxb_model_desc& d = m.d;
     hipStream_t st = g_rt.stream;
     OxbQkParams qp;
@@ -552,6 +633,7 @@ static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t
     ap.window = m.window;
     ap.sinks = m.sinks;
     ap.out = out;
+    ap.op = op ? *op : OxbOperandOut{nullptr, 0, 0, 0};
     ap.M = M;
     ap.pos_start = pos_start;
     ap.nq = d.nq;
@@ -573,6 +655,7 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
     hipStream_t st = g_rt.stream;
     const uint32_t qd = d.nq * d.hd, kd = d.nkv * d.hd, qkv_rows = qd + 2 * kd;
     int rc = OXB_HIP_OK;
+    OXB_TRY(g_rt.gemm_ws.xh.ensure(oxb_xh_bytes(qd > d.h ? qd : d.h, M)));
     OxbPackSum sum = {nullptr, 0, 0};  // partial sums that the next pack adds to m.pf_hidden
     for (uint32_t L = 0; L < d.n_layers; L++) {
         const oxb_layer_ids& ly = m.layers[L];
@@ -586,13 +669,15 @@ static int encode_prefill(Model& m, uint32_t seq, uint32_t M, uint32_t pos_start
         const Weight* wdn = mat_ptr(ly.down, d.fmt, d.h, d.inter, "down", &rc);
         if (rc) return rc;
         OXB_TRY(gemm_device(*wqkv, m.pf_hidden, d.h, m.pf_qkv, M, qkv_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_RMSNORM, attn_norm, d.eps, nullptr, &sum));
-        OXB_TRY(encode_prefill_attention(m, L, seq, M, pos_start, m.pf_qkv, q_norm, k_norm, m.pf_attn));
-        OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr, &sum));
-        // SwiGLU in the epilogue of the gate || up product: the activation [M][inter] is all that is written
-        OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, nullptr, &sum));
+        // the attention leaves the O projection's operand, the SwiGLU epilogue of gate || up that of the down projection
+        OxbOperandOut op;
+        const GemmFlow fo = flow_o(m, L, g_rt.gemm_ws, M, &op);
+        OXB_TRY(encode_prefill_attention(m, L, seq, M, pos_start, m.pf_qkv, q_norm, k_norm, m.pf_attn, &op));
+        OXB_TRY(gemm_device(*wo, m.pf_attn, qd, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr, &sum, fo));
+        OXB_TRY(gemm_device(*wgu, m.pf_hidden, d.h, m.pf_gu, M, d.inter, OXB_GEMM_SWIGLU, nullptr, OXB_PACK_RMSNORM, ffn_norm, d.eps, nullptr, &sum, flow_gate_up(m, L)));
         // (no pack follows the last layer)
         OXB_TRY(gemm_device(*wdn, m.pf_gu, d.inter, m.pf_hidden, M, d.h, OXB_GEMM_RESIDUAL, m.pf_hidden, OXB_PACK_IDENT, nullptr, 0.f, nullptr,
-                            L + 1 < d.n_layers ? &sum : nullptr));
+                            L + 1 < d.n_layers ? &sum : nullptr, flow_down(m, L)));
     }
     if (!d.lm_head) return OXB_HIP_OK;  // the caller asked for the cache rows only
     // last token: final norm, LM head, greedy token (fp32-exact products, as in a decode step)

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "kv_quant_device.h"
+#include "operand_device.h"
 
 struct OxbPrefillAttnParams {
     const float* qkv;                 // [M][qkv_stride]: the raw projections, q heads first (QK-norm and RoPE happen in the kernel)
@@ -19,6 +20,7 @@ struct OxbPrefillAttnParams {
     uint32_t seq, layer;              // whose rows the queries attend to
     uint32_t window, sinks;           // sliding window with attention sinks; window 0 = off
     float* out;                       // [M][nq * hd]
+    OxbOperandOut op;                 // optional: the outputs as the packed activations of the O projection's GEMM instead
     uint32_t M, pos_start;            // query t sits at position pos_start + t and sees keys 0 .. pos_start + t
     uint32_t nq, nkv, hd, max_seq;
     float scale;                      // 1 / sqrt(hd)

@@ -56,6 +56,12 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // walk into runs of p.blocks_per_split blocks, each run leaves its un-normalised sums in p.part, and
 // attn_prefill_merge_kernel adds them in order.
 // ---------------------------------------------------------------------------
+// The upper half of the wave's `a` and the lower half of its `b` change places.
+__device__ __forceinline__ void swap_upper_lower(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+
 // p.part: maximum and sum of every (run, query, head), then from a 16-byte boundary on their outputs.
 __host__ __device__ constexpr size_t pf_part_head(size_t n_splits, size_t rows) { return (n_splits * rows * 2 + 3) & ~(size_t)3; }
 
@@ -380,10 +386,24 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
         if (tok >= p.M) continue;
         if (gridDim.y == 1) {
             const float inv = l > 0.f ? 1.0f / l : 0.f;
+            auto four = [&](int sl) -> float4 { return make_float4(O[t][sl][0] * inv, O[t][sl][1] * inv, O[t][sl][2] * inv, O[t][sl][3] * inv); };
             float* o = p.out + ((size_t)tok * p.nq + head) * HD + 4 * g;
 #pragma unroll
-            for (int sl = 0; sl < NS; sl++)
-                *reinterpret_cast<float4*>(o + 16 * sl) = make_float4(O[t][sl][0] * inv, O[t][sl][1] * inv, O[t][sl][2] * inv, O[t][sl][3] * inv);
+            for (int sl = 0; sl < NS; sl += 2) {
+                float4 a = four(sl), b = four(sl + 1);
+                const uint32_t k = head * HD + 16 * sl;
+                if (!p.op.xh) {
+                    *reinterpret_cast<float4*>(o + 16 * sl) = a;
+                    *reinterpret_cast<float4*>(o + 16 * sl + 16) = b;
+                } else if (p.op.fmt == OXB_FMT_Q1) {
+                    operand_store8(p.op, k + 4 * g, tok, a, b);
+                } else {
+                    // a piece holds rows 4 (g % 2) .. of one tile of 16 and those 8 further, in lanes g and g + 2: the lower lane
+                    // takes the piece of the first tile, the upper one that of the second
+                    swap_upper_lower(a.x, b.x), swap_upper_lower(a.y, b.y), swap_upper_lower(a.z, b.z), swap_upper_lower(a.w, b.w);
+                    operand_store8(p.op, k + 16 * (g >> 1) + 4 * (g & 1u), tok, a, b);
+                }
+            }
         } else {
             const size_t at = ((size_t)blockIdx.y * p.M + tok) * p.nq + head;
             if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_run[t], l);
@@ -398,30 +418,43 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
 }
 
 // out[t][head] = the runs' sums brought to a common exponent, added in order, over the total of their probabilities.
-// A thread owns four dimensions.
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint32_t n_splits, uint32_t rows,
-                                                                  uint32_t hd4, float* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x, row = i / hd4, c = i % hd4;
+// A thread owns the eight dimensions of a piece of the O projection's operand: two groups of four.
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint32_t n_splits, uint32_t rows, uint32_t nq,
+                                                                  uint32_t hd, float* __restrict__ out, const OxbOperandOut op) {
+    // four tokens side by side, so that the pieces leave in runs of 64 bytes
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, c = (i >> 2) % (hd / 8), j = (i >> 2) / (hd / 8);
+    const uint32_t tok = 4 * (j / nq) + (i & 3u), head = j % nq, row = tok * nq + head;
     if (row >= rows) return;
+    const bool q1 = op.fmt == OXB_FMT_Q1;
+    const uint32_t d = 32 * (c >> 2) + (q1 ? 4 * (c & 3u) : 16 * ((c >> 1) & 1u) + 4 * (c & 1u)), step = OXB_OPERAND_STEP(op.fmt);
     const float2* ml = reinterpret_cast<const float2*>(part);
-    const float4* po = reinterpret_cast<const float4*>(part + pf_part_head(n_splits, rows));
+    const float* po = part + pf_part_head(n_splits, rows);
     float m = -INFINITY;
     for (uint32_t s = 0; s < n_splits; s++) {
         const float2 v = ml[(size_t)s * rows + row];
         m = v.y == 0.f ? m : fmaxf(m, v.x);
     }
     float l = 0.f;
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
     for (uint32_t s = 0; s < n_splits; s++) {
         const float2 v = ml[(size_t)s * rows + row];
         if (v.y == 0.f) continue;
         const float w = __builtin_amdgcn_exp2f(v.x - m);
-        const float4 o = po[((size_t)s * rows + row) * hd4 + c];
+        const float* q = po + ((size_t)s * rows + row) * hd + d;
+        const float4 x = *reinterpret_cast<const float4*>(q), y = *reinterpret_cast<const float4*>(q + step);
         l = fmaf(v.y, w, l);
-        a.x = fmaf(o.x, w, a.x), a.y = fmaf(o.y, w, a.y), a.z = fmaf(o.z, w, a.z), a.w = fmaf(o.w, w, a.w);
+        a.x = fmaf(x.x, w, a.x), a.y = fmaf(x.y, w, a.y), a.z = fmaf(x.z, w, a.z), a.w = fmaf(x.w, w, a.w);
+        b.x = fmaf(y.x, w, b.x), b.y = fmaf(y.y, w, b.y), b.z = fmaf(y.z, w, b.z), b.w = fmaf(y.w, w, b.w);
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    reinterpret_cast<float4*>(out)[(size_t)row * hd4 + c] = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+    a = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+    b = make_float4(b.x * inv, b.y * inv, b.z * inv, b.w * inv);
+    if (op.xh) {
+        operand_store8(op, head * hd + d, tok, a, b);
+        return;
+    }
+    *reinterpret_cast<float4*>(out + (size_t)row * hd + d) = a;
+    *reinterpret_cast<float4*>(out + (size_t)row * hd + d + step) = b;
 }
 
 // Query tiles per wave and runs of keys.  Two tiles per wave where there are enough queries for both (from 49 on);
@@ -496,7 +529,7 @@ hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipSt
 #undef OXB_PF_CASE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || pl.n_splits == 1) return e;
-    const uint32_t rows = p.M * p.nq, hd4 = p.hd / 4;
-    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((uint32_t)(((uint64_t)rows * hd4 + 255) / 256)), dim3(256), 0, st, p.part, pl.n_splits, rows, hd4, p.out);
+    const uint32_t rows = p.M * p.nq;
+    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((uint32_t)(((uint64_t)((p.M + 3u) / 4u * 4u) * p.nq * (p.hd / 8) + 255) / 256)), dim3(256), 0, st, p.part, pl.n_splits, rows, p.nq, p.hd, p.out, p.op);
     return hipGetLastError();
 }

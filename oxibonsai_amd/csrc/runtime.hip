@@ -283,25 +283,33 @@ int gemv_device(const Weight& w, const float* d_x, float* d_y, uint32_t batch, u
 }
 
 int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uint32_t m, uint32_t ldy, int mode,
-                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws, OxbPackSum* carry) {
+                const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws, OxbPackSum* carry,
+                const GemmFlow& flow) {
     if (!ws) ws = &g_rt.gemm_ws;
     const uint32_t k = w.L.k;
     if ((uint64_t)m * k >= (1ull << 31))
         return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: %u rows of %u activations exceed one GEMM call", m, k);
     int rc;
-    if ((rc = ws->xh.ensure(oxb_xh_bytes(k, m)))) return rc;
-    if ((rc = ws->xsh.ensure(((size_t)m + 16) * sizeof(int32_t)))) return rc;
-    if ((rc = ws->rowmul.ensure(((size_t)m + 16) * sizeof(float)))) return rc;
-    hipError_t e = oxb_launch_xh_pack((int)w.L.fmt, pack_op, d_x, d_pack_w, ldx, k, eps, m, (float*)ws->rowmul.ptr,
-                                      (uint32_t*)ws->xh.ptr, (int32_t*)ws->xsh.ptr, g_rt.stream, pack_op == OXB_PACK_RMSNORM ? carry : nullptr);
-    if (e != hipSuccess) return hip_fail(e, "kernel launch failed: xh_pack");
+    const size_t rows4 = ((size_t)m + 16) * sizeof(int32_t);
+    hipError_t e = hipSuccess;
+    if (flow.in == GemmFlow::PACK) {
+        if ((rc = ws->xh.ensure(oxb_xh_bytes(k, m))) || (rc = ws->xsh.ensure(rows4)) || (rc = ws->rowmul.ensure(rows4))) return rc;
+        if (flow.out && (rc = ws->norm.ensure(rows4))) return rc;
+        e = oxb_launch_xh_pack((int)w.L.fmt, pack_op, d_x, d_pack_w, ldx, k, eps, m, (float*)ws->rowmul.ptr, (uint32_t*)ws->xh.ptr, (int32_t*)ws->xsh.ptr,
+                               g_rt.stream, pack_op == OXB_PACK_RMSNORM ? carry : nullptr, flow.out ? (int32_t*)ws->norm.ptr : nullptr);
+        if (e != hipSuccess) return hip_fail(e, "kernel launch failed: xh_pack");
+    } else if ((flow.in == GemmFlow::ATTENTION ? ws->xh.cap : ws->xh2.cap) < oxb_xh_bytes(k, m) || (carry && carry->n > 1))
+        return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: no operand of %u rows x %u", m, k);
+    if (flow.out && ((rc = ws->xh2.ensure(oxb_xh_bytes(w.L.n_rows / 2, m))) || (rc = ws->xsh2.ensure(rows4)))) return rc;
     if (carry) carry->n = 0;
     OxbGemmParams p;
     memset(&p, 0, sizeof p);
     p.codes = w.d_codes;
     p.scales = w.d_scales;
-    p.xh = (const uint32_t*)ws->xh.ptr;
-    p.xsh = (const int32_t*)ws->xsh.ptr;
+    p.xh = (const uint32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xh2.ptr : ws->xh.ptr);
+    p.xsh = flow.in == GemmFlow::ATTENTION ? nullptr : (const int32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xsh2.ptr : ws->xsh.ptr);
+    p.x_exp = flow.x_exp;
+    if (flow.out) p.xh_out = (uint32_t*)ws->xh2.ptr, p.xsh_out = (int32_t*)ws->xsh2.ptr, p.norm = (const int32_t*)ws->norm.ptr, p.w_exp = flow.w_exp;
     p.y = d_y;
     p.residual = d_residual;
     p.n_rows = w.L.n_rows;

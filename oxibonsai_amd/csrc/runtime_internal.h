@@ -26,8 +26,17 @@ struct DevBuf {  // grow-only device scratch
 // own that never move.
 struct GemmWorkspace {
     DevBuf xh, xsh, rowmul, part;
+    DevBuf norm, xh2, xsh2;  // GemmFlow: the rows' norms, and the operand that a SwiGLU product leaves for the next
     bool no_split = false;  // no room for partial sums: K stays in one piece
-    void release() { xh.release(); xsh.release(); rowmul.release(); part.release(); }
+    void release() { xh.release(); xsh.release(); rowmul.release(); part.release(); norm.release(); xh2.release(); xsh2.release(); }
+};
+
+// Products of a chain that hand their operands on instead of fp32 rows and a pack launch between (operand_device.h).
+struct GemmFlow {
+    enum In { PACK, ATTENTION, SWIGLU } in = PACK;  // where the operand comes from: packed here; left in xh (exponent x_exp in every row) or in xh2
+    int32_t x_exp = 0;
+    bool out = false;     // mode SWIGLU: the result goes to xh2 / xsh2, for a down projection of the same format
+    int32_t w_exp = 0;    // ... every row's 2-norm is below 2^w_exp
 };
 
 // One resident matrix: [codes section][scales section].  A weight uploaded as bytes alone (the reference's
@@ -40,6 +49,10 @@ struct Weight {
     uint16_t* d_scales = nullptr;
     void* d_raw = nullptr;
     size_t raw_blocks = 0;
+    // largest sum of squared scales of a row from row norm_row0 on (128 times that is the square of the largest 2-norm);
+    // negative: not worked out yet
+    uint32_t norm_row0 = 0;
+    float norm2 = -1.f;
 };
 
 struct Vector {  // a resident fp32 vector (norm weights)
@@ -94,7 +107,7 @@ uint32_t gemv_packed_min_batch(uint32_t k);
 // packs the same rows through RMSNorm in the same workspace, is given the same carry and adds them.
 int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uint32_t m, uint32_t ldy, int mode,
                 const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws = nullptr,
-                OxbPackSum* carry = nullptr);
+                OxbPackSum* carry = nullptr, const GemmFlow& flow = GemmFlow());
 void shutdown_models();
 
 // Every `int` entry point of the C ABI runs its body between these two, so that no C++ exception (a failed host
