@@ -418,43 +418,48 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
 }
 
 // out[t][head] = the runs' sums brought to a common exponent, added in order, over the total of their probabilities.
-// A thread owns the eight dimensions of a piece of the O projection's operand: two groups of four.
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint32_t n_splits, uint32_t rows, uint32_t nq,
+// A workgroup owns four tokens of 256 / hd heads, a thread four dimensions; as the O projection's operand the outputs change
+// places in LDS and leave in runs of four tokens.  (Reading in the operand's order instead, two times sixteen bytes 64 bytes
+// apart, takes 12 us where this takes 9: 301 tokens, six runs, 30 MB.)
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint32_t n_splits, uint32_t M, uint32_t nq,
                                                                   uint32_t hd, float* __restrict__ out, const OxbOperandOut op) {
-    // four tokens side by side, so that the pieces leave in runs of 64 bytes
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x, c = (i >> 2) % (hd / 8), j = (i >> 2) / (hd / 8);
-    const uint32_t tok = 4 * (j / nq) + (i & 3u), head = j % nq, row = tok * nq + head;
-    if (row >= rows) return;
-    const bool q1 = op.fmt == OXB_FMT_Q1;
-    const uint32_t d = 32 * (c >> 2) + (q1 ? 4 * (c & 3u) : 16 * ((c >> 1) & 1u) + 4 * (c & 1u)), step = OXB_OPERAND_STEP(op.fmt);
+    __shared__ __attribute__((aligned(16))) float o[1024];
+    const uint32_t tid = threadIdx.x, hd4 = hd / 4, c = tid % hd4, r = tid / hd4, hpg = 256 / hd;
+    const uint32_t tok = blockIdx.x * 4 + (r & 3u), head = blockIdx.y * hpg + (r >> 2);
+    const bool live = tok < M && head < nq;
+    const uint32_t rows = M * nq, row = live ? tok * nq + head : 0u;
     const float2* ml = reinterpret_cast<const float2*>(part);
-    const float* po = part + pf_part_head(n_splits, rows);
+    const float4* po = reinterpret_cast<const float4*>(part + pf_part_head(n_splits, rows));
     float m = -INFINITY;
     for (uint32_t s = 0; s < n_splits; s++) {
         const float2 v = ml[(size_t)s * rows + row];
         m = v.y == 0.f ? m : fmaxf(m, v.x);
     }
     float l = 0.f;
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
     for (uint32_t s = 0; s < n_splits; s++) {
         const float2 v = ml[(size_t)s * rows + row];
-        if (v.y == 0.f) continue;
+        if (v.y == 0.f) continue;  // (an empty run has left no outputs)
         const float w = __builtin_amdgcn_exp2f(v.x - m);
-        const float* q = po + ((size_t)s * rows + row) * hd + d;
-        const float4 x = *reinterpret_cast<const float4*>(q), y = *reinterpret_cast<const float4*>(q + step);
+        const float4 q = po[((size_t)s * rows + row) * hd4 + c];
         l = fmaf(v.y, w, l);
-        a.x = fmaf(x.x, w, a.x), a.y = fmaf(x.y, w, a.y), a.z = fmaf(x.z, w, a.z), a.w = fmaf(x.w, w, a.w);
-        b.x = fmaf(y.x, w, b.x), b.y = fmaf(y.y, w, b.y), b.z = fmaf(y.z, w, b.z), b.w = fmaf(y.w, w, b.w);
+        a.x = fmaf(q.x, w, a.x), a.y = fmaf(q.y, w, a.y), a.z = fmaf(q.z, w, a.z), a.w = fmaf(q.w, w, a.w);
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     a = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
-    b = make_float4(b.x * inv, b.y * inv, b.z * inv, b.w * inv);
-    if (op.xh) {
-        operand_store8(op, head * hd + d, tok, a, b);
+    if (!op.xh) {
+        if (live) reinterpret_cast<float4*>(out)[(size_t)row * hd4 + c] = a;
         return;
     }
-    *reinterpret_cast<float4*>(out + (size_t)row * hd + d) = a;
-    *reinterpret_cast<float4*>(out + (size_t)row * hd + d + step) = b;
+    reinterpret_cast<float4*>(o)[tid] = a;
+    __syncthreads();
+    if (tid >= 128) return;
+    // piece i >> 2 of the heads' values for token i % 4
+    const uint32_t t = blockIdx.x * 4 + (tid & 3u), i = tid >> 2, hl = i / (hd / 8), e = i % (hd / 8), h = blockIdx.y * hpg + hl;
+    if (t >= M || h >= nq) return;
+    const uint32_t d = 32 * (e >> 2) + (op.fmt == OXB_FMT_Q1 ? 4 * (e & 3u) : 16 * ((e >> 1) & 1u) + 4 * (e & 1u));
+    const float* q = o + (hl * 4 + (tid & 3u)) * hd + d;
+    operand_store8(op, h * hd + d, t, *reinterpret_cast<const float4*>(q), *reinterpret_cast<const float4*>(q + OXB_OPERAND_STEP(op.fmt)));
 }
 
 // Query tiles per wave and runs of keys.  Two tiles per wave where there are enough queries for both (from 49 on);
@@ -529,7 +534,7 @@ hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipSt
 #undef OXB_PF_CASE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || pl.n_splits == 1) return e;
-    const uint32_t rows = p.M * p.nq;
-    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((uint32_t)(((uint64_t)((p.M + 3u) / 4u * 4u) * p.nq * (p.hd / 8) + 255) / 256)), dim3(256), 0, st, p.part, pl.n_splits, rows, p.nq, p.hd, p.out, p.op);
+    const uint32_t hpg = 256 / p.hd;
+    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((p.M + 3) / 4, (p.nq + hpg - 1) / hpg), dim3(256), 0, st, p.part, pl.n_splits, p.M, p.nq, p.hd, p.out, p.op);
     return hipGetLastError();
 }
