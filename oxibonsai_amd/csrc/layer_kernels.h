@@ -7,19 +7,17 @@
 #include "kv_quant_device.h"
 #include "operand_device.h"
 
-struct OxbQkParams {
-    const float* qkv;      // [batch][qkv_stride]: q heads | k heads | v heads
-    uint32_t qkv_stride;
-    const float *q_norm, *k_norm;  // [hd]
+struct OxbKvStoreParams {
+    const float* qkv;              // [M][qkv_stride]: q heads | k heads | v heads, of positions pos_base .. of sequence `seq`
+    uint32_t qkv_stride, M;
+    const float* k_norm;           // [hd]
     const float *cos_t, *sin_t;    // [max_seq][hd/2]
-    const uint32_t* pos;           // [batch], device; null: row b is token pos_base + b of sequence `seq` (prefill)
     uint32_t pos_base, seq;
-    float* q_rope;                 // [batch][nq][hd]
     void *k_cache, *v_cache;       // cache rows of hd values each (fp16, or one-byte codes: kv_mode), placed by `kv`
     float *k_scale, *v_scale;      // quantised cache: one scale per row
     uint32_t kv_mode;
     OxbKvLayout kv;
-    uint32_t nq, nkv, hd, max_seq, n_layers, layer;
+    uint32_t nq, nkv, hd, layer;
     float eps;
 };
 
@@ -57,7 +55,7 @@ hipError_t oxb_launch_kv_dequantize_rows(int kv_mode, const uint8_t* d_codes, co
                                          float* d_out, hipStream_t st);
 hipError_t oxb_launch_kv_quantize_rows(int kv_mode, const float* d_x, uint32_t n_rows, uint32_t n, uint8_t* d_codes, float* d_scales,
                                        hipStream_t st);
-hipError_t oxb_launch_qk_norm_rope_store(const OxbQkParams& p, uint32_t batch, hipStream_t st);
+hipError_t oxb_launch_kv_norm_rope_store(const OxbKvStoreParams& p, hipStream_t st);
 #define OXB_ATTN_CHUNK_POSITIONS 128  // KV positions a four-wave attention workgroup covers at a time
 #define OXB_ATTN_MAX_SPLITS 64        // slots the KV sequence is split over; slot s walks chunks s, s + n_splits, ...
 #define OXB_ATTN_PART_PAD 4           // floats after the hd outputs of a slot: maximum, sum, 2 unused (16-byte rows)

@@ -18,122 +18,87 @@
 #include "gemv_pack_device.h"
 
 // ---------------------------------------------------------------------------
-// Per-head QK-RMSNorm + half-split RoPE + KV store (fp16, or quantised rows: kv_quant_device.h)
+// The new K and V rows of a prefill: K per-head RMSNorm + half-split RoPE, V as it is, to the cache rows of positions
+// pos_base + t (fp16 round-to-nearest-even, or quantised: kv_quant_device.h).
 // (fused_qk_norm_rope + fused_kv_store, gpu_backend/cuda_attn_kernels.rs:160-251;
-//  CPU: block/types/forward.rs:179-213, rope pairs (d, d + hd/2) simd_float_ops.rs:240-253).
-// Grid (head groups, rows); block = 256 threads = 4 waves, a wave takes OXB_QK_HEADS_PER_WAVE heads of one row one
-// after the other: a lane holds the rotation pairs (d, d + hd/2) for d = lane, lane + 64, every reduction stays inside
-// the wave.  Q heads go to q_rope (fp32), K heads (after RoPE) and the raw V head go to the cache row of position
-// pos[b], rounded to f16 (round-to-nearest-even) or quantised.
+//  CPU: block/types/forward.rs:179-213, rope pairs (d, d + hd/2) simd_float_ops.rs:240-253; the attention kernel norms and
+//  rotates Q itself.)
+// hd / 4 lanes hold a head's row, four values each, so that a wave takes 256 / hd heads of a token side by side; everything it
+// needs is requested at once.  What bounds it is that one round trip to memory (few tokens) and the way there and back
+// (2048 tokens x 8 heads: 25 MB).  Two heads a wave one after the other, a value per lane and request, took 5.0 us for 23 tokens,
+// 6.9 for 301 with INT8 rows and 9.0 to 10 for 2048; this form 2.8, 5.0 and 5.7 (kernel traces).
 // ---------------------------------------------------------------------------
-#define OXB_QK_HEADS_PER_WAVE 2
-template <int KVM>
-__global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(OxbQkParams p) {
-    constexpr bool QC = KVM != OXB_KV_F16;
-    constexpr int KI = 2, VI = 4;  // pairs / values per lane at head_dim 256
-    const uint32_t b = blockIdx.y, lane = threadIdx.x & 63u, hd = p.hd, half = hd >> 1;
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t pos = p.pos ? p.pos[b] : p.pos_base + b;
-    const uint32_t seq = p.pos ? b : p.seq;
-    const float* row_in = p.qkv + (size_t)b * p.qkv_stride;
-    float cs[KI], sn[KI];
-#pragma unroll
-    for (int it = 0; it < KI; it++) {
-        const uint32_t d = lane + 64 * it;
-        cs[it] = d < half ? p.cos_t[(size_t)pos * half + d] : 0.f;
-        sn[it] = d < half ? p.sin_t[(size_t)pos * half + d] : 0.f;
+// The sum / largest over groups of L lanes, in every lane.
+template <int L>
+__device__ __forceinline__ float group_sum(float v) {
+    v += dpp_f32<0xB1>(v);
+    v += dpp_f32<0x4E>(v);
+    v += dpp_f32<0x141>(v);
+    if constexpr (L >= 16) v += dpp_f32<0x140>(v);
+    if constexpr (L >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
     }
-    // without a q_rope buffer only the K and V heads are handled (the consumer of Q does its own norm + RoPE)
-    const uint32_t first_head = p.q_rope ? 0u : p.nq;
-    const uint32_t head0 = first_head + (blockIdx.x * 4 + wave) * OXB_QK_HEADS_PER_WAVE;
+    if constexpr (L >= 64) {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    return v;
+}
+template <int L>
+__device__ __forceinline__ float group_max(float v) {
+    v = fmaxf(v, dpp_f32<0xB1>(v));
+    v = fmaxf(v, dpp_f32<0x4E>(v));
+    v = fmaxf(v, dpp_f32<0x141>(v));
+    if constexpr (L >= 16) v = fmaxf(v, dpp_f32<0x140>(v));
+    if constexpr (L >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    }
+    if constexpr (L >= 64) {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    }
+    return v;
+}
+
+template <int HD, int KVM>
+__global__ __launch_bounds__(256) void kv_norm_rope_store_kernel(OxbKvStoreParams p) {
+    constexpr int L = HD / 4, HPW = 64 / L;  // lanes of a head, heads of a wave
+    const uint32_t lane = threadIdx.x & 63u, j = lane % L;
+    const uint32_t n_hg = (p.nkv + HPW - 1) / HPW, id = blockIdx.x * 4 + (threadIdx.x >> 6);  // (token, group of heads)
+    const uint32_t t = id / n_hg, head = (id % n_hg) * HPW + lane / L;
+    if (t >= p.M || head >= p.nkv) return;  // (whole groups of lanes)
+    const uint32_t pos = p.pos_base + t, at = (4 * j) % (HD / 2);  // the pair's place
+    const float* row_in = p.qkv + (size_t)t * p.qkv_stride + (size_t)(p.nq + head) * HD + 4 * j;
+    const float4 k = *reinterpret_cast<const float4*>(row_in), v = *reinterpret_cast<const float4*>(row_in + (size_t)p.nkv * HD);
+    const float4 w = *reinterpret_cast<const float4*>(p.k_norm + 4 * j);
+    const float4 cs = *reinterpret_cast<const float4*>(p.cos_t + (size_t)pos * (HD / 2) + at), sn = *reinterpret_cast<const float4*>(p.sin_t + (size_t)pos * (HD / 2) + at);
+    const size_t row = kv_row(p.kv, p.seq, p.layer, head, pos);
+    const float ss = group_sum<L>(fmaf(k.x, k.x, fmaf(k.y, k.y, fmaf(k.z, k.z, k.w * k.w))));
+    const float inv_rms = 1.0f / sqrtf(ss / (float)HD + p.eps);
+    const float a[4] = {w.x * k.x * inv_rms, w.y * k.y * inv_rms, w.z * k.z * inv_rms, w.w * k.w * inv_rms};
+    const float c4[4] = {cs.x, cs.y, cs.z, cs.w}, s4[4] = {sn.x, sn.y, sn.z, sn.w}, v4[4] = {v.x, v.y, v.z, v.w};
+    float o[4];
 #pragma unroll
-    for (uint32_t j = 0; j < OXB_QK_HEADS_PER_WAVE; j++) {
-        const uint32_t head = head0 + j;
-        if (head >= p.nq + p.nkv) break;  // wave-uniform
-        const bool is_q = head < p.nq;
-        const uint32_t hh = is_q ? head : head - p.nq;
-        const float* in = row_in + (size_t)head * hd;  // q heads, then k heads
-        const float* w = is_q ? p.q_norm : p.k_norm;
-        float lo[KI], hi[KI], ss = 0.f;
+    for (int i = 0; i < 4; i++) {
+        const float other = __shfl_xor(a[i], L / 2, 64);
+        o[i] = j < L / 2 ? a[i] * c4[i] - other * s4[i] : other * s4[i] + a[i] * c4[i];
+    }
+    if constexpr (KVM != OXB_KV_F16) {
+        const float kmax = group_max<L>(fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3]))));
+        const float vmax = group_max<L>(fmaxf(fmaxf(fabsf(v4[0]), fabsf(v4[1])), fmaxf(fabsf(v4[2]), fabsf(v4[3]))));
+        const float ks = kv_row_scale<KVM>(kmax), vs = kv_row_scale<KVM>(vmax);
+        uint32_t kw = 0, vw = 0;
 #pragma unroll
-        for (int it = 0; it < KI; it++) {
-            const uint32_t d = lane + 64 * it;
-            lo[it] = d < half ? in[d] : 0.f;
-            hi[it] = d < half ? in[d + half] : 0.f;
-            ss = fmaf(lo[it], lo[it], fmaf(hi[it], hi[it], ss));
-        }
-        ss = wave_sum_f32(ss);
-        const float inv_rms = 1.0f / sqrtf(ss / (float)hd + p.eps);
-        float o_lo[KI], o_hi[KI], kmax = 0.f;
-#pragma unroll
-        for (int it = 0; it < KI; it++) {
-            const uint32_t d = lane + 64 * it;
-            const float a = d < half ? w[d] * lo[it] * inv_rms : 0.f, c = d < half ? w[d + half] * hi[it] * inv_rms : 0.f;
-            o_lo[it] = a * cs[it] - c * sn[it];
-            o_hi[it] = a * sn[it] + c * cs[it];
-            kmax = fmaxf(kmax, fmaxf(fabsf(o_lo[it]), fabsf(o_hi[it])));
-        }
-        if (is_q) {
-            float* q = p.q_rope + ((size_t)b * p.nq + hh) * hd;
-#pragma unroll
-            for (int it = 0; it < KI; it++) {
-                const uint32_t d = lane + 64 * it;
-                if (d < half) q[d] = o_lo[it], q[d + half] = o_hi[it];
-            }
-            continue;
-        }
-        const size_t row = kv_row(p.kv, seq, p.layer, hh, pos), cache_off = row * hd;
-        const float* v = row_in + (size_t)(p.nq + p.nkv + hh) * hd;
-        float vv[VI], vmax = 0.f;
-#pragma unroll
-        for (int it = 0; it < VI; it++) {
-            const uint32_t d = lane + 64 * it;
-            vv[it] = d < hd ? v[d] : 0.f;
-            vmax = fmaxf(vmax, fabsf(vv[it]));
-        }
-        if constexpr (QC) {
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                kmax = fmaxf(kmax, __shfl_xor(kmax, o, 64));
-                vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
-            }
-            const float ks = kv_row_scale<KVM>(kmax), vs = kv_row_scale<KVM>(vmax);
-            uint8_t* kc = reinterpret_cast<uint8_t*>(p.k_cache) + cache_off;
-            uint8_t* vc = reinterpret_cast<uint8_t*>(p.v_cache) + cache_off;
-#pragma unroll
-            for (int it = 0; it < KI; it++) {
-                const uint32_t d = lane + 64 * it;
-                if (d < half) {
-                    kc[d] = (uint8_t)kv_encode<KVM>(o_lo[it], ks);
-                    kc[d + half] = (uint8_t)kv_encode<KVM>(o_hi[it], ks);
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < VI; it++) {
-                const uint32_t d = lane + 64 * it;
-                if (d < hd) vc[d] = (uint8_t)kv_encode<KVM>(vv[it], vs);
-            }
-            if (lane == 0) {
-                p.k_scale[row] = ks;
-                p.v_scale[row] = vs;
-            }
-        } else {
-            __half* kc = reinterpret_cast<__half*>(p.k_cache) + cache_off;
-            __half* vc = reinterpret_cast<__half*>(p.v_cache) + cache_off;
-#pragma unroll
-            for (int it = 0; it < KI; it++) {
-                const uint32_t d = lane + 64 * it;
-                if (d < half) {
-                    kc[d] = __float2half_rn(o_lo[it]);
-                    kc[d + half] = __float2half_rn(o_hi[it]);
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < VI; it++) {
-                const uint32_t d = lane + 64 * it;
-                if (d < hd) vc[d] = __float2half_rn(vv[it]);
-            }
-        }
+        for (int i = 0; i < 4; i++) kw |= kv_encode<KVM>(o[i], ks) << (8 * i), vw |= kv_encode<KVM>(v4[i], vs) << (8 * i);
+        reinterpret_cast<uint32_t*>(p.k_cache)[row * L + j] = kw;
+        reinterpret_cast<uint32_t*>(p.v_cache)[row * L + j] = vw;
+        if (j == 0) p.k_scale[row] = ks, p.v_scale[row] = vs;
+    } else {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        reinterpret_cast<h4*>(p.k_cache)[row * L + j] = (h4){(_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3]};
+        reinterpret_cast<h4*>(p.v_cache)[row * L + j] = (h4){(_Float16)v4[0], (_Float16)v4[1], (_Float16)v4[2], (_Float16)v4[3]};
     }
 }
 
@@ -931,13 +896,25 @@ hipError_t oxb_launch_stage_in(const float* h_hidden, uint32_t n_floats, const u
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-hipError_t oxb_launch_qk_norm_rope_store(const OxbQkParams& p, uint32_t batch, hipStream_t st) {
-    if (p.hd > 256 || p.kv_mode > OXB_KV_FP8_E4M3 || (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale))) return hipErrorInvalidValue;
-    const uint32_t per_wg = 4 * OXB_QK_HEADS_PER_WAVE;
-    const dim3 grid(((p.q_rope ? p.nq : 0u) + p.nkv + per_wg - 1) / per_wg, batch), block(256);
-    if (p.kv_mode == OXB_KV_I8) hipLaunchKernelGGL(qk_norm_rope_store_kernel<OXB_KV_I8>, grid, block, 0, st, p);
-    else if (p.kv_mode == OXB_KV_FP8_E4M3) hipLaunchKernelGGL(qk_norm_rope_store_kernel<OXB_KV_FP8_E4M3>, grid, block, 0, st, p);
-    else hipLaunchKernelGGL(qk_norm_rope_store_kernel<OXB_KV_F16>, grid, block, 0, st, p);
+hipError_t oxb_launch_kv_norm_rope_store(const OxbKvStoreParams& p, hipStream_t st) {
+    if (p.kv_mode > OXB_KV_FP8_E4M3 || (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale)) || (p.qkv_stride & 3u)) return hipErrorInvalidValue;
+#define OXB_KV_STORE(HD_)                                                                                                                       \
+    case HD_: {                                                                                                                                 \
+        constexpr uint32_t hpw = 256 / HD_;                                                                                                     \
+        const dim3 grid((uint32_t)(((uint64_t)p.M * ((p.nkv + hpw - 1) / hpw) + 3) / 4)), block(256);                                           \
+        if (p.kv_mode == OXB_KV_I8) hipLaunchKernelGGL((kv_norm_rope_store_kernel<HD_, OXB_KV_I8>), grid, block, 0, st, p);                     \
+        else if (p.kv_mode == OXB_KV_FP8_E4M3) hipLaunchKernelGGL((kv_norm_rope_store_kernel<HD_, OXB_KV_FP8_E4M3>), grid, block, 0, st, p);    \
+        else hipLaunchKernelGGL((kv_norm_rope_store_kernel<HD_, OXB_KV_F16>), grid, block, 0, st, p);                                           \
+        break;                                                                                                                                  \
+    }
+    switch (p.hd) {
+        OXB_KV_STORE(32)
+        OXB_KV_STORE(64)
+        OXB_KV_STORE(128)
+        OXB_KV_STORE(256)
+        default: return hipErrorInvalidValue;
+    }
+#undef OXB_KV_STORE
     return hipGetLastError();
 }
 

@@ -590,17 +590,15 @@ static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t
                                     const float* k_norm, float* out, const OxbOperandOut* op = nullptr) {
     const oxb_model_desc& d = m.d;
     hipStream_t st = g_rt.stream;
-    OxbQkParams qp;
+    OxbKvStoreParams qp;
     qp.qkv = qkv;
     qp.qkv_stride = (d.nq + 2 * d.nkv) * d.hd;
-    qp.q_norm = q_norm;
+    qp.M = M;
     qp.k_norm = k_norm;
     qp.cos_t = m.cos_t;
     qp.sin_t = m.sin_t;
-    qp.pos = nullptr;
     qp.pos_base = pos_start;
     qp.seq = seq;
-    qp.q_rope = nullptr;  // the attention kernel norms and rotates Q itself
     qp.k_cache = m.k_cache;
     qp.v_cache = m.v_cache;
     qp.k_scale = m.k_scale;
@@ -610,11 +608,9 @@ static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t
     qp.nq = d.nq;
     qp.nkv = d.nkv;
     qp.hd = d.hd;
-    qp.max_seq = d.max_seq;
-    qp.n_layers = d.n_layers;
     qp.layer = L;
     qp.eps = d.eps;
-    OXB_TRY_HIP(oxb_launch_qk_norm_rope_store(qp, M, st), "kernel launch failed: qk_norm_rope_store");
+    OXB_TRY_HIP(oxb_launch_kv_norm_rope_store(qp, st), "kernel launch failed: kv_norm_rope_store");
     OxbPrefillAttnParams ap;
     ap.qkv = qkv;
     ap.qkv_stride = qp.qkv_stride;
