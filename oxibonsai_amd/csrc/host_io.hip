@@ -4,8 +4,8 @@
 // or pins the pages for the transfer: 14 / 22 us for 4 KB in / out, 110 us for 256 KB, 18 GB/s out of the device for
 // large results.  Here every transfer goes through pinned memory that the library keeps and is made by a small kernel in the
 // caller's stream, so no copy engine has to be synchronised with it.  The host's side of it is a copy by several threads
-// (CopyTeam): one moves 28 to 33 GB/s to or from memory that the bus has written or will read, less than the bus itself.  The last transfer of a call raises a flag in pinned memory that the host polls:
-// three dependent launches and a poll take 12.6 us where the same three and hipStreamSynchronize take 18.
+// (CopyTeam): one moves 28 to 33 GB/s to or from memory that the bus has written or will read, less than the bus itself.  The
+// last transfer of a call raises a flag in pinned memory that the host polls: three dependent launches and a poll take 12.6 us where the same three and hipStreamSynchronize take 18.
 #include <hip/hip_runtime.h>
 
 #include <signal.h>
@@ -61,11 +61,14 @@ constexpr size_t kPoolKept = (size_t)128 << 20; // ... and kept for reuse
 // GEMV: 17.5 us at the median, 40 to 85 for one call in 256, 17.9 on average).
 constexpr uint32_t kSyncEvery = 256;
 
-// Copies of more than kSlice bytes, shared with up to kHelpers threads of the library's own.  The caller takes slices like
-// the helpers and is done when all slices are, so a helper that wakes late costs nothing; a helper looks out for the next
-// copy for kLinger and then sleeps.  Used under the library's lock, by one call at a time; io_shutdown ends the threads.
+// The copies of a transfer of more than kShared bytes, shared with up to kHelpers threads of the library's own.  The caller takes
+// slices like the helpers and is done when all slices are, so a helper that wakes late costs nothing; a helper looks out for the
+// next copy for kLinger and then sleeps.  Used under the library's lock, by one call at a time; io_shutdown ends the threads.
 // One thread -> four: 1.3 MB in and out 130 -> 112 us (77 x 4096 GEMM, host to host), 19 MB out 3.62 -> 3.40 ms (decode of
-// 32 sequences), 34 MB in 27.4 -> 26.8 ms (2048-token prefill).  Up to kSlice the copy takes 2 us, less than waking a thread.
+// 32 sequences), 34 MB in 27.4 -> 26.8 ms (2048-token prefill).  Waking them costs the caller 0.5 to 3 us:
+// shared from 64 KB on, a product with 131 KB in and out takes 33.0 us instead of 30.2, with 196 KB 37.3 instead of 37.0; with
+// 262 KB it takes 42.8 instead of 43.1, with 328 KB 50.9 instead of 49.4, with 393 KB 48.5 instead of 53.6.
+constexpr size_t kShared = (size_t)320 << 10;
 constexpr size_t kSlice = (size_t)64 << 10;
 constexpr unsigned kHelpers = 3;
 constexpr auto kLinger = std::chrono::microseconds(60);
@@ -109,8 +112,8 @@ class CopyTeam {
     }
 
 public:
-    void copy(void* dst, const void* src, size_t bytes) {
-        if (bytes > kSlice && !started) {
+    void copy(void* dst, const void* src, size_t bytes, bool share) {
+        if (share && !started) {
             started = true;
             sigset_t all, before;  // the program's signals stay with its own threads
             sigfillset(&all);
@@ -122,7 +125,7 @@ public:
             }
             pthread_sigmask(SIG_SETMASK, &before, nullptr);
         }
-        if (bytes <= kSlice || threads.empty()) {
+        if (!share || bytes <= kSlice || threads.empty()) {
             memcpy(dst, src, bytes);
             return;
         }
@@ -155,7 +158,7 @@ struct Staging {
     uint8_t *in = nullptr, *out = nullptr;
     size_t in_cap = 0, out_cap = 0, in_used = 0, out_used = 0;
     uint32_t *flag = nullptr, *arrived = nullptr, seq = 0, seq_begin = 0, calls = 0;
-    struct Late { void* dst; size_t at, bytes; uint32_t seq; };
+    struct Late { void* dst; size_t at, bytes; uint32_t seq; bool share; };
     std::vector<Late> late;  // results that wait in staging for the device
 } st;
 
@@ -275,6 +278,7 @@ int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
     if (((uintptr_t)s & 15) == 0 && is_pinned(s, bytes)) return copy(s, d, bytes, nullptr, 0);
     int rc;
     if (st.in_used == 0 && (rc = staging(&st.in, &st.in_cap, bytes))) return rc;
+    const bool share = bytes > kShared;
     while (bytes) {
         const size_t n = bytes < kChunk ? bytes : kChunk;
         if (st.in_used + n > st.in_cap) {  // every piece has been used once: wait for the device to be done with them
@@ -282,7 +286,7 @@ int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
             st.in_used = 0;
             if ((rc = staging(&st.in, &st.in_cap, bytes))) return rc;
         }
-        team.copy(st.in + st.in_used, s, n);
+        team.copy(st.in + st.in_used, s, n, share);
         if ((rc = copy(st.in + st.in_used, d, n, nullptr, 0))) return rc;
         st.in_used += (n + 255) & ~(size_t)255;
         s += n, d += n, bytes -= n;
@@ -294,19 +298,20 @@ int IoCall::download(void* dst, const void* d_src, size_t bytes) {
     if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, st.flag, ++st.seq);
     int rc;
     if (st.out_used == 0 && (rc = staging(&st.out, &st.out_cap, bytes))) return rc;
+    const bool share = bytes > kShared;
     uint8_t* d = (uint8_t*)dst;
     const uint8_t* s = (const uint8_t*)d_src;
     while (bytes) {
         const size_t n = bytes < kChunk ? bytes : kChunk;
         if (st.out_used + n > st.out_cap) {  // staging is full of results: hand them over first
             if ((rc = sync_all("output download"))) return rc;
-            for (const Staging::Late& l : st.late) team.copy(l.dst, st.out + l.at, l.bytes);
+            for (const Staging::Late& l : st.late) team.copy(l.dst, st.out + l.at, l.bytes, l.share);
             st.late.clear();
             st.out_used = 0;
             if ((rc = staging(&st.out, &st.out_cap, bytes))) return rc;
         }
         if ((rc = copy(s, st.out + st.out_used, n, st.flag, ++st.seq))) return rc;
-        st.late.push_back({d, st.out_used, n, st.seq});
+        st.late.push_back({d, st.out_used, n, st.seq, share});
         st.out_used += (n + 255) & ~(size_t)255;
         s += n, d += n, bytes -= n;
     }
@@ -318,7 +323,7 @@ int IoCall::finish(const char* what) {
     if (st.seq == st.seq_begin && (rc = sync_all(what))) return rc;  // nothing came back
     for (const Staging::Late& l : st.late) {  // one piece is copied on the host while the next ones cross the bus
         if ((rc = wait_for(l.seq, what))) return rc;
-        team.copy(l.dst, st.out + l.at, l.bytes);
+        team.copy(l.dst, st.out + l.at, l.bytes, l.share);
     }
     st.late.clear();
     if ((rc = wait_for(st.seq, what))) return rc;
