@@ -37,15 +37,6 @@ __device__ __forceinline__ float max_rows4(float v) {
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-// The larger of two as the median with +infinity: fmaxf makes the compiler quiet every operand that comes from a matrix
-// instruction or a lane swap first, an instruction each.  A NaN is passed over where the other operand is a number.
-__device__ __forceinline__ float max_raw(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
-__device__ __forceinline__ float max_rows4_raw(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = max_raw(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return max_raw(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 __device__ __forceinline__ float wave_sum_f32(float v) {
     v += dpp_f32<0xB1>(v);
     v += dpp_f32<0x4E>(v);

@@ -41,11 +41,18 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // wait in registers and are widened on their way.  Rows are stored without padding, their 16-byte pieces permuted by an
 // XOR with the row number, which keeps both kinds of read free of bank conflicts.
 //
-// What bounds it: the SIMDs' issue slots.  With 16 queries per wave and 32-key blocks the kernel issued about 200 vector
-// instructions around 24 MFMAs per block.  Two query tiles per wave halve the LDS reads per MFMA; the accumulators of a tile
-// are rescaled only in blocks that bring a new maximum for one of its 16 queries; the visibility tests run only in blocks that
-// some query of the wave sees in part.  Per layer of the 8B shape, in a kernel trace: 90 us for 2048 tokens, 86 us (and 9 for
-// the merge) for 301 tokens behind 6000 INT8 positions.
+// What bounds it: the SIMDs' issue slots, where there are workgroups for the chip, and the latency of a block's chain of reads,
+// products, maximum and products where there are not.  Two forms:
+//  - QT = 1: one query tile per wave, 93 registers (head_dim 64) to 138 (128, one-byte rows), so three or four waves of a SIMD
+//    fill each other's waits.
+//  - QT = 2 (head_dim 128): two tiles share every K and V operand, which halves the LDS reads and the widening of one-byte rows
+//    per product, and 64-key blocks halve the maxima.  That takes the registers of two waves per SIMD and the LDS of a CU: the
+//    eight waves are two walkers, four waves each, that take the blocks in turn and add their sums in LDS at the end.
+// In both the scores start from -m (the products' C operand), so a block without a new maximum for any query of a tile costs no
+// rescaling, and the visibility tests run only in blocks that some query of the wave sees in part.
+// us per layer, 32 q heads and 8 kv heads of 128, merge included, one form for all (two tiles, four waves) -> these two:
+// fp16 rows, 100 tokens 12.6 -> 9.6, 300 18.7 -> 15.8, 1000 43.8 -> 34.0, 2048 88 -> 73, 32 behind 6000 31.9 -> 26.8; INT8 rows,
+// 300 behind 6000 93 -> 81, 2048 behind 6000 459 -> 426.  Heads of 64: 1400 behind 4000 161 -> 112.
 //
 // Options as in the decode attention: quantised cache rows (template KVM; the codes are widened to exact fp16
 // numbers on their way into LDS, V already multiplied by its row scale there, the K row scale multiplies the
@@ -65,26 +72,31 @@ __device__ __forceinline__ void swap_upper_lower(float& a, float& b) {
 // p.part: maximum and sum of every (run, query, head), then from a 16-byte boundary on their outputs.
 __host__ __device__ constexpr size_t pf_part_head(size_t n_splits, size_t rows) { return (n_splits * rows * 2 + 3) & ~(size_t)3; }
 
-// Keys per block: 64, or 32 where the LDS (4 x KB x 2 HD bytes) or the registers that hold a block of codes leave no room.
-constexpr int pf_block_keys(int hd, bool quantised) { return hd == 256 || (hd == 128 && quantised) ? 32 : 64; }
+// Keys per block: 64, or 32 where four (head_dim 128) or two (256) workgroups to a CU share its LDS, 4 x KB x 2 HD bytes each.
+constexpr int pf_block_keys(int hd, int qt) { return hd == 256 || (hd == 128 && qt == 1) ? 32 : 64; }
 
 template <int HD, int KVM, bool OPT, int QT>  // OPT: a window and / or a paged cache may be in use (else neither costs anything)
-__global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(OxbPrefillAttnParams p, uint32_t hpw) {
+__global__ __launch_bounds__(256 * QT, HD == 256 ? 1 : 2) void attn_prefill_kernel(OxbPrefillAttnParams p, uint32_t hpw) {
     constexpr bool QC = KVM != OXB_KV_F16;
-    constexpr int KS = HD / 32, NS = HD / 16, KB = pf_block_keys(HD, QC);
+    constexpr int WK = QT;                                           // walkers: groups of four waves that take the keys' blocks in turn
+    constexpr int KS = HD / 32, NS = HD / 16, KB = pf_block_keys(HD, QT);
     constexpr int RPW = KB / 4;                                      // rows of a block that a wave fetches
     constexpr int PPR = HD / 8;                                      // 16-byte pieces of an LDS row
     constexpr int RB = PPR >= 16 ? 1 : 16 / PPR, PM = (PPR < 16 ? PPR : 16) - 1;  // rows per 256 bytes; mask of the permutation
     constexpr int NI = QC ? (RPW * HD / 16 + 63) / 64 : RPW * PPR / 64;  // 16-byte pieces per lane and block, of K and of V
-    __shared__ __attribute__((aligned(16))) _Float16 ks0[KB * HD], ks1[KB * HD], vs0[KB * HD], vs1[KB * HD];
-    __shared__ __attribute__((aligned(16))) float kscale0[KB], kscale1[KB];  // K row scales of the block (quantised cache)
+    __shared__ __attribute__((aligned(16))) _Float16 ks0_all[WK * KB * HD], ks1_all[WK * KB * HD], vs0_all[WK * KB * HD], vs1_all[WK * KB * HD];
+    __shared__ __attribute__((aligned(16))) float kscale0_all[WK * KB], kscale1_all[WK * KB];  // K row scales of the block (quantised cache)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, qi = lane & 15u, g = lane >> 4;
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t wave8 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), wave = wave8 & 3u, walker = WK == 1 ? 0u : wave8 >> 2;
+    _Float16 *const ks0 = ks0_all + walker * (KB * HD), *const ks1 = ks1_all + walker * (KB * HD);
+    _Float16 *const vs0 = vs0_all + walker * (KB * HD), *const vs1 = vs1_all + walker * (KB * HD);
+    float *const kscale0 = kscale0_all + walker * KB, *const kscale1 = kscale1_all + walker * KB;
     const uint32_t tpw = 4u / hpw, n_qt = (p.M + 15u) / 16u, per_wg = tpw * QT, n_tg = (n_qt + per_wg - 1) / per_wg, hq = p.nq / hpw;
-    // Late query tiles walk more keys than early ones.  Workgroups are handed out in order, one to a CU, then a second
-    // one to each: the first half of the tiles goes from the latest down, the second half from the earliest up, so that the
-    // longest walk shares its CU with the shortest.
-    const uint32_t tb = blockIdx.x / hq, tg = 2 * tb < n_tg ? n_tg - 1 - tb : tb - (n_tg + 1) / 2;
+    // Late query tiles walk more keys than early ones.  With two walkers a CU holds one workgroup, and takes the next one when it
+    // is done: the longest walks go first.  Else workgroups are handed out in order, one to a CU, then a second one to each, and
+    // so on: the first half of the tiles goes from the latest down, the second half from the earliest up, so that the longest
+    // walk shares its CU with the shortest.
+    const uint32_t tb = blockIdx.x / hq, tg = WK == 2 || 2 * tb < n_tg ? n_tg - 1 - tb : tb - (n_tg + 1) / 2;
     const uint32_t head = (blockIdx.x % hq) * hpw + wave % hpw;
     const uint32_t kvh = head / (p.nq / p.nkv);                           // the same for the four waves
     const uint32_t t_first = (tg * per_wg + (wave / hpw) * QT) * 16;      // first query of this wave
@@ -156,8 +168,8 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
         }
         if constexpr (QC) ksreg = p.k_scale[row + min(lane & (RPW - 1), lim)];
     };
-    auto deliver = [&](_Float16* kd, _Float16* vd, float* scd) {
-        if constexpr (QC) {
+    auto deliver = [&](_Float16* kd, _Float16* vd, float* scd, bool there) {
+        if (QC && there) {
             uint32_t l = lane;
             asm volatile("" : "+v"(l));
 #pragma unroll
@@ -189,7 +201,9 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
         // the barrier that ends a block: every wave has read it, and the next one is complete in LDS
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
-    if (i0 < i1) request(key_of(i0), ks0, vs0);
+    const uint32_t steps = i0 < i1 ? (i1 - i0 + WK - 1) / WK : 0u;  // the same for both walkers: they meet at every barrier
+    auto mine = [&](uint32_t j) -> uint32_t { return i0 + j * WK + walker; };
+    if (mine(0) < i1) request(key_of(mine(0)), ks0, vs0);
 
     // Q of this lane's queries: per-head RMSNorm, RoPE on the pairs (d, d + hd/2), times log2(e)/sqrt(hd)
     // (fused_qk_norm_rope, gpu_backend/cuda_attn_kernels.rs:160-226), then split into fp16 hi + lo.  The lane holds
@@ -256,127 +270,204 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
     const uint32_t k_at = (qi * PPR + (g ^ ((qi / RB) & PM))) * 8;
     const uint32_t v_row = 4 * g + (qi >> 2), v_at = (v_row * PPR + (((qi >> 1) & 1u) ^ ((v_row / RB) & PM))) * 8 + (qi & 1u) * 4;
     v4f O[QT][NS];
-    float m_run[QT], lsum[QT];  // running maximum of the tile's queries; this lane's share of the sum of their probabilities
+    // The running maximum m of the tile's queries: -m, which the scores start from (fp16 rows: the score products' C operand;
+    // quantised ones: the addend of the row scale), and `seen`, 0 once there is one and -infinity before.  This lane's share
+    // of the sum of the probabilities.
+    v4f neg_m[QT];
+    float seen[QT], lsum[QT];
 #pragma unroll
     for (int t = 0; t < QT; t++) {
 #pragma unroll
         for (int i = 0; i < NS; i++) O[t][i] = (v4f){0.f, 0.f, 0.f, 0.f};
+        neg_m[t] = (v4f){0.f, 0.f, 0.f, 0.f};
         lsum[t] = 0.f;
-        m_run[t] = -INFINITY;
+        seen[t] = -INFINITY;
     }
+    // The larger of two as the median with an infinity that the compiler does not know (it would make the median a maximum and
+    // quiet every operand that comes from a matrix instruction or a lane swap first, an instruction each).
+    float inf;
+    asm volatile("s_mov_b32 %0, 0x7f800000" : "=s"(inf));
+    auto max2 = [&](float a, float b) -> float { return __builtin_amdgcn_fmed3f(a, b, inf); };
+    auto max_rows = [&](float v) -> float {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = max2(__uint_as_float(a[0]), __uint_as_float(a[1]));
+        const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return max2(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    };
     auto block = [&](const _Float16* kb, const _Float16* vb, const float* ksc, uint32_t blk_key0) {
         uint32_t ka = k_at, va = v_at;
         asm volatile("" : "+v"(ka), "+v"(va));  // (the XORs below stay in the loop: their results would cost 12 registers)
-        constexpr int NH = KB / 32, NV = QC && QT == 2 && NS >= 4 ? NS / 4 : NS / 2;  // (V operands read ahead: rows waiting in registers leave room for fewer)
+        constexpr int NH = KB / 32, NT = KB / 16, NP = NH * NS;  // 32-key steps, key tiles, V operands of a block
+        constexpr int VB = QC && QT == 2 && NS >= 4 ? 2 : NP < 4 ? NP : 4;  // V operands read ahead (rows waiting in registers leave room for fewer)
         // (where rows wait in registers there is no room to hold the requests' order: the compiler's own has no spills)
         constexpr bool FENCE = !QC || QT == 1;
+        auto fence = [&]() {
+            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
+        };
         v8h K[2][KS];
-        auto read_k = [&](int hb) {
+        auto read_k = [&](int hb, int s) {
 #pragma unroll
-            for (int s = 0; s < KS; s++)
-#pragma unroll
-                for (int kt = 0; kt < 2; kt++) K[kt][s] = *reinterpret_cast<const v8h*>(kb + (ka ^ (32u * s)) + (2 * hb + kt) * 16 * HD);
+            for (int kt = 0; kt < 2; kt++) K[kt][s] = *reinterpret_cast<const v8h*>(kb + (ka ^ (32u * s)) + (2 * hb + kt) * 16 * HD);
         };
-        auto read_v = [&](int hb, int sl) -> v8h {
-            const _Float16* tile = vb + (va ^ (16u * sl)) + hb * 32 * HD;
-            const v4h_t t0 = lds_read_tr16(tile), t1 = lds_read_tr16(tile + 16 * HD);
-            return (v8h){t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
+        v8h V[2][VB];
+        auto read_v = [&](int j) {  // the j-th group of V operands: step i / NS, dimensions 16 (i % NS) ..
+#pragma unroll
+            for (int u = 0; u < VB; u++) {
+                const int i = j * VB + u;
+                const _Float16* tile = vb + (va ^ (16u * (i % NS))) + (i / NS) * 32 * HD;
+                const v4h_t t0 = lds_read_tr16(tile), t1 = lds_read_tr16(tile + 16 * HD);
+                V[j & 1][u] = (v8h){t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
+            }
         };
-        read_k(0);
 #pragma unroll
-        for (int hb = 0; hb < NH; hb++) {  // 32 keys at a time
-            const uint32_t key0 = blk_key0 + hb * 32;
-            if (hb && key0 > q_hi) continue;  // (wave-uniform) above the diagonal of every query of the wave
-            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);  // all K operands have been requested: their latency is paid once
-            v4f S[QT][2];
+        for (int s = 0; s < KS; s++) read_k(0, s);
+        fence();  // all K operands have been requested: their latency is paid once
+        v4f S[QT][NT];
 #pragma unroll
-            for (int t = 0; t < QT; t++) S[t][0] = S[t][1] = (v4f){0.f, 0.f, 0.f, 0.f};
-            // four independent chains of products at a time
+        for (int t = 0; t < QT; t++)
 #pragma unroll
-            for (int s = 0; s < KS; s++)
+            for (int kt = 0; kt < NT; kt++) S[t][kt] = QC ? (v4f){0.f, 0.f, 0.f, 0.f} : neg_m[t];
+        // four independent chains of products at a time; a K operand is read again for the next step right after its last use
+#pragma unroll
+        for (int hb = 0; hb < NH; hb++)
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
 #pragma unroll
                 for (int hl = 0; hl < 2; hl++)
 #pragma unroll
                     for (int kt = 0; kt < 2; kt++)
 #pragma unroll
                         for (int t = 0; t < QT; t++)
-                            S[t][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(K[kt][s], hl ? ql[t][s] : qh[t][s], S[t][kt], 0, 0, 0);
-            // the next half's K and the first V operands travel while the probabilities are worked out
-            if (hb + 1 < NH) read_k(hb + 1);
-            v8h V[NV];
-#pragma unroll
-            for (int sl = 0; sl < NV; sl++) V[sl] = read_v(hb, sl);
-            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
-            if constexpr (QC) {
-#pragma unroll
-                for (int kt = 0; kt < 2; kt++) {
-                    const float4 a = *reinterpret_cast<const float4*>(ksc + 16 * (2 * hb + kt) + 4 * g);
-#pragma unroll
-                    for (int t = 0; t < QT; t++) S[t][kt][0] *= a.x, S[t][kt][1] *= a.y, S[t][kt][2] *= a.z, S[t][kt][3] *= a.w;
+                            S[t][2 * hb + kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(K[kt][s], hl ? ql[t][s] : qh[t][s], S[t][2 * hb + kt], 0, 0, 0);
+                if (hb + 1 < NH) {
+                    read_k(hb + 1, s);
+                    fence();
                 }
             }
-            // (wave-uniform) every query of the wave sees all of these keys, or the tests run
-            const bool all = key0 + 31 <= q_lo && (!window || key0 + 32 <= p.sinks || q_hi - key0 < budget);
-            if (!all) {
+        read_v(0);  // the first V operands travel while the probabilities are worked out
+        fence();
+        if constexpr (QC) {
 #pragma unroll
-                for (int t = 0; t < QT; t++)
+            for (int kt = 0; kt < NT; kt++) {
+                const float4 a = *reinterpret_cast<const float4*>(ksc + 16 * kt + 4 * g);
 #pragma unroll
-                    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            const uint32_t key = key0 + 16 * kt + 4 * g + v;
-                            const bool vis = key <= qpos[t] && (!window || key < p.sinks || qpos[t] - key < budget);
-                            S[t][kt][v] = vis ? S[t][kt][v] : -INFINITY;
-                        }
-            }
-            v8h P[QT];
-#pragma unroll
-            for (int t = 0; t < QT; t++) {
-                const float m0 = max_raw(max_raw(S[t][0][0], S[t][0][1]), max_raw(S[t][0][2], S[t][0][3]));
-                const float m1 = max_raw(max_raw(S[t][1][0], S[t][1][1]), max_raw(S[t][1][2], S[t][1][3]));
-                const float mx = max_rows4_raw(max_raw(m0, m1));
-                if (__builtin_amdgcn_ballot_w64(mx > m_run[t])) {  // a new maximum for some query of the tile
-                    const float m_new = max_raw(m_run[t], mx);
-                    const float alpha = m_run[t] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[t] - m_new);
-                    m_run[t] = m_new;
-#pragma unroll
-                    for (int sl = 0; sl < NS; sl++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) O[t][sl][v] *= alpha;
-                    lsum[t] *= alpha;
+                for (int t = 0; t < QT; t++) {
+                    S[t][kt][0] = fmaf(S[t][kt][0], a.x, neg_m[t][0]), S[t][kt][1] = fmaf(S[t][kt][1], a.y, neg_m[t][0]);
+                    S[t][kt][2] = fmaf(S[t][kt][2], a.z, neg_m[t][0]), S[t][kt][3] = fmaf(S[t][kt][3], a.w, neg_m[t][0]);
                 }
-                // (a query that has seen nothing yet keeps its empty state: every probability 0)
-                const float m = m_run[t] == -INFINITY ? 0.f : m_run[t];
+            }
+        }
+        // (wave-uniform) every query of the wave sees all of these keys, or the tests run
+        const bool all = blk_key0 + KB - 1 <= q_lo && (!window || blk_key0 + KB <= p.sinks || q_hi - blk_key0 < budget);
+        if (!all) {
+#pragma unroll
+            for (int t = 0; t < QT; t++)
+#pragma unroll
+                for (int kt = 0; kt < NT; kt++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const uint32_t key = blk_key0 + 16 * kt + 4 * g + v;
+                        const bool vis = key <= qpos[t] && (!window || key < p.sinks || qpos[t] - key < budget);
+                        S[t][kt][v] = vis ? S[t][kt][v] : -INFINITY;
+                    }
+        }
+        v8h P[QT][NH];
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+            float mk[NT];
+#pragma unroll
+            for (int kt = 0; kt < NT; kt++) mk[kt] = max2(max2(S[t][kt][0], S[t][kt][1]), max2(S[t][kt][2], S[t][kt][3]));
+            float mx = max2(mk[0], mk[1]);
+#pragma unroll
+            for (int kt = 2; kt < NT; kt += 2) mx = max2(mx, max2(mk[kt], mk[kt + 1]));
+            mx = max_rows(mx);
+            if (__builtin_amdgcn_ballot_w64(mx > seen[t])) {  // a new maximum for some query of the tile
+                // by how much it moves; the first one of a query may lie below 0, and finds nothing to rescale
+                const float by = mx > seen[t] ? mx : 0.f, alpha = __builtin_amdgcn_exp2f(fminf(-by, 0.f));
+                seen[t] = mx > seen[t] ? 0.f : seen[t];
+                neg_m[t][0] -= by;
+                if constexpr (!QC) neg_m[t][1] = neg_m[t][2] = neg_m[t][3] = neg_m[t][0];
+#pragma unroll
+                for (int sl = 0; sl < NS; sl++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) O[t][sl][v] *= alpha;
+                lsum[t] *= alpha;
+#pragma unroll
+                for (int kt = 0; kt < NT; kt++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) S[t][kt][v] -= by;
+            }
+            // (a query that has seen nothing yet keeps its empty state: every score -infinity, every probability 0)
+#pragma unroll
+            for (int hb = 0; hb < NH; hb++) {
                 float pe[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    pe[e] = __builtin_amdgcn_exp2f(S[t][e >> 2][e & 3] - m);
-                    P[t][e] = (_Float16)pe[e];
+                    pe[e] = __builtin_amdgcn_exp2f(S[t][2 * hb + (e >> 2)][e & 3]);
+                    P[t][hb][e] = (_Float16)pe[e];
                 }
                 lsum[t] += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
             }
-            v8h V2[NS - NV];
+        }
 #pragma unroll
-            for (int sl = NV; sl < NS; sl++) V2[sl - NV] = read_v(hb, sl);
-            if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < NP / VB; j++) {
+            if (j + 1 < NP / VB) read_v(j + 1);
+            fence();
 #pragma unroll
-            for (int sl = 0; sl < NS; sl++)
+            for (int u = 0; u < VB; u++)
 #pragma unroll
-                for (int t = 0; t < QT; t++)
-                    O[t][sl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl < NV ? V[sl < NV ? sl : 0] : V2[sl < NV ? 0 : sl - NV], P[t], O[t][sl], 0, 0, 0);
+                for (int t = 0; t < QT; t++) {
+                    const int i = j * VB + u;
+                    O[t][i % NS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(V[j & 1][u], P[t][i / NS], O[t][i % NS], 0, 0, 0);
+                }
         }
     };
-    if (i0 < i1) {
-        deliver(ks0, vs0, kscale0);
-        for (uint32_t i = i0;;) {
-            if (i + 1 < i1) request(key_of(i + 1), ks1, vs1);
-            block(ks0, vs0, kscale0, key_of(i));
-            if (++i == i1) break;
-            deliver(ks1, vs1, kscale1);
-            if (i + 1 < i1) request(key_of(i + 1), ks0, vs0);
-            block(ks1, vs1, kscale1, key_of(i));
-            if (++i == i1) break;
-            deliver(ks0, vs0, kscale0);
+    if (steps) {
+        deliver(ks0, vs0, kscale0, mine(0) < i1);
+        for (uint32_t j = 0;;) {
+            if (mine(j + 1) < i1) request(key_of(mine(j + 1)), ks1, vs1);
+            if (mine(j) < i1) block(ks0, vs0, kscale0, key_of(mine(j)));
+            if (++j == steps) break;
+            deliver(ks1, vs1, kscale1, mine(j) < i1);
+            if (mine(j + 1) < i1) request(key_of(mine(j + 1)), ks0, vs0);
+            if (mine(j) < i1) block(ks1, vs1, kscale1, key_of(mine(j)));
+            if (++j == steps) break;
+            deliver(ks0, vs0, kscale0, mine(j) < i1);
+        }
+    }
+    if constexpr (WK == 2) {
+        // The second walker's sums go through the stages (nothing is in flight: the last block's requests were waited for), the
+        // first one brings both to a common reference.
+        __shared__ float2 ex_ml[4][QT][64];
+        constexpr int PER = (int)sizeof(ks0_all) / 4096;  // dimension tiles of four waves that a stage holds
+        static_assert(4 * PER >= QT * NS, "the sums fit the four stages");
+        _Float16* const stages[4] = {ks0_all, ks1_all, vs0_all, vs1_all};
+        __syncthreads();
+        if (walker) {
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                ex_ml[wave][t][lane] = make_float2(seen[t] - neg_m[t][0], lsum[t]);
+#pragma unroll
+                for (int sl = 0; sl < NS; sl++)
+                    reinterpret_cast<v4f*>(stages[(t * NS + sl) / PER])[(wave * PER + (t * NS + sl) % PER) * 64 + lane] = O[t][sl];
+            }
+        }
+        __syncthreads();
+        if (walker) return;
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+            const float2 ml = ex_ml[wave][t][lane];
+            const float m0 = seen[t] - neg_m[t][0], m = fmaxf(m0, ml.x);
+            const float a0 = m0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m0 - m), a1 = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+            seen[t] = m == -INFINITY ? m : 0.f;
+            neg_m[t][0] = m == -INFINITY ? 0.f : -m;
+            lsum[t] = lsum[t] * a0 + ml.y * a1;
+#pragma unroll
+            for (int sl = 0; sl < NS; sl++) {
+                const v4f o = reinterpret_cast<v4f*>(stages[(t * NS + sl) / PER])[(wave * PER + (t * NS + sl) % PER) * 64 + lane];
+#pragma unroll
+                for (int v = 0; v < 4; v++) O[t][sl][v] = O[t][sl][v] * a0 + o[v] * a1;
+            }
         }
     }
 #pragma unroll
@@ -406,7 +497,7 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_prefill_kernel(Ox
             }
         } else {
             const size_t at = ((size_t)blockIdx.y * p.M + tok) * p.nq + head;
-            if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(m_run[t], l);
+            if (g == 0) reinterpret_cast<float2*>(p.part)[at] = make_float2(seen[t] - neg_m[t][0], l);
             if (!(l == 0.f)) {  // (an empty run is left out of the merge)
                 float* o = p.part + pf_part_head(gridDim.y, (size_t)p.M * p.nq) + at * HD + 4 * g;
 #pragma unroll
@@ -430,20 +521,33 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
     const uint32_t rows = M * nq, row = live ? tok * nq + head : 0u;
     const float2* ml = reinterpret_cast<const float2*>(part);
     const float4* po = reinterpret_cast<const float4*>(part + pf_part_head(n_splits, rows));
+    // (what eight runs hold is requested together; 32 runs one after the other took 14 us, 16 this way take 8: 32 tokens)
     float m = -INFINITY;
-    for (uint32_t s = 0; s < n_splits; s++) {
-        const float2 v = ml[(size_t)s * rows + row];
-        m = v.y == 0.f ? m : fmaxf(m, v.x);
+    for (uint32_t s0 = 0; s0 < n_splits; s0 += 8) {
+        float2 v[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) v[u] = s0 + u < n_splits ? ml[(size_t)(s0 + u) * rows + row] : make_float2(0.f, 0.f);
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) m = v[u].y == 0.f ? m : fmaxf(m, v[u].x);
     }
     float l = 0.f;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t s = 0; s < n_splits; s++) {
-        const float2 v = ml[(size_t)s * rows + row];
-        if (v.y == 0.f) continue;  // (an empty run has left no outputs)
-        const float w = __builtin_amdgcn_exp2f(v.x - m);
-        const float4 q = po[((size_t)s * rows + row) * hd4 + c];
-        l = fmaf(v.y, w, l);
-        a.x = fmaf(q.x, w, a.x), a.y = fmaf(q.y, w, a.y), a.z = fmaf(q.z, w, a.z), a.w = fmaf(q.w, w, a.w);
+    for (uint32_t s0 = 0; s0 < n_splits; s0 += 8) {
+        float2 v[8];
+        float4 q[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) {
+            const bool there = s0 + u < n_splits;
+            v[u] = there ? ml[(size_t)(s0 + u) * rows + row] : make_float2(0.f, 0.f);
+            q[u] = there ? po[((size_t)(s0 + u) * rows + row) * hd4 + c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) {
+            if (v[u].y == 0.f) continue;  // (an empty run has left no outputs)
+            const float w = __builtin_amdgcn_exp2f(v[u].x - m);
+            l = fmaf(v[u].y, w, l);
+            a.x = fmaf(q[u].x, w, a.x), a.y = fmaf(q[u].y, w, a.y), a.z = fmaf(q[u].z, w, a.z), a.w = fmaf(q[u].w, w, a.w);
+        }
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     a = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
@@ -462,28 +566,51 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
     operand_store8(op, h * hd + d, t, *reinterpret_cast<const float4*>(q), *reinterpret_cast<const float4*>(q + OXB_OPERAND_STEP(op.fmt)));
 }
 
-// Query tiles per wave and runs of keys.  Two tiles per wave where there are enough queries for both (from 49 on);
-// keys are split where a walk by one workgroup per tile would leave the chip idle: the cost of a plan is (rounds of
-// workgroups, two to a CU) x blocks of the longest run, 64 keys counting 1 us, and a split adds the merge: 6 us and the
-// partial sums' way to memory and back at 3 TB/s.
+// Which of the two forms, and into how many runs the keys are split: the cheapest of all, in us.  Measured with 1 to 2048
+// queries behind up to 8000 keys, every form alone, and what the rule makes of them is within 4 % of the better form there:
+//  - one tile: 7 us (launch, Q, the first keys' way), then per 32 keys of head_dim 128 with k workgroups on the CU 0.84, 0.98,
+//    1.29, 1.72 us (fp16 rows; four fit), 0.93, 1.31, 1.69 us (one-byte rows; three fit).  Heads of 64 take 0.55 of it.
+//    No CU is done before its longest walk, nor before its share of all walks, counted in whole rounds.
+//  - two tiles, two walkers: 14 us, and 0.64 to 0.78 us (one-byte rows 0.75 to 0.93) per 32 keys, the more the more CUs work;
+//    one workgroup to a CU.  So it takes long walks by less than a chip full of workgroups, and one-byte rows.
+//  - head_dim 256: 2 us per 32 keys, one workgroup to a CU.
+//  - a split adds the merge, 4 us and 0.25 per run, and the partial sums' way to memory and back, 0.4 us per MB.
 static OxbPrefillAttnPlan plan_attn(const OxbPrefillAttnParams& p, uint32_t n_cus) {
-    const uint32_t G = p.nq / p.nkv, hpw = G % 4u == 0 ? 4u : (G % 2u == 0 ? 2u : 1u), KB = (uint32_t)pf_block_keys((int)p.hd, p.kv_mode != OXB_KV_F16);
-    const uint32_t qt = p.M > 48 && p.hd != 256 ? 2u : 1u, per_wg = (4u / hpw) * qt;
-    const uint32_t n_tg = ((p.M + 15u) / 16u + per_wg - 1) / per_wg, wgs = n_tg * (p.nq / hpw);
-    uint32_t keys = p.pos_start + p.M;
-    if (p.window) {  // sinks, window and the workgroup's own queries
-        const uint64_t seen = (uint64_t)p.sinks + p.window + per_wg * 16 + 2 * KB;
-        if (seen < keys) keys = (uint32_t)seen;
-    }
-    const uint32_t n_blk = (keys + KB - 1) / KB + (p.window ? 1 : 0);
-    OxbPrefillAttnPlan best = {hpw, qt, wgs, 1, n_blk};
-    float best_cost = 1e30f;
-    for (uint32_t s = 1; s <= OXB_PF_ATTN_MAX_SPLITS && s <= n_blk; s++) {
-        const uint32_t bps = (n_blk + s - 1) / s, used = (n_blk + bps - 1) / bps;
-        if (used != s) continue;
-        const uint32_t rounds = (uint32_t)(((uint64_t)wgs * s + 2 * n_cus - 1) / (2 * n_cus));
-        const float cost = (float)rounds * (float)(bps * KB) / 64.0f + (s > 1 ? 6.0f + 2.0f * (float)s * p.M * p.nq * p.hd * 4.0f / 3e6f : 0.f);
-        if (cost < best_cost) best_cost = cost, best.n_splits = s, best.blocks_per_split = bps;
+    const uint32_t G = p.nq / p.nkv, hpw = G % 4u == 0 ? 4u : (G % 2u == 0 ? 2u : 1u);
+    const bool qc = p.kv_mode != OXB_KV_F16;
+    OxbPrefillAttnPlan best = {hpw, 1, 0, 1, 0};
+    float best_cost = INFINITY;
+    for (uint32_t qt = 1; qt <= (p.hd == 128 ? 2u : 1u); qt++) {
+        const uint32_t per_wg = (4u / hpw) * qt, KB = (uint32_t)pf_block_keys((int)p.hd, (int)qt);
+        const uint32_t n_tg = ((p.M + 15u) / 16u + per_wg - 1) / per_wg, wgs = n_tg * (p.nq / hpw);
+        // keys that the last workgroup walks, and that one walks on average
+        uint32_t keys = p.pos_start + p.M;
+        float mean = (float)p.pos_start + 0.5f * (float)(p.M + 16 * per_wg);
+        if (p.window) {  // sinks, window and the workgroup's own queries
+            const uint64_t seen = (uint64_t)p.sinks + p.window + per_wg * 16 + 2 * KB;
+            if (seen < keys) keys = (uint32_t)seen;
+        }
+        mean = fminf(mean, (float)keys);
+        const uint32_t n_blk = (keys + KB - 1) / KB + (p.window ? 1 : 0);
+        const float part_mb = 1e-6f * (float)p.M * p.nq * p.hd * 4.0f, size = 0.1f + 0.9f * (float)p.hd / 128.0f;
+        for (uint32_t s = 1; s <= OXB_PF_ATTN_MAX_SPLITS && s <= n_blk; s++) {
+            const uint32_t bps = (n_blk + s - 1) / s, used = (n_blk + bps - 1) / bps;
+            if (used != s) continue;
+            const float per_cu = (float)wgs * (float)s / (float)n_cus, walk = mean / (float)(s * 32);
+            const float longest = (float)((bps + qt - 1) / qt * qt * KB) / 32.0f;
+            float cost = s > 1 ? 4.0f + (float)s * (0.25f + 0.4f * part_mb) : 0.f;
+            if (qt == 2) {
+                const float rounds = ceilf(per_cu), t = qc ? 0.75f + 0.18f * fminf(per_cu, 1.f) : 0.64f + 0.14f * fminf(per_cu, 1.f);
+                cost += rounds * 14.0f + t * fmaxf(longest, rounds * walk);
+            } else if (p.hd == 256) {
+                cost += 10.0f + 2.0f * fmaxf(longest, ceilf(per_cu) * walk);
+            } else {
+                const float slots = qc && p.hd == 128 ? 3.f : 4.f, n = ceilf(per_cu), full = floorf(n / slots), rest = n - full * slots;
+                auto at = [&](float k) -> float { return qc ? 0.55f + 0.38f * k : fmaxf(0.7f + 0.14f * k, 0.43f * k); };
+                cost += 7.0f + size * fmaxf(at(1.f) * longest, (full * at(slots) + (rest > 0.f ? at(rest) : 0.f)) * walk);
+            }
+            if (cost < best_cost) best_cost = cost, best = {hpw, qt, wgs, s, bps};
+        }
     }
     return best;
 }
@@ -504,34 +631,31 @@ hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipSt
     const dim3 grid(pl.wgs, pl.n_splits);
     const bool opt = p.window != 0 || p.kv.page_table != nullptr;
 #define OXB_PF_LAUNCH(HD_, KVM_, QT_)                                                                                     \
-    if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, QT_>), grid, dim3(256), 0, st, p, pl.hpw);          \
-    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, QT_>), grid, dim3(256), 0, st, p, pl.hpw);
-#define OXB_PF_KVM(HD_, QT_)                                       \
-    if (p.kv_mode == OXB_KV_I8) {                                  \
-        OXB_PF_LAUNCH(HD_, OXB_KV_I8, QT_)                         \
-    } else if (p.kv_mode == OXB_KV_FP8_E4M3) {                     \
-        OXB_PF_LAUNCH(HD_, OXB_KV_FP8_E4M3, QT_)                   \
-    } else {                                                       \
-        OXB_PF_LAUNCH(HD_, OXB_KV_F16, QT_)                        \
+    if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, QT_>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);    \
+    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, QT_>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);
+#define OXB_PF_KVM(HD_, QT_)                                  \
+    if (p.kv_mode == OXB_KV_I8) {                             \
+        OXB_PF_LAUNCH(HD_, OXB_KV_I8, QT_)                    \
+    } else if (p.kv_mode == OXB_KV_FP8_E4M3) {                \
+        OXB_PF_LAUNCH(HD_, OXB_KV_FP8_E4M3, QT_)              \
+    } else {                                                  \
+        OXB_PF_LAUNCH(HD_, OXB_KV_F16, QT_)                   \
     }
-#define OXB_PF_CASE(HD_)               \
-    case HD_:                          \
-        if (pl.qt == 2) {              \
-            OXB_PF_KVM(HD_, 2)         \
-        } else {                       \
-            OXB_PF_KVM(HD_, 1)         \
-        }                              \
-        break;
     switch (p.hd) {
-        OXB_PF_CASE(32)
-        OXB_PF_CASE(64)
-        OXB_PF_CASE(128)
+        case 32: OXB_PF_KVM(32, 1) break;
+        case 64: OXB_PF_KVM(64, 1) break;
+        case 128:
+            if (pl.qt == 2) {
+                OXB_PF_KVM(128, 2)
+            } else {
+                OXB_PF_KVM(128, 1)
+            }
+            break;
         case 256: OXB_PF_KVM(256, 1) break;
         default: return hipErrorInvalidValue;
     }
 #undef OXB_PF_LAUNCH
 #undef OXB_PF_KVM
-#undef OXB_PF_CASE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || pl.n_splits == 1) return e;
     const uint32_t hpg = 256 / p.hd;

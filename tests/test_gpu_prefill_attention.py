@@ -67,24 +67,24 @@ def _visible(pos, n, window, sinks):
 
 
 # (queries, first position, q heads, kv heads, head_dim, cache, window, sinks, page size): what the launcher makes of them is
-# noted as query tiles per wave, runs of keys x blocks per run.
+# noted as runs of keys x blocks per run (all with one query tile per wave).
 CASES = [
-    (7, 0, 2, 1, 128, KV_F16, 0, 0, 0),           # one tile, a single block
-    (130, 0, 8, 2, 64, KV_F16, 0, 0, 0),          # two tiles, 3 x 1
-    (5, 1200, 1, 1, 128, KV_F16, 0, 0, 0),        # one tile, 19 x 1: an odd number (19 x 5 x 1) of rows of sums
-    (7, 1500, 3, 3, 128, KV_F16, 0, 0, 16),       # one tile, 24 x 1, paged
-    (49, 3001, 2, 2, 64, KV_F16, 0, 0, 32),       # two tiles (the fewest queries that take two), 24 x 2, paged
-    (48, 3001, 4, 2, 128, KV_F16, 0, 0, 0),       # one tile (the most), 24 x 2
-    (64, 4000, 4, 2, 128, KV_F16, 0, 0, 0),       # two tiles, 32 x 2
-    (331, 768, 4, 2, 128, KV_I8, 0, 0, 0),        # two tiles, blocks of 32 keys, 7 x 5
+    (7, 0, 2, 1, 128, KV_F16, 0, 0, 0),           # a single block
+    (130, 0, 8, 2, 64, KV_F16, 0, 0, 0),          # 1 x 3
+    (5, 1200, 1, 1, 128, KV_F16, 0, 0, 0),        # 13 x 3: an odd number (13 x 5 x 1) of rows of sums
+    (7, 1500, 3, 3, 128, KV_F16, 0, 0, 16),       # 12 x 4, paged
+    (49, 3001, 2, 2, 64, KV_F16, 0, 0, 32),       # 12 x 4, the last workgroup one query, paged
+    (48, 3001, 4, 2, 128, KV_F16, 0, 0, 0),       # 16 x 6
+    (64, 4000, 4, 2, 128, KV_F16, 0, 0, 0),       # 16 x 8
+    (331, 768, 4, 2, 128, KV_I8, 0, 0, 0),        # 7 x 5
     (331, 768, 4, 2, 128, KV_FP8_E4M3, 0, 0, 16),
-    (33, 2900, 4, 1, 32, KV_I8, 0, 0, 64),        # one tile, 23 x 2: half a wave fetches all pieces of a block
-    (100, 3000, 4, 1, 32, KV_FP8_E4M3, 0, 0, 0),  # two tiles, 25 x 2
+    (33, 2900, 4, 1, 32, KV_I8, 0, 0, 64),        # 12 x 4: half a wave fetches all pieces of a block
+    (100, 3000, 4, 1, 32, KV_FP8_E4M3, 0, 0, 0),  # 10 x 5
     (3, 2300, 5, 1, 128, KV_I8, 0, 0, 128),       # five heads: one per workgroup
-    (21, 1000, 2, 1, 256, KV_F16, 0, 0, 0),       # 32 x 1
-    (17, 900, 2, 2, 256, KV_I8, 0, 0, 16),        # 29 x 1
-    (90, 2100, 8, 2, 64, KV_F16, 700, 5, 0),      # a window: 15 x 1, runs that some queries see nothing of
-    (50, 2500, 4, 2, 128, KV_I8, 1200, 70, 16),   # 15 x 3, sinks across a block's edge, paged
+    (21, 1000, 2, 1, 256, KV_F16, 0, 0, 0),       # 16 x 2
+    (17, 900, 2, 2, 256, KV_I8, 0, 0, 16),        # 15 x 2
+    (90, 2100, 8, 2, 64, KV_F16, 700, 5, 0),      # a window: 5 x 3, runs that some queries see nothing of
+    (50, 2500, 4, 2, 128, KV_I8, 1200, 70, 16),   # 11 x 4, sinks across a block's edge, paged
     (40, 2500, 4, 2, 64, KV_FP8_E4M3, 64, 64, 32),  # nothing visible but the sinks
 ]
 
@@ -118,6 +118,51 @@ def test_prefill_attention_matches_float64(backend, M, start, nq, nkv, hd, mode,
                 want, size = p @ V / total, p @ np.abs(V) / total
                 bound = ((3 if mode != KV_F16 else 1) * 2.0**-11 + 2.0**-15) * size + n * 2.0**-25 * np.abs(V).max() / total
                 worst = max(worst, float((np.abs(got[:, kvh * (nq // nkv) + hh] - want) / bound).max()))
+        assert worst <= 1.0, worst
+    finally:
+        gpu.close()
+
+
+# Two query tiles per wave and two walkers per workgroup, as (queries, first position, q heads, kv heads, cache, window,
+# sinks, page size), noted as before with blocks of 64 keys.
+WALKED = [
+    (1000, 3000, 28, 4, KV_F16, 0, 0, 0),         # 1 x 63: the second walker has no last block; seven heads, one per workgroup
+    (960, 2000, 28, 4, KV_F16, 2000, 70, 32),     # 1 x 38, sinks across a block's edge, paged
+    (1000, 1000, 24, 8, KV_FP8_E4M3, 1000, 70, 16),  # 1 x 22
+    (1000, 6000, 8, 2, KV_I8, 0, 0, 0),           # 4 x 28, four heads per workgroup: 1000 ends inside the last one's first tile
+    (960, 4000, 8, 2, KV_I8, 4000, 70, 64),       # 4 x 17, odd runs, some of them empty
+    (200, 6000, 24, 8, KV_I8, 0, 0, 0),           # 5 x 20, the last run 17
+]
+
+
+@pytest.mark.parametrize("M,start,nq,nkv,mode,window,sinks,page", WALKED)
+def test_two_walkers_match_float64(backend, M, start, nq, nkv, mode, window, sinks, page):
+    max_seq, layer, seq, hd = start + M, 1, 1, 128
+    gpu, w = _model(backend, nq, nkv, hd, max_seq, batch=2)
+    g = np.random.default_rng([M, start, mode])
+    try:
+        if mode != KV_F16 or window or page:
+            gpu.set_attention(mode, window, sinks, page, 2 * -(-max_seq // page) if page else 0)
+        ang = g.uniform(0, 2 * np.pi, (max_seq, hd // 2)).astype(np.float32)
+        cos, sin = np.cos(ang), np.sin(ang)
+        gpu.set_rope_rows(0, cos, sin)
+        qkv = g.standard_normal((max_seq, (nq + 2 * nkv) * hd), dtype=np.float32)
+        _attend(gpu, layer, seq, qkv[:start], 0)
+        got = _attend(gpu, layer, seq, qkv[start:], start)
+        t = np.unique(np.r_[0, 1, 15:M:31, M - 17, M - 2, M - 1])
+        q = _queries(gpu.cfg, w, layer, qkv[start + t], cos[start + t], sin[start + t])
+        vis = _visible(start + t, max_seq, window, sinks)
+        worst = 0.0
+        for kvh in (0, nkv - 1):
+            K, V = _rows(gpu, layer, kvh, max_seq, seq)
+            for hh in range(nq // nkv):
+                head = kvh * (nq // nkv) + hh
+                s = np.where(vis, q[:, head] @ K.T, -np.inf)
+                p = np.exp2(s - s.max(1, keepdims=True))
+                total = p.sum(1, keepdims=True)
+                want, size = p @ V / total, p @ np.abs(V) / total
+                bound = ((3 if mode != KV_F16 else 1) * 2.0**-11 + 2.0**-15) * size + max_seq * 2.0**-25 * np.abs(V).max() / total
+                worst = max(worst, float((np.abs(got[t, head] - want) / bound).max()))
         assert worst <= 1.0, worst
     finally:
         gpu.close()
