@@ -5,7 +5,8 @@
 // large results.  Here every transfer goes through pinned memory that the library keeps and is made by a small kernel in the
 // caller's stream, so no copy engine has to be synchronised with it.  The host's side of it is a copy by several threads
 // (CopyTeam): one moves 28 to 33 GB/s to or from memory that the bus has written or will read, less than the bus itself.  The
-// last transfer of a call raises a flag in pinned memory that the host polls: three dependent launches and a poll take 12.6 us where the same three and hipStreamSynchronize take 18.
+// last transfer of a call raises a flag in pinned memory that the host polls: three dependent launches and a poll take 12.6 us
+// where the same three and hipStreamSynchronize take 18.
 #include <hip/hip_runtime.h>
 
 #include <signal.h>
@@ -29,23 +30,29 @@
 // more than they gain (1.2 MB out: 34 us with 64 workgroups, 50 with 256).
 #define OXB_IO_GRID 64u
 
-// Pieces of 16 bytes (4, where a buffer lies otherwise), then what is left byte by byte.  With `flag`: the workgroup that finishes last stores seq there once every
-// workgroup's part is visible to the host; *arrived is 0 before and after.
+// Units of 16 bytes (4, where a buffer lies otherwise), then what is left byte by byte, piece after piece of `piece` bytes.  With
+// `flag`: the workgroup that finishes piece c last stores seq + c there once every workgroup's part of it is visible to the host;
+// arrived[c] is 0 before and after.  (A workgroup has passed piece c, its store of the flag included, before it counts itself off
+// at the next one: the flag only grows.)  One launch for all pieces of a transfer: 19.4 MB out take 387 us, where a launch for
+// each piece of 1 MB, the bus idle in between, takes 496 and one without pieces, nothing of it handed over before the end, 362.
 template <typename T>
-__global__ __launch_bounds__(256) void io_copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t bytes,
+__global__ __launch_bounds__(256) void io_copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t bytes, size_t piece,
                                                        uint32_t* arrived, uint32_t* flag, uint32_t seq) {
-    const size_t n = bytes / sizeof(T), step = (size_t)gridDim.x * 256;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step)
-        reinterpret_cast<T*>(dst)[i] = reinterpret_cast<const T*>(src)[i];
-    if (blockIdx.x == 0 && threadIdx.x < bytes % sizeof(T)) dst[n * sizeof(T) + threadIdx.x] = src[n * sizeof(T) + threadIdx.x];
-    if (!flag) return;
-    __threadfence_system();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (before == gridDim.x - 1) {
-            *arrived = 0;
-            __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (uint32_t c = 0; bytes; c++) {
+        const size_t len = bytes < piece ? bytes : piece, n = len / sizeof(T), step = (size_t)gridDim.x * 256;
+        for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step)
+            reinterpret_cast<T*>(dst)[i] = reinterpret_cast<const T*>(src)[i];
+        if (blockIdx.x == 0 && threadIdx.x < len % sizeof(T)) dst[n * sizeof(T) + threadIdx.x] = src[n * sizeof(T) + threadIdx.x];
+        src += len, dst += len, bytes -= len;
+        if (!flag) continue;
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t before = __hip_atomic_fetch_add(arrived + c, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            if (before == gridDim.x - 1) {
+                arrived[c] = 0;
+                __hip_atomic_store(flag, seq + c, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
     }
 }
@@ -55,6 +62,7 @@ namespace {
 
 constexpr size_t kChunk = (size_t)1 << 20;      // host copy of one piece while the bus moves the one before
 constexpr size_t kStaging = (size_t)32 << 20;   // per direction; larger buffers take turns in it
+constexpr size_t kPieces = kStaging / kChunk;   // of one launch, at most
 constexpr size_t kPoolOut = (size_t)512 << 20;  // result memory handed out at a time
 constexpr size_t kPoolKept = (size_t)128 << 20; // ... and kept for reuse
 // Calls after which the stream is synchronised all the same, for the runtime to retire its commands (host to host, 1024 x 2048
@@ -68,7 +76,11 @@ constexpr uint32_t kSyncEvery = 256;
 // 32 sequences), 34 MB in 27.4 -> 26.8 ms (2048-token prefill).  Waking them costs the caller 0.5 to 3 us:
 // shared from 64 KB on, a product with 131 KB in and out takes 33.0 us instead of 30.2, with 196 KB 37.3 instead of 37.0; with
 // 262 KB it takes 42.8 instead of 43.1, with 328 KB 50.9 instead of 49.4, with 393 KB 48.5 instead of 53.6.
+// Helpers that sleep take 50 us to come: transfers up to kWake that follow the last one later than kSoon are the caller's alone (a
+// decode step of one sequence, 608 KB of logits every 0.8 ms: 8 us less).
 constexpr size_t kShared = (size_t)320 << 10;
+constexpr size_t kWake = (size_t)1 << 20;
+constexpr auto kSoon = std::chrono::microseconds(100);
 constexpr size_t kSlice = (size_t)64 << 10;
 constexpr unsigned kHelpers = 3;
 constexpr auto kLinger = std::chrono::microseconds(60);
@@ -92,6 +104,7 @@ class CopyTeam {
     std::condition_variable cv;
     std::shared_ptr<Job> job;
     std::atomic<uint64_t> serial{0};
+    std::chrono::steady_clock::time_point last{};  // end of the last copy large enough to be shared
     bool stop = false, started = false;
     std::vector<std::thread> threads;
 
@@ -112,7 +125,12 @@ class CopyTeam {
     }
 
 public:
-    void copy(void* dst, const void* src, size_t bytes, bool share) {
+    void copy(void* dst, const void* src, size_t bytes, size_t transfer) {  // a piece of a transfer of so many bytes
+        if (transfer <= kShared) {
+            memcpy(dst, src, bytes);
+            return;
+        }
+        const bool share = transfer > kWake || std::chrono::steady_clock::now() - last < kSoon;
         if (share && !started) {
             started = true;
             sigset_t all, before;  // the program's signals stay with its own threads
@@ -127,6 +145,7 @@ public:
         }
         if (!share || bytes <= kSlice || threads.empty()) {
             memcpy(dst, src, bytes);
+            last = std::chrono::steady_clock::now();
             return;
         }
         const std::shared_ptr<Job> j = std::make_shared<Job>((uint8_t*)dst, (const uint8_t*)src, bytes);
@@ -140,6 +159,7 @@ public:
         while (j->done.load(std::memory_order_acquire) < bytes) __builtin_ia32_pause();
         std::lock_guard<std::mutex> lk(mu);
         job.reset();
+        last = std::chrono::steady_clock::now();
     }
     void end() {
         {
@@ -158,7 +178,7 @@ struct Staging {
     uint8_t *in = nullptr, *out = nullptr;
     size_t in_cap = 0, out_cap = 0, in_used = 0, out_used = 0;
     uint32_t *flag = nullptr, *arrived = nullptr, seq = 0, seq_begin = 0, calls = 0;
-    struct Late { void* dst; size_t at, bytes; uint32_t seq; bool share; };
+    struct Late { void* dst; size_t at, bytes; uint32_t seq; size_t transfer; };
     std::vector<Late> late;  // results that wait in staging for the device
 } st;
 
@@ -182,8 +202,8 @@ int staging(uint8_t** p, size_t* cap, size_t want) {  // grows to a power of two
 int ensure_flag() {
     if (st.flag) return OXB_HIP_OK;
     // (the null stream that clears has no order with the stream whose kernels count on it: the clear is waited for)
-    if (hipHostMalloc((void**)&st.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&st.arrived, 4) != hipSuccess ||
-        hipMemset(st.arrived, 0, 4) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+    if (hipHostMalloc((void**)&st.flag, 64, hipHostMallocCoherent) != hipSuccess || hipMalloc((void**)&st.arrived, kPieces * 4) != hipSuccess ||
+        hipMemset(st.arrived, 0, kPieces * 4) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
         (void)hipGetLastError();
         if (st.flag) (void)hipHostFree(st.flag);
         if (st.arrived) (void)hipFree(st.arrived);
@@ -194,13 +214,13 @@ int ensure_flag() {
     return OXB_HIP_OK;
 }
 
-int copy(const void* src, void* dst, size_t bytes, uint32_t* flag, uint32_t seq) {
-    const size_t wgs = (bytes / 16 + 255) / 256;
+int copy(const void* src, void* dst, size_t bytes, size_t piece, uint32_t* flag, uint32_t seq) {
+    const size_t wgs = ((bytes < piece ? bytes : piece) / 16 + 255) / 256;
     const uint32_t grid = wgs < 1 ? 1u : wgs < OXB_IO_GRID ? (uint32_t)wgs : OXB_IO_GRID;
     const uintptr_t at = (uintptr_t)src | (uintptr_t)dst;
     if (at & 3) return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: a buffer of %zu bytes is not aligned to 4", bytes);
-    if (at & 15) hipLaunchKernelGGL(io_copy_kernel<uint32_t>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, st.arrived, flag, seq);
-    else hipLaunchKernelGGL(io_copy_kernel<uint4>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, st.arrived, flag, seq);
+    if (at & 15) hipLaunchKernelGGL(io_copy_kernel<uint32_t>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, piece, st.arrived, flag, seq);
+    else hipLaunchKernelGGL(io_copy_kernel<uint4>, dim3(grid), dim3(256), 0, g_rt.stream, (const uint8_t*)src, (uint8_t*)dst, bytes, piece, st.arrived, flag, seq);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? OXB_HIP_OK : hip_fail(e, "kernel launch failed: io_copy");
 }
@@ -275,10 +295,10 @@ IoCall::~IoCall() {
 int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
     const uint8_t* s = (const uint8_t*)src;
     uint8_t* d = (uint8_t*)d_dst;
-    if (((uintptr_t)s & 15) == 0 && is_pinned(s, bytes)) return copy(s, d, bytes, nullptr, 0);
+    if (((uintptr_t)s & 15) == 0 && is_pinned(s, bytes)) return copy(s, d, bytes, bytes, nullptr, 0);
     int rc;
     if (st.in_used == 0 && (rc = staging(&st.in, &st.in_cap, bytes))) return rc;
-    const bool share = bytes > kShared;
+    const size_t transfer = bytes;
     while (bytes) {
         const size_t n = bytes < kChunk ? bytes : kChunk;
         if (st.in_used + n > st.in_cap) {  // every piece has been used once: wait for the device to be done with them
@@ -286,8 +306,8 @@ int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
             st.in_used = 0;
             if ((rc = staging(&st.in, &st.in_cap, bytes))) return rc;
         }
-        team.copy(st.in + st.in_used, s, n, share);
-        if ((rc = copy(st.in + st.in_used, d, n, nullptr, 0))) return rc;
+        team.copy(st.in + st.in_used, s, n, transfer);
+        if ((rc = copy(st.in + st.in_used, d, n, n, nullptr, 0))) return rc;
         st.in_used += (n + 255) & ~(size_t)255;
         s += n, d += n, bytes -= n;
     }
@@ -295,25 +315,29 @@ int IoCall::upload(void* d_dst, const void* src, size_t bytes) {
 }
 
 int IoCall::download(void* dst, const void* d_src, size_t bytes) {
-    if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, st.flag, ++st.seq);
+    if (((uintptr_t)dst & 15) == 0 && is_pinned(dst, bytes)) return copy(d_src, dst, bytes, bytes, st.flag, ++st.seq);
     int rc;
     if (st.out_used == 0 && (rc = staging(&st.out, &st.out_cap, bytes))) return rc;
-    const bool share = bytes > kShared;
+    const size_t transfer = bytes;
     uint8_t* d = (uint8_t*)dst;
     const uint8_t* s = (const uint8_t*)d_src;
     while (bytes) {
-        const size_t n = bytes < kChunk ? bytes : kChunk;
-        if (st.out_used + n > st.out_cap) {  // staging is full of results: hand them over first
+        if (st.out_used + (bytes < kChunk ? bytes : kChunk) > st.out_cap) {  // staging is full of results: hand them over first
             if ((rc = sync_all("output download"))) return rc;
-            for (const Staging::Late& l : st.late) team.copy(l.dst, st.out + l.at, l.bytes, l.share);
+            for (const Staging::Late& l : st.late) team.copy(l.dst, st.out + l.at, l.bytes, l.transfer);
             st.late.clear();
             st.out_used = 0;
             if ((rc = staging(&st.out, &st.out_cap, bytes))) return rc;
         }
-        if ((rc = copy(s, st.out + st.out_used, n, st.flag, ++st.seq))) return rc;
-        st.late.push_back({d, st.out_used, n, st.seq, share});
-        st.out_used += (n + 255) & ~(size_t)255;
-        s += n, d += n, bytes -= n;
+        // one launch for all that fits
+        const size_t room = st.out_cap - st.out_used, all = bytes <= room ? bytes : room / kChunk * kChunk;
+        if ((rc = copy(s, st.out + st.out_used, all, kChunk, st.flag, st.seq + 1))) return rc;
+        for (size_t at = 0; at < all; at += kChunk) {
+            const size_t n = std::min(kChunk, all - at);
+            st.late.push_back({d + at, st.out_used, n, ++st.seq, transfer});
+            st.out_used += (n + 255) & ~(size_t)255;
+        }
+        s += all, d += all, bytes -= all;
     }
     return OXB_HIP_OK;
 }
@@ -323,7 +347,7 @@ int IoCall::finish(const char* what) {
     if (st.seq == st.seq_begin && (rc = sync_all(what))) return rc;  // nothing came back
     for (const Staging::Late& l : st.late) {  // one piece is copied on the host while the next ones cross the bus
         if ((rc = wait_for(l.seq, what))) return rc;
-        team.copy(l.dst, st.out + l.at, l.bytes, l.share);
+        team.copy(l.dst, st.out + l.at, l.bytes, l.transfer);
     }
     st.late.clear();
     if ((rc = wait_for(st.seq, what))) return rc;
