@@ -191,8 +191,10 @@ typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 //  * sliding window with attention sinks (is_in_window, crates/oxibonsai-model/src/layers/sliding_window.rs:173-189):
 //    the first `sinks` keys stay visible, the others while pos - key < window - sinks; chunks without a visible key
 //    are not walked.  window == 0: every key up to pos is visible.
+// The outputs as fp32 (p.out), as those and superblocks of the O projection's packed GEMV (p.pack_out), or as its GEMM's operand (p.op).
+enum { OXB_ATTN_OUT_F32 = 0, OXB_ATTN_OUT_PACK = 1, OXB_ATTN_OUT_XH = 2 };
 #define OXB_ATTN_MERGE_LDS_BYTES(heads, threads) ((heads) * 65 * 4 + 12 + (threads) * 16)  // LDS attn_merge_heads needs
-template <uint32_t NT>
+template <uint32_t NT, int OUT>
 __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t used, float* sm);
 __device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32_t b, uint32_t h_first, const float* kf);
 
@@ -223,7 +225,9 @@ __device__ __forceinline__ bool attn_last_arrival(const OxbAttnParams& p, uint32
     return *flag != 0u;
 }
 
-template <int HD, int KVM, uint32_t NW, bool OPT>  // NW: waves; OPT: a window and / or a paged cache may be in use (else neither costs anything)
+// NW: waves; OPT: a window and / or a paged cache may be in use (else neither costs anything); OUT: what the outputs leave as.
+// (With tests of the fields instead 23 scalar registers are spilled: one fp16 sequence at 700 8.7 us against 8.4.)
+template <int HD, int KVM, uint32_t NW, bool OPT, int OUT>
 __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParams p) {
     constexpr uint32_t NT = 64 * NW, CH = 32 * NW;  // threads, KV positions of a chunk
     constexpr bool QC = KVM != OXB_KV_F16;
@@ -651,7 +655,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         ml[wave * 16 + qi] = l_run;
     }
     __syncthreads();
-    const bool pack = p.pack_out != nullptr && G * HD == 512u;
+    constexpr bool pack = OUT == OXB_ATTN_OUT_PACK;  // (G * HD is 512)
     float* keep = reinterpret_cast<float*>(&qs[0][0]);  // a single slot's outputs, for the quantiser
     static_assert(sizeof(qs) >= 512 * sizeof(float), "room for them");
     for (uint32_t i = tid; i < G * HD; i += NT) {
@@ -668,7 +672,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         }
         if (used == 1) {  // the only slot: what the merge would compute (weight 1, times 1 / sum)
             o *= l > 0.f ? 1.0f / l : 0.f;
-            if (p.op.xh) p.op.xh[oxb_operand_index(p.op.fmt, (h0 + h) * HD + d, b, p.op.M_pad)] = (_Float16)ldexpf(o, p.op.shift);
+            if constexpr (OUT == OXB_ATTN_OUT_XH) p.op.xh[oxb_operand_index(p.op.fmt, (h0 + h) * HD + d, b, p.op.M_pad)] = (_Float16)ldexpf(o, p.op.shift);
             else p.out[((size_t)b * p.nq + h0 + h) * HD + d] = o;
             if (pack) keep[i] = o;
             continue;
@@ -687,7 +691,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         return;
     }
     if (attn_last_arrival(p, b, kvh, used, &last_flag))  // (the barrier inside also retires mo / mm / ml)
-        attn_merge_heads<NT>(p, b, h0, G, used, reinterpret_cast<float*>(&vs_all[0][0]));
+        attn_merge_heads<NT, OUT>(p, b, h0, G, used, reinterpret_cast<float*>(&vs_all[0][0]));
 }
 
 // One wave quantises the 512 outputs of a kv head's q heads (LDS) for the O projection: superblock h_first * hd / 512 of
@@ -720,7 +724,7 @@ __device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32
 // as far as the threads allow for the heads' nh * hd / 4 groups.
 // sm: nh * 65 floats of LDS ([head][64] slot weights | [head] 1 / sum), then NT float4 for the partial sums.
 // The slot results were written by other workgroups of this same launch: agent-coherent loads.
-template <uint32_t NT>
+template <uint32_t NT, int OUT>
 __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t used, float* sm) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, hd = p.hd, qd = p.nq * hd;
     const uint32_t stride = hd + OXB_ATTN_PART_PAD;
@@ -730,7 +734,7 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
     // The merged outputs once more, for the quantiser at the end: 128 groups of four, in the entries of `sums` that the
     // partial sums never use (those are written by threads tg and up, and with 128 groups tg >= 128).
     float4* keep = sums;
-    const bool pack = p.pack_out != nullptr && nh * hd == 512u;
+    constexpr bool pack = OUT == OXB_ATTN_OUT_PACK;  // (nh * hd is 512)
     const uint32_t e0 = h_first * hd;
     const float* part = p.part + (size_t)b * p.nq * p.n_splits * stride;
     const __amdgpu_buffer_rsrc_t r_part = make_rsrc(part, p.nq * p.n_splits * stride * 4u);
@@ -816,7 +820,7 @@ __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_
         if (live && !sh) {
             const float il = inv_l[hh];
             acc.x *= il, acc.y *= il, acc.z *= il, acc.w *= il;
-            if (p.op.xh) operand_store4(p.op, e, b, acc.x, acc.y, acc.z, acc.w);
+            if constexpr (OUT == OXB_ATTN_OUT_XH) operand_store4(p.op, e, b, acc.x, acc.y, acc.z, acc.w);
             else *reinterpret_cast<float4*>(p.out + (size_t)b * qd + e) = acc;
             if (pack) keep[eg] = acc;
         }
@@ -925,11 +929,15 @@ hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStr
         (p.kv.page_table ? (p.kv.page_shift < 4 || p.kv.page_shift > 7) : (p.kv.row_stride % 128 != 0 || p.kv.row_stride < p.max_seq)))
         return hipErrorInvalidValue;
     const dim3 grid(p.n_splits, p.nkv, batch), block(p.wide ? 512 : 256);
-    const bool opt = p.window != 0 || p.kv.page_table != nullptr;
+    const bool opt = p.window != 0 || p.kv.page_table != nullptr, pack = p.pack_out != nullptr && p.nq / p.nkv * p.hd == 512u;
     switch (p.hd) {
+#define OXB_ATTN_LAUNCH_AS(HD_, KVM_, NW_, OUT_)                                                                     \
+    if (opt) hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, true, OUT_>), grid, block, 0, st, p);      \
+    else hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, false, OUT_>), grid, block, 0, st, p);
 #define OXB_ATTN_LAUNCH(HD_, KVM_, NW_)                                                                              \
-    if (opt) hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, true>), grid, block, 0, st, p);            \
-    else hipLaunchKernelGGL((attn_decode_fused_kernel<HD_, KVM_, NW_, false>), grid, block, 0, st, p);
+    if (p.op.xh) { OXB_ATTN_LAUNCH_AS(HD_, KVM_, NW_, OXB_ATTN_OUT_XH) }                                             \
+    else if (pack) { OXB_ATTN_LAUNCH_AS(HD_, KVM_, NW_, OXB_ATTN_OUT_PACK) }                                         \
+    else { OXB_ATTN_LAUNCH_AS(HD_, KVM_, NW_, OXB_ATTN_OUT_F32) }
 #define OXB_ATTN_CASE(HD_)                                                                            \
     case HD_:                                                                                         \
         if (p.kv_mode == OXB_KV_F16) {                                                                \
@@ -951,6 +959,7 @@ hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStr
         OXB_ATTN_CASE(128)
         OXB_ATTN_CASE(256)
 #undef OXB_ATTN_LAUNCH
+#undef OXB_ATTN_LAUNCH_AS
 #undef OXB_ATTN_CASE
         default: return hipErrorInvalidValue;
     }
