@@ -14,6 +14,7 @@
 
 #include "device_utils.h"
 #include "kv_quant_device.h"
+#include "kv_row_device.h"
 #include "layer_kernels.h"
 #include "gemv_pack_device.h"
 
@@ -28,40 +29,6 @@
 // (2048 tokens x 8 heads: 25 MB).  Two heads a wave one after the other, a value per lane and request, took 5.0 us for 23 tokens,
 // 6.9 for 301 with INT8 rows and 9.0 to 10 for 2048; this form 2.8, 5.0 and 5.7 (kernel traces).
 // ---------------------------------------------------------------------------
-// The sum / largest over groups of L lanes, in every lane.
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-    v += dpp_f32<0xB1>(v);
-    v += dpp_f32<0x4E>(v);
-    v += dpp_f32<0x141>(v);
-    if constexpr (L >= 16) v += dpp_f32<0x140>(v);
-    if constexpr (L >= 32) {
-        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    }
-    if constexpr (L >= 64) {
-        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    }
-    return v;
-}
-template <int L>
-__device__ __forceinline__ float group_max(float v) {
-    v = fmaxf(v, dpp_f32<0xB1>(v));
-    v = fmaxf(v, dpp_f32<0x4E>(v));
-    v = fmaxf(v, dpp_f32<0x141>(v));
-    if constexpr (L >= 16) v = fmaxf(v, dpp_f32<0x140>(v));
-    if constexpr (L >= 32) {
-        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    }
-    if constexpr (L >= 64) {
-        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    }
-    return v;
-}
-
 template <int HD, int KVM>
 __global__ __launch_bounds__(256) void kv_norm_rope_store_kernel(OxbKvStoreParams p) {
     constexpr int L = HD / 4, HPW = 64 / L;  // lanes of a head, heads of a wave
@@ -69,37 +36,10 @@ __global__ __launch_bounds__(256) void kv_norm_rope_store_kernel(OxbKvStoreParam
     const uint32_t n_hg = (p.nkv + HPW - 1) / HPW, id = blockIdx.x * 4 + (threadIdx.x >> 6);  // (token, group of heads)
     const uint32_t t = id / n_hg, head = (id % n_hg) * HPW + lane / L;
     if (t >= p.M || head >= p.nkv) return;  // (whole groups of lanes)
-    const uint32_t pos = p.pos_base + t, at = (4 * j) % (HD / 2);  // the pair's place
-    const float* row_in = p.qkv + (size_t)t * p.qkv_stride + (size_t)(p.nq + head) * HD + 4 * j;
-    const float4 k = *reinterpret_cast<const float4*>(row_in), v = *reinterpret_cast<const float4*>(row_in + (size_t)p.nkv * HD);
+    const uint32_t pos = p.pos_base + t;
+    const KvRowIn in = kv_row_load<HD>(p.qkv + (size_t)t * p.qkv_stride, p.nq, p.nkv, head, j, p.cos_t, p.sin_t, pos);
     const float4 w = *reinterpret_cast<const float4*>(p.k_norm + 4 * j);
-    const float4 cs = *reinterpret_cast<const float4*>(p.cos_t + (size_t)pos * (HD / 2) + at), sn = *reinterpret_cast<const float4*>(p.sin_t + (size_t)pos * (HD / 2) + at);
-    const size_t row = kv_row(p.kv, p.seq, p.layer, head, pos);
-    const float ss = group_sum<L>(fmaf(k.x, k.x, fmaf(k.y, k.y, fmaf(k.z, k.z, k.w * k.w))));
-    const float inv_rms = 1.0f / sqrtf(ss / (float)HD + p.eps);
-    const float a[4] = {w.x * k.x * inv_rms, w.y * k.y * inv_rms, w.z * k.z * inv_rms, w.w * k.w * inv_rms};
-    const float c4[4] = {cs.x, cs.y, cs.z, cs.w}, s4[4] = {sn.x, sn.y, sn.z, sn.w}, v4[4] = {v.x, v.y, v.z, v.w};
-    float o[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float other = __shfl_xor(a[i], L / 2, 64);
-        o[i] = j < L / 2 ? a[i] * c4[i] - other * s4[i] : other * s4[i] + a[i] * c4[i];
-    }
-    if constexpr (KVM != OXB_KV_F16) {
-        const float kmax = group_max<L>(fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3]))));
-        const float vmax = group_max<L>(fmaxf(fmaxf(fabsf(v4[0]), fabsf(v4[1])), fmaxf(fabsf(v4[2]), fabsf(v4[3]))));
-        const float ks = kv_row_scale<KVM>(kmax), vs = kv_row_scale<KVM>(vmax);
-        uint32_t kw = 0, vw = 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) kw |= kv_encode<KVM>(o[i], ks) << (8 * i), vw |= kv_encode<KVM>(v4[i], vs) << (8 * i);
-        reinterpret_cast<uint32_t*>(p.k_cache)[row * L + j] = kw;
-        reinterpret_cast<uint32_t*>(p.v_cache)[row * L + j] = vw;
-        if (j == 0) p.k_scale[row] = ks, p.v_scale[row] = vs;
-    } else {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        reinterpret_cast<h4*>(p.k_cache)[row * L + j] = (h4){(_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3]};
-        reinterpret_cast<h4*>(p.v_cache)[row * L + j] = (h4){(_Float16)v4[0], (_Float16)v4[1], (_Float16)v4[2], (_Float16)v4[3]};
-    }
+    kv_row_store<HD, KVM>(kv_row_make<HD, KVM>(in, w, p.eps, j), p.k_cache, p.v_cache, p.k_scale, p.v_scale, kv_row(p.kv, p.seq, p.layer, head, pos), j);
 }
 
 // Rows of f32 values -> quantised cache rows (codes + scale), one wave per row; the arithmetic of the attention

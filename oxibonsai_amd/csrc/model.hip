@@ -610,11 +610,13 @@ static int encode_prefill_attention(Model& m, uint32_t L, uint32_t seq, uint32_t
     qp.hd = d.hd;
     qp.layer = L;
     qp.eps = d.eps;
-    OXB_TRY_HIP(oxb_launch_kv_norm_rope_store(qp, st), "kernel launch failed: kv_norm_rope_store");
+    const bool stores = oxb_attn_prefill_can_store(d.hd, pos_start, M);
+    if (!stores) OXB_TRY_HIP(oxb_launch_kv_norm_rope_store(qp, st), "kernel launch failed: kv_norm_rope_store");
     OxbPrefillAttnParams ap;
     ap.qkv = qkv;
     ap.qkv_stride = qp.qkv_stride;
     ap.q_norm = q_norm;
+    ap.k_norm = stores ? k_norm : nullptr;
     ap.cos_t = m.cos_t;
     ap.sin_t = m.sin_t;
     ap.eps = d.eps;

@@ -13,6 +13,7 @@ struct OxbPrefillAttnParams {
     const float* q_norm;              // [hd]
     const float *cos_t, *sin_t;       // [max_seq][hd/2]
     float eps;
+    const float* k_norm;              // null: the new rows are in the cache; else (oxb_attn_prefill_can_store) the launch stores them
     const void *k_cache, *v_cache;    // cache rows of hd values each (fp16 or one-byte codes), placed by `kv`
     const float *k_scale, *v_scale;   // quantised cache: one scale per row
     uint32_t kv_mode;                 // OXB_KV_* (kv_quant_device.h)
@@ -32,5 +33,7 @@ struct OxbPrefillAttnParams {
 struct OxbPrefillAttnPlan { uint32_t hpw, qt, wgs, n_splits, blocks_per_split; };
 #define OXB_PF_ATTN_MAX_SPLITS 32u
 
+// Whether the launch can work out and store the new positions' K and V itself.
+bool oxb_attn_prefill_can_store(uint32_t hd, uint32_t pos_start, uint32_t M);
 size_t oxb_attn_prefill_part_bytes(const OxbPrefillAttnParams& p, uint32_t n_cus);
 hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipStream_t st);

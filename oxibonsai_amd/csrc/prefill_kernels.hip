@@ -13,6 +13,7 @@
 
 #include "device_utils.h"
 #include "kv_quant_device.h"
+#include "kv_row_device.h"
 #include "prefill_kernels.h"
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -75,7 +76,10 @@ __host__ __device__ constexpr size_t pf_part_head(size_t n_splits, size_t rows) 
 // Keys per block: 64, or 32 where four (head_dim 128) or two (256) workgroups to a CU share its LDS, 4 x KB x 2 HD bytes each.
 constexpr int pf_block_keys(int hd, int qt) { return hd == 256 || (hd == 128 && qt == 1) ? 32 : 64; }
 
-template <int HD, int KVM, bool OPT, int QT>  // OPT: a window and / or a paged cache may be in use (else neither costs anything)
+// OPT: a window and / or a paged cache may be in use (else neither costs anything).
+// NEW: a prompt's first tokens, one block of keys: the cache holds none of them yet.  Every workgroup works its kv head's rows out from
+// the projection, keeps them in LDS as the cache will hold them, and one workgroup of each kv head stores them.
+template <int HD, int KVM, bool OPT, int QT, bool NEW>
 __global__ __launch_bounds__(256 * QT, HD == 256 ? 1 : 2) void attn_prefill_kernel(OxbPrefillAttnParams p, uint32_t hpw) {
     constexpr bool QC = KVM != OXB_KV_F16;
     constexpr int WK = QT;                                           // walkers: groups of four waves that take the keys' blocks in turn
@@ -203,7 +207,38 @@ __global__ __launch_bounds__(256 * QT, HD == 256 ? 1 : 2) void attn_prefill_kern
     };
     const uint32_t steps = i0 < i1 ? (i1 - i0 + WK - 1) / WK : 0u;  // the same for both walkers: they meet at every barrier
     auto mine = [&](uint32_t j) -> uint32_t { return i0 + j * WK + walker; };
-    if (mine(0) < i1) request(key_of(mine(0)), ks0, vs0);
+    if (!NEW && mine(0) < i1) request(key_of(mine(0)), ks0, vs0);
+    if constexpr (NEW) {
+        constexpr int L = HD / 4, RPI = 64 / L, IT = RPW / RPI;  // lanes of a row, rows of a wave at a time
+        const uint32_t j = lane % L;
+        const float4 w = *reinterpret_cast<const float4*>(p.k_norm + 4 * j);
+        KvRowIn in[IT];
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const uint32_t t = min(wave * RPW + it * RPI + lane / L, last);  // (rows past the last one repeat it)
+            in[it] = kv_row_load<HD>(p.qkv + (size_t)t * p.qkv_stride, p.nq, p.nkv, kvh, j, p.cos_t, p.sin_t, t);
+        }
+        const bool stores = blockIdx.x < hq && blockIdx.x * hpw % (p.nq / p.nkv) == 0;
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const uint32_t t = wave * RPW + it * RPI + lane / L;
+            const KvRowOut r = kv_row_make<HD, KVM>(in[it], w, p.eps, j);
+            if (stores && t < p.M) kv_row_store<HD, KVM>(r, const_cast<void*>(p.k_cache), const_cast<void*>(p.v_cache), const_cast<float*>(p.k_scale), const_cast<float*>(p.v_scale), kv_row(p.kv, p.seq, p.layer, kvh, t), j);
+            uint2 kw = r.k, vw = r.v;
+            if constexpr (QC) {  // as deliver() widens them
+                kv_dec4<KVM>(r.k.x, kw.x, kw.y);
+                kv_dec4<KVM>(r.v.x, vw.x, vw.y);
+                const _Float16 sc = (_Float16)r.vs;
+                const kvh2_t sc2 = {sc, sc};
+                vw.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvh2_t, vw.x) * sc2);
+                vw.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvh2_t, vw.y) * sc2);
+                if (j == 0) kscale0[t] = r.ks;
+            }
+            const uint32_t at = (t * PPR + ((j >> 1) ^ ((t / RB) & PM))) * 8 + (j & 1u) * 4;
+            *reinterpret_cast<uint2*>(ks0 + at) = kw;
+            *reinterpret_cast<uint2*>(vs0 + at) = vw;
+        }
+    }
 
     // Q of this lane's queries: per-head RMSNorm, RoPE on the pairs (d, d + hd/2), times log2(e)/sqrt(hd)
     // (fused_qk_norm_rope, gpu_backend/cuda_attn_kernels.rs:160-226), then split into fp16 hi + lo.  The lane holds
@@ -422,7 +457,10 @@ __global__ __launch_bounds__(256 * QT, HD == 256 ? 1 : 2) void attn_prefill_kern
                 }
         }
     };
-    if (steps) {
+    if constexpr (NEW) {
+        lds_barrier();
+        block(ks0, vs0, kscale0, 0);
+    } else if (steps) {
         deliver(ks0, vs0, kscale0, mine(0) < i1);
         for (uint32_t j = 0;;) {
             if (mine(j + 1) < i1) request(key_of(mine(j + 1)), ks1, vs1);
@@ -615,6 +653,11 @@ static OxbPrefillAttnPlan plan_attn(const OxbPrefillAttnParams& p, uint32_t n_cu
     return best;
 }
 
+// Up to one block of keys with one query tile per wave (which is what plan_attn takes for so few).  23 tokens, 16 q heads and 8 kv
+// heads of 128, us per layer in a kernel trace: 2.7 for the rows' own launch and 6.5 for the attention, 7.0 for both in one.
+// With more keys every workgroup would work out more rows than its share of the waves can hold in flight.
+bool oxb_attn_prefill_can_store(uint32_t hd, uint32_t pos_start, uint32_t M) { return pos_start == 0 && M <= (uint32_t)pf_block_keys((int)hd, 1); }
+
 size_t oxb_attn_prefill_part_bytes(const OxbPrefillAttnParams& p, uint32_t n_cus) {
     const OxbPrefillAttnPlan pl = plan_attn(p, n_cus);
     const size_t rows = (size_t)p.M * p.nq;
@@ -625,14 +668,18 @@ hipError_t oxb_launch_attn_prefill(OxbPrefillAttnParams p, uint32_t n_cus, hipSt
     if (p.M == 0 || p.nq == 0 || p.nkv == 0 || p.nq % p.nkv || !p.qkv || !p.q_norm || !p.cos_t || !p.sin_t || p.pos_start + p.M > p.max_seq || p.kv_mode > OXB_KV_FP8_E4M3 ||
         (p.kv_mode != OXB_KV_F16 && (!p.k_scale || !p.v_scale)) || (p.kv.page_table && (p.kv.page_shift < 4 || p.kv.page_shift > 7)))
         return hipErrorInvalidValue;
+    if (p.k_norm && !oxb_attn_prefill_can_store(p.hd, p.pos_start, p.M)) return hipErrorInvalidValue;
     const OxbPrefillAttnPlan pl = plan_attn(p, n_cus);
-    if (pl.n_splits > 1 && !p.part) return hipErrorInvalidValue;
+    if ((pl.n_splits > 1 && !p.part) || (p.k_norm && (pl.qt != 1 || pl.n_splits != 1))) return hipErrorInvalidValue;
     p.blocks_per_split = pl.blocks_per_split;
     const dim3 grid(pl.wgs, pl.n_splits);
     const bool opt = p.window != 0 || p.kv.page_table != nullptr;
 #define OXB_PF_LAUNCH(HD_, KVM_, QT_)                                                                                     \
-    if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, QT_>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);    \
-    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, QT_>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);
+    if (QT_ == 1 && p.k_norm) {                                                                                                                \
+        if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, 1, true>), grid, dim3(256), 0, st, p, pl.hpw);                   \
+        else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, 1, true>), grid, dim3(256), 0, st, p, pl.hpw);                      \
+    } else if (opt) hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, true, QT_, false>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);    \
+    else hipLaunchKernelGGL((attn_prefill_kernel<HD_, KVM_, false, QT_, false>), grid, dim3(256 * QT_), 0, st, p, pl.hpw);
 #define OXB_PF_KVM(HD_, QT_)                                  \
     if (p.kv_mode == OXB_KV_I8) {                             \
         OXB_PF_LAUNCH(HD_, OXB_KV_I8, QT_)                    \

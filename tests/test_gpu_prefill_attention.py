@@ -69,7 +69,15 @@ def _visible(pos, n, window, sinks):
 # (queries, first position, q heads, kv heads, head_dim, cache, window, sinks, page size): what the launcher makes of them is
 # noted as runs of keys x blocks per run (all with one query tile per wave).
 CASES = [
-    (7, 0, 2, 1, 128, KV_F16, 0, 0, 0),           # a single block
+    (7, 0, 2, 1, 128, KV_F16, 0, 0, 0),           # a single block, whose rows the launch stores itself, as in the next seven
+    (32, 0, 8, 2, 128, KV_I8, 0, 0, 0),           # the longest of head_dim 128: two workgroups of a kv head
+    (17, 0, 3, 3, 128, KV_F16, 0, 0, 0),          # one head per workgroup, three kv heads
+    (31, 0, 5, 1, 128, KV_FP8_E4M3, 9, 2, 16),    # five workgroups of one kv head, windowed, paged
+    (64, 0, 8, 2, 64, KV_F16, 0, 0, 64),          # the longest of head_dim 64, paged
+    (50, 0, 4, 1, 32, KV_I8, 0, 0, 0),
+    (32, 0, 2, 1, 256, KV_FP8_E4M3, 0, 0, 0),     # the longest of head_dim 256
+    (1, 0, 4, 2, 64, KV_I8, 0, 0, 0),
+    (33, 0, 4, 2, 128, KV_I8, 0, 0, 0),           # one row more than the launch stores: 1 x 2
     (130, 0, 8, 2, 64, KV_F16, 0, 0, 0),          # 1 x 3
     (5, 1200, 1, 1, 128, KV_F16, 0, 0, 0),        # 13 x 3: an odd number (13 x 5 x 1) of rows of sums
     (7, 1500, 3, 3, 128, KV_F16, 0, 0, 16),       # 12 x 4, paged
