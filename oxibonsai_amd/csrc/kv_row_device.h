@@ -67,7 +67,10 @@ __device__ __forceinline__ KvRowOut kv_row_make(const KvRowIn& in, const float4&
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const float other = __shfl_xor(a[i], L / 2, 64);
-        o[i] = j < L / 2 ? a[i] * c4[i] - other * s4[i] : other * s4[i] + a[i] * c4[i];
+        // (written out, and an fp32 number before it becomes anything else: the same bits wherever this is inlined - the compiler
+        // rounds some of these sums to fp16 inside the multiply-add)
+        o[i] = fmaf(j < L / 2 ? -other : other, s4[i], a[i] * c4[i]);
+        asm("" : "+v"(o[i]));
     }
     KvRowOut r = {make_uint2(0, 0), make_uint2(0, 0), 1.f, 1.f};
     if constexpr (KVM != OXB_KV_F16) {

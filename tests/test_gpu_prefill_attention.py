@@ -176,6 +176,24 @@ def test_two_walkers_match_float64(backend, M, start, nq, nkv, mode, window, sin
         gpu.close()
 
 
+@pytest.mark.parametrize("mode", [KV_F16, KV_I8, KV_FP8_E4M3])
+@pytest.mark.parametrize("hd,n", [(128, 32), (64, 64), (32, 64), (256, 32), (128, 1)])
+def test_a_short_prompt_stores_the_rows_that_a_longer_one_does(backend, hd, n, mode):
+    # n tokens: the attention launch works the new rows out; one more than it takes: a launch of their own does.
+    gpu, _ = _model(backend, 12, 3, hd, 80, batch=2)
+    try:
+        if mode != KV_F16:
+            gpu.set_attention(mode, 0, 0, 16, 2 * 5)
+        x = np.random.default_rng([hd, n, mode]).standard_normal((65 if hd < 128 else 33, 18 * hd)).astype(np.float32)
+        _attend(gpu, 1, 0, x[:n], 0)
+        _attend(gpu, 1, 1, x, 0)
+        for head in range(3):
+            for a, b in zip(gpu.read_kv(1, head, 0, n, 0), gpu.read_kv(1, head, 0, n, 1)):
+                assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    finally:
+        gpu.close()
+
+
 @pytest.mark.parametrize("shape", ["spread", "sink", "far sink", "late peak"])
 @pytest.mark.parametrize("M", [16, 64])
 def test_prefill_attention_weights_are_relative_to_the_row_maximum(backend, M, shape):
