@@ -30,7 +30,7 @@ struct OxbGemmParams {
     int mode;
     // Mode SWIGLU, optional: instead of y the packed activations of the product that follows (n_rows / 2 values a row, a multiple
     // of 128; its format is this matrix's) and their exponents.  norm: |a|_2 < 2^norm of every row (oxb_launch_xh_pack),
-    // w_exp: the 2-norm of every row of the matrix is below 2^w_exp.
+    // w_exp: |gate row j|_2 |up row j|_2 < 2^w_exp for every j.
     uint32_t* xh_out;
     int32_t* xsh_out;
     const int32_t* norm;
@@ -54,8 +54,9 @@ bool oxb_pack_can_sum(uint32_t k, uint32_t M);
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
                               uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr,
                               int32_t* d_norm = nullptr);  // d_norm (RMSNORM): [M] exponents, the 2-norm of a row's activations is below 2^norm
-// Largest sum of squared scales of a row, as float bits, joined by maximum with what *d_out holds.
-hipError_t oxb_launch_row_norm(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t* d_out, hipStream_t st);
+// d_out[i] = 2-norm of matrix row row0 + i (a bound: weights are +-d or 0), infinity where a scale is not finite; with `pair` times
+// that of row row0 + pair + i.  row0, n_rows and pair are multiples of 16.
+hipError_t oxb_launch_row_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t pair, float* d_out, hipStream_t st);
 // What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16, or the wide one
 // with rt row tiles per wave, tpw per workgroup, 16 ct tokens per tile; K in ksplit slices of sb_per_split superblocks.
 struct OxbGemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };

@@ -545,9 +545,9 @@ __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A
 // Exponent that undoes the scaling of token row m, INT32_MIN for a row that holds something non-finite.
 __device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) { return p.xsh ? p.xsh[m] : p.x_exp; }
 
-// SWIGLU with the next product's operand as the output: |gate|, |up| < 2^(w_exp + norm) (Cauchy-Schwarz; a factor of two is
-// left for the roundings), so silu(gate) up 2^shift lies below 2^15.
-__device__ __forceinline__ int swiglu_shift(const OxbGemmParams& p, uint32_t m) { return 14 - 2 * (p.w_exp + p.norm[m]); }
+// SWIGLU with the next product's operand as the output: |silu(gate) up| <= |gate up| < 2^(w_exp + 2 norm) (Cauchy-Schwarz), so that
+// times 2^shift it lies below 2^14, far enough from fp16's end for the roundings on the way.
+__device__ __forceinline__ int swiglu_shift(const OxbGemmParams& p, uint32_t m) { return 14 - p.w_exp - 2 * p.norm[m]; }
 
 // What else the operand of n_rows / 2 values a row needs: the rows' exponents, and zeros in the blocks up to a whole superblock.
 // By one workgroup for `rows` rows from m0 on.
@@ -1006,29 +1006,35 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     reinterpret_cast<float4*>(y)[i] = a;
 }
 
-// Largest sum of squares of the fp16 scales of a row among row tiles [t0, t1), one workgroup per tile; 128 times that bounds the
-// square of every row's 2-norm (weights are +-d or 0).  The maximum of non-negative floats is that of their bits.
-__global__ __launch_bounds__(256) void row_norm_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t t0, uint32_t* __restrict__ out) {
-    __shared__ float part[16][17];
+// 2-norms of the rows of a tile, one workgroup per tile: 128 times the sum of the squares of a row's fp16 scales is the square of
+// its 2-norm (weights are +-d or 0: with zeros among them a bound).  pair_tiles: each times that of the row so many tiles on.
+__global__ __launch_bounds__(256) void row_norms_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t t0, uint32_t pair_tiles, float* __restrict__ out) {
+    __shared__ float part[2][16][17];
     const uint32_t tid = threadIdx.x, r = tid & 15u, j = tid >> 4;
-    const _Float16* s = reinterpret_cast<const _Float16*>(scales) + (size_t)(t0 + blockIdx.x) * n_sb * 64u + r * 4u;
-    float a = 0.f;
-    for (uint32_t sb = j; sb < n_sb; sb += 16)
-        for (int q = 0; q < 4; q++) a = fmaf((float)s[sb * 64u + q], (float)s[sb * 64u + q], a);
-    part[j][r] = a;
-    __syncthreads();
-    if (tid < 16) {
-        for (int i = 1; i < 16; i++) a += part[i][tid];
-        atomicMax(out, a == a ? __float_as_uint(a) : 0x7F800000u);  // (a NaN scale: no bound)
+    for (uint32_t f = 0; f < (pair_tiles ? 2u : 1u); f++) {
+        const _Float16* s = reinterpret_cast<const _Float16*>(scales) + (size_t)(t0 + blockIdx.x + f * pair_tiles) * n_sb * 64u + r * 4u;
+        float a = 0.f;
+        for (uint32_t sb = j; sb < n_sb; sb += 16)
+            for (int q = 0; q < 4; q++) a = fmaf((float)s[sb * 64u + q], (float)s[sb * 64u + q], a);
+        part[f][j][r] = a;
     }
+    __syncthreads();
+    if (tid >= 16) return;
+    float norm = 1.f;
+    for (uint32_t f = 0; f < (pair_tiles ? 2u : 1u); f++) {
+        float a = 0.f;
+        for (int i = 0; i < 16; i++) a += part[f][i][tid];
+        norm *= sqrtf(128.f * a);
+    }
+    out[blockIdx.x * 16u + tid] = norm == norm ? norm : __builtin_inff();
 }
 
 // ---------------------------------------------------------------------------
 // Host-side launchers.
 // ---------------------------------------------------------------------------
-hipError_t oxb_launch_row_norm(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t* d_out, hipStream_t st) {
-    const uint32_t t0 = row0 / 16, t1 = (row0 + n_rows + 15) / 16;
-    hipLaunchKernelGGL(row_norm_kernel, dim3(t1 - t0), dim3(256), 0, st, d_scales, n_sb, t0, d_out);
+hipError_t oxb_launch_row_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t pair, float* d_out, hipStream_t st) {
+    if (((row0 | n_rows | pair) & 15u) != 0 || n_rows == 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(row_norms_kernel, dim3(n_rows / 16), dim3(256), 0, st, d_scales, n_sb, row0 / 16, pair / 16, d_out);
     return hipGetLastError();
 }
 

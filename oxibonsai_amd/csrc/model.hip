@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -80,8 +81,8 @@ struct Model {
                         // nothing else writes it, so the slots of a last vector group's absent vectors stay zero vectors
     // a model loaded from a file owns the weights it uploaded
     std::vector<uint64_t> owned_mats, owned_vecs;
-    // Bounds for the products that hand their operands on (GemmFlow): every gate and up row's 2-norm is below 2^gate_up, every
-    // value row of the cache below 2^value; NO_BOUND where there is none that helps.
+    // Bounds for the products that hand their operands on (GemmFlow): the product of gate row j's and up row j's 2-norms is below
+    // 2^gate_up, every value row of the cache below 2^value; NO_BOUND where there is none that helps.
     struct Bounds { int32_t gate_up, value; };
     std::vector<Bounds> bounds;
     DevBuf norm_buf;
@@ -240,47 +241,67 @@ static int encode_ffn(float* hidden, const float* attn_out, const float* ffn_nor
 // Sequences per pass of the GEMV-based step: all of them up to eight.
 static uint32_t decode_chunk(uint32_t batch) { return batch <= OXB_GEMV_PACKED_MAX_BATCH ? batch : OXB_GEMV_PACKED_MAX_BATCH; }
 
-// Exponent E with sqrt(128 norm2) * by < 2^E.
+// Exponent E with b < 2^E.
 constexpr int32_t NO_BOUND = 1000;
-static int32_t bound_exp(float norm2, double by) {
-    const double b = std::sqrt(128.0 * (double)norm2) * by;
+static int32_t bound_exp(double b) {
     int e = 0;
     if (!std::isfinite(b)) return NO_BOUND;
     if (b > 0.0) (void)std::frexp(b, &e);
     return e < -50 ? -50 : e > 50 ? NO_BOUND : e;
 }
 
+// A bound from a matrix's loudest row helps only where it says something about the others: an operand value v that is stored as
+// fp16(v 2^shift) has its 11 bits down to 2^-14, and the bound puts the largest possible value at 2^14.  What is met lies below
+// that by what Cauchy-Schwarz gives away (about sqrt(h) for each factor, 2^12 for gate times up at h = 4096) and by how much louder
+// the loudest row is than the row in the middle.  Relative error of a product behind the operand, h = 4096, one gate row R times as
+// loud, with the row's own maximum / this bound: R = 16 2.0e-4 / 2.0e-4, 256 2.2e-4 / 2.2e-4, 4096 1.86e-4 / 1.9e-4 and 16 % of the
+// values below 2^-14.  So R = 16 leaves 2^8 for rows of activations that meet the matrix at a worse angle than random ones.  More
+// uneven matrices keep the pack, which finds every row's own maximum.
+constexpr float kEvenRows = 16.f;
+static bool even_rows(const Weight::RowNorms& n) { return n.max <= kEvenRows * n.median; }
+
+static bool row_norms_known(const Weight& w, uint32_t row0, uint32_t pair) { return w.norms.max >= 0.f && w.norms.row0 == row0 && w.norms.pair == pair; }
+
 // Bounds of every layer, from the scales of gate || up and of the value rows of Q || K || V: |W a| <= |W row|_2 |a|_2, and the
 // normalised rows of a layer's input have |a|_2 <= max |norm weight| sqrt(h).  A matrix is looked at once.
 static int find_bounds(Model& m) {
     const oxb_model_desc& d = m.d;
-    const uint32_t v0 = (d.nq + d.nkv) * d.hd;
-    std::vector<Weight*> todo;
+    const uint32_t v0 = (d.nq + d.nkv) * d.hd, kd = d.nkv * d.hd;
+    struct Todo { Weight* w; uint32_t row0, n, pair; };
+    std::vector<Todo> todo;
+    size_t total = 0;
     for (const oxb_layer_ids& ly : m.layers) {
-        Weight *gu = find_weight(ly.gate_up), *qkv = find_weight(ly.qkv);
-        if (gu->norm2 < 0.f || gu->norm_row0 != 0) gu->norm_row0 = 0, gu->norm2 = -1.f, todo.push_back(gu);
-        if (qkv->norm2 < 0.f || qkv->norm_row0 != v0) qkv->norm_row0 = v0, qkv->norm2 = -1.f, todo.push_back(qkv);
+        const Todo t[2] = {{find_weight(ly.gate_up), 0, d.inter, d.inter}, {find_weight(ly.qkv), v0, kd, 0}};
+        for (const Todo& x : t)
+            if (!row_norms_known(*x.w, x.row0, x.pair)) todo.push_back(x), total += x.n;
     }
     if (!todo.empty()) {
-        OXB_TRY(m.norm_buf.ensure(todo.size() * sizeof(float)));
-        OXB_TRY_HIP(clear_now(m.norm_buf.ptr, todo.size() * sizeof(float)), "norm buffer clear");
-        for (size_t i = 0; i < todo.size(); i++) {
-            const Weight& w = *todo[i];
-            OXB_TRY_HIP(oxb_launch_row_norm(w.d_scales, w.L.n_sb, w.norm_row0, w.L.n_rows - w.norm_row0, (uint32_t*)m.norm_buf.ptr + i, g_rt.stream),
-                        "kernel launch failed: row_norm");
+        OXB_TRY(m.norm_buf.ensure(total * sizeof(float)));
+        size_t at = 0;
+        for (const Todo& x : todo) {
+            OXB_TRY_HIP(oxb_launch_row_norms(x.w->d_scales, x.w->L.n_sb, x.row0, x.n, x.pair, (float*)m.norm_buf.ptr + at, g_rt.stream), "kernel launch failed: row_norms");
+            at += x.n;
         }
-        std::vector<float> h(todo.size());
-        OXB_TRY_HIP(hipMemcpyAsync(h.data(), m.norm_buf.ptr, h.size() * sizeof(float), hipMemcpyDeviceToHost, g_rt.stream), "norm download");
+        std::vector<float> h(total);
+        OXB_TRY_HIP(hipMemcpyAsync(h.data(), m.norm_buf.ptr, total * sizeof(float), hipMemcpyDeviceToHost, g_rt.stream), "norm download");
         OXB_TRY_HIP(hipStreamSynchronize(g_rt.stream), "norm download");
-        for (size_t i = 0; i < todo.size(); i++) todo[i]->norm2 = h[i];
+        m.norm_buf.release();
+        auto first = h.begin();
+        for (const Todo& x : todo) {
+            const auto last = first + x.n, mid = first + x.n / 2;
+            std::nth_element(first, mid, last);
+            x.w->norms = {x.row0, x.pair, *std::max_element(mid, last), *mid};
+            first = last;
+        }
     }
     m.bounds.resize(m.layers.size(), {NO_BOUND, -NO_BOUND});
     for (size_t L = 0; L < m.layers.size(); L++) {
         const oxb_layer_ids& ly = m.layers[L];
-        m.bounds[L].gate_up = bound_exp(find_weight(ly.gate_up)->norm2, 1.0);
+        const Weight::RowNorms &gu = find_weight(ly.gate_up)->norms, &v = find_weight(ly.qkv)->norms;
+        m.bounds[L].gate_up = even_rows(gu) ? bound_exp(gu.max) : NO_BOUND;
         // (rows that an earlier matrix wrote may still be in the cache: the bound only grows)
-        const int32_t v = bound_exp(find_weight(ly.qkv)->norm2, (double)g_rt.vectors[ly.attn_norm].absmax * std::sqrt((double)d.h));
-        if (v > m.bounds[L].value) m.bounds[L].value = v;
+        const int32_t e = bound_exp((double)v.max * (double)g_rt.vectors[ly.attn_norm].absmax * std::sqrt((double)d.h));
+        if (e > m.bounds[L].value) m.bounds[L].value = e;
     }
     return OXB_HIP_OK;
 }

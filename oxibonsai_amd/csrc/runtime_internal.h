@@ -36,7 +36,7 @@ struct GemmFlow {
     enum In { PACK, ATTENTION, SWIGLU } in = PACK;  // where the operand comes from: packed here; left in xh (exponent x_exp in every row) or in xh2
     int32_t x_exp = 0;
     bool out = false;     // mode SWIGLU: the result goes to xh2 / xsh2, for a down projection of the same format
-    int32_t w_exp = 0;    // ... every row's 2-norm is below 2^w_exp
+    int32_t w_exp = 0;    // ... the product of gate row j's and up row j's 2-norms is below 2^w_exp for every j
 };
 
 // One resident matrix: [codes section][scales section].  A weight uploaded as bytes alone (the reference's
@@ -49,10 +49,9 @@ struct Weight {
     uint16_t* d_scales = nullptr;
     void* d_raw = nullptr;
     size_t raw_blocks = 0;
-    // largest sum of squared scales of a row from row norm_row0 on (128 times that is the square of the largest 2-norm);
-    // negative: not worked out yet
-    uint32_t norm_row0 = 0;
-    float norm2 = -1.f;
+    // Largest and median of the 2-norms of the rows from row `row0` on, or with `pair` of the products of those of rows row0 + i and
+    // row0 + pair + i; negative: not worked out yet.
+    struct RowNorms { uint32_t row0 = 0, pair = 0; float max = -1.f, median = -1.f; } norms;
 };
 
 struct Vector {  // a resident fp32 vector (norm weights)
