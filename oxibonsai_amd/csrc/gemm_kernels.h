@@ -29,11 +29,12 @@ struct OxbGemmParams {
     uint32_t codes_bytes, scales_bytes, xh_bytes;  // buffer extents (loads beyond them read 0)
     int mode;
     // Mode SWIGLU, optional: instead of y the packed activations of the product that follows (n_rows / 2 values a row, a multiple
-    // of 128; its format is this matrix's) and their exponents.  norm: |a|_2 < 2^norm of every row (oxb_launch_xh_pack),
-    // w_exp: |gate row j|_2 |up row j|_2 < 2^w_exp for every j.
+    // of 128; its format is this matrix's) and their exponents.  norm2: |a|_2^2 of every row at most (OxbPackNorm);
+    // |gate row j|_2 |up row j|_2 <= w_mant 2^w_exp for every j, w_mant in [0.5, 1).
     uint32_t* xh_out;
     int32_t* xsh_out;
-    const int32_t* norm;
+    const float* norm2;
+    float w_mant;
     int32_t w_exp;
     bool no_split;           // keep K in one piece (a caller without room for partial sums)
     bool sum_later;          // mode RESIDUAL: with K in slices leave the sums in `part`, the next pack of y adds them (OxbPackSum)
@@ -51,9 +52,12 @@ enum { OXB_PACK_IDENT = 0, OXB_PACK_RMSNORM = 1 };
 // result of: x += planes 0 .. n - 1, in that order, then as above; x is written back.
 struct OxbPackSum { const float* part; uint32_t n; size_t plane; };
 bool oxb_pack_can_sum(uint32_t k, uint32_t M);
+// RMSNORM, optional: norm2[m] is no less than the square of the 2-norm of row m's activations (and never 0); cap is such a bound for
+// every row, from the norm weights: max |w|^2 k.
+struct OxbPackNorm { float* norm2; float cap; };
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
                               uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr,
-                              int32_t* d_norm = nullptr);  // d_norm (RMSNORM): [M] exponents, the 2-norm of a row's activations is below 2^norm
+                              OxbPackNorm norm = {nullptr, 0.f});
 // d_out[i] = 2-norm of matrix row row0 + i (a bound: weights are +-d or 0), infinity where a scale is not finite; with `pair` times
 // that of row row0 + pair + i.  row0, n_rows and pair are multiples of 16.
 hipError_t oxb_launch_row_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t pair, float* d_out, hipStream_t st);

@@ -51,13 +51,13 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 __device__ __forceinline__ float sum_sq(const float4& a, float s) { return fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, fmaf(a.w, a.w, s)))); }
 __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
-// What the packer says about one token row: its multiplier, the exponent that undoes the power of two, and (RMSNORM) an
-// exponent above the 2-norm of its activations, |a|_2 < 2^norm.
-struct RowScale { float mul; int32_t xsh, norm; };
+// What the packer says about one token row: its multiplier, the exponent that undoes the power of two, and (RMSNORM) no less than
+// the square of the 2-norm of its activations.
+struct RowScale { float mul; int32_t xsh; float norm2; };
 // ... from the row's sum of squares, that of its |a| before the producer's scalar, the largest of those and whether it holds
 // something non-finite.
 template <int OP>
-__device__ __forceinline__ RowScale row_scale(float ss, float sa, float mx, int bad, uint32_t k, float eps) {
+__device__ __forceinline__ RowScale row_scale(float ss, float sa, float mx, int bad, uint32_t k, float eps, float cap) {
     float scalar = 1.0f;
     if (OP == OXB_PACK_RMSNORM) {
         scalar = 1.0f / sqrtf(ss / (float)k + eps);
@@ -67,25 +67,27 @@ __device__ __forceinline__ RowScale row_scale(float ss, float sa, float mx, int 
     int E = 0;
     if (mx > 0.0f) (void)frexpf(mx, &E);  // mx = f * 2^E, f in [0.5, 1)
     const int shift = mx > 0.0f ? 15 - E : 0;
-    int N = -64;
-    if (OP == OXB_PACK_RMSNORM) {
-        // (a sum of squares that overflows comes from values whose norm the products' fp32 sums could not hold either)
-        const float norm = sqrtf(sa) * scalar;
-        if (norm > 0.0f) (void)frexpf(fminf(norm, 3.402823466e38f), &N);
-        N = N < -64 ? -64 : N;
+    float norm2 = 1.0f;
+    if (OP == OXB_PACK_RMSNORM && !bad) {
+        // The squares are added up before the scalar: where their sum has left fp32's range at either end (a residual of 1e18 under a
+        // norm weight of 20, a row of 1e-24 under a tiny eps) the largest |a| and the norm weights' bound take its place.  The
+        // latter needs a sum of squares of x that has lost nothing to the lower end.
+        norm2 = sa >= 0x1p-100f && sa <= 3.402823466e38f ? sa * scalar * scalar : (float)k * mx * mx;
+        if (ss >= 0x1p-100f) norm2 = fminf(norm2, cap);
+        norm2 = fmaxf(fminf(norm2, 3.402823466e38f), (float)k * 0x1p-126f);  // (products below that are lost to the lower end)
     }
-    return {bad ? 0.0f : ldexpf(scalar, shift), bad ? INT32_MIN : -shift, bad ? 0 : N};
+    return {bad ? 0.0f : ldexpf(scalar, shift), bad ? INT32_MIN : -shift, norm2};
 }
 
 // The threads' partial results (sums of squares of x and of a, largest |a|, non-finite seen) joined; all 256 threads of the
 // workgroup call it, thread 0 gets the result.
 struct RowRed { float s[4], a[4], m[4]; int b[4]; };
 template <int OP>
-__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, RowRed& red);
+__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, float cap, RowRed& red);
 
 // The same with the pass over the row in front: a float4 per thread and step, in row order.
 template <int OP>
-__device__ __forceinline__ RowScale row_stats(const float* __restrict__ xr, const float* __restrict__ w, uint32_t k, float eps, RowRed& red) {
+__device__ __forceinline__ RowScale row_stats(const float* __restrict__ xr, const float* __restrict__ w, uint32_t k, float eps, float cap, RowRed& red) {
     const uint32_t tid = threadIdx.x;
     float ss = 0.f, sa = 0.f, mx = 0.f;
     int bad = 0;
@@ -102,32 +104,32 @@ __device__ __forceinline__ RowScale row_stats(const float* __restrict__ xr, cons
                !(fabsf(a.w) <= 3.402823466e38f);
         mx = fmaxf(fmaxf(mx, fmaxf(fabsf(a.x), fabsf(a.y))), fmaxf(fabsf(a.z), fabsf(a.w)));
     }
-    return row_finish<OP>(ss, sa, mx, bad, k, eps, red);
+    return row_finish<OP>(ss, sa, mx, bad, k, eps, cap, red);
 }
 
 template <int OP>
-__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, RowRed& red) {
+__device__ __forceinline__ RowScale row_finish(float ss, float sa, float mx, int bad, uint32_t k, float eps, float cap, RowRed& red) {
     const uint32_t tid = threadIdx.x;
     if (OP == OXB_PACK_RMSNORM) ss = wave_sum_f32(ss), sa = wave_sum_f32(sa);  // DPP and lane swaps: no trips through the LDS pipeline
     mx = wave_max_f32(mx);
     bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
     if ((tid & 63u) == 0) red.s[tid >> 6] = ss, red.a[tid >> 6] = sa, red.m[tid >> 6] = mx, red.b[tid >> 6] = bad;
     __syncthreads();
-    if (tid) return {0.f, 0, 0};
+    if (tid) return {0.f, 0, 0.f};
     return row_scale<OP>(red.s[0] + red.s[1] + red.s[2] + red.s[3], red.a[0] + red.a[1] + red.a[2] + red.a[3],
-                         fmaxf(fmaxf(red.m[0], red.m[1]), fmaxf(red.m[2], red.m[3])), red.b[0] | red.b[1] | red.b[2] | red.b[3], k, eps);
+                         fmaxf(fmaxf(red.m[0], red.m[1]), fmaxf(red.m[2], red.m[3])), red.b[0] | red.b[1] | red.b[2] | red.b[3], k, eps, cap);
 }
 
 template <int OP>
 __global__ __launch_bounds__(256) void row_stats_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                          uint32_t ldx, uint32_t k, float eps, float* __restrict__ rowmul,
-                                                         int32_t* __restrict__ xsh, int32_t* __restrict__ norm) {
+                                                         int32_t* __restrict__ xsh, const OxbPackNorm norm) {
     __shared__ RowRed red;
     const uint32_t m = blockIdx.x;
-    const RowScale r = row_stats<OP>(x + (size_t)m * ldx, w, k, eps, red);
+    const RowScale r = row_stats<OP>(x + (size_t)m * ldx, w, k, eps, norm.cap, red);
     if (threadIdx.x) return;
     rowmul[m] = r.mul, xsh[m] = r.xsh;
-    if (norm) norm[m] = r.norm;
+    if (norm.norm2) norm.norm2[m] = r.norm2;
 }
 
 // The eight activations of token row xr that chunk c = 4g + s of block blk holds, scaled by mul, as four fp16 pairs.
@@ -172,7 +174,7 @@ __device__ __forceinline__ float4 add4(const float4& a, const float4& b) { retur
 template <int FMT, int OP, int NI, bool SUM>
 __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float* __restrict__ w, uint32_t ldx,
                                                             uint32_t k, float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, int32_t* __restrict__ norm, uint4* __restrict__ xh, const OxbPackSum sum) {
+                                                            int32_t* __restrict__ xsh, const OxbPackNorm norm, uint4* __restrict__ xh, const OxbPackSum sum) {
     __shared__ RowRed red;
     __shared__ float mul_s;
     const uint32_t m = blockIdx.x, tid = threadIdx.x, n_items = nblk_pad * 16;
@@ -253,10 +255,10 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
             mx = fmaxf(mx, fabsf(v[e]));
         }
     }
-    const RowScale rs = row_finish<OP>(ss, sa, mx, bad, k, eps, red);
+    const RowScale rs = row_finish<OP>(ss, sa, mx, bad, k, eps, norm.cap, red);
     if (tid == 0) {
         mul_s = rs.mul, xsh[m] = rs.xsh;
-        if (OP == OXB_PACK_RMSNORM && norm) norm[m] = rs.norm;
+        if (OP == OXB_PACK_RMSNORM && norm.norm2) norm.norm2[m] = rs.norm2;
     }
     __syncthreads();
     const float mul = mul_s;
@@ -281,7 +283,7 @@ __global__ __launch_bounds__(256) void xh_pack_rows_kernel(float* x, const float
 template <int FMT, int OP, int RPW, int NI, bool SUM>
 __global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float* __restrict__ w, uint32_t ldx, uint32_t k,
                                                             float eps, uint32_t M, uint32_t M_pad, uint32_t nblk_pad,
-                                                            int32_t* __restrict__ xsh, int32_t* __restrict__ norm, uint4* __restrict__ xh, const OxbPackSum sum) {
+                                                            int32_t* __restrict__ xsh, const OxbPackNorm norm, uint4* __restrict__ xh, const OxbPackSum sum) {
     constexpr int WPR = 8 / RPW, SEG = NI <= 16 ? NI : NI == 48 ? 16 : 12;
     static_assert(NI % SEG == 0, "whole segments");
     constexpr uint32_t VALS = SEG * 256 * WPR, STR = VALS + 16;  // values of a row in a segment; LDS row stride (32 bytes of padding spread the rows over the banks)
@@ -346,11 +348,11 @@ __global__ __launch_bounds__(512) void xh_pack_wide_kernel(float* x, const float
 #pragma unroll
         for (int i = 1; i < WPR; i++) ss += red_s[wr * WPR + i], sa += red_a[wr * WPR + i], mx = fmaxf(mx, red_m[wr * WPR + i]), bad |= red_b[wr * WPR + i];
     }
-    const RowScale rs = row_scale<OP>(ss, sa, mx, bad, k, eps);
+    const RowScale rs = row_scale<OP>(ss, sa, mx, bad, k, eps, norm.cap);
     const float mul = live ? rs.mul : 0.f;
     if (live && part == 0 && lane == 0) {
         xsh[m] = rs.xsh;
-        if (OP == OXB_PACK_RMSNORM && norm) norm[m] = rs.norm;
+        if (OP == OXB_PACK_RMSNORM && norm.norm2) norm.norm2[m] = rs.norm2;
     }
 #pragma unroll
     for (int i0 = 0; i0 < NI; i0 += SEG) {
@@ -545,9 +547,13 @@ __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A
 // Exponent that undoes the scaling of token row m, INT32_MIN for a row that holds something non-finite.
 __device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) { return p.xsh ? p.xsh[m] : p.x_exp; }
 
-// SWIGLU with the next product's operand as the output: |silu(gate) up| <= |gate up| < 2^(w_exp + 2 norm) (Cauchy-Schwarz), so that
-// times 2^shift it lies below 2^14, far enough from fp16's end for the roundings on the way.
-__device__ __forceinline__ int swiglu_shift(const OxbGemmParams& p, uint32_t m) { return 14 - p.w_exp - 2 * p.norm[m]; }
+// SWIGLU with the next product's operand as the output: |silu(gate) up| <= |gate up| <= w_mant 2^w_exp norm2 (Cauchy-Schwarz), so that
+// times 2^shift it lies below 2^15: a factor of two from fp16's end for the roundings on the way.
+__device__ __forceinline__ int swiglu_shift(const OxbGemmParams& p, uint32_t m) {
+    int e;
+    (void)frexpf(p.w_mant * p.norm2[m], &e);
+    return 15 - p.w_exp - e;
+}
 
 // What else the operand of n_rows / 2 values a row needs: the rows' exponents, and zeros in the blocks up to a whole superblock.
 // By one workgroup for `rows` rows from m0 on.
@@ -1047,17 +1053,17 @@ size_t oxb_xh_bytes(uint32_t k, uint32_t M) {
 
 template <int OP, bool SUM>
 static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, uint32_t k, uint32_t M, uint32_t M_pad,
-                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, int32_t* d_norm, const OxbPackSum& sum, hipStream_t st) {
+                           uint32_t nblk_pad, float eps, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, OxbPackNorm norm, const OxbPackSum& sum, hipStream_t st) {
     const uint32_t per_thread = (nblk_pad * 16 + 255) / 256;  // items of a row per thread of the one-launch packer
     if (M <= OXB_PACK_ROWS_MAX && per_thread <= 8) {
 #define OXB_ROWS_CASE(NI)                                                                                                      \
     if (per_thread <= NI) {                                                                                                    \
         if (fmt == OXB_FMT_Q1)                                                                                                 \
             hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_Q1, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
+                               M_pad, nblk_pad, d_xsh, norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         else                                                                                                                   \
             hipLaunchKernelGGL((xh_pack_rows_kernel<OXB_FMT_TQ2, OP, NI, SUM>), dim3(M_pad), dim3(256), 0, st, d_x, d_w, ldx, k, eps, M, \
-                               M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
+                               M_pad, nblk_pad, d_xsh, norm, reinterpret_cast<uint4*>(d_xh), sum);                                   \
         return;                                                                                                                \
     }
         OXB_ROWS_CASE(1) OXB_ROWS_CASE(2) OXB_ROWS_CASE(4)
@@ -1073,10 +1079,10 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
     if (rpw == RPW && per_lane <= NI) {                                                                                            \
         if (fmt == OXB_FMT_Q1)                                                                                                     \
             hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_Q1, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
         else                                                                                                                       \
             hipLaunchKernelGGL((xh_pack_wide_kernel<OXB_FMT_TQ2, OP, RPW, NI, SUM>), dim3(M_pad / RPW), dim3(512), 0, st, d_x, d_w, ldx, \
-                               k, eps, M, M_pad, nblk_pad, d_xsh, d_norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
+                               k, eps, M, M_pad, nblk_pad, d_xsh, norm, reinterpret_cast<uint4*>(d_xh), sum);                            \
         return;                                                                                                                    \
     }
     OXB_WIDE_CASE(4, 8) OXB_WIDE_CASE(4, 16)
@@ -1086,7 +1092,7 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
     // (rows of more than 12288 values take two launches)
 #undef OXB_WIDE_CASE
     if constexpr (!SUM) {
-        hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh, d_norm);
+        hipLaunchKernelGGL(row_stats_kernel<OP>, dim3(M), dim3(256), 0, st, d_x, d_w, ldx, k, eps, d_rowmul, d_xsh, norm);
         const dim3 grid(M_pad / 16, nblk_pad < 16 ? nblk_pad : 16);
         if (fmt == OXB_FMT_Q1)
             hipLaunchKernelGGL((xh_pack_kernel<OXB_FMT_Q1, OP>), grid, dim3(256), 0, st, d_x, d_w, ldx, k, M, M_pad, nblk_pad, d_rowmul,
@@ -1100,7 +1106,7 @@ static void launch_pack_op(int fmt, float* d_x, const float* d_w, uint32_t ldx, 
 bool oxb_pack_can_sum(uint32_t k, uint32_t M) { return k <= (M <= OXB_PACK_ROWS_MAX ? 8192u : 12288u) && (k % OXB_QK) == 0; }
 
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
-                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum, int32_t* d_norm) {
+                              uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum, OxbPackNorm norm) {
     if (M == 0 || k == 0 || (k % OXB_QK) != 0 || (ldx & 3u) != 0) return hipErrorInvalidValue;
     if (op == OXB_PACK_RMSNORM && !d_w) return hipErrorInvalidValue;
     const uint32_t nblk_pad = ((k + 511u) / 512u) * 4u, M_pad = (M + 15u) / 16u * 16u;
@@ -1108,13 +1114,13 @@ hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_
     float* x = const_cast<float*>(d_x);  // (written with `sum` only)
     if (sum && sum->n > 1) {
         if (op != OXB_PACK_RMSNORM || !oxb_pack_can_sum(k, M) || ldx != k) return hipErrorInvalidValue;
-        launch_pack_op<OXB_PACK_RMSNORM, true>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, *sum, st);
+        launch_pack_op<OXB_PACK_RMSNORM, true>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, norm, *sum, st);
         return hipGetLastError();
     }
     const OxbPackSum none = {nullptr, 0, 0};
     switch (op) {
-        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, none, st); break;
-        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, d_norm, none, st); break;
+        case OXB_PACK_IDENT: launch_pack_op<OXB_PACK_IDENT, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, norm, none, st); break;
+        case OXB_PACK_RMSNORM: launch_pack_op<OXB_PACK_RMSNORM, false>(fmt, x, d_w, ldx, k, M, M_pad, nblk_pad, eps, d_rowmul, d_xh, d_xsh, norm, none, st); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1241,7 +1247,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     if (p.M == 0 || p.n_rows == 0) return hipSuccess;
     if (p.n_sb == 0 || (uint64_t)p.n_tiles * p.n_sb * 2048ull >= 0xFFFFFFF0ull) return hipErrorInvalidValue;
     if (p.mode == OXB_GEMM_SWIGLU && (p.n_rows & 31u) != 0) return hipErrorInvalidValue;  // whole gate and up row tiles
-    if (p.xh_out && (p.mode != OXB_GEMM_SWIGLU || (p.n_rows & 255u) != 0 || !p.xsh_out || !p.norm)) return hipErrorInvalidValue;  // whole blocks
+    if (p.xh_out && (p.mode != OXB_GEMM_SWIGLU || (p.n_rows & 255u) != 0 || !p.xsh_out || !p.norm2)) return hipErrorInvalidValue;  // whole blocks
     p.M_pad = (p.M + 15u) / 16u * 16u;
     const OxbGemmPlan plan = oxb_gemm_plan(fmt, p, n_cus);
     p.ksplit = plan.ksplit;

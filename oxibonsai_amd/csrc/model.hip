@@ -81,9 +81,10 @@ struct Model {
                         // nothing else writes it, so the slots of a last vector group's absent vectors stay zero vectors
     // a model loaded from a file owns the weights it uploaded
     std::vector<uint64_t> owned_mats, owned_vecs;
-    // Bounds for the products that hand their operands on (GemmFlow): the product of gate row j's and up row j's 2-norms is below
-    // 2^gate_up, every value row of the cache below 2^value; NO_BOUND where there is none that helps.
-    struct Bounds { int32_t gate_up, value; };
+    // Bounds for the products that hand their operands on (GemmFlow): the product of gate row j's and up row j's 2-norms is at most
+    // gate_up, the square of an FFN input's at most norm2_cap, every value row of the cache below 2^value; 0 (NO_BOUND) where there is
+    // none that helps.
+    struct Bounds { float gate_up, norm2_cap; int32_t value; };
     std::vector<Bounds> bounds;
     DevBuf norm_buf;
     DevBuf tok_hist, tok_ids;  // token history of the on-device generation loop; prompt ids of a token prefill
@@ -251,7 +252,7 @@ static int32_t bound_exp(double b) {
 }
 
 // A bound from a matrix's loudest row helps only where it says something about the others: an operand value v that is stored as
-// fp16(v 2^shift) has its 11 bits down to 2^-14, and the bound puts the largest possible value at 2^14.  What is met lies below
+// fp16(v 2^shift) has its 11 bits down to 2^-14, and the bound puts the largest possible value at 2^15.  What is met lies below
 // that by what Cauchy-Schwarz gives away (about sqrt(h) for each factor, 2^12 for gate times up at h = 4096) and by how much louder
 // the loudest row is than the row in the middle.  Relative error of a product behind the operand, h = 4096, one gate row R times as
 // loud, with the row's own maximum / this bound: R = 16 2.0e-4 / 2.0e-4, 256 2.2e-4 / 2.2e-4, 4096 1.86e-4 / 1.9e-4 and 16 % of the
@@ -294,11 +295,14 @@ static int find_bounds(Model& m) {
             first = last;
         }
     }
-    m.bounds.resize(m.layers.size(), {NO_BOUND, -NO_BOUND});
+    m.bounds.resize(m.layers.size(), {0.f, 0.f, -NO_BOUND});
     for (size_t L = 0; L < m.layers.size(); L++) {
         const oxb_layer_ids& ly = m.layers[L];
         const Weight::RowNorms &gu = find_weight(ly.gate_up)->norms, &v = find_weight(ly.qkv)->norms;
-        m.bounds[L].gate_up = even_rows(gu) ? bound_exp(gu.max) : NO_BOUND;
+        // (the range that the products' exponents are worked out in: far wider than that of weights and norms in use)
+        const double w = g_rt.vectors[ly.ffn_norm].absmax, cap = w * w * d.h;
+        m.bounds[L].gate_up = even_rows(gu) && gu.max < 0x1p50f && cap < 0x1p50 ? std::max(gu.max, 0x1p-50f) : 0.f;
+        m.bounds[L].norm2_cap = (float)cap * (1.f + 0x1p-10f);
         // (rows that an earlier matrix wrote may still be in the cache: the bound only grows)
         const int32_t e = bound_exp((double)v.max * (double)g_rt.vectors[ly.attn_norm].absmax * std::sqrt((double)d.h));
         if (e > m.bounds[L].value) m.bounds[L].value = e;
@@ -310,8 +314,9 @@ static int find_bounds(Model& m) {
 static bool attn_hands_on(const Model& m, uint32_t L) { return m.bounds[L].value < NO_BOUND && (m.d.nq * m.d.hd) % 512u == 0; }
 static GemmFlow flow_gate_up(const Model& m, uint32_t L) {
     GemmFlow f;
-    f.out = m.bounds[L].gate_up < NO_BOUND && m.d.inter % OXB_QK == 0;
-    f.w_exp = m.bounds[L].gate_up;
+    f.out = m.bounds[L].gate_up > 0.f && m.d.inter % OXB_QK == 0;
+    f.w_norm2 = m.bounds[L].gate_up;
+    f.norm2_cap = m.bounds[L].norm2_cap;
     return f;
 }
 static GemmFlow flow_down(const Model& m, uint32_t L) {

@@ -296,7 +296,7 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
         if ((rc = ws->xh.ensure(oxb_xh_bytes(k, m))) || (rc = ws->xsh.ensure(rows4)) || (rc = ws->rowmul.ensure(rows4))) return rc;
         if (flow.out && (rc = ws->norm.ensure(rows4))) return rc;
         e = oxb_launch_xh_pack((int)w.L.fmt, pack_op, d_x, d_pack_w, ldx, k, eps, m, (float*)ws->rowmul.ptr, (uint32_t*)ws->xh.ptr, (int32_t*)ws->xsh.ptr,
-                               g_rt.stream, pack_op == OXB_PACK_RMSNORM ? carry : nullptr, flow.out ? (int32_t*)ws->norm.ptr : nullptr);
+                               g_rt.stream, pack_op == OXB_PACK_RMSNORM ? carry : nullptr, flow.out ? OxbPackNorm{(float*)ws->norm.ptr, flow.norm2_cap} : OxbPackNorm{nullptr, 0.f});
         if (e != hipSuccess) return hip_fail(e, "kernel launch failed: xh_pack");
     } else if ((flow.in == GemmFlow::ATTENTION ? ws->xh.cap : ws->xh2.cap) < oxb_xh_bytes(k, m) || (carry && carry->n > 1))
         return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: no operand of %u rows x %u", m, k);
@@ -309,7 +309,7 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
     p.xh = (const uint32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xh2.ptr : ws->xh.ptr);
     p.xsh = flow.in == GemmFlow::ATTENTION ? nullptr : (const int32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xsh2.ptr : ws->xsh.ptr);
     p.x_exp = flow.x_exp;
-    if (flow.out) p.xh_out = (uint32_t*)ws->xh2.ptr, p.xsh_out = (int32_t*)ws->xsh2.ptr, p.norm = (const int32_t*)ws->norm.ptr, p.w_exp = flow.w_exp;
+    if (flow.out) p.xh_out = (uint32_t*)ws->xh2.ptr, p.xsh_out = (int32_t*)ws->xsh2.ptr, p.norm2 = (const float*)ws->norm.ptr, p.w_mant = frexpf(flow.w_norm2, &p.w_exp);
     p.y = d_y;
     p.residual = d_residual;
     p.n_rows = w.L.n_rows;

@@ -26,7 +26,7 @@ struct DevBuf {  // grow-only device scratch
 // own that never move.
 struct GemmWorkspace {
     DevBuf xh, xsh, rowmul, part;
-    DevBuf norm, xh2, xsh2;  // GemmFlow: the rows' norms, and the operand that a SwiGLU product leaves for the next
+    DevBuf norm, xh2, xsh2;  // GemmFlow: the squares of the rows' norms, and the operand that a SwiGLU product leaves for the next
     bool no_split = false;  // no room for partial sums: K stays in one piece
     void release() { xh.release(); xsh.release(); rowmul.release(); part.release(); norm.release(); xh2.release(); xsh2.release(); }
 };
@@ -36,7 +36,7 @@ struct GemmFlow {
     enum In { PACK, ATTENTION, SWIGLU } in = PACK;  // where the operand comes from: packed here; left in xh (exponent x_exp in every row) or in xh2
     int32_t x_exp = 0;
     bool out = false;     // mode SWIGLU: the result goes to xh2 / xsh2, for a down projection of the same format
-    int32_t w_exp = 0;    // ... the product of gate row j's and up row j's 2-norms is below 2^w_exp for every j
+    float w_norm2 = 0.f, norm2_cap = 0.f;  // ... at most the product of gate row j's and up row j's 2-norms for every j; OxbPackNorm::cap
 };
 
 // One resident matrix: [codes section][scales section].  A weight uploaded as bytes alone (the reference's

@@ -320,3 +320,36 @@ def test_uneven_rows_leave_the_other_outputs_their_precision(backend, fmt, ctx, 
             lw["down"] = _scaled(fmt, lw["down"], 1152, slice(None), 1 / loud, block=0)
     err = _second_layer_errors(backend, cfg, w, _rows(31, ctx + n * batch, 512), ctx, batch)
     assert np.median(err) <= 1.4e-3
+
+
+# One residual of 1e18 where the FFN's norm weight is 20: the sum of the squares in front of the division by the root mean square is
+# beyond fp32's range, the normalised activations are not.  Rows of 1e-22 with an eps to match and norm weights of 0.01: their squares are 0.
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("n,batch", [(1, 1), (21, 1), (70, 1), (1, 9)])
+@pytest.mark.parametrize("case", ["loud", "quiet"])
+def test_swiglu_outputs_of_rows_at_the_ends_of_the_range(backend, fmt, n, batch, case):
+    """The logits have a few fp16 roundings of the FFN's values behind them, 2^-12 of each at most: 1e-3 of the row."""
+    cfg = dict(fmt=fmt, n_layers=1, h=512, inter=1152, nq=8, nkv=2, hd=64, vocab=96, max_seq=n + 8, eps=1e-6 if case == "loud" else 2e-38, rope_theta=1e6)
+    w = synth.make_model(cfg, 5)
+    lw, rows = w["layers"][0], _rows(17, n * batch, 512)
+    if case == "loud":
+        rows[:, 5] = 1e18
+        lw["ffn_norm"] = lw["ffn_norm"].copy()
+        lw["ffn_norm"][5] = 20.0
+        w["final_norm"] = w["final_norm"].copy()
+        w["final_norm"][5] = 0.0           # the logits are those of the other 511 values
+    else:
+        rows *= np.float32(1e-22)
+        lw["ffn_norm"] = lw["ffn_norm"] * np.float32(0.01)
+        lw["o"] = _scaled(fmt, lw["o"], 512, slice(None), 0.0)
+    cpu = oracle.OracleModel(cfg, w, kv_f16=True)
+    gpu = HipModel(backend, cfg, w, batch=batch)
+    try:
+        got = gpu.forward(rows, 0)[0] if batch > 1 else gpu.prefill(rows, 0)[0][None]
+        for b in range(batch):
+            want = cpu.forward(rows[b], 0) if batch > 1 else _oracle_logits(cpu, rows)
+            err = np.sqrt(np.mean((got[b].astype(np.float64) - want) ** 2) / np.mean(want.astype(np.float64) ** 2))
+            print(f"{err:.2e}")
+            assert err <= 1e-3
+    finally:
+        gpu.close()
