@@ -58,9 +58,12 @@ struct OxbPackNorm { float* norm2; float cap; };
 hipError_t oxb_launch_xh_pack(int fmt, int op, const float* d_x, const float* d_w, uint32_t ldx, uint32_t k, float eps,
                               uint32_t M, float* d_rowmul, uint32_t* d_xh, int32_t* d_xsh, hipStream_t st, const OxbPackSum* sum = nullptr,
                               OxbPackNorm norm = {nullptr, 0.f});
-// d_out[i] = 2-norm of matrix row row0 + i (a bound: weights are +-d or 0), infinity where a scale is not finite; with `pair` times
-// that of row row0 + pair + i.  row0, n_rows and pair are multiples of 16.
-hipError_t oxb_launch_row_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t pair, float* d_out, hipStream_t st);
+// d_out[i] = the 2-norm of matrix row i times that of row n + i, i < n (bounds: weights are +-d or 0), infinity where a scale is not
+// finite.  n is a multiple of 16.
+hipError_t oxb_launch_pair_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t n, float* d_out, hipStream_t st);
+// d_out[i] = the 2-norm of matrix row row0 + i with column j times w[j], i < n, and d_out[n + i] the same with no |w[j]| taken as more
+// than `typical`.  row0 and n are multiples of 16.
+hipError_t oxb_launch_weighted_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n, const float* d_w, uint32_t k, float typical, float* d_out, hipStream_t st);
 // What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16, or the wide one
 // with rt row tiles per wave, tpw per workgroup, 16 ct tokens per tile; K in ksplit slices of sb_per_split superblocks.
 struct OxbGemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };

@@ -1012,35 +1012,64 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     reinterpret_cast<float4*>(y)[i] = a;
 }
 
-// 2-norms of the rows of a tile, one workgroup per tile: 128 times the sum of the squares of a row's fp16 scales is the square of
-// its 2-norm (weights are +-d or 0: with zeros among them a bound).  pair_tiles: each times that of the row so many tiles on.
-__global__ __launch_bounds__(256) void row_norms_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t t0, uint32_t pair_tiles, float* __restrict__ out) {
-    __shared__ float part[2][16][17];
+// The square of the 2-norm of each row of a tile (weights are +-d or 0: with zeros among them a bound), in threads 0 .. 15: the sum
+// over its blocks of the scale's square times weight(block), 128 where all inputs count alike.
+template <class F>
+__device__ __forceinline__ float tile_row_norms2(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t tile, float (&part)[16][17], F weight) {
     const uint32_t tid = threadIdx.x, r = tid & 15u, j = tid >> 4;
-    for (uint32_t f = 0; f < (pair_tiles ? 2u : 1u); f++) {
-        const _Float16* s = reinterpret_cast<const _Float16*>(scales) + (size_t)(t0 + blockIdx.x + f * pair_tiles) * n_sb * 64u + r * 4u;
-        float a = 0.f;
-        for (uint32_t sb = j; sb < n_sb; sb += 16)
-            for (int q = 0; q < 4; q++) a = fmaf((float)s[sb * 64u + q], (float)s[sb * 64u + q], a);
-        part[f][j][r] = a;
-    }
+    const _Float16* s = reinterpret_cast<const _Float16*>(scales) + (size_t)tile * n_sb * 64u + r * 4u;
+    float a = 0.f;
+    for (uint32_t sb = j; sb < n_sb; sb += 16)
+        for (uint32_t q = 0; q < 4; q++) {
+            const float d = (float)s[sb * 64u + q];
+            a = fmaf(d * d, weight(sb * 4u + q), a);
+        }
     __syncthreads();
-    if (tid >= 16) return;
-    float norm = 1.f;
-    for (uint32_t f = 0; f < (pair_tiles ? 2u : 1u); f++) {
-        float a = 0.f;
-        for (int i = 0; i < 16; i++) a += part[f][i][tid];
-        norm *= sqrtf(128.f * a);
+    part[j][r] = a;
+    __syncthreads();
+    a = 0.f;
+    if (tid < 16)
+        for (int i = 0; i < 16; i++) a += part[i][tid];
+    return a;
+}
+__device__ __forceinline__ float norm_or_inf(float n) { return n == n ? n : __builtin_inff(); }
+
+__global__ __launch_bounds__(256) void pair_norms_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t pair_tiles, float* __restrict__ out) {
+    __shared__ float part[16][17];
+    auto all = [](uint32_t) -> float { return 128.f; };
+    const float a = tile_row_norms2(scales, n_sb, blockIdx.x, part, all), b = tile_row_norms2(scales, n_sb, blockIdx.x + pair_tiles, part, all);
+    if (threadIdx.x < 16) out[blockIdx.x * 16u + threadIdx.x] = norm_or_inf(sqrtf(a) * sqrtf(b));
+}
+
+__global__ __launch_bounds__(256) void weighted_norms_kernel(const uint16_t* __restrict__ scales, uint32_t n_sb, uint32_t t0, const float* __restrict__ w,
+                                                             uint32_t k, float typical, float* __restrict__ out) {
+    __shared__ float part[16][17];
+    for (uint32_t f = 0; f < 2; f++) {
+        const float most = f ? typical : __builtin_inff();
+        const float a = tile_row_norms2(scales, n_sb, t0 + blockIdx.x, part, [&](uint32_t blk) -> float {
+            float s = 0.f;
+            for (uint32_t i = blk * 128u; i < blk * 128u + 128u && i < k; i++) {
+                const float v = fabsf(w[i]) > most ? most : w[i];
+                s = fmaf(v, v, s);
+            }
+            return s;
+        });
+        if (threadIdx.x < 16) out[(f * gridDim.x + blockIdx.x) * 16u + threadIdx.x] = norm_or_inf(sqrtf(a));
     }
-    out[blockIdx.x * 16u + tid] = norm == norm ? norm : __builtin_inff();
 }
 
 // ---------------------------------------------------------------------------
 // Host-side launchers.
 // ---------------------------------------------------------------------------
-hipError_t oxb_launch_row_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n_rows, uint32_t pair, float* d_out, hipStream_t st) {
-    if (((row0 | n_rows | pair) & 15u) != 0 || n_rows == 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(row_norms_kernel, dim3(n_rows / 16), dim3(256), 0, st, d_scales, n_sb, row0 / 16, pair / 16, d_out);
+hipError_t oxb_launch_pair_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t n, float* d_out, hipStream_t st) {
+    if ((n & 15u) != 0 || n == 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pair_norms_kernel, dim3(n / 16), dim3(256), 0, st, d_scales, n_sb, n / 16, d_out);
+    return hipGetLastError();
+}
+
+hipError_t oxb_launch_weighted_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n, const float* d_w, uint32_t k, float typical, float* d_out, hipStream_t st) {
+    if (((row0 | n) & 15u) != 0 || n == 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(weighted_norms_kernel, dim3(n / 16), dim3(256), 0, st, d_scales, n_sb, row0 / 16, d_w, k, typical, d_out);
     return hipGetLastError();
 }
 

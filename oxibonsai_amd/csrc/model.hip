@@ -83,8 +83,8 @@ struct Model {
     std::vector<uint64_t> owned_mats, owned_vecs;
     // Bounds for the products that hand their operands on (GemmFlow): the product of gate row j's and up row j's 2-norms is at most
     // gate_up, the square of an FFN input's at most norm2_cap, every value row of the cache below 2^value; 0 (NO_BOUND) where there is
-    // none that helps.
-    struct Bounds { float gate_up, norm2_cap; int32_t value; };
+    // none that helps.  value_least: the least that `value` would have been since the cache was made.
+    struct Bounds { float gate_up, norm2_cap; int32_t value, value_least; };
     std::vector<Bounds> bounds;
     DevBuf norm_buf;
     DevBuf tok_hist, tok_ids;  // token history of the on-device generation loop; prompt ids of a token prefill
@@ -261,57 +261,72 @@ static int32_t bound_exp(double b) {
 constexpr float kEvenRows = 16.f;
 static bool even_rows(const Weight::RowNorms& n) { return n.max <= kEvenRows * n.median; }
 
-static bool row_norms_known(const Weight& w, uint32_t row0, uint32_t pair) { return w.norms.max >= 0.f && w.norms.row0 == row0 && w.norms.pair == pair; }
-
-// Bounds of every layer, from the scales of gate || up and of the value rows of Q || K || V: |W a| <= |W row|_2 |a|_2, and the
-// normalised rows of a layer's input have |a|_2 <= max |norm weight| sqrt(h).  A matrix is looked at once.
+// Bounds of every layer by Cauchy-Schwarz.  gate times up: from the norms of gate row j and up row j and of the row of activations.
+// The value rows of the cache: V = W (w * x) with the attention norm's weights w and |x|_2 <= sqrt(h), so that the rows' norms
+// with every column times its weight count; the row in the middle with no weight counted as more than the one in the middle, for
+// a loud weight need not meet a loud x.  A matrix is looked at once.
 static int find_bounds(Model& m) {
     const oxb_model_desc& d = m.d;
     const uint32_t v0 = (d.nq + d.nkv) * d.hd, kd = d.nkv * d.hd;
-    struct Todo { Weight* w; uint32_t row0, n, pair; };
+    struct Todo { Weight* w; uint32_t n; Weight::RowNorms norms; const Vector* v; };
     std::vector<Todo> todo;
+    std::vector<Weight::RowNorms> found(2 * m.layers.size());
+    std::vector<size_t> where;  // todo i is found[where[i]]
     size_t total = 0;
-    for (const oxb_layer_ids& ly : m.layers) {
-        const Todo t[2] = {{find_weight(ly.gate_up), 0, d.inter, d.inter}, {find_weight(ly.qkv), v0, kd, 0}};
-        for (const Todo& x : t)
-            if (!row_norms_known(*x.w, x.row0, x.pair)) todo.push_back(x), total += x.n;
+    for (size_t L = 0; L < m.layers.size(); L++) {
+        const Vector& nw = g_rt.vectors[m.layers[L].attn_norm];
+        const Todo t[2] = {{find_weight(m.layers[L].gate_up), d.inter, {0, 0, -1.f, -1.f}, nullptr}, {find_weight(m.layers[L].qkv), kd, {v0, nw.serial, -1.f, -1.f}, &nw}};
+        for (size_t i = 0; i < 2; i++) {
+            const Weight::RowNorms& known = t[i].w->norms;
+            found[2 * L + i] = known;
+            if (known.max >= 0.f && known.row0 == t[i].norms.row0 && known.vector == t[i].norms.vector) continue;
+            todo.push_back(t[i]), where.push_back(2 * L + i), total += t[i].v ? 2 * t[i].n : t[i].n;
+        }
     }
     if (!todo.empty()) {
         OXB_TRY(m.norm_buf.ensure(total * sizeof(float)));
-        size_t at = 0;
+        float* at = (float*)m.norm_buf.ptr;
         for (const Todo& x : todo) {
-            OXB_TRY_HIP(oxb_launch_row_norms(x.w->d_scales, x.w->L.n_sb, x.row0, x.n, x.pair, (float*)m.norm_buf.ptr + at, g_rt.stream), "kernel launch failed: row_norms");
-            at += x.n;
+            OXB_TRY_HIP(x.v ? oxb_launch_weighted_norms(x.w->d_scales, x.w->L.n_sb, x.norms.row0, x.n, x.v->d, d.h, x.v->absmedian, at, g_rt.stream)
+                            : oxb_launch_pair_norms(x.w->d_scales, x.w->L.n_sb, x.n, at, g_rt.stream), "kernel launch failed: row norms");
+            at += x.v ? 2 * x.n : x.n;
         }
         std::vector<float> h(total);
         OXB_TRY_HIP(hipMemcpyAsync(h.data(), m.norm_buf.ptr, total * sizeof(float), hipMemcpyDeviceToHost, g_rt.stream), "norm download");
         OXB_TRY_HIP(hipStreamSynchronize(g_rt.stream), "norm download");
         m.norm_buf.release();
         auto first = h.begin();
-        for (const Todo& x : todo) {
-            const auto last = first + x.n, mid = first + x.n / 2;
-            std::nth_element(first, mid, last);
-            x.w->norms = {x.row0, x.pair, *std::max_element(mid, last), *mid};
-            first = last;
+        for (size_t i = 0; i < todo.size(); i++) {
+            Todo& x = todo[i];
+            x.norms.max = *std::max_element(first, first + x.n);
+            if (x.v) first += x.n;
+            std::nth_element(first, first + x.n / 2, first + x.n);
+            x.norms.median = first[x.n / 2];
+            first += x.n;
+            x.w->norms = found[where[i]] = x.norms;
         }
     }
-    m.bounds.resize(m.layers.size(), {0.f, 0.f, -NO_BOUND});
+    m.bounds.resize(m.layers.size(), {0.f, 0.f, -NO_BOUND, NO_BOUND});
     for (size_t L = 0; L < m.layers.size(); L++) {
-        const oxb_layer_ids& ly = m.layers[L];
-        const Weight::RowNorms &gu = find_weight(ly.gate_up)->norms, &v = find_weight(ly.qkv)->norms;
+        const Weight::RowNorms &gu = found[2 * L], &v = found[2 * L + 1];
+        Model::Bounds& b = m.bounds[L];
         // (the range that the products' exponents are worked out in: far wider than that of weights and norms in use)
-        const double w = g_rt.vectors[ly.ffn_norm].absmax, cap = w * w * d.h;
-        m.bounds[L].gate_up = even_rows(gu) && gu.max < 0x1p50f && cap < 0x1p50 ? std::max(gu.max, 0x1p-50f) : 0.f;
-        m.bounds[L].norm2_cap = (float)cap * (1.f + 0x1p-10f);
-        // (rows that an earlier matrix wrote may still be in the cache: the bound only grows)
-        const int32_t e = bound_exp((double)v.max * (double)g_rt.vectors[ly.attn_norm].absmax * std::sqrt((double)d.h));
-        if (e > m.bounds[L].value) m.bounds[L].value = e;
+        const double w = g_rt.vectors[m.layers[L].ffn_norm].absmax, cap = w * w * d.h;
+        b.gate_up = even_rows(gu) && gu.max < 0x1p50f && cap < 0x1p50 ? std::max(gu.max, 0x1p-50f) : 0.f;
+        b.norm2_cap = (float)cap * (1.f + 0x1p-10f);
+        // (rows that an earlier matrix wrote may still be in the cache)
+        const int32_t e = even_rows(v) ? bound_exp((double)v.max * std::sqrt((double)d.h)) : NO_BOUND;
+        b.value = std::max(b.value, e), b.value_least = std::min(b.value_least, e);
     }
     return OXB_HIP_OK;
 }
 
 // Whether the attention of layer L leaves the O projection's operand, and gate || up that of the down projection.
-static bool attn_hands_on(const Model& m, uint32_t L) { return m.bounds[L].value < NO_BOUND && (m.d.nq * m.d.hd) % 512u == 0; }
+// (a matrix replaced by one 16 times as quiet leaves the old bound as little to say as an uneven one)
+static bool attn_hands_on(const Model& m, uint32_t L) {
+    const Model::Bounds& b = m.bounds[L];
+    return b.value < NO_BOUND && b.value - b.value_least <= 4 && (m.d.nq * m.d.hd) % 512u == 0;
+}
 static GemmFlow flow_gate_up(const Model& m, uint32_t L) {
     GemmFlow f;
     f.out = m.bounds[L].gate_up > 0.f && m.d.inter % OXB_QK == 0;
@@ -324,10 +339,10 @@ static GemmFlow flow_down(const Model& m, uint32_t L) {
     if (flow_gate_up(m, L).out) f.in = GemmFlow::SWIGLU;
     return f;
 }
-// (the bound leaves a factor of two below 2^15 for the roundings on the way)
+// (2^15 is a factor of two from fp16's end, for the roundings on the way and those of one-byte rows)
 static GemmFlow flow_o(const Model& m, uint32_t L, const GemmWorkspace& ws, uint32_t M, OxbOperandOut* op) {
     GemmFlow f;
-    *op = {nullptr, (uint32_t)m.d.fmt, (M + 15u) / 16u * 16u, 14 - m.bounds[L].value};
+    *op = {nullptr, (uint32_t)m.d.fmt, (M + 15u) / 16u * 16u, 15 - m.bounds[L].value};
     if (!attn_hands_on(m, L)) return f;
     op->xh = (_Float16*)ws.xh.ptr;
     f.in = GemmFlow::ATTENTION;
@@ -736,6 +751,11 @@ int oxb_hip_upload_f32(uint64_t* id, const float* w, size_t n) {
         const float a = fabsf(w[i]);
         if (a > v.absmax || a != a) v.absmax = a;  // a NaN sticks
     }
+    std::vector<float> a(n);
+    for (size_t i = 0; i < n; i++) a[i] = w[i] == w[i] ? fabsf(w[i]) : INFINITY;
+    std::nth_element(a.begin(), a.begin() + n / 2, a.end());
+    v.absmedian = a[n / 2];
+    v.serial = ++g_rt.vector_serial;
     if (hipMalloc((void**)&v.d, n * sizeof(float)) != hipSuccess)
         return fail(OXB_HIP_OUT_OF_MEMORY, "out of device memory: requested %zu bytes on device %d", n * sizeof(float), g_rt.device);
     hipError_t e = hipMemcpy(v.d, w, n * sizeof(float), hipMemcpyHostToDevice);
@@ -964,6 +984,9 @@ int oxb_hip_model_set_attention(uint64_t model, const oxb_attention_options* opt
             if (alloc_kv_cache(*m, OXB_KV_F16, 0, 0)) free_kv_cache(*m);
             return rc;
         }
+        // no row of an earlier matrix is left
+        m->bounds.clear();
+        m->checked_gen = ~0ull;
     }
     m->window = opt->window_size;
     m->sinks = opt->sink_tokens;

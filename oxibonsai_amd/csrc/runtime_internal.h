@@ -49,15 +49,17 @@ struct Weight {
     uint16_t* d_scales = nullptr;
     void* d_raw = nullptr;
     size_t raw_blocks = 0;
-    // Largest and median of the 2-norms of the rows from row `row0` on, or with `pair` of the products of those of rows row0 + i and
-    // row0 + pair + i; negative: not worked out yet.
-    struct RowNorms { uint32_t row0 = 0, pair = 0; float max = -1.f, median = -1.f; } norms;
+    // What the bounds of a product's outputs come from (find_bounds, model.hip): the largest norm of the rows from row0 on and the one in
+    // the middle, for inputs that went through the norm weights of that serial number; max < 0: not worked out yet.
+    struct RowNorms { uint32_t row0 = 0; uint64_t vector = 0; float max = -1.f, median = -1.f; } norms;
 };
 
 struct Vector {  // a resident fp32 vector (norm weights)
     float* d = nullptr;
     size_t n = 0;
     float absmax = 0.f;  // max |value|, the RMSNorm kernel's bound for its output range
+    float absmedian = 0.f;
+    uint64_t serial = 0;  // another for every upload
 };
 
 struct Runtime {
@@ -72,6 +74,7 @@ struct Runtime {
     // Counts every free or replacement of a resident matrix or vector.  A captured decode graph holds their device
     // pointers; a model compares the count it captured under with this one and captures again when they differ.
     uint64_t weights_gen = 0;
+    uint64_t vector_serial = 0;
     DevBuf ws_x, ws_y, ws_aux;
     DevBuf gemv_pack;  // quantised activation vectors of one GEMV call (gemv_launch with pack_ws)
     void* static_scratch = nullptr;  // device address of the library's file-scope scratch array on g_rt.device

@@ -353,3 +353,64 @@ def test_swiglu_outputs_of_rows_at_the_ends_of_the_range(backend, fmt, n, batch,
             assert err <= 1e-3
     finally:
         gpu.close()
+
+
+# What is uneven: a value row `loud` times the rest, whose outputs the O projection takes as much quieter; or a norm weight in front of
+# Q || K || V that meets zeros
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("ctx,n,batch,hd", [(0, 130, 1, 64), (0, 17, 1, 128), (1600, 40, 1, 128), (60, 1, 9, 128)])
+@pytest.mark.parametrize("what", ["value row", "norm weight", "both"])
+def test_uneven_value_rows_leave_the_attention_its_precision(backend, fmt, ctx, n, batch, hd, what):
+    """The same for the attention's outputs in front of the O projection; the FFN is silent, so that they are what the second layer's
+    rows are made of."""
+    nq, loud = 1024 // hd, 2048
+    cfg = dict(fmt=fmt, n_layers=2, h=512, inter=512, nq=nq, nkv=nq // 4, hd=hd, vocab=64, max_seq=ctx + n + 8, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 78)
+    rows = _rows(32, ctx + n * batch, 512)
+    for lw in w["layers"]:
+        lw["down"] = _scaled(fmt, lw["down"], 512, slice(None), 0.0)
+        if what != "norm weight":
+            lw["v"] = _scaled(fmt, lw["v"], 512, [3], loud)
+            lw["o"] = _scaled(fmt, lw["o"], 1024, slice(None), 1 / loud, block=slice(0, 4 * hd // 128))   # its four q heads
+        if what != "value row":
+            lw["attn_norm"] = lw["attn_norm"].copy()
+            lw["attn_norm"][7] = 2.0 ** 24
+    if what != "value row":
+        rows[:, 7] = 0.0
+        for lw in w["layers"]:
+            lw["o"] = _scaled(fmt, lw["o"], 1024, [7], 0.0)
+    err = _second_layer_errors(backend, cfg, w, rows, ctx, batch)
+    assert np.median(err) <= 1.4e-3
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("n,batch", [(40, 1), (1, 9)])
+def test_quieter_value_rows_in_place_of_loud_ones(backend, fmt, n, batch):
+    """Q || K || V of a live model is replaced by one whose value rows are 2^24 times as quiet: what the old ones could reach says nothing
+    about the new ones' precision."""
+    cfg = dict(fmt=fmt, n_layers=2, h=512, inter=512, nq=8, nkv=2, hd=128, vocab=64, max_seq=n + 8, eps=1e-14, rope_theta=1e6)
+    w = synth.make_model(cfg, 79)
+    for lw in w["layers"]:
+        lw["down"] = _scaled(fmt, lw["down"], 512, slice(None), 0.0)
+    quiet = {**w, "layers": [{**lw, "v": _scaled(fmt, lw["v"], 512, slice(None), 1 / 4096)} for lw in w["layers"]]}
+    loud = {**w, "layers": [{**lw, "v": _scaled(fmt, lw["v"], 512, slice(None), 4096)} for lw in w["layers"]]}
+    rows = _rows(33, n * batch, 512) * np.float32(1e-5)
+    cpu = oracle.OracleModel(cfg, quiet, kv_f16=True, simd=True)
+    gpu = HipModel(backend, cfg, loud, batch=batch)
+    try:
+        up = backend.upload_weights_raw if fmt == Q1 else backend.upload_weights_ternary
+        run = (lambda: gpu.forward(rows, 0)) if batch > 1 else (lambda: gpu.prefill(rows, 0))
+        run()
+        for i, lw in enumerate(quiet["layers"]):
+            up(np.concatenate([lw["q"], lw["k"], lw["v"]]), 1536, 512, handle_id=gpu._ids[i].qkv)
+        run()
+        err = []
+        for seq in range(batch):
+            cpu.forward_batch(rows[seq:seq + n], 0, want_logits=False)
+            for head in range(2):
+                for a, b in zip(gpu.read_kv(1, head, 0, n, seq=seq)[:2], cpu.cache_rows(1, head, 0, n)):
+                    err += list(np.sqrt(np.mean((a.astype(np.float64) - b) ** 2, axis=1) / np.mean(b.astype(np.float64) ** 2, axis=1)))
+        print(f"median row {np.median(err):.2e}, worst {max(err):.2e}")
+        assert np.median(err) <= 1.4e-3
+    finally:
+        gpu.close()
