@@ -1400,6 +1400,11 @@ int oxb_hip_model_prefill_attention(uint64_t model, uint32_t layer, uint32_t seq
     OXB_TRY(kv_reserve(m, seq, (uint64_t)pos_start + n_tokens));
     OXB_TRY(kv_sync_table(m));
     OXB_TRY(ensure_prefill_buffers(m, n_tokens));
+    if (m.bounds[layer].value != NO_BOUND) {  // the caller's value rows know no bound; the captured step has the old one
+        m.bounds[layer].value = NO_BOUND;
+        if (m.graph_exec) (void)hipGraphExecDestroy(m.graph_exec);
+        m.graph_exec = nullptr;
+    }
     IoCall io;
     OXB_TRY(io.begin());
     OXB_TRY(io.upload(m.pf_qkv, qkv, (size_t)n_tokens * (d.nq + 2 * d.nkv) * d.hd * 4));

@@ -14,7 +14,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from helpers import Q1
+from helpers import Q1, TQ2
 from oracle import oracle
 from oxibonsai_amd import _lib, synth
 from oxibonsai_amd.backend import _check
@@ -234,3 +234,33 @@ def test_prefill_attention_weights_are_relative_to_the_row_maximum(backend, M, s
         assert err <= 1.25 * ref + 3e-6, (err, ref)
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+def test_steps_behind_value_rows_larger_than_the_model_makes(backend, fmt):
+    # Rows that the caller stores may be larger than anything the model's own value rows and norms can make, the outputs of the
+    # attention with them.  Nine sequences and prompts (fp16 products) against a single sequence's steps (fp32): 1e-2, as for any prefill.
+    cfg = dict(fmt=fmt, n_layers=2, h=512, inter=512, nq=4, nkv=2, hd=128, vocab=96, max_seq=64, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 12)
+    g = np.random.default_rng(3)
+    qkv = g.standard_normal((20, 8 * 128)).astype(np.float32)
+    qkv[:, 6 * 128:] *= 1e4
+    rows = g.standard_normal((9, 512)).astype(np.float32)
+    one, nine = HipModel(backend, cfg, w), HipModel(backend, cfg, w, batch=9)
+    try:
+        nine.forward(rows, 0)           # a captured step that is in use already
+        for seq in range(9):
+            for layer in range(2):
+                _attend(nine, layer, seq, qkv, 0)
+        for layer in range(2):
+            _attend(one, layer, 0, qkv, 0)
+        got = nine.forward(rows, 20)[0]
+        want = np.stack([one.forward(r, 20)[0][0] for r in rows])
+        assert np.all(np.abs(got - want) <= 1e-2 * np.maximum(1.0, np.abs(want)))
+        for i, r in enumerate(rows):
+            last = one.forward(r, 20 + i)[0][0]
+        got = one.prefill(rows, 20)[0]
+        assert np.all(np.abs(got - last) <= 1e-2 * np.maximum(1.0, np.abs(last)))
+    finally:
+        one.close()
+        nine.close()
