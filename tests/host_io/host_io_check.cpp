@@ -4,9 +4,12 @@
 #include <cstdarg>
 #include <cstdio>
 #include <deque>
+#include <filesystem>
 #include <map>
 #include <thread>
 #include <vector>
+
+#include <sched.h>
 
 #include "../../include/oxb_hip.h"
 #include "../../oxibonsai_amd/csrc/host_io.h"
@@ -263,9 +266,54 @@ static void pool_of_results() {
     CHECK(fake::host_bytes == 0);
 }
 
+static size_t threads() {
+    size_t n = 0;
+    for (const auto& e : std::filesystem::directory_iterator("/proc/self/task")) (void)e, n++;
+    return n;
+}
+
+static void there_and_back(size_t n, unsigned seed) {
+    static std::vector<uint8_t> dev(32 * MiB);
+    std::vector<uint8_t> src = bytes(n, seed), dst(n, 0);
+    IoCall io;
+    CHECK(io.begin() == 0);
+    CHECK(io.upload(dev.data(), src.data(), n) == 0 && io.download(dst.data(), dev.data(), n) == 0 && io.finish("there and back") == 0);
+    CHECK(src == dst);
+}
+
+// A caller that may run on one CPU gets no helpers; on two it gets one; and with all threads on one CPU while helpers are there
+// the copies end.
+static void few_cpus() {
+    cpu_set_t all, some;
+    CHECK(sched_getaffinity(0, sizeof all, &all) == 0);
+    std::vector<int> cpus;
+    for (int i = 0; i < CPU_SETSIZE; i++)
+        if (CPU_ISSET(i, &all)) cpus.push_back(i);
+    there_and_back(64, 1);  // (the stand-in's device has its thread)
+    const size_t before = threads();
+    CPU_ZERO(&some);
+    CPU_SET(cpus[0], &some);
+    CHECK(sched_setaffinity(0, sizeof some, &some) == 0);
+    for (unsigned i = 0; i < 4; i++) there_and_back(20 * MiB + 4, i);
+    CHECK(threads() == before);
+    if (cpus.size() > 1) {
+        CPU_SET(cpus[1], &some);
+        CHECK(sched_setaffinity(0, sizeof some, &some) == 0);
+        for (unsigned i = 0; i < 4; i++) there_and_back(20 * MiB + 4, i);
+        CHECK(threads() == before + 1);
+        CPU_CLR(cpus[1], &some);
+        for (const auto& e : std::filesystem::directory_iterator("/proc/self/task"))
+            CHECK(sched_setaffinity(std::stoi(e.path().filename()), sizeof some, &some) == 0);
+        for (unsigned i = 0; i < 4; i++) there_and_back(20 * MiB + 4, i);
+    }
+    io_shutdown();
+    for (int i = 0; i < 1000 && threads() != before; i++) std::this_thread::sleep_for(std::chrono::milliseconds(1));  // (the system's list lags behind)
+    CHECK(threads() == before);
+}
+
 int main(int argc, char** argv) {
     g_rt.stream = g_rt.own_stream = (hipStream_t)&g_rt;
-    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}, {"first_call", first_call}, {"pool_of_results", pool_of_results}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"round_trip", round_trip}, {"error_exit", error_exit}, {"first_call", first_call}, {"pool_of_results", pool_of_results}, {"few_cpus", few_cpus}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.run();

@@ -17,7 +17,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["round_trip", "error_exit", "first_call", "pool_of_results"])
+@pytest.mark.parametrize("check", ["round_trip", "error_exit", "first_call", "pool_of_results", "few_cpus"])
 def test_host_io(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
