@@ -70,10 +70,9 @@ struct Model {
     bool want_logits_in_graph = true;
     size_t logits_cap = 0;  // floats m.logits holds
     std::vector<void*> allocs;
-    // prefill activations for up to pf_cap token rows (allocated on first use)
+    // prefill activations for up to pf_cap token rows (allocated on first use, each when a call needs it)
     uint32_t pf_cap = 0;
     float *pf_hidden = nullptr, *pf_qkv = nullptr, *pf_attn = nullptr, *pf_gu = nullptr;
-    std::vector<void*> pf_allocs;
     DevBuf pf_part;     // the prefill attention's sums of runs of keys
     GemmWorkspace gws;  // GEMM scratch of the captured large-batch decode step: sized at creation, never moved
     DevBuf gpack;       // quantised activation vectors of the captured GEMV-based step (batches of two to eight): likewise
@@ -130,6 +129,8 @@ static void free_kv_cache(Model& m) {
     m.table_dirty = false;
 }
 
+static void free_prefill_buffers(Model& m);
+
 static void free_model(Model& m) {
     if (m.graph_exec) (void)hipGraphExecDestroy(m.graph_exec);
     m.graph_exec = nullptr;
@@ -139,9 +140,7 @@ static void free_model(Model& m) {
     m.h_pos = m.h_tokens = nullptr;
     for (void* p : m.allocs) (void)hipFree(p);
     m.allocs.clear();
-    for (void* p : m.pf_allocs) (void)hipFree(p);
-    m.pf_allocs.clear();
-    m.pf_cap = 0;
+    free_prefill_buffers(m);
     m.pf_part.release();
     m.gws.release();
     m.gpack.release();
@@ -602,26 +601,36 @@ static int encode_decode_step(Model& m, bool with_lm_head) {
     return OXB_HIP_OK;
 }
 
-// Prefill buffers for `rows` token rows.
-static int ensure_prefill_buffers(Model& m, uint32_t rows) {
-    if (rows <= m.pf_cap) return OXB_HIP_OK;
-    (void)hipStreamSynchronize(g_rt.stream);
-    for (void* p : m.pf_allocs) (void)hipFree(p);
-    m.pf_allocs.clear();
+static void free_prefill_buffers(Model& m) {
+    float** bufs[4] = {&m.pf_hidden, &m.pf_qkv, &m.pf_attn, &m.pf_gu};
+    for (float** p : bufs) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
     m.pf_cap = 0;
+}
+
+// Prefill buffers for `rows` token rows.  The fp32 rows in front of the O and down projections (at 2048 tokens of the 8B shape
+// 34 and 101 MB) only where a layer does not hand their operand on, or where attn_out asks for the former.
+static int ensure_prefill_buffers(Model& m, uint32_t rows, bool attn_out = false) {
     const oxb_model_desc& d = m.d;
-    const size_t R = (rows + 127u) / 128u * 128u, qd = (size_t)d.nq * d.hd, qkv_rows = qd + 2 * (size_t)d.nkv * d.hd;
-    struct { float** p; size_t n; } bufs[] = {{&m.pf_hidden, R * d.h}, {&m.pf_qkv, R * qkv_rows},
-                                             {&m.pf_attn, R * qd},    {&m.pf_gu, R * d.inter}};
-    for (auto& b : bufs) {
+    bool act = false;
+    for (uint32_t L = 0; L < d.n_layers; L++) attn_out |= !attn_hands_on(m, L), act |= !flow_gate_up(m, L).out;
+    if (rows > m.pf_cap) {
+        (void)hipStreamSynchronize(g_rt.stream);
+        free_prefill_buffers(m);
+        m.pf_cap = (rows + 127u) / 128u * 128u;
+    }
+    const size_t R = m.pf_cap, qd = (size_t)d.nq * d.hd, qkv_rows = qd + 2 * (size_t)d.nkv * d.hd;
+    const struct { float** p; size_t n; bool used; } bufs[] = {{&m.pf_hidden, R * d.h, true}, {&m.pf_qkv, R * qkv_rows, true}, {&m.pf_attn, R * qd, attn_out}, {&m.pf_gu, R * d.inter, act}};
+    for (const auto& b : bufs) {
+        if (*b.p || !b.used) continue;
         if (hipMalloc((void**)b.p, b.n * sizeof(float)) != hipSuccess) {
-            for (void* p : m.pf_allocs) (void)hipFree(p);
-            m.pf_allocs.clear();
+            *b.p = nullptr;
+            free_prefill_buffers(m);
             return fail(OXB_HIP_OUT_OF_MEMORY, "out of device memory: requested %zu bytes on device %d", b.n * sizeof(float), g_rt.device);
         }
-        m.pf_allocs.push_back(*b.p);
     }
-    m.pf_cap = (uint32_t)R;
     return OXB_HIP_OK;
 }
 
@@ -1399,7 +1408,7 @@ int oxb_hip_model_prefill_attention(uint64_t model, uint32_t layer, uint32_t seq
     if (rc) return rc;
     OXB_TRY(kv_reserve(m, seq, (uint64_t)pos_start + n_tokens));
     OXB_TRY(kv_sync_table(m));
-    OXB_TRY(ensure_prefill_buffers(m, n_tokens));
+    OXB_TRY(ensure_prefill_buffers(m, n_tokens, true));
     if (m.bounds[layer].value != NO_BOUND) {  // the caller's value rows know no bound; the captured step has the old one
         m.bounds[layer].value = NO_BOUND;
         if (m.graph_exec) (void)hipGraphExecDestroy(m.graph_exec);

@@ -414,3 +414,36 @@ def test_quieter_value_rows_in_place_of_loud_ones(backend, fmt, n, batch):
         assert np.median(err) <= 1.4e-3
     finally:
         gpu.close()
+
+
+def _free_bytes():
+    import ctypes as C
+    from oxibonsai_amd import _lib
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert _lib.lib().oxb_hip_device_info(None, 0, C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_buffers_that_a_prefill_has_no_use_for(backend):
+    """Where SwiGLU outputs and attention outputs go to the next product's operand their fp32 rows take no memory: 2048 tokens x (24576 +
+    1024) values, 210 MB.  What a prefill allocates is the operand in fp16 (with a quarter to spare), the projections and smaller things.
+    A layer that is uneven all of a sudden gets its rows."""
+    cfg = dict(fmt=Q1, n_layers=2, h=128, inter=24576, nq=8, nkv=2, hd=128, vocab=64, max_seq=2100, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 6)
+    uneven = {**w, "layers": [dict(w["layers"][0], gate=_scaled(Q1, w["layers"][0]["gate"], 128, [9], 64),
+                                   v=_scaled(Q1, w["layers"][0]["v"], 128, [9], 64)), w["layers"][1]]}
+    rows = _rows(7, 2048, 128)
+    gpu, other = HipModel(backend, cfg, w), HipModel(backend, cfg, uneven)
+    try:
+        before = _free_bytes()
+        gpu.prefill(rows)
+        used = before - _free_bytes()
+        print(f"{used / 2**20:.0f} MiB")
+        assert used <= 2048 * (1.25 * 2 * (24576 + 1024) + 4 * (1536 + 128)) + (32 << 20)   # (sums of K slices and what rounding up adds)
+        lw = uneven["layers"][0]
+        backend.upload_weights_raw(np.concatenate([lw["gate"], lw["up"]]), 2 * 24576, 128, handle_id=gpu._ids[0].gate_up)
+        backend.upload_weights_raw(np.concatenate([lw["q"], lw["k"], lw["v"]]), 1536, 128, handle_id=gpu._ids[0].qkv)
+        assert np.array_equal(gpu.prefill(rows)[0], other.prefill(rows)[0])
+    finally:
+        gpu.close()
+        other.close()
