@@ -81,12 +81,14 @@ constexpr uint32_t kSyncEvery = 256;
 // The copies of a transfer of more than kShared bytes, shared with up to kHelpers threads of the library's own.  The caller takes
 // slices like the helpers and is done when all slices are, so a helper that wakes late costs nothing; a helper looks out for the
 // next copy for kLinger and then sleeps.  Used under the library's lock, by one call at a time; io_shutdown ends the threads.
-// One thread -> four: 1.3 MB in and out 130 -> 112 us (77 x 4096 GEMM, host to host), 19 MB out 3.62 -> 3.40 ms (decode of
+// One thread -> four: 1.3 MB in and out 132 -> 117 us (77 x 4096 GEMM, host to host, call after call), 19 MB out 3.62 -> 3.40 ms (decode of
 // 32 sequences), 34 MB in 27.4 -> 26.8 ms (2048-token prefill).  Waking them costs the caller 0.5 to 3 us:
 // shared from 64 KB on, a product with 131 KB in and out takes 33.0 us instead of 30.2, with 196 KB 37.3 instead of 37.0; with
 // 262 KB it takes 42.8 instead of 43.1, with 328 KB 50.9 instead of 49.4, with 393 KB 48.5 instead of 53.6.
-// Helpers that sleep take 50 us to come: transfers up to kWake that follow the last one later than kSoon are the caller's alone (a
-// decode step of one sequence, 608 KB of logits every 0.8 ms: 8 us less).
+// Helpers that sleep take up to 50 us to come: transfers up to kWake that follow the last one later than kSoon are the caller's alone (a
+// decode step of one sequence, 608 KB of logits every 0.8 ms: 8 us less).  A product with so much in and out, 0.3 ms after the last
+// one, the caller alone / helpers woken: 0.9 MB 106 / 110 us, 1.0 MB 114 / 117, 1.15 MB 129 / 109 to 127, 1.3 MB 136 / 113 to 132,
+// 1.6 MB 153 / 134 to 149, 2.1 MB 170 / 159 to 168, 4.2 MB 277 / 267.
 constexpr size_t kShared = (size_t)320 << 10;
 constexpr size_t kWake = (size_t)1 << 20;
 constexpr auto kSoon = std::chrono::microseconds(100);
