@@ -255,7 +255,7 @@ static int32_t bound_exp(double b) {
 // that by what Cauchy-Schwarz gives away (about sqrt(h) for each factor, 2^12 for gate times up at h = 4096) and by how much louder
 // the loudest row is than the row in the middle.  Relative error of a product behind the operand, h = 4096, one gate row R times as
 // loud, with the row's own maximum / this bound: R = 16 2.0e-4 / 2.0e-4, 256 2.2e-4 / 2.2e-4, 4096 1.86e-4 / 1.9e-4 and 16 % of the
-// values below 2^-14.  So R = 16 leaves 2^8 for rows of activations that meet the matrix at a worse angle than random ones.  More
+// values below 2^-14.  So R = 16 leaves 2^9 for rows of activations that meet the matrix at a worse angle than random ones.  More
 // uneven matrices keep the pack, which finds every row's own maximum.
 constexpr float kEvenRows = 16.f;
 static bool even_rows(const Weight::RowNorms& n) { return n.max <= kEvenRows * n.median; }
