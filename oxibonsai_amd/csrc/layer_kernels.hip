@@ -212,11 +212,14 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
     cache_t* Vc = reinterpret_cast<cache_t*>(p.v_cache);
     float* Ksc = p.k_scale;  // one scale per row
     float* Vsc = p.v_scale;
-    // Row of a position of this (sequence, layer, kv head): an offset in a contiguous cache; in a paged one the page
-    // number comes from the sequence's table.  Pages hold 16 positions or more, so the 32 keys of a wave's block lie in
-    // at most two pages - those of keys key0 .. key0 + 15 and key0 + 16 .. key0 + 31, the same for every lane - which
-    // are looked up (one broadcast load each) one chunk before the rows are requested, so that no row load waits for
-    // a lookup.  (Keeping the table in LDS instead was measured slower: the 8 KB cost a workgroup per CU.)
+    // Rows of this (sequence, layer, kv head).  A wave's block of 32 keys is two tiles of 16, each contiguous (pages hold 16 positions or more):
+    // where a tile lies is the same for every lane, so its rows are read through a buffer descriptor that begins there, at offsets that never
+    // change, and that ends with the sequence: rows past the last key read as zeros and take no bandwidth (their scores are masked).  Per-lane
+    // addresses and a test of every key's visibility were a third of a chunk's 400 to 500 vector instructions; without them, us per launch (8B
+    // shape): FP8 in pages of 16 at 32 000 23.1 -> 21.4, INT8 there 21.6 -> 20.5, 32 of INT8 at 2048 33.0 -> 32.3, eight at 4000 21.9 -> 21.0; fp16,
+    // one at 2048 9.2 -> 8.9, six 16.9 -> 16.4, one of 16 heads at 700 7.6 -> 7.3.  In a paged cache the two page numbers come from the sequence's
+    // table, one broadcast load each, one chunk before the rows are requested, so that no row load waits for a lookup.  (Keeping the table in
+    // LDS instead was measured slower: the 8 KB cost a workgroup per CU.)
     const bool paged = OPT && p.kv.page_table != nullptr;
     const uint32_t pshift = p.kv.page_shift, pmask = (1u << pshift) - 1u;
     const size_t row0 = paged ? ((size_t)(p.layer * p.nkv + kvh) * p.kv.n_pages) << pshift : kv_row(p.kv, b, p.layer, kvh, 0);
@@ -228,49 +231,61 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         pa = (uint32_t)__builtin_amdgcn_readfirstlane((int)tbl[i0]);
         pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)tbl[i1]);
     };
-    // key: a position of the block that starts at key0 (or, for a block past the end, the last position, whose row
-    // is then read from a wrong but existing page: such a block is masked as a whole)
-    auto row_of = [&](uint32_t key, uint32_t key0, uint32_t pa, uint32_t pb) -> size_t {
-        if (!paged) return row0 + key;
-        return row0 + ((size_t)(((key - key0) & 16u) ? pb : pa) << pshift) + (key & pmask);
+    struct Tile { size_t row; uint32_t n; };  // first row, and how many of the 16 are there
+    auto tile_of = [&](uint32_t key, uint32_t page) -> Tile {
+        const uint32_t n = key < seq_len ? min(seq_len - key, 16u) : 0u;
+        return {paged ? row0 + ((size_t)page << pshift) + (key & pmask) : row0 + key, n};
     };
 
     // K rows of the two 16-key tiles (A operands) and this lane's pieces of the 32-key V block of a chunk.
-    // Rows past the last key repeat it; their scores are masked.
     v8h_t k0r[QC ? 1 : KS], k1r[QC ? 1 : KS];
     kvi2_t k0q[QC ? KS : 1], k1q[QC ? KS : 1];
     float4 ksc0, ksc1, vsc0, vsc1;  // row scales of the lane's keys 4g .. 4g+3 and 16+4g .. 16+4g+3
     v4i vr[VL];
+    constexpr uint32_t RB = HD * sizeof(cache_t);  // bytes of a row
+    const uint32_t k_at = qi * RB + g * (QC ? HD / 4 : 16), v_at = (lane / VPR) * RB + (lane % VPR) * 16;
+    auto scales = [&](const float* s, const Tile& t) -> float4 {
+        const v4i v = buf_load_b128(make_rsrc(s + t.row, t.n * 4u), 16u * g);
+        return make_float4(__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z), __int_as_float(v.w));
+    };
     auto load_k = [&](uint32_t chunk, uint32_t pa, uint32_t pb) {
         const uint32_t key0 = chunk * CH + 32 * wave;
-        const size_t kr0 = row_of(min(key0 + qi, seq_len - 1), key0, pa, pb), kr1 = row_of(min(key0 + 16 + qi, seq_len - 1), key0, pa, pb);
+        const Tile t0 = tile_of(key0, pa), t1 = tile_of(key0 + 16, pb);
+        const __amdgpu_buffer_rsrc_t r0 = make_rsrc(Kc + t0.row * HD, t0.n * RB), r1 = make_rsrc(Kc + t1.row * HD, t1.n * RB);
+        if constexpr (QC && KS % 2 == 0) {
 #pragma unroll
-        for (int s = 0; s < KS; s++) {
-            if constexpr (QC) {
-                k0q[s] = *reinterpret_cast<const kvi2_t*>(Kc + kr0 * HD + (HD / 4) * g + 8 * s);
-                k1q[s] = *reinterpret_cast<const kvi2_t*>(Kc + kr1 * HD + (HD / 4) * g + 8 * s);
-            } else {
-                k0r[s] = *reinterpret_cast<const v8h_t*>(Kc + kr0 * HD + 32 * s + 8 * g);
-                k1r[s] = *reinterpret_cast<const v8h_t*>(Kc + kr1 * HD + 32 * s + 8 * g);
+            for (int s = 0; s < KS; s += 2) {
+                const v4i a = buf_load_b128(r0, k_at + 8 * s), c = buf_load_b128(r1, k_at + 8 * s);
+                k0q[s] = (kvi2_t){a.x, a.y}, k0q[QC ? s + 1 : 0] = (kvi2_t){a.z, a.w};
+                k1q[s] = (kvi2_t){c.x, c.y}, k1q[QC ? s + 1 : 0] = (kvi2_t){c.z, c.w};
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                if constexpr (QC) {
+                    const v2u a = __builtin_amdgcn_raw_buffer_load_b64(r0, (int)(k_at + 8 * s), 0, 0), c = __builtin_amdgcn_raw_buffer_load_b64(r1, (int)(k_at + 8 * s), 0, 0);
+                    k0q[s] = (kvi2_t){(int)a.x, (int)a.y}, k1q[s] = (kvi2_t){(int)c.x, (int)c.y};
+                } else {
+                    k0r[s] = __builtin_bit_cast(v8h_t, buf_load_b128(r0, k_at + 64 * s));
+                    k1r[s] = __builtin_bit_cast(v8h_t, buf_load_b128(r1, k_at + 64 * s));
+                }
             }
         }
-        if constexpr (QC) {  // scales of positions past the last key are never used (their scores are masked)
-            ksc0 = *reinterpret_cast<const float4*>(Ksc + row_of(min(key0 + 4 * g, (seq_len - 1) & ~3u), key0, pa, pb));
-            ksc1 = *reinterpret_cast<const float4*>(Ksc + row_of(min(key0 + 16 + 4 * g, (seq_len - 1) & ~3u), key0, pa, pb));
-        }
+        if constexpr (QC) ksc0 = scales(Ksc, t0), ksc1 = scales(Ksc, t1);
     };
     auto load_v = [&](uint32_t chunk, uint32_t pa, uint32_t pb) {
         const uint32_t key0 = chunk * CH + 32 * wave;
+        const Tile t0 = tile_of(key0, pa), t1 = tile_of(key0 + 16, pb);
+        const __amdgpu_buffer_rsrc_t r0 = make_rsrc(Vc + t0.row * HD, t0.n * RB), r1 = make_rsrc(Vc + t1.row * HD, t1.n * RB);
+        // piece i: rows i * 64 / VPR + lane / VPR of the block
+        if constexpr (VL == 1) {  // (rows of 32 bytes: one piece a lane, its tile by lane)
+            const v4i a = buf_load_b128(r0, lane < 32 ? v_at : OXB_OOB), c = buf_load_b128(r1, lane < 32 ? OXB_OOB : v_at - 16 * RB);
+            vr[0] = (v4i){a.x | c.x, a.y | c.y, a.z | c.z, a.w | c.w};
+        } else {
 #pragma unroll
-        for (int i = 0; i < VL; i++) {
-            const uint32_t id = i * 64 + lane, col = id % VPR;
-            const size_t row = row_of(min(key0 + id / VPR, seq_len - 1), key0, pa, pb);
-            vr[i] = *reinterpret_cast<const v4i*>(reinterpret_cast<const uint8_t*>(Vc + row * HD) + col * 16);
+            for (int i = 0; i < VL; i++) vr[i] = buf_load_b128(i < VL / 2 ? r0 : r1, v_at + (i % (VL / 2 ? VL / 2 : 1)) * (64 / VPR) * RB);
         }
-        if constexpr (QC) {
-            vsc0 = *reinterpret_cast<const float4*>(Vsc + row_of(min(key0 + 4 * g, (seq_len - 1) & ~3u), key0, pa, pb));
-            vsc1 = *reinterpret_cast<const float4*>(Vsc + row_of(min(key0 + 16 + 4 * g, (seq_len - 1) & ~3u), key0, pa, pb));
-        }
+        if constexpr (QC) vsc0 = scales(Vsc, t0), vsc1 = scales(Vsc, t1);
     };
 
     // The rows of the first chunk are requested before anything else, so that their way from HBM overlaps the Q prologue.
@@ -434,6 +449,13 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         i += used;
         const bool more = i < n_walk;
         const uint32_t nxt = chunk_of(i);
+        if (patch) {  // (uniform)
+#pragma unroll
+            for (int j = 0; j < VL; j++) {
+                const uint32_t id = j * 64 + lane;
+                if (key0 + id / VPR == pos) vr[j] = *reinterpret_cast<const v4i*>(&kv_new[1][(id % VPR) * (QC ? 16 : 8)]);
+            }
+        }
         // stage the V block in the wave's LDS slice (the previous block's gathers were issued before: LDS runs in
         // order) and request the next chunk's
 #pragma unroll
@@ -441,8 +463,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
             const uint32_t id = j * 64 + lane;
             if constexpr (QC) {
                 uint32_t d[8];
-                v4i piece = vr[j];
-                if (patch && key0 + id / VPR >= pos) piece = *reinterpret_cast<const v4i*>(&kv_new[1][(id % VPR) * 16]);
+                const v4i piece = vr[j];
                 kv_dec4<KVM>((uint32_t)piece.x, d[0], d[1]);
                 kv_dec4<KVM>((uint32_t)piece.y, d[2], d[3]);
                 kv_dec4<KVM>((uint32_t)piece.z, d[4], d[5]);
@@ -451,9 +472,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
                 *reinterpret_cast<v4i*>(dst) = (v4i){(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
                 *reinterpret_cast<v4i*>(dst + 8) = (v4i){(int)d[4], (int)d[5], (int)d[6], (int)d[7]};
             } else {
-                v4i piece = vr[j];
-                if (patch && key0 + id / VPR >= pos) piece = *reinterpret_cast<const v4i*>(&kv_new[1][(id % VPR) * 8]);
-                *reinterpret_cast<v4i*>(vs + (id / VPR) * VSTR + (id % VPR) * 8) = piece;
+                *reinterpret_cast<v4i*>(vs + (id / VPR) * VSTR + (id % VPR) * 8) = vr[j];
             }
         }
         float4 vc0 = vsc0, vc1 = vsc1;
@@ -469,25 +488,28 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         }
         if (more) load_v(nxt, na, nb);
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+        if (patch) {  // (uniform)
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                if constexpr (QC) {
+                    const kvi2_t cn = *reinterpret_cast<const kvi2_t*>(&kv_new[0][(HD / 4) * g + 8 * s]);
+                    if (key0 + qi == pos) k0q[s] = cn;
+                    if (key0 + 16 + qi == pos) k1q[s] = cn;
+                } else {
+                    if (key0 + qi == pos) k0r[s] = *reinterpret_cast<const v8h_t*>(&kv_new[0][32 * s + 8 * g]);
+                    if (key0 + 16 + qi == pos) k1r[s] = *reinterpret_cast<const v8h_t*>(&kv_new[0][32 * s + 8 * g]);
+                }
+            }
+        }
 #pragma unroll
         for (int s = 0; s < KS; s++) {
             v8h_t a0, a1;
             if constexpr (QC) {
-                kvi2_t c0 = k0q[s], c1 = k1q[s];
-                if (patch) {
-                    const kvi2_t cn = *reinterpret_cast<const kvi2_t*>(&kv_new[0][(HD / 4) * g + 8 * s]);
-                    if (key0 + qi >= pos) c0 = cn;
-                    if (key0 + 16 + qi >= pos) c1 = cn;
-                }
-                a0 = kv_dec8<KVM>(c0);
-                a1 = kv_dec8<KVM>(c1);
+                a0 = kv_dec8<KVM>(k0q[s]);
+                a1 = kv_dec8<KVM>(k1q[s]);
             } else {
                 a0 = k0r[s];
                 a1 = k1r[s];
-                if (patch) {
-                    if (key0 + qi >= pos) a0 = *reinterpret_cast<const v8h_t*>(&kv_new[0][32 * s + 8 * g]);
-                    if (key0 + 16 + qi >= pos) a1 = *reinterpret_cast<const v8h_t*>(&kv_new[0][32 * s + 8 * g]);
-                }
             }
             s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qh[s], s0, 0, 0, 0);
             s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, ql[s], s0, 0, 0, 0);
@@ -506,29 +528,30 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         // this wave's part of the chunk holds no visible key (past the end, or outside the window)
         if (!(key0 < sink_n || max(key0, lo) < min(key0 + 32, seq_len))) continue;
         // this lane: head qi, keys key0 + 4g + v and key0 + 16 + 4g + v
+        const bool whole = (key0 >= lo && key0 + 32 <= seq_len) || (OPT && key0 + 32 <= sink_n);  // every key of the block is visible
         float sv[8];
-        bool vis[8];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const uint32_t ka = key0 + 4 * g + v, kb = ka + 16;
-            vis[v] = ka < sink_n || (ka >= lo && ka < seq_len);
-            vis[4 + v] = kb < sink_n || (kb >= lo && kb < seq_len);
-        }
         if constexpr (QC) {
             const float ka[8] = {kc0.x, kc0.y, kc0.z, kc0.w, kc1.x, kc1.y, kc1.z, kc1.w};
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                s0[v] *= ka[v];
-                s1[v] *= ka[4 + v];
-            }
-        }
+            for (int v = 0; v < 4; v++) sv[v] = s0[v] * ka[v], sv[4 + v] = s1[v] * ka[4 + v];
+        } else {
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            sv[v] = vis[v] ? s0[v] : -INFINITY;
-            sv[4 + v] = vis[4 + v] ? s1[v] : -INFINITY;
-            mx = fmaxf(mx, fmaxf(sv[v], sv[4 + v]));
+            for (int v = 0; v < 4; v++) sv[v] = s0[v], sv[4 + v] = s1[v];
         }
+        if (!whole) {  // (uniform) an invisible key's score and V row scale count for nothing
+            float va[8] = {vc0.x, vc0.y, vc0.z, vc0.w, vc1.x, vc1.y, vc1.z, vc1.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t key = key0 + (e >> 2) * 16 + 4 * g + (e & 3);
+                const bool vis = key < sink_n || (key >= lo && key < seq_len);
+                sv[e] = vis ? sv[e] : -INFINITY;
+                va[e] = vis ? va[e] : 0.f;
+            }
+            if (QC) vc0 = make_float4(va[0], va[1], va[2], va[3]), vc1 = make_float4(va[4], va[5], va[6], va[7]);
+        }
+        float mx = sv[0];
+#pragma unroll
+        for (int e = 1; e < 8; e++) mx = fmaxf(mx, sv[e]);
         mx = max_rows4(mx);
         const float m_new = fmaxf(m_run, mx);      // finite: the block holds a visible key
         float alpha = __expf(m_run - m_new);         // 0 for the wave's first block
@@ -537,12 +560,12 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
             const float va[8] = {vc0.x, vc0.y, vc0.z, vc0.w, vc1.x, vc1.y, vc1.z, vc1.w};
             float vmx = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; e++) vmx = fmaxf(vmx, vis[e] ? va[e] : 0.f);
+            for (int e = 0; e < 8; e++) vmx = fmaxf(vmx, va[e]);
             vmx = max_rows4(vmx);
             const float u_new = fmaxf(u_run, vmx);  // > 0: a visible row's scale is at least f32::EPSILON
             const float inv_u = 1.0f / u_new;
 #pragma unroll
-            for (int e = 0; e < 8; e++) vw[e] = vis[e] ? va[e] * inv_u : 0.f;
+            for (int e = 0; e < 8; e++) vw[e] = va[e] * inv_u;
             l_run = l_run * alpha;                  // the sum is rescaled by the softmax factor only
             alpha *= u_run * inv_u;                 // the accumulator also changes its unit
             u_run = u_new;

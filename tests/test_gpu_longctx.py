@@ -401,6 +401,30 @@ def test_paged_prefill_equals_contiguous_bit_for_bit(backend, mode, window, sink
         gpu.close()
 
 
+@pytest.mark.parametrize("mode,hd", [(KV_F16, 128), (KV_F16, 64), (KV_I8, 128), (KV_FP8_E4M3, 128), (KV_I8, 32), (KV_FP8_E4M3, 256)])
+@pytest.mark.parametrize("page_size", [0, 16, 128])
+def test_rows_behind_the_end_of_a_sequence_count_for_nothing(backend, mode, hd, page_size):
+    """The decode attention reads tiles of 16 rows of which the last is there in part: what an earlier prompt left behind the end - here rows
+    of NaN, which no weight of 0 makes harmless - changes no bit of the logits, wherever in a tile, a block of 32 or a chunk the sequence ends."""
+    cfg = dict(fmt=Q1, n_layers=2, h=256, inter=256, nq=256 // hd * 4, nkv=max(256 // hd, 1), hd=hd, vocab=64, max_seq=300, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 12)
+    rows = _rows(5, 140, 256)
+    fresh, used = HipModel(backend, cfg, w), HipModel(backend, cfg, w)
+    try:
+        for m in (fresh, used):
+            if mode != KV_F16 or page_size:
+                m.set_attention(mode, 0, 0, page_size, -(-300 // page_size) if page_size else 0)
+        used.prefill(np.full((299, 256), np.nan, dtype=np.float32), 0, want_logits=False)
+        for m in (fresh, used):
+            m.prefill(rows[:14], 0, want_logits=False)
+        for pos in range(14, 140):
+            a, b = (m.forward(rows[pos], pos)[0] for m in (fresh, used))
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b), pos
+    finally:
+        fresh.close()
+        used.close()
+
+
 def test_page_pool_accounting(backend):
     """The bookkeeping of crates/oxibonsai-model/tests/paged_kv_cache_tests.rs: lazy allocation, capacity in whole
     pages, exhaustion, pages returning to the pool when a sequence is dropped."""
