@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "attn_walk.h"
 #include "layout.h"
 
 #define OXB_GEMV_MAX_BATCH 4         // activation vectors per pass over the weights when the kernel quantises them itself
@@ -11,7 +12,9 @@
 
 // What the kernel's prologue does with x before quantising it, and what its epilogue does with the row sums.
 enum { OXB_GEMV_PRO_F32 = 0,        // a = x
-       OXB_GEMV_PRO_RMSNORM = 1 };  // a = norm_w * x / sqrt(mean(x^2) + eps)        (simd_float_ops.rs:204-215)
+       OXB_GEMV_PRO_RMSNORM = 1,    // a = norm_w * x / sqrt(mean(x^2) + eps)        (simd_float_ops.rs:204-215)
+       OXB_GEMV_PRO_SLOTS = 2 };    // a = the decode attention's output: x, or the slots that it has left (one vector)
+#define OXB_GEMV_MAX_SLOTS 8        // OxbAttnSlots::most
 enum { OXB_GEMV_STORE = 0,          // y = W a
        OXB_GEMV_ACCUM = 1,          // y += W a
        OXB_GEMV_RESIDUAL = 2,       // y = residual + W a
@@ -35,6 +38,7 @@ struct OxbGemvParams {
     uint32_t tpw;                 // filled by the launcher: tile slots per workgroup
     uint32_t codes_bytes, scales_bytes;  // buffer extents (loads beyond them read 0)
     int pro, epi;
+    OxbAttnSlots slots;           // OXB_GEMV_PRO_SLOTS only
 };
 
 // One launch covers at most OXB_GEMV_MAX_SB superblocks of K; the caller splits longer rows (first launch with the

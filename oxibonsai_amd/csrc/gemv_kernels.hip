@@ -690,6 +690,60 @@ __device__ __forceinline__ v4f mfma_f4_double_b(const v4i a, const v4i b, const 
 // value - the same digits against a constant -1 - takes the digit sums off again.  No shifts by bit position and no
 // sign turns: every weight reads the same.  A block costs 8 + 4 vector instructions and one MFMA (the int8 route: 15
 // and two).
+// The O projection behind the decode attention of one sequence.  While its slots are few they are added up here, by the
+// waves that quantise the sums, instead of by the last workgroup of each kv head to arrive, whose wait for the stores, count,
+// loads and weights are a chain of four trips to memory.  How many there are hangs on the position, which is requested with
+// the attention's own output, what counts in the other case; the slots then behind the weights.  us per step, merged by the attention /
+// here: 16 q heads of 128 (28 layers) with three slots of fp16 (300 positions) 811 / 789, with six (700) 811 / 791; 32 q heads (36
+// layers), FP8, with eight (1800) 1256 / 1214.  With room for 16 slots (twice the requests, most of them for nothing): six 812, eight 1268,
+// 12 slots of 16 heads 844 / 820.  The other case goes straight on: a jump costs it an instruction fetch, 0.3 us.
+// A lane adds up eight outputs in a row of one head (slots in ascending order, weight e^(m - M) as the attention's merge
+// has it); the wave's LDS slice turns them into the lane's share as above.
+template <int NSBW>
+__device__ __forceinline__ void merge_slots(const OxbGemvParams& p, uint32_t pos, uint32_t sb0, int sb_lim, float* buf, float (&xe)[NSBW][8]) {
+    const OxbAttnSlots& a = p.slots;
+    const uint32_t used = oxb_attn_slots_used(oxb_attn_walk(pos, a.window, a.sinks, a.chunk).n_walk, a.n_splits);
+    if (__builtin_expect(used < 2 || used > a.most, 1)) return;
+    const uint32_t lane = threadIdx.x & 63u, hd = 1u << a.hd_shift, stride = (hd + OXB_ATTN_PART_PAD) * 4u;
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(a.part, (p.k >> a.hd_shift) * a.n_splits * stride);
+#pragma unroll
+    for (int i = 0; i < NSBW; i++) {
+        const uint32_t e0 = (sb0 + i) * 512u + 8u * lane, d = e0 & (hd - 1);
+        const bool in = i < sb_lim && e0 < p.k;
+        const uint32_t at = (e0 >> a.hd_shift) * a.n_splits * stride;
+        v4f o[OXB_GEMV_MAX_SLOTS][2];
+        float m[OXB_GEMV_MAX_SLOTS], l[OXB_GEMV_MAX_SLOTS];
+#pragma unroll
+        for (uint32_t t = 0; t < OXB_GEMV_MAX_SLOTS; t++) {  // (entries past the last slot read 0)
+            const uint32_t row = in && t < used ? at + t * stride : OXB_OOB_BASE;
+            const v2u ml = __builtin_amdgcn_raw_buffer_load_b64(r, (int)(row + hd * 4u), 0, 0);
+            m[t] = t < used ? __uint_as_float(ml.x) : -INFINITY, l[t] = __uint_as_float(ml.y);
+            o[t][0] = __builtin_bit_cast(v4f, buf_load_b128(r, row + d * 4u)), o[t][1] = __builtin_bit_cast(v4f, buf_load_b128(r, row + d * 4u + 16u));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every request before the first use
+        float M = m[0], L = 0.f, v[8] = {};
+#pragma unroll
+        for (uint32_t t = 1; t < OXB_GEMV_MAX_SLOTS; t++) M = fmaxf(M, m[t]);
+#pragma unroll
+        for (uint32_t t = 0; t < OXB_GEMV_MAX_SLOTS; t++) {
+            const float w = __expf(m[t] - M);  // 0 past the last slot
+            L = fmaf(w, l[t], L);
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = fmaf(o[t][e >> 2][e & 3], w, v[e]);
+        }
+        const float inv = L > 0.f ? 1.0f / L : 0.f;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            *reinterpret_cast<v4f*>(&buf[8 * lane + 4 * (lane >> 2) + 4 * h]) = (v4f){v[4 * h] * inv, v[4 * h + 1] * inv, v[4 * h + 2] * inv, v[4 * h + 3] * inv};
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int e = 0; e < 8; e++) xe[i][e] = buf[(lane >> 2) * 36 + (lane & 3u) + 4 * e];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 template <int FMT, int NSBW, int TG, int PRO>
 __global__ __launch_bounds__(512) void gemv_f4_kernel(const OxbGemvParams p) {
     extern __shared__ uint32_t smem[];
@@ -727,6 +781,8 @@ __global__ __launch_bounds__(512) void gemv_f4_kernel(const OxbGemvParams p) {
     const __amdgpu_buffer_rsrc_t r_x = make_rsrc(p.x, p.k * 4u);
     const __amdgpu_buffer_rsrc_t r_w = make_rsrc(p.norm_w, PRO == OXB_GEMV_PRO_RMSNORM ? p.k * 4u : 0u);
     float xe[NSBW][8], we[NSBW][8];
+    uint32_t pos = 0;
+    if (PRO == OXB_GEMV_PRO_SLOTS) pos = buf_load_b32(make_rsrc(p.slots.pos, 4u), 0u);
 #pragma unroll
     for (int i = 0; i < NSBW; i++) {
         const uint32_t off = i < sb_lim ? (sb0 + i) * 2048u + koff : OXB_OOB_BASE;  // beyond k the buffer returns 0
@@ -754,6 +810,7 @@ __global__ __launch_bounds__(512) void gemv_f4_kernel(const OxbGemvParams p) {
     // it does not change which power of two the slices get and is applied to the row sums at the end (the waves
     // leave their sums of squares in LDS and go on: no barrier, no wait for the other slices in the prologue).
     uint32_t bad = 0;
+    if (PRO == OXB_GEMV_PRO_SLOTS) merge_slots<NSBW>(p, (uint32_t)__builtin_amdgcn_readfirstlane((int)pos), sb0, sb_lim, reinterpret_cast<float*>(stage), xe);
     if (PRO == OXB_GEMV_PRO_RMSNORM) {
         float ss = 0.f;
 #pragma unroll
@@ -1096,6 +1153,8 @@ static hipError_t launch_gemv_f4_t(const OxbGemvParams& p, const GemvPlan& pl, h
     const size_t shm = oxb_gemv_f4_lds_bytes(pl.S, TG);
     if (p.pro == OXB_GEMV_PRO_RMSNORM)
         hipLaunchKernelGGL((gemv_f4_kernel<FMT, NSBW, TG, OXB_GEMV_PRO_RMSNORM>), dim3(pl.grid), dim3(pl.S * 64), shm, st, p);
+    else if (p.pro == OXB_GEMV_PRO_SLOTS)
+        hipLaunchKernelGGL((gemv_f4_kernel<FMT, NSBW, TG, OXB_GEMV_PRO_SLOTS>), dim3(pl.grid), dim3(pl.S * 64), shm, st, p);
     else
         hipLaunchKernelGGL((gemv_f4_kernel<FMT, NSBW, TG, OXB_GEMV_PRO_F32>), dim3(pl.grid), dim3(pl.S * 64), shm, st, p);
     return hipGetLastError();
@@ -1137,7 +1196,8 @@ static bool check_gemv_args(const OxbGemvParams& p) {
     if (p.nvec == 0 || p.nvec > (p.xq ? OXB_GEMV_PACKED_MAX_BATCH : OXB_GEMV_MAX_BATCH)) return false;
     if (p.xq && (p.nvg != (p.nvec + 3) / 4 || p.xq_bytes < oxb_gemv_pack_dwords(p.n_sb, p.nvg) * 4)) return false;
     if (p.codes_bytes >= 0x7FFFFFFFull || (uint64_t)p.k * 4 >= OXB_OOB_BASE) return false;
-    if (p.pro != OXB_GEMV_PRO_F32 && p.pro != OXB_GEMV_PRO_RMSNORM) return false;
+    if (p.pro != OXB_GEMV_PRO_F32 && p.pro != OXB_GEMV_PRO_RMSNORM && p.pro != OXB_GEMV_PRO_SLOTS) return false;
+    if (p.pro == OXB_GEMV_PRO_SLOTS && (p.nvec != 1 || p.xq || !p.slots.part || !p.slots.pos || p.slots.most > OXB_GEMV_MAX_SLOTS || p.slots.hd_shift < 3)) return false;
     if (p.pro == OXB_GEMV_PRO_RMSNORM && !p.norm_w) return false;
     if (p.epi == OXB_GEMV_RESIDUAL && !p.residual) return false;
     if (p.epi == OXB_GEMV_SWIGLU && (p.sb_begin != 0 || p.sb_count != p.n_sb)) return false;  // needs the whole K

@@ -4,6 +4,7 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include "attn_walk.h"
 #include "kv_quant_device.h"
 #include "operand_device.h"
 
@@ -38,6 +39,8 @@ struct OxbAttnParams {
     uint32_t* done;                      // n_splits > 1: [batch][nkv] arrival counters, zero before the launch; the kernel leaves them zero
     const uint32_t* pos;                 // [batch], device; seq_len = pos + 1
     uint32_t nq, nkv, hd, max_seq, n_layers, layer, n_splits;
+    uint32_t leave;                      // fp32 outputs: so many slots at most are left in p.part as they are (OxbAttnSlots::most).  Beside
+                                         // n_splits, which is read early: 0.15 us for the merge otherwise
     uint32_t wide;                       // eight waves (256 positions at a time) instead of four (128): one-byte rows and hd <= 128 only
     float scale;                         // 1 / sqrt(hd)
     // Optional: the workgroup that merges the slots of (sequence b, kv head) also leaves its 512 outputs quantised for
@@ -58,7 +61,6 @@ hipError_t oxb_launch_kv_quantize_rows(int kv_mode, const float* d_x, uint32_t n
 hipError_t oxb_launch_kv_norm_rope_store(const OxbKvStoreParams& p, hipStream_t st);
 #define OXB_ATTN_CHUNK_POSITIONS 128  // KV positions a four-wave attention workgroup covers at a time
 #define OXB_ATTN_MAX_SPLITS 64        // slots the KV sequence is split over; slot s walks chunks s, s + n_splits, ...
-#define OXB_ATTN_PART_PAD 4           // floats after the hd outputs of a slot: maximum, sum, 2 unused (16-byte rows)
 // QK-norm, RoPE, KV store of the new position, split-KV attention (at most 16 q heads per kv head) into p.part and
 // the merge of the slots into the fp32 attention output p.out [batch][nq * hd], all in one launch.
 hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStream_t st);

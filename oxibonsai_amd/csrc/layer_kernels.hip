@@ -138,14 +138,6 @@ template <uint32_t NT, int OUT>
 __device__ __forceinline__ void attn_merge_heads(const OxbAttnParams& p, uint32_t b, uint32_t h_first, uint32_t nh, uint32_t used, float* sm);
 __device__ __forceinline__ void attn_pack_outputs(const OxbAttnParams& p, uint32_t b, uint32_t h_first, const float* kf);
 
-// Slots in use for a walk of n_walk chunks.  A second slot saves a chunk's time and costs a merge, and the two are about
-// equal (one fp16 sequence at 200, 128-position chunks: 7.6 us with one slot, 8.2 with two; six: 8.6 and 9.7): two
-// chunks stay with one workgroup, also where eight waves make them 256 positions each (INT8 at 350: one sequence
-// 9.5 and 9.7, four 10.2 and 10.5; FP8, eight at 500: 10.6 and 11.3).
-__device__ __forceinline__ uint32_t attn_slots_used(uint32_t n_walk, uint32_t n_splits) {
-    return n_walk <= 2 ? 1u : min(n_walk, n_splits);
-}
-
 // The workgroups of one (sequence, kv head) count themselves off once their slot results are written; the last one
 // to arrive merges the slots of the group's heads into the attention output, so that no second launch is needed.
 // The counter returns to 0 for the next launch.  The slot results travel between workgroups (other CUs, other XCDs)
@@ -188,16 +180,11 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
     const uint32_t slot = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const uint32_t G = p.nq / p.nkv, h0 = kvh * G, half = HD / 2;
     const uint32_t pos = p.pos[b], seq_len = pos + 1;
-    // visible keys: [0, sink_n) and [lo, seq_len)
-    const uint32_t window = OPT ? p.window : 0u;
-    const uint32_t budget = window > p.sinks ? window - p.sinks : 0u;
-    const uint32_t lo = window ? (seq_len > budget ? seq_len - budget : 0u) : 0u;
-    const uint32_t sink_n = window ? min(p.sinks, seq_len) : 0u;
-    // the chunks that hold a visible key, in ascending order: `skip_at` of them, then a gap, then up to the new position's
-    const uint32_t lo_chunk = min(lo, pos) / CH, skip_at = min((sink_n + CH - 1) / CH, lo_chunk), gap = lo_chunk - skip_at;
-    const uint32_t n_walk = (seq_len + CH - 1) / CH - gap;
+    // visible keys: [0, sink_n) and [lo, seq_len); the chunks that hold one
+    const OxbAttnWalk walk = oxb_attn_walk(pos, OPT ? p.window : 0u, p.sinks, CH);
+    const uint32_t lo = walk.lo, sink_n = walk.sink_n, skip_at = walk.skip_at, gap = walk.gap, n_walk = walk.n_walk;
     auto chunk_of = [&](uint32_t i) -> uint32_t { return OPT && i >= skip_at ? i + gap : i; };
-    const uint32_t used = attn_slots_used(n_walk, p.n_splits);
+    const uint32_t used = oxb_attn_slots_used(n_walk, p.n_splits);
     if (slot >= used) return;  // never read by the merge
     const bool owner = (n_walk - 1) % used == slot;  // this workgroup stores the new position
     float* part = p.part + (((size_t)b * p.nq + h0) * p.n_splits + slot) * (HD + OXB_ATTN_PART_PAD);
@@ -653,6 +640,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
         }
         return;
     }
+    if (OUT == OXB_ATTN_OUT_F32 && used <= p.leave) return;  // (few slots: the O projection adds them up)
     if (attn_last_arrival(p, b, kvh, used, &last_flag))  // (the barrier inside also retires mo / mm / ml)
         attn_merge_heads<NT, OUT>(p, b, h0, G, used, reinterpret_cast<float*>(&vs_all[0][0]));
 }

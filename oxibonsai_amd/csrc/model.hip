@@ -225,9 +225,11 @@ static int gate_up_swiglu(const Weight& gate_up, const float* x, uint32_t ldx, u
 // one pack launch in front of each where the vectors are quantised ahead.
 static int encode_ffn(float* hidden, const float* attn_out, const float* ffn_norm, float eps, const Weight& o,
                       const Weight& gate_up, const Weight& down, float* gu, float* act, uint32_t h, uint32_t inter,
-                      uint32_t attn_k, uint32_t nb, DevBuf* pack, DevBuf* o_prepacked = nullptr) {
-    // (o_prepacked: the attention kernel has left attn_out quantised there)
-    OXB_TRY(proj(o, attn_out, attn_k, nb, hidden, h, OXB_GEMV_PRO_F32, nullptr, 0.f, OXB_GEMV_RESIDUAL, hidden, o_prepacked ? o_prepacked : pack,
+                      uint32_t attn_k, uint32_t nb, DevBuf* pack, DevBuf* o_prepacked = nullptr,
+                      const OxbAttnSlots* slots = nullptr) {
+    // (o_prepacked: the attention kernel has left attn_out quantised there; slots: or its slot results where they are few)
+    if (slots) OXB_TRY(gemv_launch(o, attn_out, attn_k, nb, hidden, h, OXB_GEMV_PRO_SLOTS, nullptr, 0.f, OXB_GEMV_RESIDUAL, hidden, nullptr, false, slots));
+    else OXB_TRY(proj(o, attn_out, attn_k, nb, hidden, h, OXB_GEMV_PRO_F32, nullptr, 0.f, OXB_GEMV_RESIDUAL, hidden, o_prepacked ? o_prepacked : pack,
                  o_prepacked != nullptr));
     OXB_TRY(gate_up_swiglu(gate_up, hidden, h, nb, ffn_norm, eps, gu, act, inter, pack));
     OXB_TRY(proj(down, act, inter, nb, hidden, h, OXB_GEMV_PRO_F32, nullptr, 0.f, OXB_GEMV_RESIDUAL, hidden, pack));
@@ -469,12 +471,15 @@ static int kv_sync_table(Model& m) {
     return OXB_HIP_OK;
 }
 
+// KV positions that a workgroup of the decode attention walks at a time.
+static uint32_t attn_chunk(const Model& m) { return OXB_ATTN_CHUNK_POSITIONS * (m.attn_wide ? 2u : 1u); }
+
 // QK-norm + RoPE + KV store + split-KV attention of one layer for the whole decode batch, one launch; leaves the
 // slot results in m.attn_part and the parameters the merge needs in *ap.
 // One launch: QK-norm, RoPE, the store of the new rows, attention over the cache and the merge of the KV slots into
 // m.attn_out (with a single slot per sequence the kernel writes its output directly).
 static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, const float* k_norm, const Weight* pack_for = nullptr,
-                                   const OxbOperandOut* op = nullptr) {
+                                   const OxbOperandOut* op = nullptr, uint32_t leave = 0) {
     const oxb_model_desc& d = m.d;
     OxbAttnParams ap;
     ap.op = op ? *op : OxbOperandOut{nullptr, 0, 0, 0};
@@ -505,6 +510,7 @@ static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, co
     ap.layer = L;
     ap.n_splits = m.n_splits;
     ap.wide = m.attn_wide ? 1u : 0u;
+    ap.leave = leave;
     ap.scale = 1.0f / sqrtf((float)d.hd);
     ap.pack_out = pack_for ? (uint32_t*)m.gpack_o.ptr : nullptr;  // the O projection's operands, written by the merging workgroups
     ap.pack_fmt = pack_for ? (uint32_t)pack_for->L.fmt : 0;
@@ -579,12 +585,15 @@ static int encode_decode_step(Model& m, bool with_lm_head) {
         // quantised ahead of that GEMV, the attention kernel's merging workgroups do the quantising: no pack launch.
         const bool fuse_o = m.gpack_o.ptr && d.batch <= OXB_GEMV_PACKED_MAX_BATCH && d.batch >= gemv_packed_min_batch(qd) &&
                             (d.nq / d.nkv) * d.hd == 512u && m.gpack_o.cap >= oxb_gemv_pack_bytes(qd, d.batch);
-        OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm, fuse_o ? wo : nullptr));
+        // One sequence: up to so many slots are added up by the O projection.
+        const OxbAttnSlots slots = {m.attn_part, m.pos, (uint32_t)__builtin_ctz(d.hd), m.n_splits, attn_chunk(m), m.window, m.sinks, OXB_GEMV_MAX_SLOTS};
+        const bool leave = d.batch == 1 && !fuse_o;
+        OXB_TRY(encode_decode_attention(m, L, q_norm, k_norm, fuse_o ? wo : nullptr, nullptr, leave ? slots.most : 0u));
         for (uint32_t b0 = 0; b0 < d.batch; b0 += chunk) {
             const uint32_t nb = (d.batch - b0) < chunk ? (d.batch - b0) : chunk;
             OXB_TRY(encode_ffn(m.hidden + (size_t)b0 * d.h, m.attn_out + (size_t)b0 * qd, ffn_norm, d.eps, *wo, *wgu, *wdn,
                                m.gu + (size_t)b0 * 2 * d.inter, m.act + (size_t)b0 * d.inter, d.h, d.inter, qd, nb, pack,
-                               fuse_o ? &m.gpack_o : nullptr));
+                               fuse_o ? &m.gpack_o : nullptr, leave ? &slots : nullptr));
         }
     }
     if (with_lm_head) {

@@ -208,9 +208,11 @@ int upload_weight(uint64_t* id, int fmt, const uint8_t* aos, size_t n_bytes, uin
 // One GEMV over resident weights, any K: launches of at most OXB_GEMV_MAX_SB superblocks, the first with the wanted
 // epilogue, the rest accumulating.  nvec <= OXB_GEMV_MAX_BATCH vectors share each pass over the weights.
 int gemv_launch(const Weight& w, const float* d_x, uint32_t ldx, uint32_t nvec, float* d_y, uint32_t ldy, int pro,
-                const float* d_norm_w, float eps, int epi, const float* d_residual, DevBuf* pack_ws, bool prepacked) {
+                const float* d_norm_w, float eps, int epi, const float* d_residual, DevBuf* pack_ws, bool prepacked,
+                const OxbAttnSlots* slots) {
     OxbGemvParams p;
     memset(&p, 0, sizeof p);
+    if (slots) p.slots = *slots;
     if (pack_ws) {  // quantise the vectors once, in a launch of its own; the GEMV then loads its operands
         const size_t need = oxb_gemv_pack_bytes(w.L.k, nvec);
         if (prepacked) {  // (the kernel that produced the vectors has left them quantised in pack_ws)

@@ -9,6 +9,7 @@
 #include <unordered_map>
 
 #include "gemm_kernels.h"
+#include "attn_walk.h"
 #include "layout.h"
 
 namespace oxb {
@@ -100,7 +101,8 @@ int gemv_device(const Weight& w, const float* d_x, float* d_y, uint32_t batch, u
 // (grown on demand: never inside a stream capture) and the GEMV loads its operands from there; with `prepacked` the
 // buffer already holds them (left there by the kernel that produced the vectors) and no pack launch is made.
 int gemv_launch(const Weight& w, const float* d_x, uint32_t ldx, uint32_t nvec, float* d_y, uint32_t ldy, int pro,
-                const float* d_norm_w, float eps, int epi, const float* d_residual, DevBuf* pack_ws = nullptr, bool prepacked = false);
+                const float* d_norm_w, float eps, int epi, const float* d_residual, DevBuf* pack_ws = nullptr, bool prepacked = false,
+                const OxbAttnSlots* slots = nullptr);  // slots: OXB_GEMV_PRO_SLOTS only
 uint32_t gemv_packed_min_batch(uint32_t k);
 // x (device, [m][ldx]) -> y (device, [m][ldy]) through the fp16 packer + MFMA GEMM.  pack_op (OXB_PACK_*) names the
 // row-wise producer fused into the packer: RMSNorm with weights d_pack_w and eps, or SwiGLU of x = [gate | up].

@@ -425,6 +425,34 @@ def test_rows_behind_the_end_of_a_sequence_count_for_nothing(backend, mode, hd, 
         used.close()
 
 
+@pytest.mark.parametrize("mode,hd,window,sinks,page_size", [(KV_F16, 128, 0, 0, 0), (KV_F16, 64, 0, 0, 16), (KV_I8, 32, 0, 0, 0), (KV_FP8_E4M3, 256, 0, 0, 128),
+                                                            (KV_F16, 128, 700, 130, 0), (KV_I8, 128, 0, 0, 0)])
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+def test_few_slots_are_added_up_by_the_o_projection(backend, fmt, mode, hd, window, sinks, page_size):
+    """One sequence's slots are merged by the O projection while there are two to eight, by the attention otherwise; with two sequences
+    always by the attention.  Positions on both sides of every line: two and three chunks, eight and nine, of 128 and (one-byte rows and a long
+    context) 256 positions.  The routes differ in the order of a few fp32 sums and in how the activations are cut into digits (2^-26 of
+    the largest and less), 1e-6 each; a slot left out or counted twice moves the sums by an eighth or more."""
+    cfg = dict(fmt=fmt, n_layers=2, h=256, inter=256, nq=640 // hd // 2 * 2, nkv=2 if hd < 256 else 1, hd=hd, vocab=320, max_seq=2400 if mode != KV_I8 else 40000, eps=1e-6, rope_theta=1e6)
+    w = synth.make_model(cfg, 13)
+    edges = [200, 255, 256, 300, 511, 512, 900, 1023, 1024, 1151, 1152, 2047, 2048, 2303]
+    rows = _rows(6, edges[-1] + 1, 256)
+    one, two = HipModel(backend, cfg, w), HipModel(backend, cfg, w, batch=2)
+    try:
+        for m, n in ((one, 1), (two, 2)):
+            if mode != KV_F16 or window or page_size:
+                m.set_attention(mode, window, sinks, page_size, n * -(-cfg["max_seq"] // page_size) if page_size else 0)
+            for seq in range(n):
+                m.prefill(rows, 0, seq=seq, want_logits=False)
+        for pos in reversed(edges):
+            a = one.forward(rows[pos], pos)[0][0]
+            b = two.forward(np.stack([rows[pos], rows[pos // 2]]), np.array([pos, pos // 2]))[0][0]
+            assert np.abs(a - b).max() <= 2e-5 * np.abs(b).max(), (pos, np.abs(a - b).max(), np.abs(b).max())
+    finally:
+        one.close()
+        two.close()
+
+
 def test_page_pool_accounting(backend):
     """The bookkeeping of crates/oxibonsai-model/tests/paged_kv_cache_tests.rs: lazy allocation, capacity in whole
     pages, exhaustion, pages returning to the pool when a sequence is dropped."""
