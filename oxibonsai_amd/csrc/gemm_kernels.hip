@@ -425,12 +425,21 @@ __device__ __forceinline__ void load_half(HalfRegs<FMT>& H, __amdgpu_buffer_rsrc
 
 // Per (row tile, block) state prepared once and used by the four MFMA steps of the block.
 struct BlockDec {
-    uint32_t w0, w1;  // Q1: w0 = inverted sign bits (xor the scale's sign); TQ2: fields of the 16-weight halves as value+1
-    uint32_t d2;      // Q1: |d| in both halves of the dword; TQ2: d in both halves
+    uint32_t w0, w1;  // Q1: w0 = inverted sign bits (xor the scale's sign); TQ2: fields of the 16-weight halves as sign and magnitude bits
+    uint32_t d2;      // Q1: |d| in both halves of the dword; TQ2: d (times dmul) in both halves
 };
 
+// TQ2.  A field with both bits inverted is a sign bit above a magnitude bit (-1 = 3, 0 = 2, which is minus 0, +1 = 1); those at in-byte
+// position 3 are that as they are (two's complement: 3, 0, 1).  Shifted to the top of a half and masked it is the fp16 number +-2 or
+// +-0, and one packed multiplication by d makes the weight, twice as large as it is: three instructions for two weights where
+// building 1024 + field, subtracting 1025 and multiplying takes four.  The factor goes into the row's exponent (row_exp); a
+// matrix with a scale of 2^15 or more, twice which fp16 does not hold, has its scales halved instead (dmul, one of 1 and 1/2).
+// us, TQ2, four instructions / three: gate || up 19456 x 2560 at 64 / 301 / 512 / 2048 rows 17.0 / 38.3 / 52 / 191.5 and 15.2 / 35.7 / 52 /
+// 189; 2560 x 9728 at 16 / 128 / 512 rows 6.4 / 19.7 / 40.8 and 5.8 / 18.4 / 38.5; 5120 x 2560 at 23 / 301 / 512 rows 5.7 / 17.2 / 23.3
+// and 5.1 / 15.6 / 21.9; 2048 x 6144 at 2048 rows 60 and 55.
+
 template <int FMT>
-__device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e) {
+__device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e, uint32_t dmul) {
     BlockDec B;
     const uint32_t dbits = H.d[e];
     const uint32_t dd = (dbits & 0xFFFFu) * 0x00010001u;
@@ -441,12 +450,9 @@ __device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e)
         B.w1 = 0;
         B.d2 = dd & 0x7FFF7FFFu;
     } else {
-        // fields at in-byte position 3 are 2-bit two's complement (3, 0, 1 for -1, 0, +1): adding 1 modulo 4
-        // turns them into value+1 like the others
-        const uint32_t a = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e], b = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e + 1];
-        B.w0 = (a & 0x3F3F3F3Fu) | (((a & 0xC0C0C0C0u) + 0x40404040u) & 0xC0C0C0C0u);
-        B.w1 = (b & 0x3F3F3F3Fu) | (((b & 0xC0C0C0C0u) + 0x40404040u) & 0xC0C0C0C0u);
-        B.d2 = dd;
+        B.w0 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e] ^ 0x3F3F3F3Fu;
+        B.w1 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e + 1] ^ 0x3F3F3F3Fu;
+        B.d2 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, dd) * __builtin_bit_cast(v2h, dmul));
     }
     return B;
 }
@@ -458,7 +464,7 @@ __device__ __forceinline__ void decode_step(const BlockDec (&B)[RT], int s, v8h 
     uint32_t o[RT][4];
     // The masks live in registers (VOP3 encodings take no literal), opaque to the compiler so that
     // (x & mask) | y stays one v_and_or_b32.
-    uint32_t kmask, kmagic;
+    uint32_t kmask;
     if (FMT == OXB_FMT_Q1) {
         asm volatile("s_mov_b32 %0, 0x80008000" : "=s"(kmask));
 #pragma unroll
@@ -470,26 +476,19 @@ __device__ __forceinline__ void decode_step(const BlockDec (&B)[RT], int s, v8h 
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) o[rt][p] = (o[rt][p] & kmask) | B[rt].d2;
     } else {
-        asm volatile("s_mov_b32 %0, 0x00030003" : "=s"(kmask));
-        asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(kmagic));
-        const v2h bias = {(_Float16)1025.0f, (_Float16)1025.0f};
-        v2h v[RT][4];
+        asm volatile("s_mov_b32 %0, 0xC000C000" : "=s"(kmask));
 #pragma unroll
         for (int p = 0; p < 4; p++)
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) o[rt][p] = ((s >> 1) ? B[rt].w1 : B[rt].w0) >> (2 * (4 * (s & 1) + p));
+            for (int rt = 0; rt < RT; rt++) o[rt][p] = ((s >> 1) ? B[rt].w1 : B[rt].w0) << (14 - 2 * (4 * (s & 1) + p));
 #pragma unroll
         for (int p = 0; p < 4; p++)
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) o[rt][p] = (o[rt][p] & kmask) | kmagic;  // fp16 1024 + field
+            for (int rt = 0; rt < RT; rt++) o[rt][p] &= kmask;  // fp16 2, -2, 0 or -0
 #pragma unroll
         for (int p = 0; p < 4; p++)
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) v[rt][p] = __builtin_bit_cast(v2h, o[rt][p]) - bias;  // exact: field - 1
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) o[rt][p] = __builtin_bit_cast(uint32_t, v[rt][p] * __builtin_bit_cast(v2h, B[rt].d2));
+            for (int rt = 0; rt < RT; rt++) o[rt][p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, o[rt][p]) * __builtin_bit_cast(v2h, B[rt].d2));
     }
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
@@ -545,7 +544,10 @@ __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A
 }
 
 // Exponent that undoes the scaling of token row m, INT32_MIN for a row that holds something non-finite.
-__device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) { return p.xsh ? p.xsh[m] : p.x_exp; }
+__device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) {
+    const int e = p.xsh ? p.xsh[m] : p.x_exp;
+    return e == INT32_MIN ? e : e - p.w_twice;
+}
 
 // SWIGLU with the next product's operand as the output: |silu(gate) up| <= |gate up| <= w_mant 2^w_exp norm2 (Cauchy-Schwarz), so that
 // times 2^shift it lies below 2^15: a factor of two from fp16's end for the roundings on the way.
@@ -601,6 +603,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
+    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
 
     v4f acc[RT][CT];
 #pragma unroll
@@ -652,7 +655,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
     BlockDec bd[RT], bdn[RT];
     v8h A[RT];
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][0], 0);
+    for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][0], 0, dmul);
     decode_step<FMT, RT>(bd, 0, A);
     const uint32_t boff = g * 4 * BM + r;  // this lane's B operand of step s, token tile ct: xs[boff + s*BM + 16 ct]
     const v8h* x0 = reinterpret_cast<const v8h*>(xs0);
@@ -662,7 +665,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
         // block 0 of the superblock
         stage_x(sb * 4 + 1, xs1);
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) bdn[rt] = prepare_block<FMT>(H[rt][0], 1);
+        for (int rt = 0; rt < RT; rt++) bdn[rt] = prepare_block<FMT>(H[rt][0], 1, dmul);
         block_steps<FMT, RT, CT>(x0, A, bd, bdn, acc, boff);
         publish();
         // block 1: half 0 is consumed; reload it for the next superblock
@@ -671,7 +674,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][1], 0);
+            bdn[rt] = prepare_block<FMT>(H[rt][1], 0, dmul);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][0], rc, rs, tile_at(rt), (uint32_t)rt < n_valid, p.n_sb, sb + 1, 0, lane);
@@ -683,7 +686,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][1], 1);
+            bdn[rt] = prepare_block<FMT>(H[rt][1], 1, dmul);
         }
         block_steps<FMT, RT, CT>(x0, A, bd, bdn, acc, boff);
         publish();
@@ -693,7 +696,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][0], 0);
+            bdn[rt] = prepare_block<FMT>(H[rt][0], 0, dmul);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][1], rc, rs, tile_at(rt), (uint32_t)rt < n_valid, p.n_sb, sb + 1, 1, lane);
@@ -837,6 +840,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     const uint32_t per = (s1 - s0 + 7u) / 8u, h0 = s0 + wave * per, h1 = min(h0 + per, s1);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
+    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
 
     v4f acc[RT][CT];
 #pragma unroll
@@ -884,7 +888,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
                 for (int bi = 0; bi < 2; bi++)
 #pragma unroll
-                    for (int rt = 0; rt < RT; rt++) bd[EARLY ? bi : 0][rt] = prepare_block<FMT>(H[rt][hh], bi);
+                    for (int rt = 0; rt < RT; rt++) bd[EARLY ? bi : 0][rt] = prepare_block<FMT>(H[rt][hh], bi, dmul);
                 if (REFILL) refill();
             }
 #pragma unroll
@@ -895,7 +899,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
                 }
                 if (!EARLY) {
 #pragma unroll
-                    for (int rt = 0; rt < RT; rt++) bd[0][rt] = prepare_block<FMT>(H[rt][hh], bi);
+                    for (int rt = 0; rt < RT; rt++) bd[0][rt] = prepare_block<FMT>(H[rt][hh], bi, dmul);
                     if (REFILL && bi) refill();
                 }
 #pragma unroll

@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(OxbLayout L, const uint32_
 // unit, one thread per output dword: stores are contiguous, the 2-byte-aligned block bytes are read as halves.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void repack_kernel(OxbLayout L, const uint16_t* __restrict__ aos,
-                                                     uint32_t* __restrict__ codes, uint16_t* __restrict__ scales) {
+                                                     uint32_t* __restrict__ codes, uint16_t* __restrict__ scales, uint32_t* loud) {
     const uint32_t bpr = L.k / OXB_QK;
     const uint32_t tile = blockIdx.x / L.n_sb, sb = blockIdx.x % L.n_sb;
     const uint32_t t = threadIdx.x;
@@ -1073,6 +1073,7 @@ __global__ __launch_bounds__(256) void repack_kernel(OxbLayout L, const uint16_t
             const uint16_t* b = aos + ((size_t)row * bpr + blk) * halves;
             d = L.fmt == OXB_FMT_Q1 ? b[0] : b[16];
         }
+        if ((d & 0x7FFFu) >= 0x7800u) *loud = 1;  // 2^15 and more
         scales[(size_t)blockIdx.x * 64 + t] = d;
     }
     for (uint32_t dwi = t; dwi < L.unit_dwords; dwi += 256) {
@@ -1276,11 +1277,11 @@ hipError_t oxb_launch_dequant(const OxbLayout& L, const uint32_t* d_codes, const
     return hipGetLastError();
 }
 
-hipError_t oxb_launch_repack(const OxbLayout& L, const uint8_t* d_aos, uint32_t* d_codes, uint16_t* d_scales, hipStream_t st) {
+hipError_t oxb_launch_repack(const OxbLayout& L, const uint8_t* d_aos, uint32_t* d_codes, uint16_t* d_scales, uint32_t* d_loud, hipStream_t st) {
     const uint64_t units = (uint64_t)L.n_tiles * L.n_sb;
     if (units == 0) return hipSuccess;
     if (units > 0x7FFFFFFFull) return hipErrorInvalidValue;
     hipLaunchKernelGGL(repack_kernel, dim3((uint32_t)units), dim3(256), 0, st, L, reinterpret_cast<const uint16_t*>(d_aos),
-                       d_codes, d_scales);
+                       d_codes, d_scales, d_loud);
     return hipGetLastError();
 }

@@ -162,14 +162,18 @@ int bind_shape(Weight& w, uint32_t n_rows, uint32_t k) {
         return fail(OXB_HIP_INVALID_ARGUMENT,
                     "invalid argument: a weight uploaded without a shape cannot be bound inside a stream capture; call once before capturing");
     const OxbLayout L = oxb_make_layout(w.L.fmt, n_rows, k);
-    const size_t total = L.codes_bytes + L.scales_bytes;
+    const size_t flag_at = (L.codes_bytes + L.scales_bytes + 3) / 4 * 4, total = flag_at + 4;
     void* base = nullptr;
     hipError_t e = hipMalloc(&base, total);
     if (e != hipSuccess)
         return fail(OXB_HIP_OUT_OF_MEMORY, "out of device memory: requested %zu bytes on device %d", total, g_rt.device);
     uint32_t* codes = reinterpret_cast<uint32_t*>(base);
     uint16_t* scales = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(base) + L.codes_bytes);
-    e = oxb_launch_repack(L, reinterpret_cast<const uint8_t*>(w.d_raw), codes, scales, g_rt.stream);
+    uint32_t* flag = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(base) + flag_at);
+    uint32_t loud = 0;
+    e = hipMemsetAsync(flag, 0, 4, g_rt.stream);
+    if (e == hipSuccess) e = oxb_launch_repack(L, reinterpret_cast<const uint8_t*>(w.d_raw), codes, scales, flag, g_rt.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&loud, flag, 4, hipMemcpyDeviceToHost, g_rt.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g_rt.stream);
     if (e != hipSuccess) {
         (void)hipFree(base);
@@ -181,6 +185,7 @@ int bind_shape(Weight& w, uint32_t n_rows, uint32_t k) {
     w.d_base = base;
     w.d_codes = codes;
     w.d_scales = scales;
+    w.loud = loud != 0;
     return OXB_HIP_OK;
 }
 
@@ -311,6 +316,7 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
     p.xh = (const uint32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xh2.ptr : ws->xh.ptr);
     p.xsh = flow.in == GemmFlow::ATTENTION ? nullptr : (const int32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xsh2.ptr : ws->xsh.ptr);
     p.x_exp = flow.x_exp;
+    p.w_twice = w.L.fmt == OXB_FMT_TQ2 && !w.loud;
     if (flow.out) p.xh_out = (uint32_t*)ws->xh2.ptr, p.xsh_out = (int32_t*)ws->xsh2.ptr, p.norm2 = (const float*)ws->norm.ptr, p.w_mant = frexpf(flow.w_norm2, &p.w_exp);
     p.y = d_y;
     p.residual = d_residual;

@@ -50,6 +50,7 @@ struct Weight {
     uint16_t* d_scales = nullptr;
     void* d_raw = nullptr;
     size_t raw_blocks = 0;
+    bool loud = false;  // a scale is 2^15 or more: twice that is no fp16 number
     // What the bounds of a product's outputs come from (find_bounds, model.hip): the largest norm of the rows from row0 on and the one in
     // the middle, for inputs that went through the norm weights of that serial number; max < 0: not worked out yet.
     struct RowNorms { uint32_t row0 = 0; uint64_t vector = 0; float max = -1.f, median = -1.f; } norms;

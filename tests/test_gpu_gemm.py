@@ -258,3 +258,17 @@ def test_gemm_subnormal_fp16_scales(backend, fmt):
     got = _gemm(backend, fmt, a, x, m, n, k)
     _check_against_truth(got, dense_f64(fmt, a, n, k), x)
     assert np.count_nonzero(got) == got.size
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 128), (23, 40, 640), (70, 48, 384), (130, 330, 1152), (300, 70, 2048)])
+@pytest.mark.parametrize("loudest", [32752.0, 32768.0, 65504.0])
+def test_gemm_ternary_scales_on_both_sides_of_a_doubled_weight(backend, m, n, k, loudest):
+    # weights enter the products twice as large where fp16 holds that, as they are in a matrix that has one scale it does not hold
+    rng = np.random.default_rng(int(loudest) + m)
+    scales = rng.choice([0.004, 0.7, 300.0, -2.5], n * k // 128)
+    scales[rng.integers(0, n * k // 128)] = -loudest
+    a = np.concatenate([tq2_block(float(s), rng.integers(0, 256, 32, dtype=np.uint8)) for s in scales])
+    x = synth.normal_f32(12, m * k).reshape(m, k)
+    got = _gemm(backend, TQ2, a, x, m, n, k)
+    assert np.all(np.isfinite(got))
+    _check_against_truth(got, dense_f64(TQ2, a, n, k), x)
