@@ -220,7 +220,12 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
     };
     struct Tile { size_t row; uint32_t n; };  // first row, and how many of the 16 are there
     auto tile_of = [&](uint32_t key, uint32_t page) -> Tile {
-        const uint32_t n = key < seq_len ? min(seq_len - key, 16u) : 0u;
+        // (Opaque: of key < seq_len ? min(seq_len - key, 16) : 0 the compiler drops the test, for it takes the difference in the minimum
+        // for one that never wraps; other ways to write it become vector instructions, and the descriptors loops: six sequences
+        // 16.7 -> 18.4 us.)
+        uint32_t left = seq_len - key;
+        asm("" : "+s"(left));
+        const uint32_t n = key < seq_len ? min(left, 16u) : 0u;
         return {paged ? row0 + ((size_t)page << pshift) + (key & pmask) : row0 + key, n};
     };
 
