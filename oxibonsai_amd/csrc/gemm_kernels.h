@@ -65,7 +65,8 @@ hipError_t oxb_launch_pair_norms(const uint16_t* d_scales, uint32_t n_sb, uint32
 // d_out[i] = the 2-norm of matrix row row0 + i with column j times w[j], i < n, and d_out[n + i] the same with no |w[j]| taken as more
 // than `typical`.  row0 and n are multiples of 16.
 hipError_t oxb_launch_weighted_norms(const uint16_t* d_scales, uint32_t n_sb, uint32_t row0, uint32_t n, const float* d_w, uint32_t k, float typical, float* d_out, hipStream_t st);
-// What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16, or the wide one
+// What the launcher runs for p: the narrow kernel with rt row tiles per workgroup and ct token tiles of 16 (rt 0: the tall one with
+// tpw row tiles per workgroup), or the wide one
 // with rt row tiles per wave, tpw per workgroup, 16 ct tokens per tile; K in ksplit slices of sb_per_split superblocks.
 struct OxbGemmPlan { bool narrow; uint32_t rt, tpw, ct, ksplit, sb_per_split; };
 OxbGemmPlan oxb_gemm_plan(int fmt, const OxbGemmParams& p, uint32_t n_cus);

@@ -998,6 +998,119 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     if (sw && p.xh_out && ng == 0) finish_operand(p, 0, p.M_pad, tid, OXB_GEMM_NARROW_THREADS);
 }
 
+// ---------------------------------------------------------------------------
+// The same for matrices of many rows (an LM head) and 17 to 32 token rows, K up to 4096.  With a workgroup for each group of row tiles the
+// kernel above takes all of the activations in again and waits for its first weights every time, one workgroup on a CU: 11 us
+// each.  Here one workgroup per CU stays: a wave keeps the activations of its superblock in registers (64 for each 16 token rows) and its
+// share of the tiles streams past in pairs, RING tiles ahead.  The waves' sums of a pair meet in LDS as [token][row], two pairs' worth,
+// a barrier for each; every thread adds up a few outputs and stores them, 16 rows of a token side by side.  Reads of the sums
+// one behind the other cost 5 us of 56, stores in branches, whose number nobody knows where the next weights are waited for, 3.
+// us, 32 rows, kernel above / this one: Q1 151936 x 4096 65.4 / 50.7, x 2048 46.2 / 34.8, TQ2 84.2 / 57.3 and 52.3 / 38.3;
+// 65536 x 2560 25.3 / 21.9 and 33.7 / 25.5.
+// ---------------------------------------------------------------------------
+template <int FMT>
+__global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_tall_kernel(const OxbGemmParams p) {
+    constexpr int CT = 2, RING = 4;  // token tiles; row tiles in flight
+    __shared__ __attribute__((aligned(16))) float red[2][8][2][CT * 256];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, g = lane >> 4, threads = blockDim.x, S = threads >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));  // its superblock
+    const uint32_t t_begin = blockIdx.x * p.tpw, t_end = min(t_begin + p.tpw, p.n_tiles);
+    const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
+    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(p.y, ((p.M - 1) * p.ldy + p.n_rows) * 4u);
+    const uint32_t b_off = (4u * g * p.M_pad + r) * 16u, blk_stride = 16u * p.M_pad * 16u;
+    v8h B[4][4][CT];  // [block][step][token tile]
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) B[b][s][ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, b_off + ct * 256u, (wave * 4u + b) * blk_stride + s * p.M_pad * 16u));
+    HalfRegs<FMT> H[RING][2];
+    auto request = [&](HalfRegs<FMT> (&h)[2], uint32_t t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) load_half<FMT>(h[hh], rc, rs, t, t < t_end, p.n_sb, wave, hh, lane);
+    };
+#pragma unroll
+    for (int i = 0; i < RING; i++) request(H[i], t_begin + i);
+    // the outputs of this thread: value o = tid + i threads of a tile, row o % 16 of token o / 16
+    int e[CT];
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+        const uint32_t m = (tid + i * threads) / 16u;
+        e[i] = m < p.M ? row_exp(p, m) : 0;
+    }
+    for (uint32_t t0 = t_begin, pair = 0; t0 < t_end; t0 += RING) {
+#pragma unroll
+        for (int i = 0; i < RING; i += 2, pair++) {
+            const uint32_t t = t0 + i;
+            if (t >= t_end) break;  // (the same for all waves)
+            v4f acc[2][CT];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) acc[j][ct] = (v4f){0.f, 0.f, 0.f, 0.f};
+            // a step's weights are expanded while the products of the one before run: one product, then its share of the expansion
+            BlockDec bd[2] = {prepare_block<FMT>(H[i][0], 0, dmul), prepare_block<FMT>(H[i + 1][0], 0, dmul)};
+            v8h A[2];
+            decode_step<FMT, 2>(bd, 0, A);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < 16; st++) {
+                const int b = st >> 2, s = st & 3;
+                v8h An[2];
+                if (s == 3 && b < 3) {
+                    bd[0] = prepare_block<FMT>(H[i][(b + 1) >> 1], (b + 1) & 1, dmul);
+                    bd[1] = prepare_block<FMT>(H[i + 1][(b + 1) >> 1], (b + 1) & 1, dmul);
+                }
+                if (st < 15) decode_step<FMT, 2>(bd, (s + 1) & 3, An);
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) acc[j][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[j], B[b][s][ct], acc[j][ct], 0, 0, 0);
+                if (st < 15) A[0] = An[0], A[1] = An[1];
+#pragma unroll
+                for (int k = 0; k < 2 * CT; k++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, (FMT == OXB_FMT_Q1 ? 16 : 24) / (2 * CT), 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            request(H[i], t + RING);
+            request(H[i + 1], t + RING + 1);
+            float(*const mine)[CT * 256] = red[pair & 1u][wave];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) *reinterpret_cast<v4f*>(&mine[j][ct * 256 + r * 16 + 4 * g]) = acc[j][ct];
+            // (one barrier a pair: a wave writes the pair after next here only when all have added this one up)
+            lds_barrier();
+            // (all the reads before the first sum; a wave that does not exist adds nothing)
+            float v[2][CT][8];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int k = 0; k < CT; k++)
+#pragma unroll
+                    for (uint32_t w = 0; w < 8; w++) v[j][k][w] = red[pair & 1u][w < S ? w : 0u][j][min(tid + k * threads, CT * 256u - 1)];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int k = 0; k < CT; k++) {
+                    const uint32_t o = tid + k * threads, m = o / 16u, n = (t + j) * 16u + (o & 15u);
+                    float a = v[j][k][0];
+#pragma unroll
+                    for (uint32_t w = 1; w < 8; w++) a += w < S ? v[j][k][w] : 0.f;
+                    a = e[k] == INT32_MIN ? __int_as_float(0x7FC00000) : ldexpf(a, e[k]);
+                    // (no branch: how many stores are under way is known where the next weights are waited for)
+                    const bool there = m < p.M && n < p.n_rows && t + j < t_end;
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), ry, (int)(there ? (m * p.ldy + n) * 4u : OXB_OOB_BASE), 0, 0);
+                }
+        }
+    }
+}
+
 // y = (residual +) the K slices' partial sums, added in slice order (deterministic): where no pack of the result follows.
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, uint32_t ksplit, size_t plane,
                                                                   const float* __restrict__ residual, float* __restrict__ y,
@@ -1205,12 +1318,24 @@ static float narrow_cost(bool tq2, const OxbGemmParams& p, uint32_t rt, uint32_t
     return 1.91f + (float)(q / R) * (lat + R * busy) + (q % R ? lat + (q % R) * busy : 0.f);
 }
 
+// 16 row tiles and more for every CU, two token tiles and a wave for every superblock (four to eight).  With half the rows, 32768, the two
+// kernels are about equal (Q1 x 4096 15.2 / 15.6 us, x 2048 10.7 / 10.9, TQ2 19.6 / 17.8 and 12.2 / 12.1), with one token tile often the
+// other is faster (Q1 65536 x 2560 16.4 / 17.8 us, 151936 x 4096 42.6 / 41.5).
+static bool tall(const OxbGemmParams& p, uint32_t n_cus) {
+    return p.mode == OXB_GEMM_STORE && p.M > 16 && p.M <= 32 && p.n_sb >= 4 && p.n_sb <= 8 && p.n_tiles >= 16 * n_cus &&
+           (uint64_t)p.M * p.ldy * 4 < OXB_OOB_BASE;
+}
+
 // The narrow kernel up to OXB_GEMM_NARROW_MAX_M token rows (the wide one would spend its time on barriers and padding),
 // the cheaper of the two up to 128, the wide one beyond.
 OxbGemmPlan oxb_gemm_plan(int fmt, const OxbGemmParams& p, uint32_t n_cus) {
     const bool tq2 = fmt == OXB_FMT_TQ2, sw = p.mode == OXB_GEMM_SWIGLU;
     OxbGemmPlan best = {true, 0, 0, 0, 1, p.n_sb};
     float best_us = 1e30f;
+    if (tall(p, n_cus)) {
+        best.ct = (p.M + 15) / 16, best.tpw = (p.n_tiles + n_cus - 1) / n_cus;
+        return best;
+    }
     if (p.M <= 128) {
         // row tiles per workgroup: as many as the registers hold next to the token tiles (six: Q1 only), two or more with SWIGLU
         static const uint32_t choices[4] = {1, 2, 4, 6};
@@ -1286,6 +1411,13 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     p.ksplit = plan.ksplit;
     p.sb_per_split = plan.sb_per_split;
     if (p.ksplit > 1 && !p.part) return hipErrorInvalidValue;
+    if (plan.narrow && plan.rt == 0) {
+        p.tpw = plan.tpw;
+        const dim3 grid((p.n_tiles + p.tpw - 1) / p.tpw), block(64 * p.n_sb);
+        if (fmt == OXB_FMT_Q1) hipLaunchKernelGGL(gemm_tall_kernel<OXB_FMT_Q1>, grid, block, 0, st, p);
+        else hipLaunchKernelGGL(gemm_tall_kernel<OXB_FMT_TQ2>, grid, block, 0, st, p);
+        return hipGetLastError();
+    }
     if (plan.narrow) return launch_gemm_narrow(fmt, p, plan.rt, st);
     p.n_mt = (p.M + 16 * plan.ct - 1) / (16 * plan.ct);
     p.tpw = plan.tpw;

@@ -7,7 +7,7 @@ Inputs that are exact in fp16 must give bit-exact results, which pins the k orde
 import numpy as np
 import pytest
 
-from helpers import GEMM_FORMS, Q1, TQ2, dense_f64, parity_violations, q1_block, tq2_block
+from helpers import GEMM_FORMS, Q1, TQ2, dense_f64, gemm_plan, parity_violations, q1_block, tq2_block
 from oracle import oracle
 from oxibonsai_amd import GpuError, synth
 
@@ -272,3 +272,20 @@ def test_gemm_ternary_scales_on_both_sides_of_a_doubled_weight(backend, m, n, k,
     got = _gemm(backend, TQ2, a, x, m, n, k)
     assert np.all(np.isfinite(got))
     _check_against_truth(got, dense_f64(TQ2, a, n, k), x)
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("m,n,k", [(17, 65521, 1664), (32, 65536, 2048), (25, 65537, 2304), (31, 67777, 4096), (32, 70000, 3584), (20, 98304, 2560)])
+def test_gemm_few_rows_of_a_matrix_with_many(backend, fmt, m, n, k):
+    # an LM head's shape: a workgroup walks its share of the row tiles (16 and more: even and odd shares, one that ends early, a last tile
+    # in part), four to eight waves; the last share and the rows on both sides of a share's end, and some in between
+    assert gemm_plan(fmt, m, n, k)[:2] == (1, 0)
+    a = synth.make_blocks(fmt, 4000 + m, n, k)
+    x = synth.normal_f32(13 + k, m * k).reshape(m, k)
+    got = _gemm(backend, fmt, a, x, m, n, k)
+    per = -(-(-(-n // 16)) // 256) * 16
+    rows = np.unique(np.concatenate([np.arange(40), np.arange(per - 20, per + 20), np.arange(128 * per - 20, 128 * per + 20).clip(0, n - 1),
+                                     np.arange(0, n, 997), np.arange(n - 60, n)]))
+    sub = a.reshape(n, -1)[rows]
+    _check_against_truth(got[:, rows], dense_f64(fmt, np.ascontiguousarray(sub).reshape(-1), rows.size, k), x)
+    assert np.all(np.isfinite(got))
