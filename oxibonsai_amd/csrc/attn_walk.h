@@ -11,7 +11,7 @@
 // chunks stay with one workgroup, also where eight waves make them 256 positions each (INT8 at 350: one sequence
 // 9.5 and 9.7, four 10.2 and 10.5; FP8, eight at 500: 10.6 and 11.3).
 __device__ __forceinline__ uint32_t oxb_attn_slots_used(uint32_t n_walk, uint32_t n_splits) {
-    return n_walk <= 2 ? 1u : min(n_walk, n_splits);
+    return n_walk <= 2 ? 1u : n_walk < n_splits ? n_walk : n_splits;
 }
 
 // The keys that position `pos` sees are [0, sink_n) and [lo, pos].  The chunks of `ch` positions that hold one of them, in
@@ -23,9 +23,9 @@ __device__ __forceinline__ OxbAttnWalk oxb_attn_walk(uint32_t pos, uint32_t wind
     OxbAttnWalk w;
     const uint32_t seq_len = pos + 1, budget = window > sinks ? window - sinks : 0u;
     w.lo = window ? (seq_len > budget ? seq_len - budget : 0u) : 0u;
-    w.sink_n = window ? min(sinks, seq_len) : 0u;
-    const uint32_t lo_chunk = min(w.lo, pos) / ch;
-    w.skip_at = min((w.sink_n + ch - 1) / ch, lo_chunk);
+    w.sink_n = window ? (sinks < seq_len ? sinks : seq_len) : 0u;
+    const uint32_t lo_chunk = (w.lo < pos ? w.lo : pos) / ch, sink_chunks = (w.sink_n + ch - 1) / ch;
+    w.skip_at = sink_chunks < lo_chunk ? sink_chunks : lo_chunk;
     w.gap = lo_chunk - w.skip_at;
     w.n_walk = (seq_len + ch - 1) / ch - w.gap;
     return w;
