@@ -111,9 +111,10 @@ def parity_violations(a: np.ndarray, b: np.ndarray, tol: float = 1e-3) -> int:
 from oxibonsai_amd.gguf import GGUF_F16, GGUF_F32, GGUF_MAGIC, GGUF_Q1, GGUF_TQ2, gguf_bytes, model_gguf  # noqa: E402,F401
 
 
-# Products (format, token rows, rows, k) that between them run every form of the two GEMM kernels that the launcher picks on
-# 256 compute units: (narrow, row tiles, token tiles, K in slices).  Token rows and rows off the tiles' multiples, K of an
-# odd number of half superblocks.  tests/test_host.py holds the list to the launcher's own plans.
+# Products (format, token rows, rows, k) that between them run every form of the GEMM kernels that the launcher picks on
+# 256 compute units: (narrow, row tiles, token tiles, K in slices); no row tiles is the kernel that walks its share of a matrix
+# with very many.  Token rows and rows off the tiles' multiples, K of an odd number of half superblocks.  tests/test_host.py
+# holds the list to the launcher's own plans.
 GEMM_FORMS = {
     (Q1, 1, 1, 1, False): (1, 20, 896), (TQ2, 1, 1, 1, False): (5, 31, 640),
     (Q1, 1, 1, 2, False): (19, 17, 640), (TQ2, 1, 1, 2, False): (31, 19, 640),
@@ -135,6 +136,7 @@ GEMM_FORMS = {
     (Q1, 1, 4, 3, False): (34, 8242, 640), (TQ2, 1, 4, 3, False): (33, 8342, 640),
     (Q1, 1, 4, 4, False): (50, 8194, 640), (TQ2, 1, 4, 4, False): (49, 8205, 640),
     (Q1, 1, 6, 1, False): (1, 20605, 640), (Q1, 1, 6, 2, False): (17, 16440, 640),
+    (Q1, 1, 0, 2, False): (18, 65530, 1664), (TQ2, 1, 0, 2, False): (29, 65600, 1792),
     (Q1, 0, 1, 4, False): (142, 19, 640), (TQ2, 0, 1, 4, False): (143, 27, 640),
     (Q1, 0, 1, 4, True): (209, 20, 1152), (TQ2, 0, 1, 4, True): (136, 20, 1408),
     (Q1, 0, 1, 5, False): (129, 5557, 640), (TQ2, 0, 1, 5, False): (130, 5602, 640),
