@@ -289,6 +289,26 @@ int gemv_device(const Weight& w, const float* d_x, float* d_y, uint32_t batch, u
     return OXB_HIP_OK;
 }
 
+// What every GEMM launch on w takes from the matrix and the shape; its operand, workspace and epilogue's inputs are the caller's.
+static OxbGemmParams gemm_params(const Weight& w, float* d_y, uint32_t m, uint32_t ldy, int mode) {
+    OxbGemmParams p;
+    memset(&p, 0, sizeof p);
+    p.codes = w.d_codes;
+    p.scales = w.d_scales;
+    p.w_twice = w.L.fmt == OXB_FMT_TQ2 && !w.loud;
+    p.y = d_y;
+    p.n_rows = w.L.n_rows;
+    p.n_tiles = w.L.n_tiles;
+    p.n_sb = w.L.n_sb;
+    p.M = m;
+    p.ldy = ldy;
+    p.codes_bytes = (uint32_t)w.L.codes_bytes;
+    p.scales_bytes = (uint32_t)w.L.scales_bytes;
+    p.xh_bytes = (uint32_t)oxb_xh_bytes(w.L.k, m);
+    p.mode = mode;
+    return p;
+}
+
 int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uint32_t m, uint32_t ldy, int mode,
                 const float* d_residual, int pack_op, const float* d_pack_w, float eps, GemmWorkspace* ws, OxbPackSum* carry,
                 const GemmFlow& flow) {
@@ -309,26 +329,12 @@ int gemm_device(const Weight& w, const float* d_x, uint32_t ldx, float* d_y, uin
         return fail(OXB_HIP_INVALID_ARGUMENT, "internal error: no operand of %u rows x %u", m, k);
     if (flow.out && ((rc = ws->xh2.ensure(oxb_xh_bytes(w.L.n_rows / 2, m))) || (rc = ws->xsh2.ensure(rows4)))) return rc;
     if (carry) carry->n = 0;
-    OxbGemmParams p;
-    memset(&p, 0, sizeof p);
-    p.codes = w.d_codes;
-    p.scales = w.d_scales;
+    OxbGemmParams p = gemm_params(w, d_y, m, ldy, mode);
     p.xh = (const uint32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xh2.ptr : ws->xh.ptr);
     p.xsh = flow.in == GemmFlow::ATTENTION ? nullptr : (const int32_t*)(flow.in == GemmFlow::SWIGLU ? ws->xsh2.ptr : ws->xsh.ptr);
     p.x_exp = flow.x_exp;
-    p.w_twice = w.L.fmt == OXB_FMT_TQ2 && !w.loud;
     if (flow.out) p.xh_out = (uint32_t*)ws->xh2.ptr, p.xsh_out = (int32_t*)ws->xsh2.ptr, p.norm2 = (const float*)ws->norm.ptr, p.w_mant = frexpf(flow.w_norm2, &p.w_exp);
-    p.y = d_y;
     p.residual = d_residual;
-    p.n_rows = w.L.n_rows;
-    p.n_tiles = w.L.n_tiles;
-    p.n_sb = w.L.n_sb;
-    p.M = m;
-    p.ldy = ldy;
-    p.codes_bytes = (uint32_t)w.L.codes_bytes;
-    p.scales_bytes = (uint32_t)w.L.scales_bytes;
-    p.xh_bytes = (uint32_t)oxb_xh_bytes(k, m);
-    p.mode = mode;
     p.no_split = ws->no_split;
     p.sum_later = carry && mode == OXB_GEMM_RESIDUAL && ldy == w.L.n_rows && oxb_pack_can_sum(ldy, m);
     const uint32_t ksplit = oxb_gemm_ksplit((int)w.L.fmt, p, g_rt.n_cus);
@@ -734,22 +740,9 @@ int oxb_hip_profile_gemm(uint64_t id, const float* d_x, float* d_y, uint32_t m, 
     if (!d_x || !d_y || !avg_us || m == 0 || iters == 0)
         return fail(OXB_HIP_INVALID_ARGUMENT, "invalid argument: null buffer or zero count");
     if ((rc = gemm_device(*w, d_x, k, d_y, m, n_rows, OXB_GEMM_STORE, nullptr, OXB_PACK_IDENT, nullptr, 0.f))) return rc;  // packs x, warms up
-    OxbGemmParams p;
-    memset(&p, 0, sizeof p);
-    p.codes = w->d_codes;
-    p.scales = w->d_scales;
+    OxbGemmParams p = gemm_params(*w, d_y, m, n_rows, OXB_GEMM_STORE);
     p.xh = (const uint32_t*)g_rt.gemm_ws.xh.ptr;
     p.xsh = (const int32_t*)g_rt.gemm_ws.xsh.ptr;
-    p.y = d_y;
-    p.n_rows = n_rows;
-    p.n_tiles = w->L.n_tiles;
-    p.n_sb = w->L.n_sb;
-    p.M = m;
-    p.ldy = n_rows;
-    p.codes_bytes = (uint32_t)w->L.codes_bytes;
-    p.scales_bytes = (uint32_t)w->L.scales_bytes;
-    p.xh_bytes = (uint32_t)oxb_xh_bytes(k, m);
-    p.mode = OXB_GEMM_STORE;
     p.part = (float*)g_rt.gemm_ws.part.ptr;  // sized by the gemm_device call above
     hipEvent_t ev0, ev1;
     hipError_t e;

@@ -4,12 +4,14 @@ Tolerance: 1e-2 relative under the reference's gate form (abs_err < tol || |a-b|
 tightened by the bound the arithmetic implies: weights and products are exact, so an output differs from the
 float64 product by at most 2^-11 * sum_k |w_k x_k| (activation rounding to fp16) plus fp32 summation error.
 Inputs that are exact in fp16 must give bit-exact results, which pins the k order of both operands."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from helpers import GEMM_FORMS, Q1, TQ2, dense_f64, gemm_plan, parity_violations, q1_block, tq2_block
+from helpers import GEMM_FORMS, Q1, TQ2, DeviceBuffer, block, dense_f64, gemm_plan, parity_violations, q1_block, tq2_block
 from oracle import oracle
-from oxibonsai_amd import GpuError, synth
+from oxibonsai_amd import GpuError, _lib, synth
 
 pytestmark = pytest.mark.gpu
 GEMM_REL_TOL = 1e-2
@@ -258,6 +260,31 @@ def test_gemm_subnormal_fp16_scales(backend, fmt):
     got = _gemm(backend, fmt, a, x, m, n, k)
     _check_against_truth(got, dense_f64(fmt, a, n, k), x)
     assert np.count_nonzero(got) == got.size
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("m,n,k", [(23, 40, 640), (300, 70, 2048)])
+def test_timed_gemm_launches_are_those_of_a_call(backend, fmt, m, n, k):
+    # the launches that oxb_hip_profile_gemm times leave the bits of oxb_hip_gemm_dev, on scales that any rounding on the way changes too
+    L = _lib.lib()
+    rng = np.random.default_rng(14)
+    a = np.concatenate([block(fmt, float(s), rng.integers(0, 256, 16 if fmt == Q1 else 32, dtype=np.uint8)) for s in rng.choice([2.0**-24, 3 * 2.0**-24, 1023 * 2.0**-24, 0.7], n * k // 128)])
+    x = synth.normal_f32(15, m * k).reshape(m, k)
+    h = _upload(backend, fmt, a, n, k)
+    d_x, d_y, us = DeviceBuffer.from_numpy(x), DeviceBuffer(m * n * 4), C.c_float()
+    try:
+        outs = []
+        for run in (lambda: L.oxb_hip_gemm_dev(int(h), d_x.ptr, d_y.ptr, m, n, k),
+                    lambda: L.oxb_hip_profile_gemm(int(h), d_x.ptr, d_y.ptr, m, n, k, 1, 2, C.byref(us))):
+            d_y.fill(0xFF)
+            assert run() == 0, _lib.last_error()
+            assert L.oxb_hip_synchronize() == 0
+            outs.append(d_y.to_numpy(np.uint32, (m, n)))
+        assert np.array_equal(*outs) and us.value > 0
+    finally:
+        d_x.free()
+        d_y.free()
+        backend.free_weights(h)
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (23, 40, 640), (70, 48, 384), (130, 330, 1152), (300, 70, 2048)])
