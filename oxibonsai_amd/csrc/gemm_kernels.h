@@ -16,7 +16,7 @@ struct OxbGemmParams {
     const uint32_t* xh;      // packed fp16 activations (oxb_launch_xh_pack)
     const int32_t* xsh;      // [M] exponent that undoes the row scaling, INT32_MIN for a non-finite row; null: x_exp for all rows
     int32_t x_exp;
-    int32_t w_twice;         // TQ2: 1, the weights enter the products twice as large; 0 (and the kernel halves the scales) where one of these is 2^15 or more
+    int32_t loud;            // TQ2: 1 where a scale is 2^15 or more: the weights then do not enter the products twice as large
     float* y;                // [M][ldy]
     const float* residual;   // [M][ldy], mode RESIDUAL only
     uint32_t n_rows, n_tiles, n_sb;

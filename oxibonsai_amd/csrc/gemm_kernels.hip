@@ -395,6 +395,11 @@ __global__ __launch_bounds__(256) void xh_pack_kernel(const float* __restrict__ 
 // ---------------------------------------------------------------------------
 // GEMM.
 // ---------------------------------------------------------------------------
+// How a kernel expands its weights (template FMT): by the matrix's format, and one more for a ternary matrix with a scale of 2^15 or
+// more, twice which fp16 does not hold (decode_step).
+enum { GEMM_TQ2_LOUD = OXB_FMT_TQ2 + 1 };
+static_assert(OXB_FMT_Q1 == 0 && OXB_FMT_TQ2 == 1, "the forms of a matrix's weights");
+
 // Codes and scales of one row tile for half a superblock (two 128-weight blocks), as loaded: the unit of the
 // in-place register ring (half 0 is reloaded for the next superblock while half 1 is still being consumed).
 template <int FMT>
@@ -426,20 +431,21 @@ __device__ __forceinline__ void load_half(HalfRegs<FMT>& H, __amdgpu_buffer_rsrc
 // Per (row tile, block) state prepared once and used by the four MFMA steps of the block.
 struct BlockDec {
     uint32_t w0, w1;  // Q1: w0 = inverted sign bits (xor the scale's sign); TQ2: fields of the 16-weight halves as sign and magnitude bits
-    uint32_t d2;      // Q1: |d| in both halves of the dword; TQ2: d (times dmul) in both halves
+    uint32_t d2;      // Q1: |d| in both halves of the dword; TQ2: d in both halves
 };
 
 // TQ2.  A field with both bits inverted is a sign bit above a magnitude bit (-1 = 3, 0 = 2, which is minus 0, +1 = 1); those at in-byte
 // position 3 are that as they are (two's complement: 3, 0, 1).  Shifted to the top of a half and masked it is the fp16 number +-2 or
 // +-0, and one packed multiplication by d makes the weight, twice as large as it is: three instructions for two weights where
-// building 1024 + field, subtracting 1025 and multiplying takes four.  The factor goes into the row's exponent (row_exp); a
-// matrix with a scale of 2^15 or more, twice which fp16 does not hold, has its scales halved instead (dmul, one of 1 and 1/2).
+// building 1024 + field, subtracting 1025 and multiplying takes four.  The factor goes into the row's exponent (row_exp).
+// A matrix with a scale of 2^15 or more (GEMM_TQ2_LOUD) has these numbers halved first, which is exact, and the weights as they are:
+// an instruction more.  (Half the scale instead would round the ones below 2^-13.)
 // us, TQ2, four instructions / three: gate || up 19456 x 2560 at 64 / 301 / 512 / 2048 rows 17.0 / 38.3 / 52 / 191.5 and 15.2 / 35.7 / 52 /
 // 189; 2560 x 9728 at 16 / 128 / 512 rows 6.4 / 19.7 / 40.8 and 5.8 / 18.4 / 38.5; 5120 x 2560 at 23 / 301 / 512 rows 5.7 / 17.2 / 23.3
 // and 5.1 / 15.6 / 21.9; 2048 x 6144 at 2048 rows 60 and 55.
 
 template <int FMT>
-__device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e, uint32_t dmul) {
+__device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e) {
     BlockDec B;
     const uint32_t dbits = H.d[e];
     const uint32_t dd = (dbits & 0xFFFFu) * 0x00010001u;
@@ -452,7 +458,7 @@ __device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e,
     } else {
         B.w0 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e] ^ 0x3F3F3F3Fu;
         B.w1 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e + 1] ^ 0x3F3F3F3Fu;
-        B.d2 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, dd) * __builtin_bit_cast(v2h, dmul));
+        B.d2 = dd;
     }
     return B;
 }
@@ -485,6 +491,13 @@ __device__ __forceinline__ void decode_step(const BlockDec (&B)[RT], int s, v8h 
         for (int p = 0; p < 4; p++)
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) o[rt][p] &= kmask;  // fp16 2, -2, 0 or -0
+        if (FMT == GEMM_TQ2_LOUD) {
+            const v2h half = {(_Float16)0.5f, (_Float16)0.5f};
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) o[rt][p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, o[rt][p]) * half);
+        }
 #pragma unroll
         for (int p = 0; p < 4; p++)
 #pragma unroll
@@ -544,9 +557,10 @@ __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A
 }
 
 // Exponent that undoes the scaling of token row m, INT32_MIN for a row that holds something non-finite.
+template <int FMT>
 __device__ __forceinline__ int row_exp(const OxbGemmParams& p, uint32_t m) {
     const int e = p.xsh ? p.xsh[m] : p.x_exp;
-    return e == INT32_MIN ? e : e - p.w_twice;
+    return e == INT32_MIN || FMT != OXB_FMT_TQ2 ? e : e - 1;
 }
 
 // SWIGLU with the next product's operand as the output: |silu(gate) up| <= |gate up| <= w_mant 2^w_exp norm2 (Cauchy-Schwarz), so that
@@ -603,7 +617,6 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
-    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
 
     v4f acc[RT][CT];
 #pragma unroll
@@ -655,7 +668,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
     BlockDec bd[RT], bdn[RT];
     v8h A[RT];
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][0], 0, dmul);
+    for (int rt = 0; rt < RT; rt++) bd[rt] = prepare_block<FMT>(H[rt][0], 0);
     decode_step<FMT, RT>(bd, 0, A);
     const uint32_t boff = g * 4 * BM + r;  // this lane's B operand of step s, token tile ct: xs[boff + s*BM + 16 ct]
     const v8h* x0 = reinterpret_cast<const v8h*>(xs0);
@@ -665,7 +678,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
         // block 0 of the superblock
         stage_x(sb * 4 + 1, xs1);
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) bdn[rt] = prepare_block<FMT>(H[rt][0], 1, dmul);
+        for (int rt = 0; rt < RT; rt++) bdn[rt] = prepare_block<FMT>(H[rt][0], 1);
         block_steps<FMT, RT, CT>(x0, A, bd, bdn, acc, boff);
         publish();
         // block 1: half 0 is consumed; reload it for the next superblock
@@ -674,7 +687,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][1], 0, dmul);
+            bdn[rt] = prepare_block<FMT>(H[rt][1], 0);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][0], rc, rs, tile_at(rt), (uint32_t)rt < n_valid, p.n_sb, sb + 1, 0, lane);
@@ -686,7 +699,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][1], 1, dmul);
+            bdn[rt] = prepare_block<FMT>(H[rt][1], 1);
         }
         block_steps<FMT, RT, CT>(x0, A, bd, bdn, acc, boff);
         publish();
@@ -696,7 +709,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             bd[rt] = bdn[rt];
-            bdn[rt] = prepare_block<FMT>(H[rt][0], 0, dmul);
+            bdn[rt] = prepare_block<FMT>(H[rt][0], 0);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) load_half<FMT>(H[rt][1], rc, rs, tile_at(rt), (uint32_t)rt < n_valid, p.n_sb, sb + 1, 1, lane);
@@ -728,7 +741,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
                     const int ct = ps * CH + ci;
                     if (ct >= CT) continue;
                     const uint32_t m = m0 + ct * 16 + r;
-                    const int e = m < p.M ? row_exp(p, m) : 0;
+                    const int e = m < p.M ? row_exp<FMT>(p, m) : 0;
 #pragma unroll
                     for (int rt = 0; rt < RT; rt++) {
                         float o[4];
@@ -749,7 +762,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
                     };
                     if (p.xh_out) {
                         if (g_first + 2 * pr >= half_tiles) continue;  // (whole blocks of 128 rows: pairs are complete)
-                        const OxbOperandOut out = {(_Float16*)p.xh_out, FMT, p.M_pad, swiglu_shift(p, m)};
+                        const OxbOperandOut out = {(_Float16*)p.xh_out, FMT == OXB_FMT_Q1 ? OXB_FMT_Q1 : OXB_FMT_TQ2, p.M_pad, swiglu_shift(p, m)};
                         // lane 16 s + r writes piece s of the 32 rows
                         const uint32_t k0 = (g_first + 2 * pr) * 16;
                         if constexpr (FMT == OXB_FMT_Q1) operand_store8(out, k0 + 4 * g, m, four(0, lane), four(1, lane));
@@ -775,7 +788,7 @@ __global__ __launch_bounds__(OXB_GEMM_THREADS, RT == 3 ? 2 : 1) void gemm_mfma_k
     for (int ct = 0; ct < CT; ct++) {
         const uint32_t m = m0 + ct * 16 + r;
         if (m >= p.M) continue;
-        const int e = row_exp(p, m);
+        const int e = row_exp<FMT>(p, m);
         // with K split over workgroups, slice ks writes its partial sums to plane ks of the workspace
         float* yr = p.ksplit > 1 ? p.part + ((size_t)ks * p.M + m) * p.ldy : p.y + (size_t)m * p.ldy;
         const float* rr = (p.mode == OXB_GEMM_RESIDUAL && p.ksplit == 1) ? p.residual + (size_t)m * p.ldy : nullptr;
@@ -840,7 +853,6 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
     const uint32_t per = (s1 - s0 + 7u) / 8u, h0 = s0 + wave * per, h1 = min(h0 + per, s1);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
-    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
 
     v4f acc[RT][CT];
 #pragma unroll
@@ -888,7 +900,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
                 for (int bi = 0; bi < 2; bi++)
 #pragma unroll
-                    for (int rt = 0; rt < RT; rt++) bd[EARLY ? bi : 0][rt] = prepare_block<FMT>(H[rt][hh], bi, dmul);
+                    for (int rt = 0; rt < RT; rt++) bd[EARLY ? bi : 0][rt] = prepare_block<FMT>(H[rt][hh], bi);
                 if (REFILL) refill();
             }
 #pragma unroll
@@ -899,7 +911,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
                 }
                 if (!EARLY) {
 #pragma unroll
-                    for (int rt = 0; rt < RT; rt++) bd[0][rt] = prepare_block<FMT>(H[rt][hh], bi, dmul);
+                    for (int rt = 0; rt < RT; rt++) bd[0][rt] = prepare_block<FMT>(H[rt][hh], bi);
                     if (REFILL && bi) refill();
                 }
 #pragma unroll
@@ -965,7 +977,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
         const uint32_t q = idx / CT, ct = idx % CT, m = ct * 16 + r;
         const uint32_t rt = (uint32_t)pass_rt(ps, (int)q);
         if (!valid((int)rt) || m >= p.M) continue;
-        const int e = row_exp(p, m);
+        const int e = row_exp<FMT>(p, m);
         float o[4];
         total(idx, o, e);
         if (sw) {  // y[m][row] = silu(gate) * up, rows counted within the gate half
@@ -974,7 +986,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
 #pragma unroll
             for (int v = 0; v < 4; v++) o[v] = silu_mul(o[v], u[v]);
             if (p.xh_out) {
-                operand_store4({(_Float16*)p.xh_out, FMT, p.M_pad, swiglu_shift(p, m)}, (t0 + rt) * 16 + 4 * g, m, o[0], o[1], o[2], o[3]);
+                operand_store4({(_Float16*)p.xh_out, FMT == OXB_FMT_Q1 ? OXB_FMT_Q1 : OXB_FMT_TQ2, p.M_pad, swiglu_shift(p, m)}, (t0 + rt) * 16 + 4 * g, m, o[0], o[1], o[2], o[3]);
                 continue;
             }
         }
@@ -1017,7 +1029,6 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_tall_kernel(cons
     const uint32_t t_begin = blockIdx.x * p.tpw, t_end = min(t_begin + p.tpw, p.n_tiles);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.codes, p.codes_bytes), rs = make_rsrc(p.scales, p.scales_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xh, p.xh_bytes);
-    const uint32_t dmul = p.w_twice ? 0x3C003C00u : 0x38003800u;
     const __amdgpu_buffer_rsrc_t ry = make_rsrc(p.y, ((p.M - 1) * p.ldy + p.n_rows) * 4u);
     const uint32_t b_off = (4u * g * p.M_pad + r) * 16u, blk_stride = 16u * p.M_pad * 16u;
     v8h B[4][4][CT];  // [block][step][token tile]
@@ -1039,7 +1050,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_tall_kernel(cons
 #pragma unroll
     for (int i = 0; i < CT; i++) {
         const uint32_t m = (tid + i * threads) / 16u;
-        e[i] = m < p.M ? row_exp(p, m) : 0;
+        e[i] = m < p.M ? row_exp<FMT>(p, m) : 0;
     }
     for (uint32_t t0 = t_begin, pair = 0; t0 < t_end; t0 += RING) {
 #pragma unroll
@@ -1052,7 +1063,7 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_tall_kernel(cons
 #pragma unroll
                 for (int ct = 0; ct < CT; ct++) acc[j][ct] = (v4f){0.f, 0.f, 0.f, 0.f};
             // a step's weights are expanded while the products of the one before run: one product, then its share of the expansion
-            BlockDec bd[2] = {prepare_block<FMT>(H[i][0], 0, dmul), prepare_block<FMT>(H[i + 1][0], 0, dmul)};
+            BlockDec bd[2] = {prepare_block<FMT>(H[i][0], 0), prepare_block<FMT>(H[i + 1][0], 0)};
             v8h A[2];
             decode_step<FMT, 2>(bd, 0, A);
             __builtin_amdgcn_sched_barrier(0);
@@ -1061,8 +1072,8 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_tall_kernel(cons
                 const int b = st >> 2, s = st & 3;
                 v8h An[2];
                 if (s == 3 && b < 3) {
-                    bd[0] = prepare_block<FMT>(H[i][(b + 1) >> 1], (b + 1) & 1, dmul);
-                    bd[1] = prepare_block<FMT>(H[i + 1][(b + 1) >> 1], (b + 1) & 1, dmul);
+                    bd[0] = prepare_block<FMT>(H[i][(b + 1) >> 1], (b + 1) & 1);
+                    bd[1] = prepare_block<FMT>(H[i + 1][(b + 1) >> 1], (b + 1) & 1);
                 }
                 if (st < 15) decode_step<FMT, 2>(bd, (s + 1) & 3, An);
 #pragma unroll
@@ -1376,12 +1387,13 @@ static hipError_t launch_narrow_case(const OxbGemmParams& p, hipStream_t st) {
     return hipGetLastError();
 }
 
+// (fmt: OXB_FMT_* or GEMM_TQ2_LOUD)
 static hipError_t launch_gemm_narrow(int fmt, OxbGemmParams p, uint32_t rt, hipStream_t st) {
     p.n_ng = p.mode == OXB_GEMM_SWIGLU ? (p.n_tiles / 2 + rt / 2 - 1) / (rt > 1 ? rt / 2 : 1) : (p.n_tiles + rt - 1) / rt;
     const uint32_t ct = p.M_pad / 16;
 #define OXB_NARROW_CASE(F, R, C) \
     if (fmt == F && rt == R && ct == C) return launch_narrow_case<F, R, C>(p, st);
-#define OXB_NARROW_CASES(R, C) OXB_NARROW_CASE(OXB_FMT_Q1, R, C) OXB_NARROW_CASE(OXB_FMT_TQ2, R, C)
+#define OXB_NARROW_CASES(R, C) OXB_NARROW_CASE(OXB_FMT_Q1, R, C) OXB_NARROW_CASE(OXB_FMT_TQ2, R, C) OXB_NARROW_CASE(GEMM_TQ2_LOUD, R, C)
     OXB_NARROW_CASES(1, 1) OXB_NARROW_CASES(2, 1) OXB_NARROW_CASES(4, 1) OXB_NARROW_CASE(OXB_FMT_Q1, 6, 1)
     OXB_NARROW_CASES(1, 2) OXB_NARROW_CASES(2, 2) OXB_NARROW_CASES(4, 2) OXB_NARROW_CASE(OXB_FMT_Q1, 6, 2)
     OXB_NARROW_CASES(1, 3) OXB_NARROW_CASES(2, 3) OXB_NARROW_CASES(4, 3)
@@ -1411,11 +1423,13 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     p.ksplit = plan.ksplit;
     p.sb_per_split = plan.sb_per_split;
     if (p.ksplit > 1 && !p.part) return hipErrorInvalidValue;
+    if (p.loud && fmt == OXB_FMT_TQ2) fmt = GEMM_TQ2_LOUD;
     if (plan.narrow && plan.rt == 0) {
         p.tpw = plan.tpw;
         const dim3 grid((p.n_tiles + p.tpw - 1) / p.tpw), block(64 * p.n_sb);
         if (fmt == OXB_FMT_Q1) hipLaunchKernelGGL(gemm_tall_kernel<OXB_FMT_Q1>, grid, block, 0, st, p);
-        else hipLaunchKernelGGL(gemm_tall_kernel<OXB_FMT_TQ2>, grid, block, 0, st, p);
+        else if (fmt == OXB_FMT_TQ2) hipLaunchKernelGGL(gemm_tall_kernel<OXB_FMT_TQ2>, grid, block, 0, st, p);
+        else hipLaunchKernelGGL(gemm_tall_kernel<GEMM_TQ2_LOUD>, grid, block, 0, st, p);
         return hipGetLastError();
     }
     if (plan.narrow) return launch_gemm_narrow(fmt, p, plan.rt, st);
@@ -1426,7 +1440,7 @@ hipError_t oxb_launch_gemm(int fmt, OxbGemmParams p, uint32_t n_cus, hipStream_t
     hipError_t err = hipErrorInvalidValue;
 #define OXB_GEMM_CASE(R, C)                                                                        \
     if (plan.rt == R && plan.ct == C)                                                              \
-        err = fmt == OXB_FMT_Q1 ? launch_gemm_case<OXB_FMT_Q1, R, C>(p, grid, st) : launch_gemm_case<OXB_FMT_TQ2, R, C>(p, grid, st);
+        err = fmt == OXB_FMT_Q1 ? launch_gemm_case<OXB_FMT_Q1, R, C>(p, grid, st) : fmt == OXB_FMT_TQ2 ? launch_gemm_case<OXB_FMT_TQ2, R, C>(p, grid, st) : launch_gemm_case<GEMM_TQ2_LOUD, R, C>(p, grid, st);
     OXB_GEMM_CASE(2, 8) OXB_GEMM_CASE(3, 8) OXB_GEMM_CASE(4, 8) OXB_GEMM_CASE(5, 8)
     OXB_GEMM_CASE(1, 5) OXB_GEMM_CASE(2, 5) OXB_GEMM_CASE(3, 5) OXB_GEMM_CASE(4, 5)
     OXB_GEMM_CASE(1, 4) OXB_GEMM_CASE(2, 4) OXB_GEMM_CASE(3, 4) OXB_GEMM_CASE(4, 4)

@@ -295,7 +295,7 @@ static OxbGemmParams gemm_params(const Weight& w, float* d_y, uint32_t m, uint32
     memset(&p, 0, sizeof p);
     p.codes = w.d_codes;
     p.scales = w.d_scales;
-    p.w_twice = w.L.fmt == OXB_FMT_TQ2 && !w.loud;
+    p.loud = w.loud;
     p.y = d_y;
     p.n_rows = w.L.n_rows;
     p.n_tiles = w.L.n_tiles;

@@ -301,6 +301,31 @@ def test_gemm_ternary_scales_on_both_sides_of_a_doubled_weight(backend, m, n, k,
     _check_against_truth(got, dense_f64(TQ2, a, n, k), x)
 
 
+# by what the launcher runs: the narrow kernel with one row tile to a workgroup and with two, the wide one (130 and 300 rows: K whole and
+# in slices), and the one for very many matrix rows
+@pytest.mark.parametrize("m,n,k", [(1, 16, 128), (23, 40, 640), (17, 4163, 640), (130, 330, 1152), (300, 70, 2048), (18, 65530, 1664)])
+@pytest.mark.parametrize("loudest", [32752.0, 32768.0, 65504.0])
+def test_gemm_ternary_small_scales_beside_a_loud_one(backend, m, n, k, loudest):
+    # one loud block says nothing about the others: rows of nothing but subnormal scales, halves of which fp16 does not hold, keep the
+    # element's own bound (2^-11 of sum |w x|), and so do rows that have the loud block and meet zeros in it
+    rng = np.random.default_rng(int(loudest) + m + n)
+    bpr, tiny = k // 128, np.array([1, 3, 0x3FF, 0x401]) * 2.0**-24
+    rows = np.arange(n) if n < 5000 else np.unique(np.concatenate([np.arange(60), np.arange(0, n, 997), np.arange(n - 60, n)]))
+    d = rng.choice(tiny, (n, bpr)).astype(np.float16)
+    d[::3] = rng.choice([0.004, 0.7, 300.0, -2.5], (len(d[::3]), bpr))
+    d[:, 0] = tiny[rng.integers(0, 4, n)]
+    loud = rng.choice(rows, 2)
+    d[loud, -1] = (-loudest, 1.5)
+    a = np.empty((n, bpr, 34), dtype=np.uint8)
+    a[:, :, :32] = rng.integers(0, 256, (n, bpr, 32), dtype=np.uint8)
+    a[:, :, 32:] = d.view(np.uint8).reshape(n, bpr, 2)
+    x = synth.normal_f32(16, m * k).reshape(m, k).copy()
+    if bpr > 1:
+        x[::2, -128:] = 0.0
+    got = _gemm(backend, TQ2, a.reshape(-1), x, m, n, k)
+    _check_against_truth(got[:, rows], dense_f64(TQ2, np.ascontiguousarray(a[rows]).reshape(-1), rows.size, k), x)
+
+
 @pytest.mark.parametrize("fmt", [Q1, TQ2])
 @pytest.mark.parametrize("m,n,k", [(17, 65521, 1664), (32, 65536, 2048), (25, 65537, 2304), (31, 67777, 4096), (32, 70000, 3584), (20, 98304, 2560)])
 def test_gemm_few_rows_of_a_matrix_with_many(backend, fmt, m, n, k):

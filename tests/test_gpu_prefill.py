@@ -118,6 +118,28 @@ def test_prefill_rows_match_the_oracle(backend, fmt, h, inter, nq, nkv, hd, n, f
         gpu.close()
 
 
+@pytest.mark.parametrize("cfg,n", [(SMALL, 23), (SMALL, 130), (LONG_FFN, 500)])
+def test_prefill_of_ternary_ffn_scales_above_and_below_a_doubled_weight(backend, cfg, n):
+    # gate and up with scales up to 2^15 .. 2^16, which do not enter the products twice as large, and with half of each, which do; the
+    # norm weights in front of them take the factor off again.  Powers of two all along: the same bits.
+    cfg, logits = dict(cfg, fmt=TQ2), []
+    rows = _rows(9, n, cfg["h"])
+    for top in (14, 15):
+        w = synth.make_model(cfg, 77)
+        for ly in w["layers"]:
+            d = [ly[name].reshape(-1, 34)[:, 32:].copy().view(np.float16) for name in ("gate", "up")]
+            up = top - int(np.floor(np.log2(max(np.abs(v).max() for v in d).astype(np.float64))))
+            for name, v in zip(("gate", "up"), d):
+                ly[name].reshape(-1, 34)[:, 32:] = np.ldexp(v.astype(np.float32), up).astype(np.float16).view(np.uint8)
+            ly["ffn_norm"] = np.ldexp(ly["ffn_norm"], -up).astype(np.float32)
+        gpu = HipModel(backend, cfg, w, batch=1)
+        try:
+            logits.append(gpu.prefill(rows)[0].copy())
+        finally:
+            gpu.close()
+    assert np.all(np.isfinite(logits[0])) and np.array_equal(*logits)
+
+
 def test_chunked_prefill_equals_one_prefill(backend):
     # the reference's chunked 4 + 4 = 8 test (metal_prefill_ternary_parity_tests.rs:427-473), at tile-crossing sizes
     cfg = dict(SMALL, fmt=TQ2)
