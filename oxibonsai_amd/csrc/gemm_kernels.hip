@@ -440,9 +440,11 @@ struct BlockDec {
 // building 1024 + field, subtracting 1025 and multiplying takes four.  The factor goes into the row's exponent (row_exp).
 // A matrix with a scale of 2^15 or more (GEMM_TQ2_LOUD) has these numbers halved first, which is exact, and the weights as they are:
 // an instruction more.  (Half the scale instead would round the ones below 2^-13.)
-// us, TQ2, four instructions / three: gate || up 19456 x 2560 at 64 / 301 / 512 / 2048 rows 17.0 / 38.3 / 52 / 191.5 and 15.2 / 35.7 / 52 /
-// 189; 2560 x 9728 at 16 / 128 / 512 rows 6.4 / 19.7 / 40.8 and 5.8 / 18.4 / 38.5; 5120 x 2560 at 23 / 301 / 512 rows 5.7 / 17.2 / 23.3
-// and 5.1 / 15.6 / 21.9; 2048 x 6144 at 2048 rows 60 and 55.
+// us, TQ2, four instructions / three: 19456 x 2560 at 64 / 301 / 512 / 2048 rows 16.8 / 37.5 / 51.3 / 190 and 14.8 / 35.2 / 50.8 / 186, the
+// same as gate || up with SwiGLU 20.2 / 42.6 / 61.0 / 198 and 18.3 / 39.0 / 57.7 / 188; 12288 x 2048 with SwiGLU at 200 / 512 / 2048 24.2 /
+// 34.5 / 100.5 and 22.1 / 32.9 / 95.8; 2560 x 9728 at 16 / 128 / 512 6.3 / 18.9 / 40.6 and 5.85 / 17.6 / 38.1; 5120 x 2560 at 23 / 301 / 512
+// 5.7 / 16.6 / 23.2 and 5.15 / 14.9 / 21.5.  Equal up to 2 % slower with two row tiles and seven token tiles (97 to 112 rows of 6144 x
+// 4096 12.1 and 12.3, of 12288 x 2048 13.9 and 14.3).
 
 template <int FMT>
 __device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e) {
@@ -458,6 +460,10 @@ __device__ __forceinline__ BlockDec prepare_block(const HalfRegs<FMT>& H, int e)
     } else {
         B.w0 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e] ^ 0x3F3F3F3Fu;
         B.w1 = H.c[FMT == OXB_FMT_Q1 ? 0 : 2 * e + 1] ^ 0x3F3F3F3Fu;
+        // (Opaque, or the inversion moves into the masks that take it and the loaded codes live on: up to 30 registers more, with which
+        // three of the wide kernel's forms and <2, 7> of the narrow one spill or lose a workgroup a CU: 6144 x 4096 at 97 rows 15.0 us
+        // against 12.3, 24576 x 4096 at 400 84.7 against 71.7, gate || up 12288 x 2048 at 700 47.3 against 44.2.)
+        asm("" : "+v"(B.w0), "+v"(B.w1));
         B.d2 = dd;
     }
     return B;
@@ -873,8 +879,9 @@ __global__ __launch_bounds__(OXB_GEMM_NARROW_THREADS) void gemm_narrow_kernel(co
             for (int ct = 0; ct < CT; ct++) dst[ct] = __builtin_bit_cast(v8h, buf_load_b128(rx, at + ct * 256u, blk * blk_stride + s * p.M_pad * 16u));
         };
         // Two halves of weights in registers: a half is requested again, for the one after next, as soon as both its blocks
-        // have been prepared (with many row tiles only once the second one has: there is no room for two prepared blocks).
-        constexpr bool EARLY = RT <= 4 && RT * CT <= 12;
+        // have been prepared (with many row tiles only once the second one has: there is no room for two prepared blocks; nor with
+        // seven token tiles of a ternary matrix, 4096 x 4096 at 97 rows 11.9 against 11.5 us, while with eight the two are equal).
+        constexpr bool EARLY = RT <= 4 && RT * CT <= 12 && (FMT == OXB_FMT_Q1 || CT != 7);
         HalfRegs<FMT> H[RT][2];
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)

@@ -48,6 +48,43 @@ def test_gemm_forms_cover_what_the_launcher_picks():
         assert _lib.lib().oxb_hip_gemm_plan(*bad, 0, 0, 256, plan) == 5
 
 
+def _device_kernels():
+    """Name -> metadata (the compiler's notes) of every kernel of the built library."""
+    import msgpack
+    data, out, at = open(_lib.LIB_PATH, "rb").read(), {}, 0
+    while (at := data.find(b"\x7fELF", at + 1)) >= 0:
+        elf = data[at:]
+        if int.from_bytes(elf[18:20], "little") != 224:                       # EM_AMDGPU
+            continue
+        sh, size, n = int.from_bytes(elf[40:48], "little"), int.from_bytes(elf[58:60], "little"), int.from_bytes(elf[60:62], "little")
+        for i in range(n):
+            head = elf[sh + i * size:sh + (i + 1) * size]
+            if int.from_bytes(head[4:8], "little") != 7:                      # SHT_NOTE
+                continue
+            off, end = int.from_bytes(head[24:32], "little"), int.from_bytes(head[24:32], "little") + int.from_bytes(head[32:40], "little")
+            while off < end:
+                nn, nd, kind = (int.from_bytes(elf[off + 4 * j:off + 4 * j + 4], "little") for j in range(3))
+                desc = off + 12 + (nn + 3) // 4 * 4
+                if kind == 32:                                                # NT_AMDGPU_METADATA
+                    out.update((k[".name"], k) for k in msgpack.unpackb(elf[desc:desc + nd])["amdhsa.kernels"])
+                off = desc + (nd + 3) // 4 * 4
+    return out
+
+
+def test_gemm_kernels_keep_their_registers():
+    # what the launcher's costs take for granted: no form spills, and a ternary form leaves room for as many waves a SIMD as the one-bit
+    # form, with which it shares the table of resident workgroups (512 registers a SIMD and lane, given out in eights)
+    kernels, forms = _device_kernels(), {}
+    for name, k in kernels.items():
+        if m := re.match(r"_Z\d+gemm_(mfma|narrow|tall)_kernelILi([01])E(?:Li(\d)ELi(\d)E)?", name):
+            assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0, name
+            forms[m.groups()] = 512 // ((k[".vgpr_count"] + 7) // 8 * 8)
+    wide = [f for f in forms if f[0] == "mfma"]
+    assert len(wide) == 24 and len(forms) == 24 + 42
+    for kind, fmt, rt, ct in wide:
+        assert forms[kind, "1", rt, ct] >= forms[kind, "0", rt, ct], (rt, ct)
+
+
 def test_static_library_is_built():
     assert os.path.exists(os.path.join(os.path.dirname(_lib.LIB_PATH), "liboxb_hip.a"))
 
