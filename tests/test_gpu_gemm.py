@@ -327,7 +327,28 @@ def test_gemm_ternary_small_scales_beside_a_loud_one(backend, m, n, k, loudest):
 
 
 @pytest.mark.parametrize("fmt", [Q1, TQ2])
-@pytest.mark.parametrize("m,n,k", [(17, 65521, 1664), (32, 65536, 2048), (25, 65537, 2304), (31, 67777, 4096), (32, 70000, 3584), (20, 98304, 2560)])
+@pytest.mark.parametrize("n,k", [(65530, 1664), (66000, 3072)])
+def test_gemm_non_finite_rows_before_a_matrix_with_many(backend, fmt, n, k):
+    # as above on the kernel that walks its share of a matrix with very many rows: token rows of both tiles, the first and the last
+    m = 27
+    assert gemm_plan(fmt, m, n, k)[:2] == (1, 0)
+    a = synth.make_blocks(fmt, 53, n, k)
+    x = synth.normal_f32(54, m * k).reshape(m, k).copy()
+    h = _upload(backend, fmt, a, n, k)
+    try:
+        clean = backend.gemm_cached(h, x, m, n, k)
+        bad = [0, 15, 16, 26]
+        x[bad, [7, k - 1, 0, 130]] = (np.nan, np.inf, -np.inf, np.nan)
+        got = backend.gemm_cached(h, x, m, n, k)
+    finally:
+        backend.free_weights(h)
+    assert np.all(np.isnan(got[bad]))
+    keep = np.setdiff1d(np.arange(m), bad)
+    assert np.all(np.isfinite(clean)) and np.array_equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("fmt", [Q1, TQ2])
+@pytest.mark.parametrize("m,n,k", [(17, 65521, 1664), (32, 65536, 2048), (25, 65537, 2304), (31, 67777, 4096), (32, 70000, 3584), (20, 98304, 2560), (19, 66000, 3072), (32, 65601, 2688)])
 def test_gemm_few_rows_of_a_matrix_with_many(backend, fmt, m, n, k):
     # an LM head's shape: a workgroup walks its share of the row tiles (16 and more: even and odd shares, one that ends early, a last tile
     # in part), four to eight waves; the last share and the rows on both sides of a share's end, and some in between

@@ -432,7 +432,8 @@ def test_few_slots_are_added_up_by_the_o_projection(backend, fmt, mode, hd, wind
     """One sequence's slots are merged by the O projection while there are two to eight, by the attention otherwise; with two sequences
     always by the attention.  Positions on both sides of every line: two and three chunks, eight and nine, of 128 and (one-byte rows and a long
     context) 256 positions.  The routes differ in the order of a few fp32 sums and in how the activations are cut into digits (2^-26 of
-    the largest and less), 1e-6 each; a slot left out or counted twice moves the sums by an eighth or more."""
+    the largest and less), 1e-6 each; the smallest slot, one key of 257 or 513, moves the logits by 0.8e-3 and more (shown by
+    test_one_key_in_hundreds_shows_in_the_logits)."""
     cfg = dict(fmt=fmt, n_layers=2, h=256, inter=256, nq=640 // hd // 2 * 2, nkv=2 if hd < 256 else 1, hd=hd, vocab=320, max_seq=2400 if mode != KV_I8 else 40000, eps=1e-6, rope_theta=1e6)
     w = synth.make_model(cfg, 13)
     edges = [200, 255, 256, 300, 511, 512, 900, 1023, 1024, 1151, 1152, 2047, 2048, 2303]

@@ -244,3 +244,22 @@ def test_model_with_sliding_window_matches_float64_numpy(window, sinks):
         assert np.max(np.abs(got - want[pos])) < 2e-4 * max(1.0, np.max(np.abs(want[pos]))), pos
     moved = max(float(np.max(np.abs(a - b))) for a, b in zip(plain, want))
     assert (moved == 0.0) if window >= len(hiddens) else (moved > 1e-3)
+
+
+@pytest.mark.parametrize("fmt,hd,last", [(0, 128, 512), (0, 64, 256), (1, 128, 256), (1, 32, 256)])
+def test_one_key_in_hundreds_shows_in_the_logits(fmt, hd, last):
+    """What the tolerance of test_few_slots_are_added_up_by_the_o_projection (2e-5 of the largest logit) can tell apart: the smallest slot there
+    holds the new position alone, one key of 257 or of 513, and without its V row the logits of the same models move by ten tolerances
+    and more (0.8e-3 to 15e-3)."""
+    from oxibonsai_amd import synth
+    cfg = dict(fmt=fmt, n_layers=2, h=256, inter=256, nq=640 // hd // 2 * 2, nkv=2, hd=hd, vocab=320, max_seq=520, eps=1e-6, rope_theta=1e6)
+    rows = synth.embedding_rows(6, [(7 * i + 3) % 211 for i in range(last + 1)], 256) * 50.0
+    m = oracle.OracleModel(cfg, synth.make_model(cfg, 13), kv_f16=True)
+    m.forward_batch(rows[:last], 0, want_logits=False)
+    want = m.forward(rows[last], last)
+    for layer in range(2):
+        for head in range(2):
+            k, v = m.cache_rows(layer, head, last, 1)
+            m.load_rows(layer, head, last, k, np.zeros_like(v))
+    m.freeze()
+    assert np.abs(m.forward(rows[last], last) - want).max() > 10 * 2e-5 * np.abs(want).max()
