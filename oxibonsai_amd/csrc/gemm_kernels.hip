@@ -525,7 +525,7 @@ template <int FMT, int RT, int CT>
 __device__ __forceinline__ void block_steps(const v8h* __restrict__ xsb, v8h (&A)[RT], const BlockDec (&bd)[RT],
                                             const BlockDec (&bdn)[RT], v4f (&acc)[RT][CT], uint32_t boff) {
     constexpr int BM = 16 * CT;
-    constexpr int NV = FMT == OXB_FMT_Q1 ? 1 : 2;  // VALU instructions issued after each MFMA
+    constexpr int NV = FMT == OXB_FMT_Q1 ? 1 : 2;  // VALU instructions issued after each MFMA, while there are any (a step has 8 or 12 a row tile)
     v8h B[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) B[ct] = xsb[boff + ct * 16];
@@ -1300,7 +1300,8 @@ static hipError_t launch_gemm_case(const OxbGemmParams& p, uint32_t grid, hipStr
 // 12288, 33 .. 2048 tokens - whose best plan it names within 2 % on average (the rule before it, 128-token tiles by rounds
 // of workgroups: 12 %).  Per 128-weight block a workgroup alone on its CU needs `lone`, a latency; workgroups that share
 // one need `busy` each, a rate.  More tokens per tile amortise the expansion of the weights, more row tiles the reading of
-// the token tile out of LDS; small tiles make more workgroups and less padding.
+// the token tile out of LDS; small tiles make more workgroups and less padding.  (The ternary times here and in narrow_cost are those of
+// four instructions for two weights; with three (BlockDec) a plan takes up to 10 % less, 4 % on average, and the choice was not fitted again.)
 static float wide_cost(bool tq2, const OxbGemmParams& p, const OxbGemmPlan& g, uint32_t n_cus) {
     // [format][ct = 4, 5, 8][rt - 1]; rt = 5 goes with ct = 8 only, rt = 1 not with it (smaller token tiles always beat it)
     static const float lone_us[2][3][5] = {{{0.34f, 0.50f, 0.68f, 0.82f}, {0.40f, 0.59f, 0.81f, 0.96f}, {0.66f, 0.86f, 1.18f, 1.42f, 1.69f}},

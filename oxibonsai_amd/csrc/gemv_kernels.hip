@@ -681,15 +681,6 @@ __device__ __forceinline__ v4f mfma_f4_double_b(const v4i a, const v4i b, const 
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a8, b8, c, 4, 4, 0, 0x7F7F7F7F, 0, 0x80808080);
 }
 
-// TQ2 weights on the same route.  A stored field is value + 1 (0, 1, 2) and reads (value + 1) / 2 as an E2M1 nibble:
-// the even fields of a code dword are in place after one AND with 0x33333333, the odd ones after a shift by two - and
-// an add of 0x10101010 before the AND, which turns the two's-complement fields at in-byte position 3 into value + 1 like
-// the others (the carry runs into bits that the AND drops).  The two dwords of a lane's 32 weights give the four operand
-// registers: register j, nibble n is weight 2 n + (j & 1) + 16 (j >> 1) of the group, and the prologue's lane m = j
-// quantises exactly those eight activations.  At a block scale of 2 the MFMA sums (value + 1) * digit / 2; the start
-// value - the same digits against a constant -1 - takes the digit sums off again.  No shifts by bit position and no
-// sign turns: every weight reads the same.  A block costs 8 + 4 vector instructions and one MFMA (the int8 route: 15
-// and two).
 // The O projection behind the decode attention of one sequence.  While its slots are few they are added up here, by the
 // waves that quantise the sums, instead of by the last workgroup of each kv head to arrive, whose wait for the stores, count,
 // loads and weights are a chain of four trips to memory.  How many there are hangs on the position, which is requested with
@@ -744,6 +735,15 @@ __device__ __forceinline__ void merge_slots(const OxbGemvParams& p, uint32_t pos
     }
 }
 
+// TQ2 weights on the same route.  A stored field is value + 1 (0, 1, 2) and reads (value + 1) / 2 as an E2M1 nibble:
+// the even fields of a code dword are in place after one AND with 0x33333333, the odd ones after a shift by two - and
+// an add of 0x10101010 before the AND, which turns the two's-complement fields at in-byte position 3 into value + 1 like
+// the others (the carry runs into bits that the AND drops).  The two dwords of a lane's 32 weights give the four operand
+// registers: register j, nibble n is weight 2 n + (j & 1) + 16 (j >> 1) of the group, and the prologue's lane m = j
+// quantises exactly those eight activations.  At a block scale of 2 the MFMA sums (value + 1) * digit / 2; the start
+// value - the same digits against a constant -1 - takes the digit sums off again.  No shifts by bit position and no
+// sign turns: every weight reads the same.  A block costs 8 + 4 vector instructions and one MFMA (the int8 route: 15
+// and two).
 template <int FMT, int NSBW, int TG, int PRO>
 __global__ __launch_bounds__(512) void gemv_f4_kernel(const OxbGemvParams p) {
     extern __shared__ uint32_t smem[];

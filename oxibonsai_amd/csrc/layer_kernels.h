@@ -35,7 +35,7 @@ struct OxbAttnParams {
     OxbKvLayout kv;                      // contiguous (row_stride a multiple of 128, >= max_seq) or paged (pages of 16..128 positions)
     uint32_t window, sinks;              // sliding window with attention sinks; window 0 = off
     float* part;                         // [batch][nq][n_splits][hd + OXB_ATTN_PART_PAD]: un-normalised output, maximum, sum
-    float* out;                          // [batch][nq*hd], written by the last workgroup of each (sequence, kv head) to finish
+    float* out;                          // [batch][nq*hd], written by the last workgroup of each (sequence, kv head) to finish (but see leave)
     uint32_t* done;                      // n_splits > 1: [batch][nkv] arrival counters, zero before the launch; the kernel leaves them zero
     const uint32_t* pos;                 // [batch], device; seq_len = pos + 1
     uint32_t nq, nkv, hd, max_seq, n_layers, layer, n_splits;
@@ -62,7 +62,9 @@ hipError_t oxb_launch_kv_norm_rope_store(const OxbKvStoreParams& p, hipStream_t 
 #define OXB_ATTN_CHUNK_POSITIONS 128  // KV positions a four-wave attention workgroup covers at a time
 #define OXB_ATTN_MAX_SPLITS 64        // slots the KV sequence is split over; slot s walks chunks s, s + n_splits, ...
 // QK-norm, RoPE, KV store of the new position, split-KV attention (at most 16 q heads per kv head) into p.part and
-// the merge of the slots into the fp32 attention output p.out [batch][nq * hd], all in one launch.
+// the merge of the slots into the fp32 attention output p.out [batch][nq * hd], all in one launch.  Where two to p.leave slots are in
+// use (p.leave 0: never) p.part is the output and p.out keeps what an earlier launch left there: both are read through OxbAttnSlots
+// (oxb_launch_gemv with OXB_GEMV_PRO_SLOTS) then.
 hipError_t oxb_launch_attn_decode(const OxbAttnParams& p, uint32_t batch, hipStream_t st);
 // out[v] = w * x[v] / sqrt(mean(x[v]^2) + eps) for nvec vectors of n values; d_w == nullptr copies.
 hipError_t oxb_launch_rmsnorm(const float* d_x, const float* d_w, uint32_t n, uint32_t nvec, float eps, float* d_out, hipStream_t st);

@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_fused_kernel(OxbAttnParam
     };
 
     // The rows of the first chunk are requested before anything else, so that their way from HBM overlaps the Q prologue.
-    // The new position's row is not in the cache then (and rows past the end repeat it): in the chunk that holds it, it is
+    // The new position's row is not in the cache then (rows past the end read as zeros): in the chunk that holds it, it is
     // patched in from LDS, with the very values the cache receives, so no workgroup waits for its own stores.
     const uint32_t pos_walk = n_walk - 1;
     uint32_t na = 0, nb = 0;  // pages of the chunk whose rows are requested next

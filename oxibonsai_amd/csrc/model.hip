@@ -474,10 +474,9 @@ static int kv_sync_table(Model& m) {
 // KV positions that a workgroup of the decode attention walks at a time.
 static uint32_t attn_chunk(const Model& m) { return OXB_ATTN_CHUNK_POSITIONS * (m.attn_wide ? 2u : 1u); }
 
-// QK-norm + RoPE + KV store + split-KV attention of one layer for the whole decode batch, one launch; leaves the
-// slot results in m.attn_part and the parameters the merge needs in *ap.
-// One launch: QK-norm, RoPE, the store of the new rows, attention over the cache and the merge of the KV slots into
-// m.attn_out (with a single slot per sequence the kernel writes its output directly).
+// One launch: QK-norm, RoPE, the store of the new rows, attention over the cache of one layer for the whole decode batch and the merge
+// of the KV slots into m.attn_out (with a single slot per sequence the kernel writes its output directly).  With `leave`, two to so
+// many slots stay in m.attn_part, m.attn_out is stale, and only a product that takes both through OxbAttnSlots may follow.
 static int encode_decode_attention(Model& m, uint32_t L, const float* q_norm, const float* k_norm, const Weight* pack_for = nullptr,
                                    const OxbOperandOut* op = nullptr, uint32_t leave = 0) {
     const oxb_model_desc& d = m.d;
